@@ -81,6 +81,7 @@ void Workspace::release() {
   hot.release();
   wave_cost.release();
   wave_order.release();
+  cull_list.release();
   find_stash.release();
   find_cnt.release();
   find_over.release();
@@ -875,6 +876,14 @@ static bool sdf_mixed_pass2_fp32() {
   return e && strcmp(e, "fp32") == 0;
 }
 
+// A handle created with one of the settings above keeps the reference walk.
+static bool sdf_walk_fixed() {
+  for (const char* name : {"AXSQ_SDF_BUDGET", "AXSQ_SDF_SUSPEND_CAP", "AXSQ_SDF_EARLY_WALKS",
+                           "AXSQ_SDF_WAVE_TAIL", "AXSQ_SDF_MIXED_PASS2"})
+    if (getenv(name)) return true;
+  return false;
+}
+
 int axsq_sdf_create(axsq_sdf** out, const double* x, const double* y, const double* z,
                     int64_t nverts, const int32_t* tris, int64_t ntris, int watertight,
                     int compute_sign, int fp_mode, void* stream) {
@@ -911,6 +920,7 @@ int axsq_sdf_create(axsq_sdf** out, const double* x, const double* y, const doub
   h->mixed_pass2_fp32 = sdf_mixed_pass2_fp32();
   h->early_walks = sdf_early_walks(h->budget);
   h->wave_tail = sdf_wave_tail();
+  h->walk_fixed = sdf_walk_fixed();
   int rc = AXSQ_OK;
   auto fail = [&](int code) {
     axsq_sdf_destroy(h);
@@ -992,6 +1002,7 @@ int axsq_sdf_create_cells(axsq_sdf** out, const double* x, const double* y, cons
   h->compute_sign = compute_sign ? 1 : 0;
   h->fp_mode = AXSQ_FP64;  // the cell walk runs on FP64 nodes
   h->budget = sdf_budget(ncells);
+  h->walk_fixed = sdf_walk_fixed();
   h->susp_cap_fixed = sdf_suspend_cap();
   h->bvh = new axsq_bvh();
   h->bvh->device = h->device;
@@ -1040,6 +1051,7 @@ int axsq_sdf_destroy(axsq_sdf* h) {
   hipFree(h->early_q);
   hipFree(h->skip);
   hipFree(h->wsteps);
+  hipFree(h->cull);
   if (h->early_done) hipEventDestroy(h->early_done);
   hipFree(h->v2t_start);
   hipFree(h->v2t_end);
@@ -1075,6 +1087,7 @@ int axsq_sdf_update_vertices(axsq_sdf* h, const double* x, const double* y, cons
   }
   hipStream_t s = (hipStream_t)stream;
   const size_t nb = sizeof(double) * h->nverts;
+  h->cull_state = 0;
   AXSQ_CHECK_HIP(hipMemcpyAsync(h->vx, x, nb, hipMemcpyDefault, s));
   AXSQ_CHECK_HIP(hipMemcpyAsync(h->vy, y, nb, hipMemcpyDefault, s));
   AXSQ_CHECK_HIP(hipMemcpyAsync(h->vz, z, nb, hipMemcpyDefault, s));

@@ -1,0 +1,507 @@
+// axsq_cull.hip -- builds the oriented child boxes of axsq_cull.hpp over a
+// built tree: per leaf its normal (prefix sums, so that a node's mean normal
+// is a difference) and closest-point tolerance; per node its frame and order
+// plane; then extents, by node size: a thread per node of up to 8 leaves, a
+// wave per node of up to 1,024, and above that a workgroup per 1,024 leaves
+// that adds its share to every such node over them. Bound by memory latency
+// at small sizes (six launches) and by the triangle reads of the mid sizes at
+// large ones. The large nodes matter: with axis-aligned boxes above 512
+// leaves the 1.3M-triangle walk takes twice the steps.
+#include <algorithm>
+
+#include "axsq_cull.hpp"
+#include "axsq_internal.hpp"
+
+namespace axsq {
+
+namespace {
+
+constexpr int kSmallNode = 8;
+constexpr int kLargeNode = 1024;
+constexpr int kMaxLargePath = 256;  // large nodes over one 1,024-leaf chunk
+constexpr int kCullWave = 64;
+
+// A double as two floats is what the walk has; here the difference to the
+// float centre is taken in double and rounded once.
+struct Proj {
+  float p[3], e;
+};
+
+__device__ __forceinline__ Proj project(const CullNode& n, const double* V, float tau) {
+  const float x0 = (float)(V[0] - (double)n.c[0]);
+  const float x1 = (float)(V[1] - (double)n.c[1]);
+  const float x2 = (float)(V[2] - (double)n.c[2]);
+  Proj r;
+  r.p[0] = fmaf(x0, n.w[0], fmaf(x1, n.w[1], x2 * n.w[2]));
+  r.p[1] = fmaf(x0, n.u[0], fmaf(x1, n.u[1], x2 * n.u[2]));
+  r.p[2] = fmaf(x0, n.v[0], fmaf(x1, n.v[1], x2 * n.v[2]));
+  // rounding of x and p: under 2^-22 of the sum of |x|
+  r.e = fmaf(fabsf(x0) + fabsf(x1) + fabsf(x2), 4.76837158e-7f, tau);
+  return r;
+}
+
+struct Extents {
+  float lo[3], hi[3];
+  __device__ __forceinline__ void clear() {
+    for (int d = 0; d < 3; ++d) {
+      lo[d] = INFINITY;
+      hi[d] = -INFINITY;
+    }
+  }
+  __device__ __forceinline__ void add(const Proj& r) {
+#pragma unroll
+    for (int d = 0; d < 3; ++d) {
+      lo[d] = fminf(lo[d], r.p[d] - r.e);
+      hi[d] = fmaxf(hi[d], r.p[d] + r.e);
+    }
+  }
+};
+
+// Adds leaf pos's triangle records to the extents.
+template <bool CELLS>
+__device__ __forceinline__ void add_leaf(const CullNode& n, const TriRec* __restrict__ tris,
+                                         const float* __restrict__ tau, int32_t pos, Extents& x) {
+  const float t = tau[pos];
+  const int nrec = CELLS ? tris[2 * (int64_t)pos].pad : 1;
+  for (int e = 0; e < nrec; ++e) {
+    const double* T = tris[CELLS ? 2 * (int64_t)pos + e : (int64_t)pos].v;
+    for (int k = 0; k < 3; ++k) {
+      const double V[3] = {T[3 * k], T[3 * k + 1], T[3 * k + 2]};
+      x.add(project(n, V, t));
+    }
+  }
+}
+
+// How far a triangle's computed closest point can lie from the triangle, for
+// queries up to `reach` away; negative when no useful bound holds.
+//  - Face: the weights are ratios of differences of products of dot products.
+//    A dot product of an edge (at most L) with a difference to the query (at
+//    most R) is off by 5 u L R, a difference of two products by 22 u (L R)^2,
+//    the denominator |n|^2 by 70 u (L R)^2 (u = 2^-53), so the point is off by
+//    less than 256 u L (L R)^2 / |n|^2 where that ratio is well below 1.
+//  - Edge: the region tests allow 1e-12 (SignedDistance.hpp:647), so the
+//    parameter can leave [0, 1] by (1e-12 + 16 u L R) / |e|^2.
+// A triangle with two equal corners has |n| = 0 and never takes the face
+// branch: the equal dot products send it to an edge or a vertex.
+__device__ __forceinline__ float tri_tau(const double T[9], double reach) {
+  double e2[3], lmax = 0.0, emin = kDblMax;
+  bool same = false;
+  for (int k = 0; k < 3; ++k) {
+    const double* A = T + 3 * k;
+    const double* B = T + 3 * ((k + 1) % 3);
+    const double d0 = B[0] - A[0], d1 = B[1] - A[1], d2 = B[2] - A[2];
+    e2[k] = d0 * d0 + d1 * d1 + d2 * d2;
+    const bool eq = A[0] == B[0] && A[1] == B[1] && A[2] == B[2];
+    same = same || eq;
+    lmax = fmax(lmax, e2[k]);
+    if (!eq) emin = fmin(emin, e2[k]);
+  }
+  if (!(lmax < 1e30)) return -1.0f;  // also NaN corners
+  if (lmax == 0.0) return 0.0f;      // a point
+  if (!(emin >= 4e-12)) return -1.0f;
+  const double L = sqrt(lmax), LR = L * reach;
+  double tau = (1.1e-12 + 1.8e-15 * LR) / sqrt(emin);
+  if (!same) {
+    double n[3];
+    tri_normal(T, n);
+    const double S = n[0] * n[0] + n[1] * n[1] + n[2] * n[2];
+    const double rho = 2.9e-14 * LR * LR / S;
+    if (!(rho <= 0.25)) return -1.0f;
+    tau += rho * L;
+  }
+  return (float)(tau * 1.000001);
+}
+
+// Per leaf: tau, and the running sum of normals within its block of 256.
+template <bool CELLS>
+__global__ __launch_bounds__(kBlock) void k_cull_leaf(const TriRec* __restrict__ tris, int64_t n,
+                                                       double reach, double tau_max,
+                                                       float* __restrict__ tau,
+                                                       double* __restrict__ pre,
+                                                       double* __restrict__ totals,
+                                                       int32_t* __restrict__ ctl) {
+  __shared__ double s_w[kBlock / kCullWave][3];
+  const int64_t pos = (int64_t)blockIdx.x * kBlock + threadIdx.x;
+  double nr[3] = {0.0, 0.0, 0.0};
+  if (pos < n) {
+    float t = 0.0f;
+    const int nrec = CELLS ? tris[2 * pos].pad : (tris[pos].id >= 0 ? 1 : 0);
+    for (int e = 0; e < nrec; ++e) {
+      double T[9], m[3];
+      for (int k = 0; k < 9; ++k) T[k] = tris[CELLS ? 2 * pos + e : pos].v[k];
+      const float te = tri_tau(T, reach);
+      t = (te < 0.0f || t < 0.0f) ? -1.0f : fmaxf(t, te);
+      tri_normal(T, m);
+      for (int d = 0; d < 3; ++d) nr[d] += m[d];
+    }
+    if (!(t >= 0.0f && t <= tau_max)) {
+      atomicOr(&ctl[0], 1);
+      t = 0.0f;
+      for (int d = 0; d < 3; ++d) nr[d] = 0.0;
+    }
+    tau[pos] = t;
+  }
+  const int lane = (int)threadIdx.x % kCullWave, wv = (int)threadIdx.x / kCullWave;
+  for (int o = 1; o < kCullWave; o <<= 1)
+    for (int d = 0; d < 3; ++d) {
+      const double v = __shfl_up(nr[d], o);
+      if (lane >= o) nr[d] += v;
+    }
+  if (lane == kCullWave - 1)
+    for (int d = 0; d < 3; ++d) s_w[wv][d] = nr[d];
+  __syncthreads();
+  for (int k = 0; k < wv; ++k)
+    for (int d = 0; d < 3; ++d) nr[d] += s_w[k][d];
+  if (pos < n)
+    for (int d = 0; d < 3; ++d) pre[3 * pos + d] = nr[d];
+  if (threadIdx.x == kBlock - 1)
+    for (int d = 0; d < 3; ++d) totals[3 * (int64_t)blockIdx.x + d] = nr[d];
+}
+
+// Exclusive sums of the block totals, one block.
+__global__ __launch_bounds__(1024) void k_cull_scan(double* __restrict__ totals, int64_t nb) {
+  __shared__ double s[2][3][1024];
+  double base[3] = {0.0, 0.0, 0.0};
+  const int t = (int)threadIdx.x;
+  for (int64_t b0 = 0; b0 < nb; b0 += 1024) {
+    const int64_t b = b0 + t;
+    double own[3];
+    for (int d = 0; d < 3; ++d) own[d] = b < nb ? totals[3 * b + d] : 0.0;
+    int cur = 0;
+    for (int d = 0; d < 3; ++d) s[0][d][t] = own[d];
+    __syncthreads();
+    for (int o = 1; o < 1024; o <<= 1) {
+      for (int d = 0; d < 3; ++d)
+        s[1 - cur][d][t] = s[cur][d][t] + (t >= o ? s[cur][d][t - o] : 0.0);
+      cur = 1 - cur;
+      __syncthreads();
+    }
+    if (b < nb)
+      for (int d = 0; d < 3; ++d) totals[3 * b + d] = base[d] + s[cur][d][t] - own[d];
+    for (int d = 0; d < 3; ++d) base[d] += s[cur][d][1023];
+    __syncthreads();
+  }
+}
+
+__device__ __forceinline__ uint32_t ordered(float f) {
+  const uint32_t b = __float_as_uint(f);
+  return (b & 0x80000000u) ? ~b : (b | 0x80000000u);
+}
+__device__ __forceinline__ float unordered(uint32_t k) {
+  return __uint_as_float((k & 0x80000000u) ? (k & 0x7fffffffu) : ~k);
+}
+
+__device__ __forceinline__ void store_extents(CullNode* __restrict__ n, const Extents& l,
+                                              const Extents& r, int32_t flags) {
+  for (int d = 0; d < 3; ++d) {  // an invalid child is infinitely far
+    n->llo[d] = (flags & 1) ? l.lo[d] : INFINITY;
+    n->lhi[d] = (flags & 1) ? l.hi[d] : -INFINITY;
+    n->rlo[d] = (flags & 2) ? r.lo[d] : INFINITY;
+    n->rhi[d] = (flags & 2) ? r.hi[d] : -INFINITY;
+  }
+}
+
+// Per node: frame, order plane and links; extents of nodes of at most 8
+// leaves; the others are listed by size. ctl[1], ctl[2]: list lengths.
+template <bool CELLS>
+__global__ __launch_bounds__(kBlock) void k_cull_nodes(const Node64* __restrict__ nodes,
+                                                        int32_t ninner,
+                                                        const TriRec* __restrict__ tris,
+                                                        const float* __restrict__ tau,
+                                                        const double* __restrict__ pre,
+                                                        const double* __restrict__ base,
+                                                        CullNode* __restrict__ out,
+                                                        int32_t* __restrict__ mid_list,
+                                                        int32_t* __restrict__ large_list,
+                                                        int32_t* __restrict__ ctl) {
+  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  bool mid = false, large = false;
+  if (i < ninner) {
+    const Node64 nd = nodes[i];
+    CullNode n;
+    n.lc = nd.lc;
+    n.rc = nd.rc;
+    n.pad = 0;
+    double w[3], len = 0.0;
+    for (int d = 0; d < 3; ++d) {
+      const double hi = pre[3 * (int64_t)nd.hi + d] + base[3 * (int64_t)(nd.hi / kBlock) + d];
+      const double lo = nd.lo > 0 ? pre[3 * (int64_t)(nd.lo - 1) + d] +
+                                        base[3 * (int64_t)((nd.lo - 1) / kBlock) + d]
+                                  : 0.0;
+      w[d] = hi - lo;
+      len += w[d] * w[d];
+    }
+    const double il = len > 0.0 ? 1.0 / sqrt(len) : 0.0;
+    if (il > 0.0 && il < 1e300) {
+      for (int d = 0; d < 3; ++d) w[d] *= il;
+    } else {
+      w[0] = 1.0;
+      w[1] = w[2] = 0.0;
+    }
+    double cl[3], cr[3], D[3], dl = 0.0, tw = 0.0;
+    for (int d = 0; d < 3; ++d) {  // centroids as in BoxTests::right_first
+      cl[d] = 0.5 * (nd.l[d] + nd.l[3 + d]);
+      cr[d] = 0.5 * (nd.r[d] + nd.r[3 + d]);
+      n.c[d] = (float)(0.5 * (cl[d] + cr[d]));
+      D[d] = cr[d] - cl[d];
+      dl += D[d] * D[d];
+      tw += D[d] * w[d];
+    }
+    // second axis: the split direction in the tangent plane
+    double u[3], ul = 0.0;
+    for (int d = 0; d < 3; ++d) {
+      u[d] = D[d] - tw * w[d];
+      ul += u[d] * u[d];
+    }
+    if (ul > 1e-6 * dl && ul > 0.0 && ul < 1e300) {
+      const double iu = 1.0 / sqrt(ul);
+      for (int d = 0; d < 3; ++d) u[d] *= iu;
+    } else {  // any tangent: the axis least along w, made orthogonal
+      const int k = fabs(w[0]) <= fabs(w[1]) ? (fabs(w[0]) <= fabs(w[2]) ? 0 : 2)
+                                             : (fabs(w[1]) <= fabs(w[2]) ? 1 : 2);
+      const double wk = k == 0 ? w[0] : k == 1 ? w[1] : w[2];
+      double m = 0.0;
+      for (int d = 0; d < 3; ++d) {
+        u[d] = (d == k ? 1.0 : 0.0) - wk * w[d];
+        m += u[d] * u[d];
+      }
+      const double iu = 1.0 / sqrt(m);
+      for (int d = 0; d < 3; ++d) u[d] *= iu;
+    }
+    double v[3];
+    cross3(w, u, v);
+    const double dlen = sqrt(dl), idl = dl > 0.0 ? 1.0 / dlen : 0.0;
+    const bool plane = idl > 0.0 && idl < 1e30;
+    double t = 0.0;
+    for (int d = 0; d < 3; ++d) {
+      n.w[d] = (float)w[d];
+      n.u[d] = (float)u[d];
+      n.v[d] = (float)v[d];
+      n.dn[d] = plane ? (float)(D[d] * idl) : 0.0f;
+      t += plane ? D[d] * idl * (0.5 * (cl[d] + cr[d]) - (double)n.c[d]) : 0.0;
+    }
+    n.dt = (float)t;
+    n.inv_d = plane ? (float)(idl * 1.000001) : INFINITY;
+    Extents xl, xr;
+    xl.clear();
+    xr.clear();
+    const int32_t size = nd.hi - nd.lo + 1;
+    large = size > kLargeNode;
+    mid = !large && size > kSmallNode;
+    if (!large && !mid) {
+      for (int32_t p = nd.lo; p <= nd.hi; ++p)
+        add_leaf<CELLS>(n, tris, tau, p, p <= nd.mid ? xl : xr);
+    }
+    store_extents(&n, xl, xr, nd.flags);
+    if (large) {  // ordered integers until k_cull_large_end
+      for (int d = 0; d < 3; ++d) {
+        n.llo[d] = n.rlo[d] = __uint_as_float(0xffffffffu);
+        n.lhi[d] = n.rhi[d] = __uint_as_float(0u);
+      }
+    }
+    out[i] = n;
+  }
+  // list entries, one atomic per wave and list
+  const int lane = (int)threadIdx.x % kCullWave;
+  const uint64_t below = lane == 0 ? 0ull : (~0ull >> (kCullWave - lane));
+  for (int k = 0; k < 2; ++k) {
+    const uint64_t m = __ballot(k == 0 ? mid : large);
+    int32_t at = 0;
+    if (lane == 0 && m) at = atomicAdd(&ctl[1 + k], __popcll(m));
+    at = __shfl(at, 0);
+    if (k == 0 ? mid : large) (k == 0 ? mid_list : large_list)[at + __popcll(m & below)] = (int32_t)i;
+  }
+}
+
+__device__ __forceinline__ void wave_reduce(Extents& x) {
+  for (int o = kCullWave / 2; o > 0; o >>= 1)
+    for (int d = 0; d < 3; ++d) {
+      x.lo[d] = fminf(x.lo[d], __shfl_xor(x.lo[d], o));
+      x.hi[d] = fmaxf(x.hi[d], __shfl_xor(x.hi[d], o));
+    }
+}
+
+// One wave per node of 9 to 1,024 leaves; the list's length is on the device,
+// so a fixed grid strides over it.
+template <bool CELLS>
+__global__ __launch_bounds__(kBlock) void k_cull_mid(const Node64* __restrict__ nodes,
+                                                      const TriRec* __restrict__ tris,
+                                                      const float* __restrict__ tau,
+                                                      const int32_t* __restrict__ list,
+                                                      const int32_t* __restrict__ ctl,
+                                                      CullNode* __restrict__ out) {
+  const int lane = (int)threadIdx.x % kCullWave;
+  const int32_t waves = (int32_t)(gridDim.x * (kBlock / kCullWave));
+  const int32_t count = ctl[1];
+  for (int32_t j = (int32_t)(blockIdx.x * (kBlock / kCullWave) + threadIdx.x / kCullWave);
+       j < count; j += waves) {
+    const int32_t i = list[j];
+    const int32_t lo = nodes[i].lo, hi = nodes[i].hi, split = nodes[i].mid;
+    const CullNode n = out[i];
+    Extents xl, xr;
+    xl.clear();
+    xr.clear();
+    for (int32_t p = lo + lane; p <= hi; p += kCullWave) {
+      Extents x;
+      x.clear();
+      add_leaf<CELLS>(n, tris, tau, p, x);
+      const bool left = p <= split;
+      for (int d = 0; d < 3; ++d) {
+        xl.lo[d] = fminf(xl.lo[d], left ? x.lo[d] : INFINITY);
+        xl.hi[d] = fmaxf(xl.hi[d], left ? x.hi[d] : -INFINITY);
+        xr.lo[d] = fminf(xr.lo[d], left ? INFINITY : x.lo[d]);
+        xr.hi[d] = fmaxf(xr.hi[d], left ? -INFINITY : x.hi[d]);
+      }
+    }
+    wave_reduce(xl);
+    wave_reduce(xr);
+    if (lane == 0) store_extents(out + i, xl, xr, nodes[i].flags);
+  }
+}
+
+// One workgroup per 1,024 leaves: its share of every larger node over them.
+template <bool CELLS>
+__global__ __launch_bounds__(kBlock) void k_cull_large(const Node64* __restrict__ nodes,
+                                                        int32_t ninner,
+                                                        const TriRec* __restrict__ tris,
+                                                        const float* __restrict__ tau,
+                                                        CullNode* __restrict__ out,
+                                                        int32_t* __restrict__ ctl) {
+  __shared__ int32_t s_list[kMaxLargePath];
+  __shared__ int32_t s_n;
+  const int32_t a = (int32_t)blockIdx.x * kLargeNode;
+  const int32_t b = min(a + kLargeNode - 1, ninner);
+  if (threadIdx.x == 0) {  // from the root down: list doubles as the stack's record
+    int32_t n = 0, done = 0;
+    bool full = false;
+    if (ninner + 1 > kLargeNode) s_list[n++] = 0;
+    while (done < n) {
+      const Node64& nd = nodes[s_list[done++]];
+      const int32_t c[2] = {nd.lc, nd.rc};
+      const int32_t lo[2] = {nd.lo, nd.mid + 1}, hi[2] = {nd.mid, nd.hi};
+      for (int k = 0; k < 2; ++k) {
+        if (c[k] < 0 || c[k] >= ninner || hi[k] < a || lo[k] > b) continue;
+        if (hi[k] - lo[k] + 1 <= kLargeNode) continue;
+        if (n < kMaxLargePath)
+          s_list[n++] = c[k];
+        else
+          full = true;
+      }
+    }
+    if (full) atomicOr(&ctl[0], 1);
+    s_n = n;
+  }
+  __syncthreads();
+  const int lane = (int)threadIdx.x % kCullWave;
+  for (int32_t j = 0; j < s_n; ++j) {
+    const int32_t i = s_list[j];
+    const int32_t lo = max(nodes[i].lo, a), hi = min(nodes[i].hi, b), split = nodes[i].mid;
+    const CullNode n = out[i];
+    Extents xl, xr;
+    xl.clear();
+    xr.clear();
+    for (int32_t p = lo + (int32_t)threadIdx.x; p <= hi; p += kBlock) {
+      Extents x;
+      x.clear();
+      add_leaf<CELLS>(n, tris, tau, p, x);
+      const bool left = p <= split;
+      for (int d = 0; d < 3; ++d) {
+        xl.lo[d] = fminf(xl.lo[d], left ? x.lo[d] : INFINITY);
+        xl.hi[d] = fmaxf(xl.hi[d], left ? x.hi[d] : -INFINITY);
+        xr.lo[d] = fminf(xr.lo[d], left ? INFINITY : x.lo[d]);
+        xr.hi[d] = fmaxf(xr.hi[d], left ? -INFINITY : x.hi[d]);
+      }
+    }
+    wave_reduce(xl);
+    wave_reduce(xr);
+    if (lane == 0) {
+      for (int d = 0; d < 3; ++d) {
+        if (xl.lo[d] <= xl.hi[d]) {
+          atomicMin(reinterpret_cast<uint32_t*>(&out[i].llo[d]), ordered(xl.lo[d]));
+          atomicMax(reinterpret_cast<uint32_t*>(&out[i].lhi[d]), ordered(xl.hi[d]));
+        }
+        if (xr.lo[d] <= xr.hi[d]) {
+          atomicMin(reinterpret_cast<uint32_t*>(&out[i].rlo[d]), ordered(xr.lo[d]));
+          atomicMax(reinterpret_cast<uint32_t*>(&out[i].rhi[d]), ordered(xr.hi[d]));
+        }
+      }
+    }
+  }
+}
+
+__global__ __launch_bounds__(kBlock) void k_cull_large_end(const Node64* __restrict__ nodes,
+                                                            const int32_t* __restrict__ list,
+                                                            const int32_t* __restrict__ ctl,
+                                                            CullNode* __restrict__ out) {
+  const int32_t count = ctl[2];
+  for (int32_t j = (int32_t)(blockIdx.x * blockDim.x + threadIdx.x); j < count;
+       j += (int32_t)(gridDim.x * blockDim.x)) {
+    CullNode* n = out + list[j];
+    Extents l, r;
+    for (int d = 0; d < 3; ++d) {
+      l.lo[d] = unordered(__float_as_uint(n->llo[d]));
+      l.hi[d] = unordered(__float_as_uint(n->lhi[d]));
+      r.lo[d] = unordered(__float_as_uint(n->rlo[d]));
+      r.hi[d] = unordered(__float_as_uint(n->rhi[d]));
+    }
+    store_extents(n, l, r, nodes[list[j]].flags);
+  }
+}
+
+template <bool CELLS>
+int build(const axsq_bvh* b, const TriRec* tris, double diag, CullNode* out, Workspace& ws,
+          int32_t* bad, hipStream_t s) {
+  const int64_t n = b->n;
+  const int32_t ninner = (int32_t)(n - 1);
+  const int64_t nb = grid_for(n);
+  const size_t lists = sizeof(int32_t) * ((size_t)ninner + (size_t)ninner / kLargeNode * 2 + 1024);
+  AXSQ_TRY(ws.k0.ensure(sizeof(float) * (size_t)n));
+  AXSQ_TRY(ws.k1.ensure(lists));
+  AXSQ_TRY(ws.v0.ensure(sizeof(double) * 3 * (size_t)n));
+  AXSQ_TRY(ws.v1.ensure(sizeof(double) * 3 * (size_t)nb));
+  AXSQ_TRY(ws.cnt.ensure(sizeof(int32_t) * 4));
+  float* tau = ws.k0.as<float>();
+  double* pre = ws.v0.as<double>();
+  double* totals = ws.v1.as<double>();
+  int32_t* ctl = ws.cnt.as<int32_t>();
+  // large_list: nodes over 1,024 leaves; at most ninner of them
+  int32_t* mid_list = ws.k1.as<int32_t>();
+  AXSQ_TRY(ws.redo.ensure(sizeof(int32_t) * (size_t)std::max<int64_t>(ninner, 1)));
+  int32_t* large_list = ws.redo.as<int32_t>();
+  AXSQ_TRY(fill_i32(ctl, 0, 4, s));
+  k_cull_leaf<CELLS><<<(unsigned)nb, kBlock, 0, s>>>(tris, n, kCullReach * diag,
+                                                     diag * (1.0 / 1024.0), tau, pre, totals, ctl);
+  AXSQ_CHECK_HIP(hipGetLastError());
+  k_cull_scan<<<1, 1024, 0, s>>>(totals, nb);
+  AXSQ_CHECK_HIP(hipGetLastError());
+  k_cull_nodes<CELLS><<<grid_for(ninner), kBlock, 0, s>>>(b->nodes, ninner, tris, tau, pre,
+                                                          totals, out, mid_list, large_list, ctl);
+  AXSQ_CHECK_HIP(hipGetLastError());
+  if (n > kSmallNode) {
+    const unsigned g = (unsigned)std::min<int64_t>((n / 6 + 3) / 4 + 1, 8192);
+    k_cull_mid<CELLS><<<g, kBlock, 0, s>>>(b->nodes, tris, tau, mid_list, ctl, out);
+    AXSQ_CHECK_HIP(hipGetLastError());
+  }
+  if (n > kLargeNode) {
+    k_cull_large<CELLS><<<(unsigned)((n + kLargeNode - 1) / kLargeNode), kBlock, 0, s>>>(
+        b->nodes, ninner, tris, tau, out, ctl);
+    AXSQ_CHECK_HIP(hipGetLastError());
+    k_cull_large_end<<<(unsigned)std::min<int64_t>(n / kLargeNode / kBlock + 1, 256), kBlock, 0,
+                       s>>>(b->nodes, large_list, ctl, out);
+    AXSQ_CHECK_HIP(hipGetLastError());
+  }
+  AXSQ_CHECK_HIP(hipMemcpyAsync(bad, ctl, sizeof(int32_t), hipMemcpyDeviceToHost, s));
+  AXSQ_CHECK_HIP(hipStreamSynchronize(s));
+  return AXSQ_OK;
+}
+
+}  // namespace
+
+int cull_build(const axsq_bvh* b, const TriRec* tris, bool cells, double diag, CullNode* out,
+               int32_t* bad, hipStream_t s) {
+  Workspace& ws = workspace();
+  return cells ? build<true>(b, tris, diag, out, ws, bad, s)
+               : build<false>(b, tris, diag, out, ws, bad, s);
+}
+
+}  // namespace axsq

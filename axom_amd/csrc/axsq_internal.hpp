@@ -4,10 +4,12 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <mutex>
 #include <string>
 #include <vector>
 
 #include "axsq.h"
+#include "axsq_cull.hpp"
 #include "axsq_device.hpp"
 
 namespace axsq {
@@ -57,6 +59,7 @@ struct Workspace {
   DevBuf box2d;                                      // 2-D boxes widened to 3-D
   DevBuf hot;                                        // tables of the longest saved walks
   DevBuf wave_cost, wave_order;                      // first pass: launch order of the waves
+  DevBuf cull_list;                                  // queries the culled walk leaves to the reference walk
   axsq_bvh* mesh_bvh = nullptr;                      // its BVH, rebuilt per call
   // one-call candidate search: the count pass keeps each query's first
   // candidates (find_stash, find_cnt) and lists the queries with more
@@ -229,6 +232,12 @@ struct axsq_sdf {
   uint64_t wave_key[5] = {0, 0, 0, 0, 0};
   bool wsteps_valid = false;
   int32_t wave_tail = 0;  // percent of waves launched last (set at creation; 0: off)
+  // oriented child boxes of the culled walk (axsq_cull.hpp), one per inner
+  // node: 0 not built for the current vertices, 1 built, -1 not usable
+  axsq::CullNode* cull = nullptr;
+  int cull_state = 0;
+  std::mutex cull_mu;       // held while a call builds them
+  bool walk_fixed = false;  // created with a setting of the reference walk: no culled walk
 };
 
 namespace axsq {
@@ -239,6 +248,11 @@ int bvh_build_into(axsq_bvh* b, const double* boxes, int64_t n, double scale, in
                    hipStream_t s, int dims = 3, bool f32 = false,
                    const float* boxes_f32 = nullptr);
 void bvh_release(axsq_bvh* b);
+// Builds the oriented child boxes of a tree over `tris` (diag: the mesh's
+// diagonal) into out, n - 1 records; *bad is set when they must not be used.
+// Returns after the stream has run them.
+int cull_build(const axsq_bvh* b, const TriRec* tris, bool cells, double diag, CullNode* out,
+               int32_t* bad, hipStream_t s);
 // n 2-D boxes (4 doubles) -> 3-D boxes with z range [0, 0] (6 doubles)
 int widen_boxes2d(const double* boxes2d, int64_t n, double* out, hipStream_t s);
 // Candidate search launches (axsq_query.hip). mode 0: count pass (keeping the

@@ -20,9 +20,11 @@
 //
 // Adjoint (no reference counterpart): see axsq_sdf_backward in axsq.h.
 #include <algorithm>
+#include <cmath>
 #include <cstring>
 #include <type_traits>
 
+#include "axsq_cull.hpp"
 #include "axsq_internal.hpp"
 #include "axsq_traverse.hpp"
 
@@ -74,6 +76,7 @@ struct SdfArgs {
   const double* qz;
   int64_t qs;
   int64_t nq;
+  int64_t npos;          // positions of the query order to walk (nq, or a list's length)
   int32_t ninner;
   const uint32_t* order;
   const int32_t* skip;  // first pass: queries whose walks run elsewhere (nonzero), or NULL
@@ -159,7 +162,7 @@ __device__ __forceinline__ void normal_term(const double T[9], int code, double 
 constexpr int kNormList = 8;
 constexpr int32_t kListOverflow = 1 << 16;
 
-__device__ __forceinline__ void check_candidate_deferred(MinCand& m, const double q[3],
+__device__ __forceinline__ bool check_candidate_deferred(MinCand& m, const double q[3],
                                                          const double T[9], int32_t pos,
                                                          bool compute_normal, lds_i32* list,
                                                          int32_t& cnt) {
@@ -178,7 +181,8 @@ __device__ __forceinline__ void check_candidate_deferred(MinCand& m, const doubl
   const double e0 = m.p[0] - cp[0], e1 = m.p[1] - cp[1], e2 = m.p[2] - cp[2];
   const bool same = near_eq(dot3(e0, e1, e2, e0, e1, e2), 0., EPS);
   bool upd;
-  if (sq < m.sq) {
+  const bool closer = sq < m.sq;
+  if (closer) {
     const bool clear = !shared || (m.type != type) || !same;
     m.sq = sq;
     m.p[0] = cp[0];
@@ -199,6 +203,7 @@ __device__ __forceinline__ void check_candidate_deferred(MinCand& m, const doubl
       cnt |= kListOverflow;
     }
   }
+  return closer || upd;  // whether the running state changed
 }
 
 // Adds the recorded terms, in order, to sn. `stride` is the distance between
@@ -362,10 +367,10 @@ __global__ __launch_bounds__(kSdfBlock) AXSQ_SDF_WAVES_ATTR void k_sdf_eval(SdfA
   int64_t t = g;  // position in the query order
   if (a.wave_order) {
     const int64_t wl = g / kWaveLanes;
-    if (wl >= (a.nq + kWaveLanes - 1) / kWaveLanes) return;
+    if (wl >= (a.npos + kWaveLanes - 1) / kWaveLanes) return;
     t = (int64_t)a.wave_order[wl] * kWaveLanes + g % kWaveLanes;
   }
-  if (t >= a.nq) return;
+  if (t >= a.npos) return;
   const int64_t i = a.order ? (int64_t)a.order[t] : t;
   if (a.skip && a.skip[i]) {  // walked beside this pass from the start
     if (a.wsteps) a.wsteps[t] = 0;
@@ -459,6 +464,291 @@ __global__ __launch_bounds__(kSdfBlock) AXSQ_SDF_WAVES_ATTR void k_sdf_eval(SdfA
 }
 
 // ---------------------------------------------------------------------------
+// Culled walk: the reference's walk without the subtrees whose oriented box
+// (axsq_cull.hpp, with the argument why the results are the reference's) is
+// farther than the running minimum. One lane per query in Morton order, on
+// the vote schedule of traverse_vote; a leaf is checked as soon as the walk
+// reaches it, since only the order of the leaves that change the state
+// matters. A pushed child keeps its box key, so an entry that the minimum has
+// passed by the time it is popped costs no node visit.
+// A query is listed for the reference walk instead when a coordinate is not
+// finite or out of the reach of the boxes' tolerance, when a leaf changed the
+// state that the reference's own box test could have pruned, when its term
+// list or stack is full, or when its wave takes kCullSteps steps (queries
+// with a large part of the surface at the same distance).
+#ifndef AXSQ_CULL_LDS
+#define AXSQ_CULL_LDS 24  // stack entries a lane keeps in LDS
+#endif
+#ifndef AXSQ_CULL_VOTE_PCT
+#define AXSQ_CULL_VOTE_PCT 50
+#endif
+constexpr int kCullLds = AXSQ_CULL_LDS;
+#ifndef AXSQ_CULL_STEPS
+#define AXSQ_CULL_STEPS 512
+#endif
+constexpr int32_t kCullSteps = AXSQ_CULL_STEPS;
+#ifndef AXSQ_COOP_QUERIES
+#define AXSQ_COOP_QUERIES 4096
+#endif
+constexpr int64_t kCoopQueries = AXSQ_COOP_QUERIES;  // batches walked one wave per query
+constexpr int64_t kCoopWaves = 4096;    // waves that share the long walks
+
+struct CullArgs {
+  const CullNode* nodes;
+  double reach2;   // squared reach: queries farther from the mesh are listed
+  float cmax;      // largest coordinate of the mesh's box, by magnitude
+  int32_t* longq;  // queries whose wave took kCullSteps steps (room for nq)
+  uint32_t* nlong;
+  uint32_t* ticket;  // k_sdf_coop: the next entry of longq to walk
+};
+
+// What the two culled walks keep per query beside the reference's state.
+struct CullQuery {
+  float qh[3], ql[3];  // the query as float pairs
+  float slack;         // added to the running distance
+  float a0, a1;        // order plane: decided beyond a0 + a1 / |D|
+  float thr;           // box keys above it are left out
+  bool ok;             // finite and within reach
+  template <bool MIXED>
+  __device__ __forceinline__ void init(const double q[3], const double dom[6], const CullArgs& c) {
+    // R: distance to the farthest corner of the mesh's box
+    double r2 = 0.0;
+    for (int d = 0; d < 3; ++d) {
+      const double e = fmax(fabs(q[d] - dom[d]), fabs(q[d] - dom[3 + d]));
+      r2 += e * e;
+    }
+    ok = !query_has_nan(q) && r2 <= c.reach2;
+    const float R = sqrtf((float)r2) * 1.00001f;
+    float qmax = c.cmax;
+    for (int d = 0; d < 3; ++d) {
+      qh[d] = (float)q[d];
+      ql[d] = (float)(q[d] - (double)qh[d]);
+      qmax = fmaxf(qmax, fabsf(qh[d]));
+    }
+    // 1e-6: ties (checkCandidate); 2^-19 R: projections; 2^-40 qmax: the pairs
+    slack = 1.01e-6f + R * 1.9073486e-6f + qmax * 9.0949470e-13f;
+    // a query at most a0 + a1 / |D| from a node's order plane reads the boxes:
+    // FP64 right_first is decided to 2^-49 R^2 / |D| and the plane's float form
+    // to 2^-20 R; the FP32 form also rounds coordinates (2^-23 of qmax)
+    a0 = MIXED ? (R + qmax) * 1.9073486e-6f : R * 9.5367432e-7f;
+    a1 = MIXED ? (R + qmax) * R * 9.5367432e-7f : R * R * 1.7763568e-15f;
+    thr = 3.402823466e38f;
+  }
+  __device__ __forceinline__ void bound(double sq) {
+    const float r = sqrtf((float)sq) * 1.0000003f + slack;
+    thr = fminf(r * r * 1.0000039f, 3.402823466e38f);
+  }
+};
+
+// A visit: the child box keys, links, and whether the right child is nearer
+// (only where both keys pass).
+struct CullVisit {
+  float kl, kr;
+  int32_t lc, rc;
+  bool right;
+};
+template <bool MIXED>
+__device__ __forceinline__ CullVisit cull_visit(const SdfArgs& a, const CullArgs& c,
+                                                const CullQuery& k, const double q[3],
+                                                int32_t cur) {
+  const float4* p = reinterpret_cast<const float4*>(c.nodes + cur);
+  const float4 f0 = p[0], f1 = p[1], f2 = p[2], f3 = p[3], f4 = p[4], f5 = p[5], f6 = p[6],
+               f7 = p[7];
+  const float x0 = (k.qh[0] - f0.x) + k.ql[0];
+  const float x1 = (k.qh[1] - f0.y) + k.ql[1];
+  const float x2 = (k.qh[2] - f0.z) + k.ql[2];
+  const float pw = fmaf(x0, f0.w, fmaf(x1, f1.x, x2 * f1.y));
+  const float pu = fmaf(x0, f1.z, fmaf(x1, f1.w, x2 * f2.x));
+  const float pv = fmaf(x0, f2.y, fmaf(x1, f2.z, x2 * f2.w));
+  const float lw = fmaxf(fmaxf(f3.x - pw, pw - f3.w), 0.0f);
+  const float lu = fmaxf(fmaxf(f3.y - pu, pu - f4.x), 0.0f);
+  const float lv = fmaxf(fmaxf(f3.z - pv, pv - f4.y), 0.0f);
+  const float rw = fmaxf(fmaxf(f4.z - pw, pw - f5.y), 0.0f);
+  const float ru = fmaxf(fmaxf(f4.w - pu, pu - f5.z), 0.0f);
+  const float rv = fmaxf(fmaxf(f5.x - pv, pv - f5.w), 0.0f);
+  CullVisit v;
+  v.kl = fmaf(lw, lw, fmaf(lu, lu, lv * lv));
+  v.kr = fmaf(rw, rw, fmaf(ru, ru, rv * rv));
+  v.lc = __float_as_int(f7.y);
+  v.rc = __float_as_int(f7.z);
+  v.right = false;
+  if (v.kl <= k.thr && v.kr <= k.thr) {
+    const float sd = fmaf(x0, f6.x, fmaf(x1, f6.y, fmaf(x2, f6.z, -f6.w)));
+    v.right = sd > 0.0f;
+    if (!(fabsf(sd) > fmaf(k.a1, f7.x, k.a0))) {
+      int32_t l2, r2, flags;
+      if constexpr (MIXED) {
+        float lb[6], rb[6];
+        load_node(a.nodes32, cur, lb, rb, l2, r2, flags);
+        v.right = BoxTests<true>(q).right_first(lb, rb);
+      } else {
+        double lb[6], rb[6];
+        load_node(a.nodes, cur, lb, rb, l2, r2, flags);
+        v.right = BoxTests<false>(q).right_first(lb, rb);
+      }
+    }
+  }
+  return v;
+}
+
+typedef __attribute__((address_space(3))) float lds_f32;
+
+// LaneStackT with a box key beside each entry.
+struct KeyedStack {
+  lds_i32* node;
+  lds_f32* key;
+  int32_t spill_node[kStack - kCullLds];
+  float spill_key[kStack - kCullLds];
+  __device__ __forceinline__ void get(int32_t sp, int32_t& n, float& k) const {
+    if (sp < kCullLds) {
+      n = node[sp * kWaveLanes];
+      k = key[sp * kWaveLanes];
+    } else {
+      n = spill_node[sp - kCullLds];
+      k = spill_key[sp - kCullLds];
+    }
+  }
+  __device__ __forceinline__ void set(int32_t sp, int32_t n, float k) {
+    if (sp < kCullLds) {
+      node[sp * kWaveLanes] = n;
+      key[sp * kWaveLanes] = k;
+    } else {
+      spill_node[sp - kCullLds] = n;
+      spill_key[sp - kCullLds] = k;
+    }
+  }
+};
+
+// The squared distance to the scaled box of a leaf, as the tree holds it
+// (k_tri_boxes / k_cell_boxes, box_scale with the default factor).
+__device__ __forceinline__ double leaf_box_key(const double q[3], const double b[6]) {
+  double x[6];
+  for (int k = 0; k < 6; ++k) x[k] = b[k];
+  box_scale(x, 1.000123);
+  return sqdist_box(q[0], q[1], q[2], x);
+}
+
+template <bool MIXED, bool CELLS>
+__global__ __launch_bounds__(kWaveLanes) void k_sdf_cull(SdfArgs a, CullArgs c) {
+  __shared__ int32_t s_node[kCullLds * kWaveLanes];
+  __shared__ float s_key[kCullLds * kWaveLanes];
+  __shared__ int32_t s_terms[kNormList * kWaveLanes];
+  const int lane = (int)threadIdx.x;
+  const int64_t t = (int64_t)blockIdx.x * kWaveLanes + lane;
+  if (t >= a.npos) return;
+  const int64_t i = a.order ? (int64_t)a.order[t] : t;
+  lds_i32* terms = (lds_i32*)(s_terms + lane);
+  KeyedStack todo;
+  todo.node = (lds_i32*)(s_node + lane);
+  todo.key = (lds_f32*)(s_key + lane);
+  const double q[3] = {a.qx[i * a.qs], a.qy[i * a.qs], a.qz[i * a.qs]};
+  const bool cn = a.compute_sign != 0;
+  MinCand m;
+  m.sq = kDblMax;
+  m.p[0] = m.p[1] = m.p[2] = 0.0;
+  m.sn[0] = m.sn[1] = m.sn[2] = 0.0;
+  m.type = -1;
+  m.pos = 0;
+  int32_t nterms = 0;
+  CullQuery k;
+  k.init<MIXED>(q, a.dom, c);
+  bool listed = !k.ok, is_long = false;
+  int32_t cur = listed ? kBarrier : 0, sp = 0;
+  todo.set(0, kBarrier, 0.0f);
+  auto pop = [&]() {
+    float key;
+    do {
+      todo.get(sp, cur, key);
+      --sp;
+    } while (key > k.thr);  // the barrier's key is 0
+  };
+  for (int32_t it = 0;; ++it) {
+    const uint64_t want_node = __ballot(cur >= 0);
+    const uint64_t want_leaf = __ballot(cur < 0 && cur != kBarrier);
+    if ((want_node | want_leaf) == 0) break;
+    if (it >= kCullSteps) {
+      is_long = cur != kBarrier;
+      break;
+    }
+    const int n_node = __popcll(want_node), n_leaf = __popcll(want_leaf);
+    if (n_leaf > 0 && 100 * n_leaf >= AXSQ_CULL_VOTE_PCT * (n_node + n_leaf)) {
+      if (cur < 0 && cur != kBarrier) {
+        const int32_t pos = min(-cur - 1, a.ninner);  // a malformed tree reads no further
+        const double before = m.sq;
+        int32_t changed = 0;
+        double T[9], bx[6];
+        int32_t ntri = 1;
+        if constexpr (CELLS) ntri = reinterpret_cast<const int32_t*>(a.tris + 2 * (int64_t)pos)[19];
+        for (int e = 0; e < (CELLS ? 2 : 1); ++e) {
+          if (e >= ntri) continue;
+          const int32_t rec = CELLS ? 2 * pos + e : pos;
+          load_tri(a.tris, rec, T);
+          changed |= check_candidate_deferred(m, q, T, rec, cn, terms, nterms) ? 1 : 0;
+        }
+        if (changed) {
+          // the reference reaches this leaf whatever its earlier minima were
+          // only if the leaf's box passes at this one
+          if constexpr (CELLS) load_tri(a.tris, 2 * pos, T);
+          for (int d = 0; d < 3; ++d) {
+            bx[d] = fmin(fmin(T[d], T[3 + d]), T[6 + d]);
+            bx[3 + d] = fmax(fmax(T[d], T[3 + d]), T[6 + d]);
+          }
+          if constexpr (CELLS) {
+            if (ntri > 1) {
+              load_tri(a.tris, 2 * pos + 1, T);
+              for (int d = 0; d < 3; ++d) {
+                bx[d] = fmin(bx[d], fmin(fmin(T[d], T[3 + d]), T[6 + d]));
+                bx[3 + d] = fmax(bx[3 + d], fmax(fmax(T[d], T[3 + d]), T[6 + d]));
+              }
+            }
+          }
+          if (!(leaf_box_key(q, bx) <= before))
+            listed = true;
+          else
+            k.bound(m.sq);
+        }
+        if (listed)
+          cur = kBarrier;
+        else
+          pop();
+      }
+    } else if (cur >= 0) {
+      if (cur >= a.ninner) {  // only from a malformed tree
+        listed = true;
+        cur = kBarrier;
+      } else {
+        const CullVisit v = cull_visit<MIXED>(a, c, k, q, cur);
+        const bool in_l = v.kl <= k.thr, in_r = v.kr <= k.thr;
+        if (in_l && in_r) {
+          ++sp;
+          if (sp >= kStack) {
+            listed = true;
+            cur = kBarrier;
+          } else {
+            todo.set(sp, v.right ? v.lc : v.rc, v.right ? v.kl : v.kr);
+            cur = v.right ? v.rc : v.lc;
+          }
+        } else if (in_l || in_r) {
+          cur = in_l ? v.lc : v.rc;
+        } else {
+          pop();
+        }
+      }
+    }
+  }
+  if (is_long) {
+    c.longq[atomicAdd(c.nlong, 1u)] = (int32_t)i;  // one slot per query
+    return;
+  }
+  if (listed || (nterms & kListOverflow)) {
+    a.redo[atomicAdd(a.nredo, 1u)] = (int32_t)i;  // one slot per query
+    return;
+  }
+  add_terms(m.sn, a.tris, (const lds_i32*)terms, kWaveLanes, nterms);
+  sdf_finish(a, i, q, m, cn);
+}
+
+// ---------------------------------------------------------------------------
 // Second pass, wave-cooperative form: one walk per wave, either a saved walk
 // or (after a term-list overflow) a walk run again from the start. The walk
 // itself is sequential (its pruning depends on every earlier leaf), so all 64
@@ -543,6 +833,225 @@ struct MemoLane {
   int32_t pn;       // this node's parent in the memo, 2 * index + (1 if right child); -1: root
   int32_t pl;       // this leaf's parent in the memo, 2 * index + (1 if right child)
 };
+
+// The culled walk of one query by a whole wave: for the queries the lanes'
+// walk gave up as long, and for batches too small to fill the chip with one
+// lane per query. The pending subtrees are a list in walk order (LDS, the
+// next one on top). Each step takes the top 64: a lane with an inner node
+// replaces it by the children that pass, nearer first; a lane with a leaf
+// keeps it; a prefix count puts the results back in order. When enough leaves
+// lead the list, the lanes check one each, and those that change the state
+// are applied one after the other, in lane order, which is walk order. A step
+// costs one node or triangle load for up to 64 visits, where a lane's walk
+// pays that for each.
+#ifndef AXSQ_COOP_LEAD
+#define AXSQ_COOP_LEAD 24  // leaves at the head of the list that are checked at once
+#endif
+constexpr int kCoopCap = 1536;
+
+template <bool MIXED, bool CELLS>
+__global__ __launch_bounds__(kWaveLanes) void k_sdf_coop(SdfArgs a, CullArgs c, int64_t nall) {
+  __shared__ int32_t s_node[kCoopCap];
+  __shared__ float s_key[kCoopCap];
+  __shared__ int32_t s_terms[kNormList];
+  const int32_t lane = (int32_t)threadIdx.x;
+  const uint64_t below = lane == 0 ? 0ull : (~0ull >> (kWaveLanes - lane));
+  const int64_t count = nall > 0 ? nall : (int64_t)*c.nlong;
+  const bool cn = a.compute_sign != 0;
+  for (int64_t j = blockIdx.x; j < count;) {
+    const int64_t i = nall > 0 ? (a.order ? (int64_t)a.order[j] : j) : (int64_t)c.longq[j];
+    const double q[3] = {a.qx[i * a.qs], a.qy[i * a.qs], a.qz[i * a.qs]};
+    CullQuery k;
+    k.init<MIXED>(q, a.dom, c);
+    bool listed = !k.ok;
+    MinCand m;
+    m.sq = kDblMax;
+    m.p[0] = m.p[1] = m.p[2] = 0.0;
+    m.sn[0] = m.sn[1] = m.sn[2] = 0.0;
+    m.type = -1;
+    m.pos = 0;
+    int32_t nterms = 0;
+    int32_t sp = listed ? 0 : 1;  // entries in the list
+    __syncthreads();
+    if (lane == 0) {
+      s_node[0] = 0;
+      s_key[0] = 0.0f;
+    }
+    __syncthreads();
+    // every step removes or expands an entry, and a node is expanded once
+    for (int64_t guard = 0; sp > 0; ++guard) {
+      if (guard > 4 * (int64_t)a.ninner + 64) {  // only a malformed tree
+        listed = true;
+        break;
+      }
+      const int32_t take = min(sp, kWaveLanes);
+      const int32_t at = sp - 1 - lane;
+      int32_t node = 0;
+      float key = INFINITY;
+      if (lane < take) {
+        node = s_node[at];
+        key = s_key[at];
+      }
+      const bool live = key <= k.thr;
+      const uint64_t m_inner = __ballot(live && node >= 0);
+      const uint64_t m_leaf = __ballot(live && node < 0);
+      const int32_t first_inner = m_inner ? __builtin_ctzll(m_inner) : kWaveLanes;
+      const uint64_t lead =
+          m_leaf & (first_inner >= kWaveLanes ? ~0ull : ((1ull << first_inner) - 1));
+      if (m_inner == 0 || __popcll(lead) >= AXSQ_COOP_LEAD) {
+        sp -= min(first_inner, take);
+        if (lead == 0) continue;
+        const bool mine = (lead >> lane) & 1ull;
+        const int32_t pos = mine ? min(-node - 1, a.ninner) : 0;
+        double sq = kDblMax, cp[3] = {0.0, 0.0, 0.0};
+        double sq2 = kDblMax, cp2[3] = {0.0, 0.0, 0.0};
+        int32_t type = 2, code = 0, type2 = 2, code2 = 0;
+        double bkey = 0.0;
+        bool two = false;
+        if (mine) {
+          double T[9], bx[6];
+          load_tri(a.tris, CELLS ? 2 * pos : pos, T);
+          leaf_record(q, T, sq, cp, type, code);
+          for (int d = 0; d < 3; ++d) {
+            bx[d] = fmin(fmin(T[d], T[3 + d]), T[6 + d]);
+            bx[3 + d] = fmax(fmax(T[d], T[3 + d]), T[6 + d]);
+          }
+          if constexpr (CELLS) {
+            two = reinterpret_cast<const int32_t*>(a.tris + 2 * (int64_t)pos)[19] > 1;
+            if (two) {
+              load_tri(a.tris, 2 * pos + 1, T);
+              leaf_record(q, T, sq2, cp2, type2, code2);
+              for (int d = 0; d < 3; ++d) {
+                bx[d] = fmin(bx[d], fmin(fmin(T[d], T[3 + d]), T[6 + d]));
+                bx[3 + d] = fmax(bx[3 + d], fmax(fmax(T[d], T[3 + d]), T[6 + d]));
+              }
+            }
+          }
+          bkey = leaf_box_key(q, bx);
+        }
+        auto changes = [&](double rsq, const double rp[3], int32_t rtype) -> bool {
+          const double e0 = m.p[0] - rp[0], e1 = m.p[1] - rp[1], e2 = m.p[2] - rp[2];
+          return (rsq < m.sq) || (cn && rtype != 2 && m.type == rtype &&
+                                  near_eq(dot3(e0, e1, e2, e0, e1, e2), 0., kSdfEps));
+        };
+        // checkCandidate's update from lane l's record, with its term deferred
+        auto apply = [&](int32_t l, double vsq, const double vp[3], int32_t vtype, int32_t vcode,
+                         int32_t vrec) {
+          const double rsq = lane_get(vsq, l);
+          const double rp[3] = {lane_get(vp[0], l), lane_get(vp[1], l), lane_get(vp[2], l)};
+          const int32_t rtype = lane_get(vtype, l), rcode = lane_get(vcode, l);
+          const int32_t rec = lane_get(vrec, l);
+          const double e0 = m.p[0] - rp[0], e1 = m.p[1] - rp[1], e2 = m.p[2] - rp[2];
+          const bool same = near_eq(dot3(e0, e1, e2, e0, e1, e2), 0., kSdfEps);
+          bool upd;
+          if (rsq < m.sq) {
+            if (cn && (rtype == 2 || m.type != rtype || !same)) nterms = 0;
+            m.sq = rsq;
+            for (int d = 0; d < 3; ++d) m.p[d] = rp[d];
+            m.type = rtype;
+            m.pos = rec;
+            upd = cn && rtype != 2;
+          } else {
+            upd = cn && rtype != 2 && m.type == rtype && same;
+          }
+          if (upd) {
+            if (nterms < kNormList) {
+              if (lane == 0)
+                s_terms[nterms] = (int32_t)((uint32_t)rec * 4u + (uint32_t)rcode);
+              ++nterms;
+            } else {
+              nterms |= kListOverflow;
+            }
+          }
+        };
+        const int32_t rec = CELLS ? 2 * pos : pos;
+        uint64_t left = lead;
+        bool any = false;
+        while (left) {
+          const bool e = mine && (changes(sq, cp, type) ||
+                                  (CELLS && two && changes(sq2, cp2, type2)));
+          const uint64_t eff = __ballot(e) & left;
+          if (!eff) break;
+          const int32_t l = __builtin_ctzll(eff);
+          if (!(lane_get(bkey, l) <= m.sq)) {
+            listed = true;
+            break;
+          }
+          apply(l, sq, cp, type, code, rec);
+          if constexpr (CELLS) {
+            if (lane_get((int32_t)two, l)) apply(l, sq2, cp2, type2, code2, rec + 1);
+          }
+          any = true;
+          left &= l >= kWaveLanes - 1 ? 0ull : ~((2ull << l) - 1);
+        }
+        if (listed) break;
+        if (any) k.bound(m.sq);
+        continue;
+      }
+      // expand the inner nodes of the top entries in place
+      int32_t n0 = node, n1 = 0;
+      float k0 = key, k1 = 0.0f;
+      bool one = live && node < 0, both = false, bad = false;
+      if (live && node >= 0) {
+        if (node >= a.ninner) {
+          bad = true;
+        } else {
+          const CullVisit v = cull_visit<MIXED>(a, c, k, q, node);
+          const bool in_l = v.kl <= k.thr, in_r = v.kr <= k.thr;
+          both = in_l && in_r;
+          one = in_l || in_r;
+          const bool r = both ? v.right : !in_l;
+          n0 = r ? v.rc : v.lc;
+          k0 = r ? v.kr : v.kl;
+          n1 = r ? v.lc : v.rc;
+          k1 = r ? v.kl : v.kr;
+        }
+      }
+      const uint64_t m_one = __ballot(one), m_both = __ballot(both);
+      const int32_t total = __popcll(m_one) + __popcll(m_both);
+      const int32_t base = sp - take;
+      if (base + total > kCoopCap || __ballot(bad)) {
+        listed = true;
+        break;
+      }
+      const int32_t dst = base + total - 1 - (__popcll(m_one & below) + __popcll(m_both & below));
+      __syncthreads();
+      if (one) {
+        s_node[dst] = n0;
+        s_key[dst] = k0;
+      }
+      if (both) {
+        s_node[dst - 1] = n1;
+        s_key[dst - 1] = k1;
+      }
+      __syncthreads();
+      sp = base + total;
+    }
+    if (listed || (nterms & kListOverflow)) {
+      if (lane == 0) a.redo[atomicAdd(a.nredo, 1u)] = (int32_t)i;
+    } else {
+      // the recorded terms, one lane each, added in their order
+      __syncthreads();
+      double t[3] = {0.0, 0.0, 0.0};
+      if (lane < nterms) {
+        const uint32_t e = (uint32_t)s_terms[lane];
+        double T[9];
+        load_tri(a.tris, (int32_t)(e >> 2), T);
+        normal_term(T, (int)(e & 3u), t);
+      }
+      for (int32_t l = 0; l < nterms; ++l)
+        for (int d = 0; d < 3; ++d) m.sn[d] += lane_get(t[d], l);
+      if (lane == 0) sdf_finish(a, i, q, m, cn);
+    }
+    if (nall > 0) {
+      j += gridDim.x;
+    } else {
+      uint32_t nx = 0;
+      if (lane == 0) nx = atomicAdd(c.ticket, 1u);
+      j = (int64_t)gridDim.x + (int64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)nx);
+    }
+  }
+}
 
 // A hot walk's tables: for its query, every leaf's record (leaf_record's
 // values) and every inner node's child-box keys and bits (MemoLane::bits),
@@ -1891,57 +2400,15 @@ static SideStream* side_stream() {
   return &ss;
 }
 
-int sdf_eval_launch(const axsq_sdf* h, const double* x, const double* y, const double* z,
-                    int64_t stride, int64_t nq, int fp_mode, double* dist, double* cp,
-                    double* normal, int32_t* elem, bool stats, hipStream_t s) {
+// The reference walk in two passes over the npos positions of a's query order:
+// every query, or (list) the queries the culled walk listed. qkey names the
+// query arrays for what a call remembers for the next one on them.
+static int sdf_eval_reference(const axsq_sdf* h, SdfArgs a, bool list, const uint64_t qkey[5],
+                              bool mixed, bool stats, hipStream_t s) {
   Workspace& ws = workspace();
   const axsq_bvh* b = h->bvh;
-  SdfArgs a{};
-  a.nodes = b->nodes;
-  a.nodes32 = b->nodes32;
-  a.ranges32 = b->ranges32;
-  a.tris = h->tris;
-  a.qx = x;
-  a.qy = y;
-  a.qz = z;
-  a.qs = stride;
-  a.nq = nq;
-  a.ninner = (int32_t)(b->n - 1);
-  a.order = nullptr;
-  a.susp_order = nullptr;
-  for (int k = 0; k < 6; ++k) a.dom[k] = h->domain[k];
-  a.watertight = h->watertight;
-  a.compute_sign = h->compute_sign;
-  a.dist = dist;
-  a.cp = cp;
-  a.normal = normal;
-  a.elem = elem;
-  a.status = b->status;
-  a.stats = h->stats_dev;
-  if (h->sort_queries && nq > 4096) {
-    AXSQ_TRY(ws.k0.ensure(sizeof(uint32_t) * nq));
-    AXSQ_TRY(ws.v0.ensure(sizeof(uint32_t) * nq));
-    AXSQ_TRY(ws.k1.ensure(sizeof(uint32_t) * nq));
-    AXSQ_TRY(ws.v1.ensure(sizeof(uint32_t) * nq));
-    double inv[3];
-    for (int d = 0; d < 3; ++d) {
-      const double ext = h->domain[3 + d] - h->domain[d];
-      inv[d] = ext > 0.0 ? 1.0 / ext : 0.0;
-    }
-    ProfRange pq("sdf_query_order", s);
-    k_query_codes<<<grid_for(nq), kBlock, 0, s>>>(x, y, z, stride, nq, h->domain[0],
-                                                  h->domain[1], h->domain[2], inv[0], inv[1],
-                                                  inv[2], ws.k0.as<uint32_t>(),
-                                                  ws.v0.as<uint32_t>());
-    AXSQ_CHECK_HIP(hipGetLastError());
-    uint32_t *sk, *sv;
-    AXSQ_TRY(radix_sort_pairs(ws.k0.as<uint32_t>(), ws.v0.as<uint32_t>(), ws.k1.as<uint32_t>(),
-                              ws.v1.as<uint32_t>(), nq, 30, ws, s, &sk, &sv));
-    pq.stop();
-    a.order = sv;
-  }
-  const bool cells = h->cells;  // quad cells: FP64 nodes, two records per leaf
-  const bool mixed = (fp_mode == AXSQ_FP32_TRAVERSAL) && !cells;
+  const bool cells = h->cells;
+  const int64_t nq = a.npos;
   // room for suspended walks (360 B each): as many as the previous call on
   // this handle suspended, plus a quarter and 4,096; on the first call an
   // eighth of the queries (at least 65,536); never more than the queries or
@@ -1966,7 +2433,6 @@ int sdf_eval_launch(const axsq_sdf* h, const double* x, const double* y, const d
   a.cap = cap;
   a.budget = h->budget;
   AXSQ_TRY(fill_i32(reinterpret_cast<int32_t*>(a.nsusp), 0, 2, s));
-  ProfRange pr(mixed ? "sdf_eval_fp32" : "sdf_eval_fp64", s);
   // Early walks: the previous call on the same query arrays listed its
   // longest walks (the first of its second pass's launch order). Their
   // queries are walked here from the start, one wave each as in the second
@@ -1974,17 +2440,15 @@ int sdf_eval_launch(const axsq_sdf* h, const double* x, const double* y, const d
   // longest walks no longer wait for the first pass to end. Which queries
   // these are changes speed only: each query is still walked once, in full.
   axsq_sdf* hm = const_cast<axsq_sdf*>(h);
-  const uint64_t qkey[5] = {(uint64_t)(uintptr_t)x, (uint64_t)(uintptr_t)y,
-                            (uint64_t)(uintptr_t)z, (uint64_t)stride, (uint64_t)nq};
-  const int64_t kEarly = cells ? 0 : h->early_walks;
-  if (kEarly == 0 || memcmp(qkey, hm->early_key, sizeof(qkey)) != 0) {
+  const int64_t kEarly = (cells || list) ? 0 : h->early_walks;
+  if (kEarly == 0 || memcmp(qkey, hm->early_key, sizeof(hm->early_key)) != 0) {
     hm->nearly = 0;
-    memcpy(hm->early_key, qkey, sizeof(qkey));
+    memcpy(hm->early_key, qkey, sizeof(hm->early_key));
   }
   const int64_t nearly = std::min<int64_t>(hm->nearly, kEarly);
   SideStream* side = nearly > 0 ? side_stream() : nullptr;
   // launch order of the waves from the previous call's steps (in query order)
-  const bool wave_on = h->wave_tail > 0 && a.order != nullptr;
+  const bool wave_on = h->wave_tail > 0 && a.order != nullptr && !list;
   if ((kEarly > 0 || wave_on) && !hm->early_done)
     AXSQ_CHECK_HIP(hipEventCreateWithFlags(&hm->early_done, hipEventDisableTiming));
   // On every way out of this call once the early walks are forked (an error
@@ -2052,7 +2516,7 @@ int sdf_eval_launch(const axsq_sdf* h, const double* x, const double* y, const d
     // the previous call may have run on another stream: its first pass
     // wrote the steps read here and rewritten by this call's
     if (hm->early_done) AXSQ_CHECK_HIP(hipStreamWaitEvent(s, hm->early_done, 0));
-    const bool same = hm->wsteps_valid && memcmp(qkey, hm->wave_key, sizeof(qkey)) == 0;
+    const bool same = hm->wsteps_valid && memcmp(qkey, hm->wave_key, sizeof(hm->wave_key)) == 0;
     if (hm->wsteps_cap < nq) {
       (void)hipFree(hm->wsteps);
       hm->wsteps = nullptr;
@@ -2074,7 +2538,7 @@ int sdf_eval_launch(const axsq_sdf* h, const double* x, const double* y, const d
       a.wave_order = ws.wave_order.as<int32_t>();
     }
     a.wsteps = hm->wsteps;
-    memcpy(hm->wave_key, qkey, sizeof(qkey));
+    memcpy(hm->wave_key, qkey, sizeof(hm->wave_key));
     hm->wsteps_valid = true;
   }
   ProfRange p1(mixed ? "sdf_eval_fp32_pass1" : "sdf_eval_fp64_pass1", s);
@@ -2186,8 +2650,157 @@ int sdf_eval_launch(const axsq_sdf* h, const double* x, const double* y, const d
     AXSQ_CHECK_HIP(hipEventRecord(hm->early_done, s));
   }
   p2.stop();
-  pr.stop();
   return AXSQ_OK;
+}
+
+// Whether a call of nq queries runs the culled walk. The boxes cost about as
+// much as a rebuild of the tree, so a call with few queries on a mesh that
+// has none yet keeps the reference walk; so do meshes so small or so large
+// that the tie radius 1e-6 or float range would count, and handles created
+// with one of the reference walk's own settings.
+static bool cull_wanted(const axsq_sdf* h, int64_t nq) {
+  if (h->walk_fixed) return false;
+  double d2 = 0.0;
+  for (int k = 0; k < 3; ++k) {
+    const double e = h->domain[3 + k] - h->domain[k];
+    d2 += e * e;
+  }
+  if (!(d2 >= 1e-4 && d2 <= 1e30)) return false;  // diagonal 0.01 .. 1e15
+  return h->cull_state == 1 || 16 * nq >= h->ntris;
+}
+
+// The tree's oriented boxes, built by the first call that wants them after
+// the mesh was set or moved; *out stays NULL where they do not hold (a
+// triangle without a useful tolerance, no memory).
+static int sdf_cull_nodes(axsq_sdf* h, hipStream_t s, const CullNode** out) {
+  std::lock_guard<std::mutex> lock(h->cull_mu);
+  if (h->cull_state == 0) {
+    const size_t n = (size_t)(h->bvh->n - 1);
+    if (!h->cull && hipMalloc((void**)&h->cull, sizeof(CullNode) * n) != hipSuccess) {
+      (void)hipGetLastError();
+      h->cull = nullptr;
+      h->cull_state = -1;
+    } else {
+      double d2 = 0.0;
+      for (int k = 0; k < 3; ++k) {
+        const double e = h->domain[3 + k] - h->domain[k];
+        d2 += e * e;
+      }
+      int32_t bad = 0;
+      ProfRange pr("sdf_cull_build", s);
+      AXSQ_TRY(cull_build(h->bvh, h->tris, h->cells, std::sqrt(d2), h->cull, &bad, s));
+      h->cull_state = bad ? -1 : 1;
+    }
+  }
+  if (h->cull_state == 1) *out = h->cull;
+  return AXSQ_OK;
+}
+
+int sdf_eval_launch(const axsq_sdf* h, const double* x, const double* y, const double* z,
+                    int64_t stride, int64_t nq, int fp_mode, double* dist, double* cp,
+                    double* normal, int32_t* elem, bool stats, hipStream_t s) {
+  Workspace& ws = workspace();
+  const axsq_bvh* b = h->bvh;
+  SdfArgs a{};
+  a.nodes = b->nodes;
+  a.nodes32 = b->nodes32;
+  a.ranges32 = b->ranges32;
+  a.tris = h->tris;
+  a.qx = x;
+  a.qy = y;
+  a.qz = z;
+  a.qs = stride;
+  a.nq = nq;
+  a.npos = nq;
+  a.ninner = (int32_t)(b->n - 1);
+  a.order = nullptr;
+  a.susp_order = nullptr;
+  for (int k = 0; k < 6; ++k) a.dom[k] = h->domain[k];
+  a.watertight = h->watertight;
+  a.compute_sign = h->compute_sign;
+  a.dist = dist;
+  a.cp = cp;
+  a.normal = normal;
+  a.elem = elem;
+  a.status = b->status;
+  a.stats = h->stats_dev;
+  const bool cells = h->cells;  // quad cells: FP64 nodes, two records per leaf
+  const bool mixed = (fp_mode == AXSQ_FP32_TRAVERSAL) && !cells;
+  const CullNode* cull = nullptr;
+  if (!stats && cull_wanted(h, nq)) AXSQ_TRY(sdf_cull_nodes(const_cast<axsq_sdf*>(h), s, &cull));
+  if (h->sort_queries && nq > 4096) {
+    AXSQ_TRY(ws.k0.ensure(sizeof(uint32_t) * nq));
+    AXSQ_TRY(ws.v0.ensure(sizeof(uint32_t) * nq));
+    AXSQ_TRY(ws.k1.ensure(sizeof(uint32_t) * nq));
+    AXSQ_TRY(ws.v1.ensure(sizeof(uint32_t) * nq));
+    double inv[3];
+    for (int d = 0; d < 3; ++d) {
+      const double ext = h->domain[3 + d] - h->domain[d];
+      inv[d] = ext > 0.0 ? 1.0 / ext : 0.0;
+    }
+    ProfRange pq("sdf_query_order", s);
+    k_query_codes<<<grid_for(nq), kBlock, 0, s>>>(x, y, z, stride, nq, h->domain[0],
+                                                  h->domain[1], h->domain[2], inv[0], inv[1],
+                                                  inv[2], ws.k0.as<uint32_t>(),
+                                                  ws.v0.as<uint32_t>());
+    AXSQ_CHECK_HIP(hipGetLastError());
+    uint32_t *sk, *sv;
+    AXSQ_TRY(radix_sort_pairs(ws.k0.as<uint32_t>(), ws.v0.as<uint32_t>(), ws.k1.as<uint32_t>(),
+                              ws.v1.as<uint32_t>(), nq, 30, ws, s, &sk, &sv));
+    pq.stop();
+    a.order = sv;
+  }
+  ProfRange pr(mixed ? "sdf_eval_fp32" : "sdf_eval_fp64", s);
+  const uint64_t qkey[5] = {(uint64_t)(uintptr_t)x, (uint64_t)(uintptr_t)y,
+                            (uint64_t)(uintptr_t)z, (uint64_t)stride, (uint64_t)nq};
+  if (!cull) return sdf_eval_reference(h, a, false, qkey, mixed, stats, s);
+  axsq_sdf* hm = const_cast<axsq_sdf*>(h);
+  AXSQ_TRY(ws.cull_list.ensure(sizeof(int32_t) * 2 * (size_t)nq));
+  AXSQ_TRY(ws.cnt.ensure(sizeof(uint32_t) * 4));
+  a.redo = ws.cull_list.as<int32_t>();
+  a.nredo = ws.cnt.as<uint32_t>();
+  AXSQ_TRY(fill_i32(reinterpret_cast<int32_t*>(a.nredo), 0, 3, s));
+  CullArgs c{};
+  c.nodes = cull;
+  double d2 = 0.0;
+  for (int k = 0; k < 3; ++k) {
+    const double e = h->domain[3 + k] - h->domain[k];
+    d2 += e * e;
+    c.cmax = std::max(c.cmax, (float)std::max(std::fabs(h->domain[k]),
+                                              std::fabs(h->domain[3 + k])) * 1.00001f);
+  }
+  c.reach2 = kCullReach * kCullReach * d2;
+  c.longq = a.redo + nq;
+  c.nlong = a.nredo + 1;
+  c.ticket = a.nredo + 2;
+  ProfRange p1(mixed ? "sdf_eval_fp32_cull" : "sdf_eval_fp64_cull", s);
+  // one lane per query, then one wave per long walk; a small batch one wave
+  // per query at once
+  const bool small = nq <= kCoopQueries;
+  const unsigned g = grid_for(nq, kWaveLanes);
+  const unsigned gc = (unsigned)(small ? nq : std::min<int64_t>(nq, kCoopWaves));
+  const int64_t nall = small ? nq : 0;
+  if (cells) {
+    if (!small) k_sdf_cull<false, true><<<g, kWaveLanes, 0, s>>>(a, c);
+    k_sdf_coop<false, true><<<gc, kWaveLanes, 0, s>>>(a, c, nall);
+  } else if (mixed) {
+    if (!small) k_sdf_cull<true, false><<<g, kWaveLanes, 0, s>>>(a, c);
+    k_sdf_coop<true, false><<<gc, kWaveLanes, 0, s>>>(a, c, nall);
+  } else {
+    if (!small) k_sdf_cull<false, false><<<g, kWaveLanes, 0, s>>>(a, c);
+    k_sdf_coop<false, false><<<gc, kWaveLanes, 0, s>>>(a, c, nall);
+  }
+  AXSQ_CHECK_HIP(hipGetLastError());
+  p1.stop();
+  uint32_t listed = 0;
+  AXSQ_CHECK_HIP(hipMemcpyAsync(&listed, a.nredo, sizeof(listed), hipMemcpyDeviceToHost, s));
+  AXSQ_CHECK_HIP(hipStreamSynchronize(s));
+  hm->last_suspended = 0;
+  hm->last_early = 0;
+  if (listed == 0) return AXSQ_OK;
+  a.order = reinterpret_cast<const uint32_t*>(ws.cull_list.p);
+  a.npos = std::min<int64_t>(listed, nq);
+  return sdf_eval_reference(h, a, true, qkey, mixed, false, s);
 }
 
 int sdf_backward_launch(const axsq_sdf* h, const double* x, const double* y, const double* z,
