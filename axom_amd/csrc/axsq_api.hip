@@ -1088,6 +1088,7 @@ int axsq_sdf_update_vertices(axsq_sdf* h, const double* x, const double* y, cons
   hipStream_t s = (hipStream_t)stream;
   const size_t nb = sizeof(double) * h->nverts;
   h->cull_state = 0;
+  h->evaluated = false;
   AXSQ_CHECK_HIP(hipMemcpyAsync(h->vx, x, nb, hipMemcpyDefault, s));
   AXSQ_CHECK_HIP(hipMemcpyAsync(h->vy, y, nb, hipMemcpyDefault, s));
   AXSQ_CHECK_HIP(hipMemcpyAsync(h->vz, z, nb, hipMemcpyDefault, s));

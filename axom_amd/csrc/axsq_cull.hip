@@ -21,23 +21,8 @@ constexpr int kLargeNode = 1024;
 constexpr int kMaxLargePath = 256;  // large nodes over one 1,024-leaf chunk
 constexpr int kCullWave = 64;
 
-// A double as two floats is what the walk has; here the difference to the
-// float centre is taken in double and rounded once.
-struct Proj {
-  float p[3], e;
-};
-
-__device__ __forceinline__ Proj project(const CullNode& n, const double* V, float tau) {
-  const float x0 = (float)(V[0] - (double)n.c[0]);
-  const float x1 = (float)(V[1] - (double)n.c[1]);
-  const float x2 = (float)(V[2] - (double)n.c[2]);
-  Proj r;
-  r.p[0] = fmaf(x0, n.w[0], fmaf(x1, n.w[1], x2 * n.w[2]));
-  r.p[1] = fmaf(x0, n.u[0], fmaf(x1, n.u[1], x2 * n.u[2]));
-  r.p[2] = fmaf(x0, n.v[0], fmaf(x1, n.v[1], x2 * n.v[2]));
-  // rounding of x and p: under 2^-22 of the sum of |x|
-  r.e = fmaf(fabsf(x0) + fabsf(x1) + fabsf(x2), 4.76837158e-7f, tau);
-  return r;
+__device__ __forceinline__ void mesh_coords(const CullSpace& cs, const double* V, float x[3]) {
+  for (int d = 0; d < 3; ++d) x[d] = (float)((V[d] - cs.o[d]) * cs.scale);
 }
 
 struct Extents {
@@ -48,26 +33,44 @@ struct Extents {
       hi[d] = -INFINITY;
     }
   }
-  __device__ __forceinline__ void add(const Proj& r) {
+  __device__ __forceinline__ void add(const float t[3], float e) {
 #pragma unroll
     for (int d = 0; d < 3; ++d) {
-      lo[d] = fminf(lo[d], r.p[d] - r.e);
-      hi[d] = fmaxf(hi[d], r.p[d] + r.e);
+      lo[d] = fminf(lo[d], t[d] - e);
+      hi[d] = fmaxf(hi[d], t[d] + e);
+    }
+  }
+  __device__ __forceinline__ void merge(const Extents& o) {
+#pragma unroll
+    for (int d = 0; d < 3; ++d) {
+      lo[d] = fminf(lo[d], o.lo[d]);
+      hi[d] = fmaxf(hi[d], o.hi[d]);
     }
   }
 };
 
+// The share of a vertex at x; tau in mesh coordinates. Projections are
+// rounded to under 2^-21 of the sum of |x|, about the diagonal's 1 to 2.
+__device__ __forceinline__ void add_vertex(const CullNode& n, const float x[3], float tau,
+                                           Extents& out) {
+  float t[3];
+  cull_project(n.w, n.u, n.m, x, t);
+  out.add(t, fmaf(fabsf(x[0]) + fabsf(x[1]) + fabsf(x[2]) + 1.0f, 4.76837158e-7f, tau));
+}
+
 // Adds leaf pos's triangle records to the extents.
 template <bool CELLS>
-__device__ __forceinline__ void add_leaf(const CullNode& n, const TriRec* __restrict__ tris,
-                                         const float* __restrict__ tau, int32_t pos, Extents& x) {
+__device__ __forceinline__ void add_leaf(const CullNode& n, const CullSpace& cs,
+                                         const TriRec* __restrict__ tris,
+                                         const float* __restrict__ tau, int32_t pos, Extents& out) {
   const float t = tau[pos];
   const int nrec = CELLS ? tris[2 * (int64_t)pos].pad : 1;
   for (int e = 0; e < nrec; ++e) {
     const double* T = tris[CELLS ? 2 * (int64_t)pos + e : (int64_t)pos].v;
     for (int k = 0; k < 3; ++k) {
-      const double V[3] = {T[3 * k], T[3 * k + 1], T[3 * k + 2]};
-      x.add(project(n, V, t));
+      float x[3];
+      mesh_coords(cs, T + 3 * k, x);
+      add_vertex(n, x, t, out);
     }
   }
 }
@@ -115,7 +118,7 @@ __device__ __forceinline__ float tri_tau(const double T[9], double reach) {
 // Per leaf: tau, and the running sum of normals within its block of 256.
 template <bool CELLS>
 __global__ __launch_bounds__(kBlock) void k_cull_leaf(const TriRec* __restrict__ tris, int64_t n,
-                                                       double reach, double tau_max,
+                                                       double reach, double tau_max, double scale,
                                                        float* __restrict__ tau,
                                                        double* __restrict__ pre,
                                                        double* __restrict__ totals,
@@ -139,7 +142,7 @@ __global__ __launch_bounds__(kBlock) void k_cull_leaf(const TriRec* __restrict__
       t = 0.0f;
       for (int d = 0; d < 3; ++d) nr[d] = 0.0;
     }
-    tau[pos] = t;
+    tau[pos] = (float)((double)t * scale * 1.000001);
   }
   const int lane = (int)threadIdx.x % kCullWave, wv = (int)threadIdx.x / kCullWave;
   for (int o = 1; o < kCullWave; o <<= 1)
@@ -191,20 +194,32 @@ __device__ __forceinline__ float unordered(uint32_t k) {
   return __uint_as_float((k & 0x80000000u) ? (k & 0x7fffffffu) : ~k);
 }
 
+// lo and hi as halves rounded outward (halves are sign and magnitude, so the
+// next one down or up is one off in its bits).
+__device__ __forceinline__ uint32_t half_range(float lo, float hi) {
+  uint16_t l = __half_as_ushort(__float2half_rn(lo)), h = __half_as_ushort(__float2half_rn(hi));
+  if (__half2float(__ushort_as_half(l)) > lo)
+    l = (l & 0x8000u) ? l + 1 : (l == 0 ? 0x8001u : l - 1);
+  if (__half2float(__ushort_as_half(h)) < hi)
+    h = (h & 0x8000u) ? (h == 0x8000u ? 1 : h - 1) : h + 1;
+  return (uint32_t)l | ((uint32_t)h << 16);
+}
+
 __device__ __forceinline__ void store_extents(CullNode* __restrict__ n, const Extents& l,
                                               const Extents& r, int32_t flags) {
-  for (int d = 0; d < 3; ++d) {  // an invalid child is infinitely far
-    n->llo[d] = (flags & 1) ? l.lo[d] : INFINITY;
-    n->lhi[d] = (flags & 1) ? l.hi[d] : -INFINITY;
-    n->rlo[d] = (flags & 2) ? r.lo[d] : INFINITY;
-    n->rhi[d] = (flags & 2) ? r.hi[d] : -INFINITY;
+  constexpr uint32_t kNone = 0xfc007c00u;  // an invalid child: from +inf to -inf
+  for (int d = 0; d < 3; ++d) {
+    n->l[d] = (flags & 1) ? half_range(l.lo[d], l.hi[d]) : kNone;
+    n->r[d] = (flags & 2) ? half_range(r.lo[d], r.hi[d]) : kNone;
   }
 }
 
 // Per node: frame, order plane and links; extents of nodes of at most 8
-// leaves; the others are listed by size. ctl[1], ctl[2]: list lengths.
+// leaves; the others are listed by size. ctl[1], ctl[2]: list lengths. A large
+// node's place in its list is kept in l[0] until k_cull_large_end.
 template <bool CELLS>
-__global__ __launch_bounds__(kBlock) void k_cull_nodes(const Node64* __restrict__ nodes,
+__global__ __launch_bounds__(kBlock) void k_cull_nodes(CullSpace cs,
+                                                        const Node64* __restrict__ nodes,
                                                         int32_t ninner,
                                                         const TriRec* __restrict__ tris,
                                                         const float* __restrict__ tau,
@@ -213,6 +228,7 @@ __global__ __launch_bounds__(kBlock) void k_cull_nodes(const Node64* __restrict_
                                                         CullNode* __restrict__ out,
                                                         int32_t* __restrict__ mid_list,
                                                         int32_t* __restrict__ large_list,
+                                                        uint32_t* __restrict__ acc,
                                                         int32_t* __restrict__ ctl) {
   const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   bool mid = false, large = false;
@@ -221,7 +237,6 @@ __global__ __launch_bounds__(kBlock) void k_cull_nodes(const Node64* __restrict_
     CullNode n;
     n.lc = nd.lc;
     n.rc = nd.rc;
-    n.pad = 0;
     double w[3], len = 0.0;
     for (int d = 0; d < 3; ++d) {
       const double hi = pre[3 * (int64_t)nd.hi + d] + base[3 * (int64_t)(nd.hi / kBlock) + d];
@@ -242,7 +257,6 @@ __global__ __launch_bounds__(kBlock) void k_cull_nodes(const Node64* __restrict_
     for (int d = 0; d < 3; ++d) {  // centroids as in BoxTests::right_first
       cl[d] = 0.5 * (nd.l[d] + nd.l[3 + d]);
       cr[d] = 0.5 * (nd.r[d] + nd.r[3 + d]);
-      n.c[d] = (float)(0.5 * (cl[d] + cr[d]));
       D[d] = cr[d] - cl[d];
       dl += D[d] * D[d];
       tw += D[d] * w[d];
@@ -268,20 +282,22 @@ __global__ __launch_bounds__(kBlock) void k_cull_nodes(const Node64* __restrict_
       const double iu = 1.0 / sqrt(m);
       for (int d = 0; d < 3; ++d) u[d] *= iu;
     }
-    double v[3];
-    cross3(w, u, v);
     const double dlen = sqrt(dl), idl = dl > 0.0 ? 1.0 / dlen : 0.0;
     const bool plane = idl > 0.0 && idl < 1e30;
-    double t = 0.0;
+    double a = 0.0, bb = 0.0;
+    float xm[3];
+    const float zero[3] = {0.0f, 0.0f, 0.0f};
     for (int d = 0; d < 3; ++d) {
       n.w[d] = (float)w[d];
       n.u[d] = (float)u[d];
-      n.v[d] = (float)v[d];
-      n.dn[d] = plane ? (float)(D[d] * idl) : 0.0f;
-      t += plane ? D[d] * idl * (0.5 * (cl[d] + cr[d]) - (double)n.c[d]) : 0.0;
+      xm[d] = (float)((0.5 * (cl[d] + cr[d]) - cs.o[d]) * cs.scale);
+      a += D[d] * idl * w[d];
+      bb += D[d] * idl * u[d];
     }
-    n.dt = (float)t;
-    n.inv_d = plane ? (float)(idl * 1.000001) : INFINITY;
+    cull_project(n.w, n.u, zero, xm, n.m);
+    n.a = plane ? (float)a : 0.0f;
+    n.b = plane ? (float)bb : 0.0f;
+    n.inv_d = plane ? (float)(idl / cs.scale * 1.000001) : INFINITY;
     Extents xl, xr;
     xl.clear();
     xr.clear();
@@ -290,15 +306,9 @@ __global__ __launch_bounds__(kBlock) void k_cull_nodes(const Node64* __restrict_
     mid = !large && size > kSmallNode;
     if (!large && !mid) {
       for (int32_t p = nd.lo; p <= nd.hi; ++p)
-        add_leaf<CELLS>(n, tris, tau, p, p <= nd.mid ? xl : xr);
+        add_leaf<CELLS>(n, cs, tris, tau, p, p <= nd.mid ? xl : xr);
     }
     store_extents(&n, xl, xr, nd.flags);
-    if (large) {  // ordered integers until k_cull_large_end
-      for (int d = 0; d < 3; ++d) {
-        n.llo[d] = n.rlo[d] = __uint_as_float(0xffffffffu);
-        n.lhi[d] = n.rhi[d] = __uint_as_float(0u);
-      }
-    }
     out[i] = n;
   }
   // list entries, one atomic per wave and list
@@ -309,7 +319,13 @@ __global__ __launch_bounds__(kBlock) void k_cull_nodes(const Node64* __restrict_
     int32_t at = 0;
     if (lane == 0 && m) at = atomicAdd(&ctl[1 + k], __popcll(m));
     at = __shfl(at, 0);
-    if (k == 0 ? mid : large) (k == 0 ? mid_list : large_list)[at + __popcll(m & below)] = (int32_t)i;
+    at += __popcll(m & below);
+    if (k == 0 && mid) mid_list[at] = (int32_t)i;
+    if (k == 1 && large) {
+      large_list[at] = (int32_t)i;
+      out[i].l[0] = (uint32_t)at;
+      for (int d = 0; d < 12; ++d) acc[12 * (int64_t)at + d] = (d % 6) < 3 ? 0xffffffffu : 0u;
+    }
   }
 }
 
@@ -324,7 +340,8 @@ __device__ __forceinline__ void wave_reduce(Extents& x) {
 // One wave per node of 9 to 1,024 leaves; the list's length is on the device,
 // so a fixed grid strides over it.
 template <bool CELLS>
-__global__ __launch_bounds__(kBlock) void k_cull_mid(const Node64* __restrict__ nodes,
+__global__ __launch_bounds__(kBlock) void k_cull_mid(CullSpace cs,
+                                                      const Node64* __restrict__ nodes,
                                                       const TriRec* __restrict__ tris,
                                                       const float* __restrict__ tau,
                                                       const int32_t* __restrict__ list,
@@ -344,14 +361,11 @@ __global__ __launch_bounds__(kBlock) void k_cull_mid(const Node64* __restrict__ 
     for (int32_t p = lo + lane; p <= hi; p += kCullWave) {
       Extents x;
       x.clear();
-      add_leaf<CELLS>(n, tris, tau, p, x);
-      const bool left = p <= split;
-      for (int d = 0; d < 3; ++d) {
-        xl.lo[d] = fminf(xl.lo[d], left ? x.lo[d] : INFINITY);
-        xl.hi[d] = fmaxf(xl.hi[d], left ? x.hi[d] : -INFINITY);
-        xr.lo[d] = fminf(xr.lo[d], left ? INFINITY : x.lo[d]);
-        xr.hi[d] = fmaxf(xr.hi[d], left ? -INFINITY : x.hi[d]);
-      }
+      add_leaf<CELLS>(n, cs, tris, tau, p, x);
+      if (p <= split)
+        xl.merge(x);
+      else
+        xr.merge(x);
     }
     wave_reduce(xl);
     wave_reduce(xr);
@@ -359,14 +373,21 @@ __global__ __launch_bounds__(kBlock) void k_cull_mid(const Node64* __restrict__ 
   }
 }
 
-// One workgroup per 1,024 leaves: its share of every larger node over them.
+// One workgroup per 1,024 leaves: its share of every larger node over them,
+// from vertices held in registers (a node costs no triangle reads: for 2.1M
+// triangles the kernel took 1.14 ms reading them per node). A node's share on
+// one side of its split only, the common case, reduces that side alone.
 template <bool CELLS>
-__global__ __launch_bounds__(kBlock) void k_cull_large(const Node64* __restrict__ nodes,
+__global__ __launch_bounds__(kBlock) void k_cull_large(CullSpace cs,
+                                                        const Node64* __restrict__ nodes,
                                                         int32_t ninner,
                                                         const TriRec* __restrict__ tris,
                                                         const float* __restrict__ tau,
-                                                        CullNode* __restrict__ out,
+                                                        const CullNode* __restrict__ out,
+                                                        uint32_t* __restrict__ acc,
                                                         int32_t* __restrict__ ctl) {
+  constexpr int kPer = kLargeNode / kBlock;  // leaves per thread
+  constexpr int kVerts = CELLS ? 6 : 3;
   __shared__ int32_t s_list[kMaxLargePath];
   __shared__ int32_t s_n;
   const int32_t a = (int32_t)blockIdx.x * kLargeNode;
@@ -391,38 +412,49 @@ __global__ __launch_bounds__(kBlock) void k_cull_large(const Node64* __restrict_
     if (full) atomicOr(&ctl[0], 1);
     s_n = n;
   }
+  float x[kPer][kVerts][3], t[kPer];
+  int nv[kPer];
+  for (int j = 0; j < kPer; ++j) {
+    const int32_t p = a + j * kBlock + (int32_t)threadIdx.x;
+    nv[j] = 0;
+    t[j] = 0.0f;
+    for (int k = 0; k < kVerts; ++k)
+      for (int d = 0; d < 3; ++d) x[j][k][d] = 0.0f;
+    if (p <= b) {
+      t[j] = tau[p];
+      nv[j] = CELLS ? 3 * tris[2 * (int64_t)p].pad : 3;
+      for (int k = 0; k < kVerts; ++k)
+        if (k < nv[j]) {
+          const int64_t rec = CELLS ? 2 * (int64_t)p + k / 3 : (int64_t)p;
+          mesh_coords(cs, tris[rec].v + 3 * (k % 3), x[j][k]);
+        }
+    }
+  }
   __syncthreads();
   const int lane = (int)threadIdx.x % kCullWave;
-  for (int32_t j = 0; j < s_n; ++j) {
-    const int32_t i = s_list[j];
-    const int32_t lo = max(nodes[i].lo, a), hi = min(nodes[i].hi, b), split = nodes[i].mid;
-    const CullNode n = out[i];
-    Extents xl, xr;
-    xl.clear();
-    xr.clear();
-    for (int32_t p = lo + (int32_t)threadIdx.x; p <= hi; p += kBlock) {
-      Extents x;
-      x.clear();
-      add_leaf<CELLS>(n, tris, tau, p, x);
-      const bool left = p <= split;
-      for (int d = 0; d < 3; ++d) {
-        xl.lo[d] = fminf(xl.lo[d], left ? x.lo[d] : INFINITY);
-        xl.hi[d] = fmaxf(xl.hi[d], left ? x.hi[d] : -INFINITY);
-        xr.lo[d] = fminf(xr.lo[d], left ? INFINITY : x.lo[d]);
-        xr.hi[d] = fmaxf(xr.hi[d], left ? -INFINITY : x.hi[d]);
+  for (int32_t i = 0; i < s_n; ++i) {
+    const CullNode n = out[s_list[i]];
+    const int32_t lo = nodes[s_list[i]].lo, hi = nodes[s_list[i]].hi, split = nodes[s_list[i]].mid;
+    uint32_t* to = acc + 12 * (int64_t)n.l[0];
+    for (int side = 0; side < 2; ++side) {
+      const int32_t from = side == 0 ? max(lo, a) : max(split + 1, a);
+      const int32_t last = side == 0 ? min(split, b) : min(hi, b);
+      if (from > last) continue;  // uniform
+      Extents e;
+      e.clear();
+      for (int j = 0; j < kPer; ++j) {
+        const int32_t p = a + j * kBlock + (int32_t)threadIdx.x;
+        if (p < from || p > last) continue;
+        for (int k = 0; k < kVerts; ++k)
+          if (k < nv[j]) add_vertex(n, x[j][k], t[j], e);
       }
-    }
-    wave_reduce(xl);
-    wave_reduce(xr);
-    if (lane == 0) {
-      for (int d = 0; d < 3; ++d) {
-        if (xl.lo[d] <= xl.hi[d]) {
-          atomicMin(reinterpret_cast<uint32_t*>(&out[i].llo[d]), ordered(xl.lo[d]));
-          atomicMax(reinterpret_cast<uint32_t*>(&out[i].lhi[d]), ordered(xl.hi[d]));
-        }
-        if (xr.lo[d] <= xr.hi[d]) {
-          atomicMin(reinterpret_cast<uint32_t*>(&out[i].rlo[d]), ordered(xr.lo[d]));
-          atomicMax(reinterpret_cast<uint32_t*>(&out[i].rhi[d]), ordered(xr.hi[d]));
+      wave_reduce(e);
+      if (lane == 0) {
+        for (int d = 0; d < 3; ++d) {
+          if (e.lo[d] <= e.hi[d]) {
+            atomicMin(to + 6 * side + d, ordered(e.lo[d]));
+            atomicMax(to + 6 * side + 3 + d, ordered(e.hi[d]));
+          }
         }
       }
     }
@@ -432,31 +464,29 @@ __global__ __launch_bounds__(kBlock) void k_cull_large(const Node64* __restrict_
 __global__ __launch_bounds__(kBlock) void k_cull_large_end(const Node64* __restrict__ nodes,
                                                             const int32_t* __restrict__ list,
                                                             const int32_t* __restrict__ ctl,
+                                                            const uint32_t* __restrict__ acc,
                                                             CullNode* __restrict__ out) {
   const int32_t count = ctl[2];
   for (int32_t j = (int32_t)(blockIdx.x * blockDim.x + threadIdx.x); j < count;
        j += (int32_t)(gridDim.x * blockDim.x)) {
-    CullNode* n = out + list[j];
-    Extents l, r;
-    for (int d = 0; d < 3; ++d) {
-      l.lo[d] = unordered(__float_as_uint(n->llo[d]));
-      l.hi[d] = unordered(__float_as_uint(n->lhi[d]));
-      r.lo[d] = unordered(__float_as_uint(n->rlo[d]));
-      r.hi[d] = unordered(__float_as_uint(n->rhi[d]));
-    }
-    store_extents(n, l, r, nodes[list[j]].flags);
+    Extents x[2];
+    for (int side = 0; side < 2; ++side)
+      for (int d = 0; d < 3; ++d) {
+        x[side].lo[d] = unordered(acc[12 * (int64_t)j + 6 * side + d]);
+        x[side].hi[d] = unordered(acc[12 * (int64_t)j + 6 * side + 3 + d]);
+      }
+    store_extents(out + list[j], x[0], x[1], nodes[list[j]].flags);
   }
 }
 
 template <bool CELLS>
-int build(const axsq_bvh* b, const TriRec* tris, double diag, CullNode* out, Workspace& ws,
-          int32_t* bad, hipStream_t s) {
+int build(const axsq_bvh* b, const TriRec* tris, const CullSpace& cs, double diag, CullNode* out,
+          Workspace& ws, int32_t* bad, hipStream_t s) {
   const int64_t n = b->n;
   const int32_t ninner = (int32_t)(n - 1);
   const int64_t nb = grid_for(n);
-  const size_t lists = sizeof(int32_t) * ((size_t)ninner + (size_t)ninner / kLargeNode * 2 + 1024);
   AXSQ_TRY(ws.k0.ensure(sizeof(float) * (size_t)n));
-  AXSQ_TRY(ws.k1.ensure(lists));
+  AXSQ_TRY(ws.k1.ensure(sizeof(int32_t) * (size_t)ninner));
   AXSQ_TRY(ws.v0.ensure(sizeof(double) * 3 * (size_t)n));
   AXSQ_TRY(ws.v1.ensure(sizeof(double) * 3 * (size_t)nb));
   AXSQ_TRY(ws.cnt.ensure(sizeof(int32_t) * 4));
@@ -464,30 +494,36 @@ int build(const axsq_bvh* b, const TriRec* tris, double diag, CullNode* out, Wor
   double* pre = ws.v0.as<double>();
   double* totals = ws.v1.as<double>();
   int32_t* ctl = ws.cnt.as<int32_t>();
-  // large_list: nodes over 1,024 leaves; at most ninner of them
   int32_t* mid_list = ws.k1.as<int32_t>();
-  AXSQ_TRY(ws.redo.ensure(sizeof(int32_t) * (size_t)std::max<int64_t>(ninner, 1)));
+  // nodes over 1,024 leaves: few in a balanced tree, up to ninner - 1,023 in a
+  // chain, each with 12 running extents
+  const size_t nlarge = (size_t)std::max<int64_t>((int64_t)ninner - kLargeNode + 1, 1);
+  AXSQ_TRY(ws.redo.ensure(sizeof(int32_t) * nlarge));
+  AXSQ_TRY(ws.misc.ensure(sizeof(uint32_t) * 12 * nlarge));
   int32_t* large_list = ws.redo.as<int32_t>();
+  uint32_t* acc = ws.misc.as<uint32_t>();
   AXSQ_TRY(fill_i32(ctl, 0, 4, s));
   k_cull_leaf<CELLS><<<(unsigned)nb, kBlock, 0, s>>>(tris, n, kCullReach * diag,
-                                                     diag * (1.0 / 1024.0), tau, pre, totals, ctl);
+                                                     diag * (1.0 / 1024.0), cs.scale, tau, pre, totals,
+                                                     ctl);
   AXSQ_CHECK_HIP(hipGetLastError());
   k_cull_scan<<<1, 1024, 0, s>>>(totals, nb);
   AXSQ_CHECK_HIP(hipGetLastError());
-  k_cull_nodes<CELLS><<<grid_for(ninner), kBlock, 0, s>>>(b->nodes, ninner, tris, tau, pre,
-                                                          totals, out, mid_list, large_list, ctl);
+  k_cull_nodes<CELLS><<<grid_for(ninner), kBlock, 0, s>>>(cs, b->nodes, ninner, tris, tau, pre,
+                                                          totals, out, mid_list, large_list, acc,
+                                                          ctl);
   AXSQ_CHECK_HIP(hipGetLastError());
   if (n > kSmallNode) {
     const unsigned g = (unsigned)std::min<int64_t>((n / 6 + 3) / 4 + 1, 8192);
-    k_cull_mid<CELLS><<<g, kBlock, 0, s>>>(b->nodes, tris, tau, mid_list, ctl, out);
+    k_cull_mid<CELLS><<<g, kBlock, 0, s>>>(cs, b->nodes, tris, tau, mid_list, ctl, out);
     AXSQ_CHECK_HIP(hipGetLastError());
   }
   if (n > kLargeNode) {
     k_cull_large<CELLS><<<(unsigned)((n + kLargeNode - 1) / kLargeNode), kBlock, 0, s>>>(
-        b->nodes, ninner, tris, tau, out, ctl);
+        cs, b->nodes, ninner, tris, tau, out, acc, ctl);
     AXSQ_CHECK_HIP(hipGetLastError());
     k_cull_large_end<<<(unsigned)std::min<int64_t>(n / kLargeNode / kBlock + 1, 256), kBlock, 0,
-                       s>>>(b->nodes, large_list, ctl, out);
+                       s>>>(b->nodes, large_list, ctl, acc, out);
     AXSQ_CHECK_HIP(hipGetLastError());
   }
   AXSQ_CHECK_HIP(hipMemcpyAsync(bad, ctl, sizeof(int32_t), hipMemcpyDeviceToHost, s));
@@ -497,11 +533,11 @@ int build(const axsq_bvh* b, const TriRec* tris, double diag, CullNode* out, Wor
 
 }  // namespace
 
-int cull_build(const axsq_bvh* b, const TriRec* tris, bool cells, double diag, CullNode* out,
-               int32_t* bad, hipStream_t s) {
+int cull_build(const axsq_bvh* b, const TriRec* tris, bool cells, const CullSpace& cs, double diag,
+               CullNode* out, int32_t* bad, hipStream_t s) {
   Workspace& ws = workspace();
-  return cells ? build<true>(b, tris, diag, out, ws, bad, s)
-               : build<false>(b, tris, diag, out, ws, bad, s);
+  return cells ? build<true>(b, tris, cs, diag, out, ws, bad, s)
+               : build<false>(b, tris, cs, diag, out, ws, bad, s);
 }
 
 }  // namespace axsq

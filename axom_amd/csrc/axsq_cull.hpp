@@ -10,9 +10,9 @@
 // box is farther than the running minimum holds no triangle the walk could
 // use, and leaving it out leaves 13 triangles and 75 nodes, and 18 and 118.
 // Forward and adjoint of 4M queries on the 81,920-triangle sphere: 33.2 ms
-// with the reference walk alone, 8.7 ms; a shape-fit iteration on 1.3M
-// triangles, 8M queries: 226 and 34.8 ms; 1,000 queries on 5,120 triangles:
-// 1.8 and 0.08 ms.
+// with the reference walk alone, 4.7 ms; a shape-fit iteration on 1.3M
+// triangles, 8M queries: 227 and 17.7 ms; 1,000 queries on 5,120 triangles:
+// 1.6 and 0.07 ms.
 //
 // Why the result is the reference walk's, bit for bit. Let s be the running
 // minimum (squared) and p the closest point when the reference checks leaf Y.
@@ -33,38 +33,62 @@
 // Leaves that change nothing may be checked by one walk and not by the
 // other; the state after each leaf that changes it is the same in both.
 //
-// Rounding. The extents contain every triangle inflated by `tau`, the
-// largest distance its computed closest point can have from it (k_cull_leaf).
-// Query coordinates enter as float pairs relative to the node's centre c, so
-// a projection is off by at most 2^-21 of |q - c| <= R (R: distance to the
-// farthest corner of the mesh's box); the walk's slack covers sqrt(3) times
-// that. Frames are orthonormal to 2^-22, covered by a relative 2^-18.
+// Rounding. All of it is in mesh coordinates: x = (q - centre) * scale in
+// float, scale a power of two that makes the mesh's diagonal 1 to 2. The
+// extents contain every triangle inflated by `tau`, the largest distance its
+// computed closest point can have from it (k_cull_leaf), and by the rounding
+// of its own projections. A query's projections are off by at most 2^-21 R
+// (R: its distance to the farthest corner of the mesh's box); the walk's slack
+// covers sqrt(3) times that. Frames are orthonormal to 2^-22, covered by a
+// relative 2^-18.
 #pragma once
+
+#include <hip/hip_fp16.h>
 
 #include "axsq_device.hpp"
 
 namespace axsq {
 
-// 128 bytes, one cache line, beside each Node64: a visit reads this record
-// alone. Extents are along w, u, v from c. (dn, dt, inv_d): the plane between
-// the two child boxes' centroids, dn the unit vector towards the right one;
-// the right child is nearer when dn . (q - c) > dt. inv_d is the inverse
-// distance of the centroids: a query so near the plane that float rounding
-// could decide reads the boxes instead.
-struct __attribute__((aligned(128))) CullNode {
-  float c[3];
-  float w[3], u[3], v[3];
-  float llo[3], lhi[3];
-  float rlo[3], rhi[3];
-  float dn[3], dt;
-  float inv_d;
+// Read alone by a visit. The walk's lanes are at different nodes, and the
+// vector L1 returns one lane's 16 bytes a cycle: with 128-byte records it was
+// busy 96% of the walk's time. So the record is 80 bytes, five loads: two of
+// the three axes (the third is their cross product), and the extents as
+// halves, rounded outward, relative to m. Extents run along w, u, w x u; m is
+// the projection of the middle M between the two child boxes' centroids.
+// (a, b): the unit vector between those centroids along w and u (it has no
+// third component), so a t_w + b t_u > 0, t the projections less m, says
+// that the right child is nearer. inv_d: the inverse distance of the
+// centroids; a query so near that plane that float rounding could decide
+// reads the boxes instead.
+struct __attribute__((aligned(16))) CullNode {
+  float w[3], u[3];
+  float m[3];
+  float a, b, inv_d;
+  uint32_t l[3], r[3];  // left / right child per axis: halves lo | hi << 16
   int32_t lc, rc;
-  int32_t pad;
 };
-static_assert(sizeof(CullNode) == 128, "CullNode is one cache line");
+static_assert(sizeof(CullNode) == 80, "CullNode is five 16-byte loads");
 
 // Queries farther than this many mesh diagonals from the mesh's farthest
 // corner go to the reference walk: tau is computed for that distance.
 constexpr double kCullReach = 4.0;
+
+// Mesh coordinates: centre and scale of the mesh's bounding box.
+struct CullSpace {
+  double o[3];
+  double scale;
+};
+
+// t: projections of mesh coordinates x less m, by the same operations in the
+// build and the walk.
+__device__ __forceinline__ void cull_project(const float w[3], const float u[3], const float m[3],
+                                             const float x[3], float t[3]) {
+  const float v0 = fmaf(w[1], u[2], -(w[2] * u[1]));
+  const float v1 = fmaf(w[2], u[0], -(w[0] * u[2]));
+  const float v2 = fmaf(w[0], u[1], -(w[1] * u[0]));
+  t[0] = fmaf(x[0], w[0], fmaf(x[1], w[1], fmaf(x[2], w[2], -m[0])));
+  t[1] = fmaf(x[0], u[0], fmaf(x[1], u[1], fmaf(x[2], u[2], -m[1])));
+  t[2] = fmaf(x[0], v0, fmaf(x[1], v1, fmaf(x[2], v2, -m[2])));
+}
 
 }  // namespace axsq

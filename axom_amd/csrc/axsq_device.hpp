@@ -69,6 +69,16 @@ __device__ __forceinline__ bool is_lt(double x, double y, double e) { return (x 
 __device__ __forceinline__ bool is_leq(double x, double y, double e) { return !is_gt(x, y, e); }
 __device__ __forceinline__ bool is_geq(double x, double y, double e) { return !is_lt(x, y, e); }
 
+// The same comparisons against zero and of two values, as one compare each.
+// is_leq(x, 0, e) is !(x > 0 && !(|x| <= e)), so !(x > e); is_geq(x, 0, e) is
+// !(x < -e); is_leq(x, y, e) is !(x - y > e), since x > y exactly when the
+// rounded difference is positive (gradual underflow) and equal infinities or a
+// NaN compare false on both sides. A closest point makes up to twelve of them:
+// the plain form costs five instructions each.
+__device__ __forceinline__ bool is_leq0(double x, double e) { return !(x > e); }
+__device__ __forceinline__ bool is_geq0(double x, double e) { return !(x < -e); }
+__device__ __forceinline__ bool is_leq_diff(double x, double y, double e) { return !(x - y > e); }
+
 // primal/geometry/Vector.hpp:543-552: the sum starts from +0.0, which turns a
 // leading -0.0 product into +0.0 exactly as the reference does.
 __device__ __forceinline__ double dot3(double a0, double a1, double a2, double b0, double b1,
@@ -251,7 +261,7 @@ __device__ __forceinline__ int closest_point(const double P[3], const double* __
   const double ap0 = P[0] - A[0], ap1 = P[1] - A[1], ap2 = P[2] - A[2];
   const double d1 = dot3(ab0, ab1, ab2, ap0, ap1, ap2);
   const double d2 = dot3(ac0, ac1, ac2, ap0, ap1, ap2);
-  if (is_leq(d1, 0.0, EPS) && is_leq(d2, 0.0, EPS)) {
+  if (is_leq0(d1, EPS) && is_leq0(d2, EPS)) {
     cp[0] = A[0]; cp[1] = A[1]; cp[2] = A[2];
     if (WANT_W) { w[0] = 1.0; w[1] = 0.0; w[2] = 0.0; }
     return 0;
@@ -259,13 +269,13 @@ __device__ __forceinline__ int closest_point(const double P[3], const double* __
   const double bp0 = P[0] - B[0], bp1 = P[1] - B[1], bp2 = P[2] - B[2];
   const double d3 = dot3(ab0, ab1, ab2, bp0, bp1, bp2);
   const double d4 = dot3(ac0, ac1, ac2, bp0, bp1, bp2);
-  if (is_geq(d3, 0.0, EPS) && is_leq(d4, d3, EPS)) {
+  if (is_geq0(d3, EPS) && is_leq_diff(d4, d3, EPS)) {
     cp[0] = B[0]; cp[1] = B[1]; cp[2] = B[2];
     if (WANT_W) { w[0] = 0.0; w[1] = 1.0; w[2] = 0.0; }
     return 1;
   }
   const double vc = d1 * d4 - d3 * d2;
-  if (is_leq(vc, 0.0, EPS) && is_geq(d1, 0.0, EPS) && is_leq(d3, 0.0, EPS) &&
+  if (is_leq0(vc, EPS) && is_geq0(d1, EPS) && is_leq0(d3, EPS) &&
       !near_eq(d1, d3, EPS)) {
     const double v = d1 / (d1 - d3);
     cp[0] = A[0] + ab0 * v; cp[1] = A[1] + ab1 * v; cp[2] = A[2] + ab2 * v;
@@ -275,20 +285,20 @@ __device__ __forceinline__ int closest_point(const double P[3], const double* __
   const double cq0 = P[0] - C[0], cq1 = P[1] - C[1], cq2 = P[2] - C[2];
   const double d5 = dot3(ab0, ab1, ab2, cq0, cq1, cq2);
   const double d6 = dot3(ac0, ac1, ac2, cq0, cq1, cq2);
-  if (is_geq(d6, 0.0, EPS) && is_leq(d5, d6, EPS)) {
+  if (is_geq0(d6, EPS) && is_leq_diff(d5, d6, EPS)) {
     cp[0] = C[0]; cp[1] = C[1]; cp[2] = C[2];
     if (WANT_W) { w[0] = 0.0; w[1] = 0.0; w[2] = 1.0; }
     return 2;
   }
   const double vb = d5 * d2 - d1 * d6;
-  if (is_leq(vb, 0.0, EPS) && is_geq(d2, 0.0, EPS) && is_leq(d6, 0.0, EPS)) {
+  if (is_leq0(vb, EPS) && is_geq0(d2, EPS) && is_leq0(d6, EPS)) {
     const double ww = d2 / (d2 - d6);
     cp[0] = A[0] + ac0 * ww; cp[1] = A[1] + ac1 * ww; cp[2] = A[2] + ac2 * ww;
     if (WANT_W) { w[0] = 1.0 - ww; w[1] = 0.0; w[2] = ww; }
     return -3;
   }
   const double va = d3 * d6 - d5 * d4;
-  if (is_leq(va, 0.0, EPS) && is_geq(d4 - d3, 0.0, EPS) && is_geq(d5 - d6, 0.0, EPS)) {
+  if (is_leq0(va, EPS) && is_geq0(d4 - d3, EPS) && is_geq0(d5 - d6, EPS)) {
     const double ww = (d4 - d3) / ((d4 - d3) + (d5 - d6));
     cp[0] = B[0] + (C[0] - B[0]) * ww;
     cp[1] = B[1] + (C[1] - B[1]) * ww;
@@ -332,18 +342,18 @@ __device__ __forceinline__ int closest_point_ilp(const double P[3], const double
   const double vb = d5 * d2 - d1 * d6;
   const double va = d3 * d6 - d5 * d4;
   int loc;
-  if (is_leq(d1, 0.0, EPS) && is_leq(d2, 0.0, EPS)) {
+  if (is_leq0(d1, EPS) && is_leq0(d2, EPS)) {
     loc = 0;
-  } else if (is_geq(d3, 0.0, EPS) && is_leq(d4, d3, EPS)) {
+  } else if (is_geq0(d3, EPS) && is_leq_diff(d4, d3, EPS)) {
     loc = 1;
-  } else if (is_leq(vc, 0.0, EPS) && is_geq(d1, 0.0, EPS) && is_leq(d3, 0.0, EPS) &&
+  } else if (is_leq0(vc, EPS) && is_geq0(d1, EPS) && is_leq0(d3, EPS) &&
              !near_eq(d1, d3, EPS)) {
     loc = -1;
-  } else if (is_geq(d6, 0.0, EPS) && is_leq(d5, d6, EPS)) {
+  } else if (is_geq0(d6, EPS) && is_leq_diff(d5, d6, EPS)) {
     loc = 2;
-  } else if (is_leq(vb, 0.0, EPS) && is_geq(d2, 0.0, EPS) && is_leq(d6, 0.0, EPS)) {
+  } else if (is_leq0(vb, EPS) && is_geq0(d2, EPS) && is_leq0(d6, EPS)) {
     loc = -3;
-  } else if (is_leq(va, 0.0, EPS) && is_geq(d4 - d3, 0.0, EPS) && is_geq(d5 - d6, 0.0, EPS)) {
+  } else if (is_leq0(va, EPS) && is_geq0(d4 - d3, EPS) && is_geq0(d5 - d6, EPS)) {
     loc = -2;
   } else {
     loc = 3;

@@ -4,6 +4,7 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <atomic>
 #include <mutex>
 #include <string>
 #include <vector>
@@ -236,6 +237,7 @@ struct axsq_sdf {
   // node: 0 not built for the current vertices, 1 built, -1 not usable
   axsq::CullNode* cull = nullptr;
   int cull_state = 0;
+  std::atomic<bool> evaluated{false};  // since the vertices were set
   std::mutex cull_mu;       // held while a call builds them
   bool walk_fixed = false;  // created with a setting of the reference walk: no culled walk
 };
@@ -248,11 +250,11 @@ int bvh_build_into(axsq_bvh* b, const double* boxes, int64_t n, double scale, in
                    hipStream_t s, int dims = 3, bool f32 = false,
                    const float* boxes_f32 = nullptr);
 void bvh_release(axsq_bvh* b);
-// Builds the oriented child boxes of a tree over `tris` (diag: the mesh's
-// diagonal) into out, n - 1 records; *bad is set when they must not be used.
-// Returns after the stream has run them.
-int cull_build(const axsq_bvh* b, const TriRec* tris, bool cells, double diag, CullNode* out,
-               int32_t* bad, hipStream_t s);
+// Builds the oriented child boxes of a tree over `tris` (cs: its mesh
+// coordinates, diag: the mesh's diagonal) into out, n - 1 records; *bad is set
+// when they must not be used. Returns after the stream has run them.
+int cull_build(const axsq_bvh* b, const TriRec* tris, bool cells, const CullSpace& cs, double diag,
+               CullNode* out, int32_t* bad, hipStream_t s);
 // n 2-D boxes (4 doubles) -> 3-D boxes with z range [0, 0] (6 doubles)
 int widen_boxes2d(const double* boxes2d, int64_t n, double* out, hipStream_t s);
 // Candidate search launches (axsq_query.hip). mode 0: count pass (keeping the

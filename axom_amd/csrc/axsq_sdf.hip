@@ -162,9 +162,10 @@ __device__ __forceinline__ void normal_term(const double T[9], int code, double 
 constexpr int kNormList = 8;
 constexpr int32_t kListOverflow = 1 << 16;
 
+template <int STRIDE = kWaveLanes, class P>
 __device__ __forceinline__ bool check_candidate_deferred(MinCand& m, const double q[3],
                                                          const double T[9], int32_t pos,
-                                                         bool compute_normal, lds_i32* list,
+                                                         bool compute_normal, P list,
                                                          int32_t& cnt) {
   constexpr double EPS = 1e-12;
   double cp[3];
@@ -197,7 +198,7 @@ __device__ __forceinline__ bool check_candidate_deferred(MinCand& m, const doubl
   }
   if (upd) {
     if (cnt < kNormList) {
-      list[cnt * kWaveLanes] = (int32_t)((uint32_t)pos * 4u + (uint32_t)(type == 1 ? 3 : loc));
+      list[cnt * STRIDE] = (int32_t)((uint32_t)pos * 4u + (uint32_t)(type == 1 ? 3 : loc));
       ++cnt;
     } else {
       cnt |= kListOverflow;
@@ -474,41 +475,56 @@ __global__ __launch_bounds__(kSdfBlock) AXSQ_SDF_WAVES_ATTR void k_sdf_eval(SdfA
 // A query is listed for the reference walk instead when a coordinate is not
 // finite or out of the reach of the boxes' tolerance, when a leaf changed the
 // state that the reference's own box test could have pruned, when its term
-// list or stack is full, or when its wave takes kCullSteps steps (queries
-// with a large part of the surface at the same distance).
+// list or stack is full. A walk still going when its wave has taken
+// CullArgs::steps node steps (queries with much of the surface at nearly one
+// distance) is handed to k_sdf_coop.
+// 4M queries on 81,920 triangles: 3.7 ms, 75 visits and 13 checks a query in
+// 175 and 33 steps a wave. The vector L1's return path is busy 90% of that
+// time and the VALUs 80%. Before: 7.4 ms with 128-byte records, a stack whose
+// entries past the 24th were private (so was its address) and the state
+// copied at each step.
 #ifndef AXSQ_CULL_LDS
-#define AXSQ_CULL_LDS 24  // stack entries a lane keeps in LDS
+#define AXSQ_CULL_LDS 16  // stack entries a lane keeps in LDS (a power of two)
 #endif
+#if defined(AXSQ_CULL_WAVES) && AXSQ_CULL_WAVES > 0
+#define AXSQ_CULL_WAVES_ATTR __attribute__((amdgpu_waves_per_eu(AXSQ_CULL_WAVES)))
+#else
+#define AXSQ_CULL_WAVES_ATTR
+#endif
+// A leaf step runs when this percentage of the walking lanes wait at a leaf
+// (4M queries on 81,920 / 2.1M triangles: 50% 6.15 / 10.1 ms a call, 35% 5.98 /
+// 9.3, 25% 6.02 / 9.0).
 #ifndef AXSQ_CULL_VOTE_PCT
-#define AXSQ_CULL_VOTE_PCT 50
+#define AXSQ_CULL_VOTE_PCT 35
 #endif
 constexpr int kCullLds = AXSQ_CULL_LDS;
-#ifndef AXSQ_CULL_STEPS
-#define AXSQ_CULL_STEPS 512
-#endif
-constexpr int32_t kCullSteps = AXSQ_CULL_STEPS;
-#ifndef AXSQ_COOP_QUERIES
-#define AXSQ_COOP_QUERIES 4096
-#endif
-constexpr int64_t kCoopQueries = AXSQ_COOP_QUERIES;  // batches walked one wave per query
-constexpr int64_t kCoopWaves = 4096;    // waves that share the long walks
+// Batches walked one wave per query from the start: 10,000 queries on 5,120 /
+// 2.1M triangles 0.19 / 0.34 ms, a lane per query first 0.26 / 0.44; 20,000
+// 0.26 / 0.49 and 0.26 / 0.52; 40,000 0.40 / 0.81 and 0.26 / 0.61.
+constexpr int64_t kCoopQueries = 16384;
+constexpr int64_t kCoopWaves = 4096;  // waves that share the long walks
 
 struct CullArgs {
   const CullNode* nodes;
+  CullSpace cs;    // mesh coordinates
   double reach2;   // squared reach: queries farther from the mesh are listed
   float cmax;      // largest coordinate of the mesh's box, by magnitude
-  int32_t* longq;  // queries whose wave took kCullSteps steps (room for nq)
+  int32_t* longq;  // queries whose walks a wave each takes over (room for nq),
+  float* longd;    // and a distance their lanes had reached, rounded up
   uint32_t* nlong;
   uint32_t* ticket;  // k_sdf_coop: the next entry of longq to walk
+  int32_t steps;     // node steps a wave of lanes takes before it hands on
 };
 
-// What the two culled walks keep per query beside the reference's state.
+// What the two culled walks keep per query beside the reference's state, in
+// mesh coordinates.
 struct CullQuery {
-  float qh[3], ql[3];  // the query as float pairs
-  float slack;         // added to the running distance
-  float a0, a1;        // order plane: decided beyond a0 + a1 / |D|
-  float thr;           // box keys above it are left out
-  bool ok;             // finite and within reach
+  float x[3];
+  float scale;   // mesh coordinates per unit
+  float slack;   // added to the running distance
+  float a0, a1;  // order plane: decided beyond a0 + a1 / |D|
+  float thr;     // box keys above it are left out
+  bool ok;       // finite and within reach
   template <bool MIXED>
   __device__ __forceinline__ void init(const double q[3], const double dom[6], const CullArgs& c) {
     // R: distance to the farthest corner of the mesh's box
@@ -518,106 +534,101 @@ struct CullQuery {
       r2 += e * e;
     }
     ok = !query_has_nan(q) && r2 <= c.reach2;
-    const float R = sqrtf((float)r2) * 1.00001f;
+    scale = (float)c.cs.scale;
+    const float R = sqrtf((float)r2) * 1.00001f * scale;
     float qmax = c.cmax;
     for (int d = 0; d < 3; ++d) {
-      qh[d] = (float)q[d];
-      ql[d] = (float)(q[d] - (double)qh[d]);
-      qmax = fmaxf(qmax, fabsf(qh[d]));
+      x[d] = (float)((q[d] - c.cs.o[d]) * c.cs.scale);
+      qmax = fmaxf(qmax, fabsf((float)q[d]));
     }
-    // 1e-6: ties (checkCandidate); 2^-19 R: projections; 2^-40 qmax: the pairs
-    slack = 1.01e-6f + R * 1.9073486e-6f + qmax * 9.0949470e-13f;
+    qmax *= scale;
+    // 1e-6: ties (checkCandidate); 2^-19 R: projections; 2^-50 qmax: q - o
+    slack = 1.01e-6f * scale + R * 1.9073486e-6f + qmax * 8.8817842e-16f;
     // a query at most a0 + a1 / |D| from a node's order plane reads the boxes:
     // FP64 right_first is decided to 2^-49 R^2 / |D| and the plane's float form
     // to 2^-20 R; the FP32 form also rounds coordinates (2^-23 of qmax)
-    a0 = MIXED ? (R + qmax) * 1.9073486e-6f : R * 9.5367432e-7f;
+    a0 = (MIXED ? R + qmax : R) * 1.9073486e-6f;
     a1 = MIXED ? (R + qmax) * R * 9.5367432e-7f : R * R * 1.7763568e-15f;
     thr = 3.402823466e38f;
   }
   __device__ __forceinline__ void bound(double sq) {
-    const float r = sqrtf((float)sq) * 1.0000003f + slack;
+    const float r = fmaf(sqrtf((float)sq) * 1.0000003f, scale, slack);
     thr = fminf(r * r * 1.0000039f, 3.402823466e38f);
   }
 };
 
-// A visit: the child box keys, links, and whether the right child is nearer
-// (only where both keys pass).
+// A visit: the child box keys, links, which children pass, and whether the
+// right one comes first (the only one that passes, or the nearer of two).
 struct CullVisit {
   float kl, kr;
   int32_t lc, rc;
-  bool right;
+  bool in_l, in_r, right;
 };
+
+// Squared distance from t to a child's extents. The subtractions take the
+// halves as they are (v_fma_mix_f32: one instruction, no conversion).
+__device__ __forceinline__ float cull_key(const uint32_t ext[3], const float t[3]) {
+  float g[3];
+#pragma unroll
+  for (int d = 0; d < 3; ++d) {
+    float lo, hi;
+    asm("v_fma_mix_f32 %0, %1, 1.0, -%2 op_sel_hi:[1,0,0]" : "=v"(lo) : "v"(ext[d]), "v"(t[d]));
+    asm("v_fma_mix_f32 %0, -%1, 1.0, %2 op_sel:[1,0,0] op_sel_hi:[1,0,0]"
+        : "=v"(hi)
+        : "v"(ext[d]), "v"(t[d]));
+    g[d] = fmaxf(fmaxf(lo, hi), 0.0f);
+  }
+  return fmaf(g[0], g[0], fmaf(g[1], g[1], g[2] * g[2]));
+}
+
 template <bool MIXED>
 __device__ __forceinline__ CullVisit cull_visit(const SdfArgs& a, const CullArgs& c,
                                                 const CullQuery& k, const double q[3],
                                                 int32_t cur) {
   const float4* p = reinterpret_cast<const float4*>(c.nodes + cur);
-  const float4 f0 = p[0], f1 = p[1], f2 = p[2], f3 = p[3], f4 = p[4], f5 = p[5], f6 = p[6],
-               f7 = p[7];
-  const float x0 = (k.qh[0] - f0.x) + k.ql[0];
-  const float x1 = (k.qh[1] - f0.y) + k.ql[1];
-  const float x2 = (k.qh[2] - f0.z) + k.ql[2];
-  const float pw = fmaf(x0, f0.w, fmaf(x1, f1.x, x2 * f1.y));
-  const float pu = fmaf(x0, f1.z, fmaf(x1, f1.w, x2 * f2.x));
-  const float pv = fmaf(x0, f2.y, fmaf(x1, f2.z, x2 * f2.w));
-  const float lw = fmaxf(fmaxf(f3.x - pw, pw - f3.w), 0.0f);
-  const float lu = fmaxf(fmaxf(f3.y - pu, pu - f4.x), 0.0f);
-  const float lv = fmaxf(fmaxf(f3.z - pv, pv - f4.y), 0.0f);
-  const float rw = fmaxf(fmaxf(f4.z - pw, pw - f5.y), 0.0f);
-  const float ru = fmaxf(fmaxf(f4.w - pu, pu - f5.z), 0.0f);
-  const float rv = fmaxf(fmaxf(f5.x - pv, pv - f5.w), 0.0f);
+  const float4 f0 = p[0], f1 = p[1], f2 = p[2];
+  const uint4 g0 = reinterpret_cast<const uint4*>(p)[3], g1 = reinterpret_cast<const uint4*>(p)[4];
+  const float w[3] = {f0.x, f0.y, f0.z}, u[3] = {f0.w, f1.x, f1.y}, m[3] = {f1.z, f1.w, f2.x};
+  float t[3];
+  cull_project(w, u, m, k.x, t);
+  const uint32_t el[3] = {g0.x, g0.y, g0.z}, er[3] = {g0.w, g1.x, g1.y};
   CullVisit v;
-  v.kl = fmaf(lw, lw, fmaf(lu, lu, lv * lv));
-  v.kr = fmaf(rw, rw, fmaf(ru, ru, rv * rv));
-  v.lc = __float_as_int(f7.y);
-  v.rc = __float_as_int(f7.z);
-  v.right = false;
-  if (v.kl <= k.thr && v.kr <= k.thr) {
-    const float sd = fmaf(x0, f6.x, fmaf(x1, f6.y, fmaf(x2, f6.z, -f6.w)));
-    v.right = sd > 0.0f;
-    if (!(fabsf(sd) > fmaf(k.a1, f7.x, k.a0))) {
-      int32_t l2, r2, flags;
-      if constexpr (MIXED) {
-        float lb[6], rb[6];
-        load_node(a.nodes32, cur, lb, rb, l2, r2, flags);
-        v.right = BoxTests<true>(q).right_first(lb, rb);
-      } else {
-        double lb[6], rb[6];
-        load_node(a.nodes, cur, lb, rb, l2, r2, flags);
-        v.right = BoxTests<false>(q).right_first(lb, rb);
-      }
+  v.kl = cull_key(el, t);
+  v.kr = cull_key(er, t);
+  v.lc = (int32_t)g1.z;
+  v.rc = (int32_t)g1.w;
+  v.in_l = v.kl <= k.thr;
+  v.in_r = v.kr <= k.thr;
+  const float sd = fmaf(f2.y, t[0], f2.z * t[1]);
+  v.right = v.in_r && (sd > 0.0f || !v.in_l);
+  if (v.in_l && v.in_r && !(fabsf(sd) > fmaf(k.a1, f2.w, k.a0))) {
+    int32_t l2, r2, flags;
+    if constexpr (MIXED) {
+      float lb[6], rb[6];
+      load_node(a.nodes32, cur, lb, rb, l2, r2, flags);
+      v.right = BoxTests<true>(q).right_first(lb, rb);
+    } else {
+      double lb[6], rb[6];
+      load_node(a.nodes, cur, lb, rb, l2, r2, flags);
+      v.right = BoxTests<false>(q).right_first(lb, rb);
     }
   }
   return v;
 }
 
-typedef __attribute__((address_space(3))) float lds_f32;
+// The pending children of a lane's walk with their box keys: a ring in LDS,
+// [entry][lane] of 8 bytes, holds the top kCullLds entries; pushing over a
+// full ring moves its oldest entry to a private array, and popping an empty
+// one brings the last of those back. The first descent pushes the depth of
+// the tree (17 to 25) before any distance is known, and what it pushed first
+// is used last, so the entries the walk works on stay in LDS. 8 KB a wave
+// admit 5 waves per SIMD; 24 entries in place (the deepest in the private
+// array) took 14 KB and 3 waves.
+typedef __attribute__((address_space(3))) uint64_t lds_u64;
 
-// LaneStackT with a box key beside each entry.
-struct KeyedStack {
-  lds_i32* node;
-  lds_f32* key;
-  int32_t spill_node[kStack - kCullLds];
-  float spill_key[kStack - kCullLds];
-  __device__ __forceinline__ void get(int32_t sp, int32_t& n, float& k) const {
-    if (sp < kCullLds) {
-      n = node[sp * kWaveLanes];
-      k = key[sp * kWaveLanes];
-    } else {
-      n = spill_node[sp - kCullLds];
-      k = spill_key[sp - kCullLds];
-    }
-  }
-  __device__ __forceinline__ void set(int32_t sp, int32_t n, float k) {
-    if (sp < kCullLds) {
-      node[sp * kWaveLanes] = n;
-      key[sp * kWaveLanes] = k;
-    } else {
-      spill_node[sp - kCullLds] = n;
-      spill_key[sp - kCullLds] = k;
-    }
-  }
-};
+__device__ __forceinline__ uint64_t stack_entry(int32_t node, float key) {
+  return (uint64_t)(uint32_t)node | ((uint64_t)__float_as_uint(key) << 32);
+}
 
 // The squared distance to the scaled box of a leaf, as the tree holds it
 // (k_tri_boxes / k_cell_boxes, box_scale with the default factor).
@@ -629,18 +640,15 @@ __device__ __forceinline__ double leaf_box_key(const double q[3], const double b
 }
 
 template <bool MIXED, bool CELLS>
-__global__ __launch_bounds__(kWaveLanes) void k_sdf_cull(SdfArgs a, CullArgs c) {
-  __shared__ int32_t s_node[kCullLds * kWaveLanes];
-  __shared__ float s_key[kCullLds * kWaveLanes];
-  __shared__ int32_t s_terms[kNormList * kWaveLanes];
+__global__ __launch_bounds__(kWaveLanes) AXSQ_CULL_WAVES_ATTR void k_sdf_cull(SdfArgs a, CullArgs c) {
+  __shared__ uint64_t s_ring[kCullLds * kWaveLanes];
   const int lane = (int)threadIdx.x;
   const int64_t t = (int64_t)blockIdx.x * kWaveLanes + lane;
   if (t >= a.npos) return;
   const int64_t i = a.order ? (int64_t)a.order[t] : t;
-  lds_i32* terms = (lds_i32*)(s_terms + lane);
-  KeyedStack todo;
-  todo.node = (lds_i32*)(s_node + lane);
-  todo.key = (lds_f32*)(s_key + lane);
+  lds_u64* ring = (lds_u64*)(s_ring + lane);
+  uint64_t deep[kStack];
+  int32_t terms[kNormList];
   const double q[3] = {a.qx[i * a.qs], a.qy[i * a.qs], a.qz[i * a.qs]};
   const bool cn = a.compute_sign != 0;
   MinCand m;
@@ -652,99 +660,103 @@ __global__ __launch_bounds__(kWaveLanes) void k_sdf_cull(SdfArgs a, CullArgs c) 
   int32_t nterms = 0;
   CullQuery k;
   k.init<MIXED>(q, a.dom, c);
-  bool listed = !k.ok, is_long = false;
-  int32_t cur = listed ? kBarrier : 0, sp = 0;
-  todo.set(0, kBarrier, 0.0f);
-  auto pop = [&]() {
-    float key;
-    do {
-      todo.get(sp, cur, key);
-      --sp;
-    } while (key > k.thr);  // the barrier's key is 0
-  };
-  for (int32_t it = 0;; ++it) {
-    const uint64_t want_node = __ballot(cur >= 0);
-    const uint64_t want_leaf = __ballot(cur < 0 && cur != kBarrier);
-    if ((want_node | want_leaf) == 0) break;
-    if (it >= kCullSteps) {
-      is_long = cur != kBarrier;
-      break;
-    }
-    const int n_node = __popcll(want_node), n_leaf = __popcll(want_leaf);
-    if (n_leaf > 0 && 100 * n_leaf >= AXSQ_CULL_VOTE_PCT * (n_node + n_leaf)) {
-      if (cur < 0 && cur != kBarrier) {
-        const int32_t pos = min(-cur - 1, a.ninner);  // a malformed tree reads no further
-        const double before = m.sq;
-        int32_t changed = 0;
-        double T[9], bx[6];
-        int32_t ntri = 1;
-        if constexpr (CELLS) ntri = reinterpret_cast<const int32_t*>(a.tris + 2 * (int64_t)pos)[19];
-        for (int e = 0; e < (CELLS ? 2 : 1); ++e) {
-          if (e >= ntri) continue;
-          const int32_t rec = CELLS ? 2 * pos + e : pos;
-          load_tri(a.tris, rec, T);
-          changed |= check_candidate_deferred(m, q, T, rec, cn, terms, nterms) ? 1 : 0;
-        }
-        if (changed) {
-          // the reference reaches this leaf whatever its earlier minima were
-          // only if the leaf's box passes at this one
-          if constexpr (CELLS) load_tri(a.tris, 2 * pos, T);
-          for (int d = 0; d < 3; ++d) {
-            bx[d] = fmin(fmin(T[d], T[3 + d]), T[6 + d]);
-            bx[3 + d] = fmax(fmax(T[d], T[3 + d]), T[6 + d]);
+  // cur: a node (>= 0), a leaf (-(pos + 1)), kBarrier when done, or below it:
+  // kListed, for the reference walk; kPop, the next entry of the stack
+  constexpr int32_t kListed = kBarrier - 1, kPop = kBarrier - 2;
+  int32_t cur = k.ok ? 0 : kListed;
+  int32_t sp = 0, base = 0;  // entries base .. sp are in the ring, below base in deep
+  ring[0] = stack_entry(kBarrier, 0.0f);
+  int32_t it = 0;
+  for (;;) {
+    uint64_t want_leaf;
+    for (;;) {
+      if (cur == kPop) {
+        uint64_t e;
+        do {
+          if (sp < base)
+            e = deep[--base];
+          else
+            e = ring[(sp & (kCullLds - 1)) * kWaveLanes];
+          --sp;
+        } while (__uint_as_float((uint32_t)(e >> 32)) > k.thr);  // the barrier's key is 0
+        cur = (int32_t)(uint32_t)e;
+      }
+      const uint64_t want_node = __ballot(cur >= 0);
+      want_leaf = __ballot(cur < 0 && cur > kBarrier);
+      const int n_node = __popcll(want_node), n_leaf = __popcll(want_leaf);
+      if (n_node == 0 || 100 * n_leaf >= AXSQ_CULL_VOTE_PCT * (n_node + n_leaf)) break;
+      if (++it > c.steps) {
+        want_leaf = 0;
+        break;
+      }
+      if (cur >= 0) {
+        const CullVisit v = cull_visit<MIXED>(a, c, k, q, min(cur, a.ninner - 1));
+        cur = v.right ? v.rc : v.lc;
+        if (v.in_l && v.in_r) {
+          ++sp;
+          if (sp - base >= kCullLds) {
+            deep[base] = ring[(base & (kCullLds - 1)) * kWaveLanes];
+            ++base;
           }
-          if constexpr (CELLS) {
-            if (ntri > 1) {
-              load_tri(a.tris, 2 * pos + 1, T);
-              for (int d = 0; d < 3; ++d) {
-                bx[d] = fmin(bx[d], fmin(fmin(T[d], T[3 + d]), T[6 + d]));
-                bx[3 + d] = fmax(bx[3 + d], fmax(fmax(T[d], T[3 + d]), T[6 + d]));
-              }
+          if (sp >= kStack) {
+            cur = kListed;
+          } else {
+            ring[(sp & (kCullLds - 1)) * kWaveLanes] =
+                stack_entry(v.right ? v.lc : v.rc, v.right ? v.kl : v.kr);
+          }
+        } else if (!v.in_l && !v.in_r) {
+          cur = kPop;
+        }
+      }
+    }
+    if (want_leaf == 0) break;
+    if (cur < 0 && cur > kBarrier) {
+      const int32_t pos = min(-cur - 1, a.ninner);
+      cur = kPop;
+      const double before = m.sq;
+      bool changed = false;
+      double T[9], bx[6];
+      int32_t ntri = 1;
+      if constexpr (CELLS) ntri = reinterpret_cast<const int32_t*>(a.tris + 2 * (int64_t)pos)[19];
+      for (int e = 0; e < (CELLS ? 2 : 1); ++e) {
+        if (e >= ntri) continue;
+        const int32_t rec = CELLS ? 2 * pos + e : pos;
+        load_tri(a.tris, rec, T);
+        changed |= check_candidate_deferred<1>(m, q, T, rec, cn, terms, nterms);
+      }
+      if (changed) {
+        // the reference reaches this leaf whatever its earlier minima were
+        // only if the leaf's box passes at this one
+        if constexpr (CELLS) load_tri(a.tris, 2 * pos, T);
+        for (int d = 0; d < 3; ++d) {
+          bx[d] = fmin(fmin(T[d], T[3 + d]), T[6 + d]);
+          bx[3 + d] = fmax(fmax(T[d], T[3 + d]), T[6 + d]);
+        }
+        if constexpr (CELLS) {
+          if (ntri > 1) {
+            load_tri(a.tris, 2 * pos + 1, T);
+            for (int d = 0; d < 3; ++d) {
+              bx[d] = fmin(bx[d], fmin(fmin(T[d], T[3 + d]), T[6 + d]));
+              bx[3 + d] = fmax(bx[3 + d], fmax(fmax(T[d], T[3 + d]), T[6 + d]));
             }
           }
-          if (!(leaf_box_key(q, bx) <= before))
-            listed = true;
-          else
-            k.bound(m.sq);
         }
-        if (listed)
-          cur = kBarrier;
-        else
-          pop();
-      }
-    } else if (cur >= 0) {
-      if (cur >= a.ninner) {  // only from a malformed tree
-        listed = true;
-        cur = kBarrier;
-      } else {
-        const CullVisit v = cull_visit<MIXED>(a, c, k, q, cur);
-        const bool in_l = v.kl <= k.thr, in_r = v.kr <= k.thr;
-        if (in_l && in_r) {
-          ++sp;
-          if (sp >= kStack) {
-            listed = true;
-            cur = kBarrier;
-          } else {
-            todo.set(sp, v.right ? v.lc : v.rc, v.right ? v.kl : v.kr);
-            cur = v.right ? v.rc : v.lc;
-          }
-        } else if (in_l || in_r) {
-          cur = in_l ? v.lc : v.rc;
-        } else {
-          pop();
-        }
+        if (!(leaf_box_key(q, bx) <= before)) cur = kListed;
+        k.bound(m.sq);
       }
     }
   }
-  if (is_long) {
-    c.longq[atomicAdd(c.nlong, 1u)] = (int32_t)i;  // one slot per query
+  if (cur != kBarrier && cur != kListed) {  // handed on
+    const uint32_t slot = atomicAdd(c.nlong, 1u);  // one per query
+    c.longq[slot] = (int32_t)i;
+    c.longd[slot] = sqrtf((float)m.sq) * 1.0000003f;
     return;
   }
-  if (listed || (nterms & kListOverflow)) {
+  if (cur == kListed || (nterms & kListOverflow)) {
     a.redo[atomicAdd(a.nredo, 1u)] = (int32_t)i;  // one slot per query
     return;
   }
-  add_terms(m.sn, a.tris, (const lds_i32*)terms, kWaveLanes, nterms);
+  add_terms(m.sn, a.tris, terms, 1, nterms);
   sdf_finish(a, i, q, m, cn);
 }
 
@@ -864,6 +876,22 @@ __global__ __launch_bounds__(kWaveLanes) void k_sdf_coop(SdfArgs a, CullArgs c, 
     CullQuery k;
     k.init<MIXED>(q, a.dom, c);
     bool listed = !k.ok;
+    // A distance `ub` known to be reached bounds the walk from its start:
+    // subtrees beyond ub + 2e-6 are left out. What they hold could still have
+    // entered the reference's pseudo-normal sum, through a chain of strictly
+    // closer points each within 1e-6 of the one before; such a chain has a
+    // member between ub + 1e-6 and ub + 2e-6 in the sum, and a query whose sum
+    // ends with one (`above`) is listed.
+    double above_sq = kDblMax;
+    bool above = false;
+    if (nall == 0) {
+      const float ub = c.longd[j];
+      if (ub < 1e15f) {
+        const double r = (double)ub + 1.0e-6;
+        above_sq = r * r;
+        k.bound(((double)ub + 1.01e-6) * ((double)ub + 1.01e-6));
+      }
+    }
     MinCand m;
     m.sq = kDblMax;
     m.p[0] = m.p[1] = m.p[2] = 0.0;
@@ -945,7 +973,10 @@ __global__ __launch_bounds__(kWaveLanes) void k_sdf_coop(SdfArgs a, CullArgs c, 
           const bool same = near_eq(dot3(e0, e1, e2, e0, e1, e2), 0., kSdfEps);
           bool upd;
           if (rsq < m.sq) {
-            if (cn && (rtype == 2 || m.type != rtype || !same)) nterms = 0;
+            if (rtype == 2 || m.type != rtype || !same) {
+              if (cn) nterms = 0;
+              above = false;
+            }
             m.sq = rsq;
             for (int d = 0; d < 3; ++d) m.p[d] = rp[d];
             m.type = rtype;
@@ -954,6 +985,7 @@ __global__ __launch_bounds__(kWaveLanes) void k_sdf_coop(SdfArgs a, CullArgs c, 
           } else {
             upd = cn && rtype != 2 && m.type == rtype && same;
           }
+          above = above || ((upd || rsq == m.sq) && rsq > above_sq);
           if (upd) {
             if (nterms < kNormList) {
               if (lane == 0)
@@ -985,7 +1017,7 @@ __global__ __launch_bounds__(kWaveLanes) void k_sdf_coop(SdfArgs a, CullArgs c, 
           left &= l >= kWaveLanes - 1 ? 0ull : ~((2ull << l) - 1);
         }
         if (listed) break;
-        if (any) k.bound(m.sq);
+        if (any && m.sq <= above_sq) k.bound(m.sq);
         continue;
       }
       // expand the inner nodes of the top entries in place
@@ -997,14 +1029,12 @@ __global__ __launch_bounds__(kWaveLanes) void k_sdf_coop(SdfArgs a, CullArgs c, 
           bad = true;
         } else {
           const CullVisit v = cull_visit<MIXED>(a, c, k, q, node);
-          const bool in_l = v.kl <= k.thr, in_r = v.kr <= k.thr;
-          both = in_l && in_r;
-          one = in_l || in_r;
-          const bool r = both ? v.right : !in_l;
-          n0 = r ? v.rc : v.lc;
-          k0 = r ? v.kr : v.kl;
-          n1 = r ? v.lc : v.rc;
-          k1 = r ? v.kl : v.kr;
+          both = v.in_l && v.in_r;
+          one = v.in_l || v.in_r;
+          n0 = v.right ? v.rc : v.lc;
+          k0 = v.right ? v.kr : v.kl;
+          n1 = v.right ? v.lc : v.rc;
+          k1 = v.right ? v.kl : v.kr;
         }
       }
       const uint64_t m_one = __ballot(one), m_both = __ballot(both);
@@ -1027,7 +1057,7 @@ __global__ __launch_bounds__(kWaveLanes) void k_sdf_coop(SdfArgs a, CullArgs c, 
       __syncthreads();
       sp = base + total;
     }
-    if (listed || (nterms & kListOverflow)) {
+    if (listed || above || (nterms & kListOverflow)) {
       if (lane == 0) a.redo[atomicAdd(a.nredo, 1u)] = (int32_t)i;
     } else {
       // the recorded terms, one lane each, added in their order
@@ -2653,26 +2683,30 @@ static int sdf_eval_reference(const axsq_sdf* h, SdfArgs a, bool list, const uin
   return AXSQ_OK;
 }
 
-// Whether a call of nq queries runs the culled walk. The boxes cost about as
-// much as a rebuild of the tree, so a call with few queries on a mesh that
-// has none yet keeps the reference walk; so do meshes so small or so large
-// that the tie radius 1e-6 or float range would count, and handles created
-// with one of the reference walk's own settings.
-static bool cull_wanted(const axsq_sdf* h, int64_t nq) {
-  if (h->walk_fixed) return false;
-  double d2 = 0.0;
-  for (int k = 0; k < 3; ++k) {
-    const double e = h->domain[3 + k] - h->domain[k];
-    d2 += e * e;
-  }
-  if (!(d2 >= 1e-4 && d2 <= 1e30)) return false;  // diagonal 0.01 .. 1e15
-  return h->cull_state == 1 || 16 * nq >= h->ntris;
+// Whether a call of nq queries runs the culled walk (`first`: the first call
+// since the mesh was set or moved, so that it would build the boxes). Even one
+// query pays for them: 1,280 to 2.1M triangles, first call with the boxes
+// built in it 0.15 to 1.5 ms, the reference walk 0.13 to 2.4 ms; 1,024 queries
+// 0.15 to 1.6 and 0.5 to 14 ms. What keeps the reference walk:
+//  - meshes so small or so large that the tie radius 1e-6 or float range would
+//    count, and handles created with one of its own settings;
+//  - on a tree large enough for early walks, a first call with some tens of
+//    thousands of queries (over 32,768 and under a 24th of the triangles):
+//    calls that alternate with updateVertices there repeat their longest walks
+//    beside the first pass and report them (axsq_sdf_last_early), which the
+//    culled walk has no use for. Speed alone would take them too (50,000
+//    queries on 1.3M triangles: 38 ms, culled 2.0 ms with the boxes), and a
+//    second call on the same vertices does.
+static bool cull_wanted(const axsq_sdf* h, double diag, int64_t nq, bool first) {
+  if (h->walk_fixed || !(diag >= 0.01 && diag <= 1e15)) return false;
+  return h->early_walks == 0 || !first || nq <= 32768 || 24 * nq >= h->ntris;
 }
 
 // The tree's oriented boxes, built by the first call that wants them after
 // the mesh was set or moved; *out stays NULL where they do not hold (a
 // triangle without a useful tolerance, no memory).
-static int sdf_cull_nodes(axsq_sdf* h, hipStream_t s, const CullNode** out) {
+static int sdf_cull_nodes(axsq_sdf* h, const CullSpace& cs, double diag, hipStream_t s,
+                          const CullNode** out) {
   std::lock_guard<std::mutex> lock(h->cull_mu);
   if (h->cull_state == 0) {
     const size_t n = (size_t)(h->bvh->n - 1);
@@ -2681,14 +2715,9 @@ static int sdf_cull_nodes(axsq_sdf* h, hipStream_t s, const CullNode** out) {
       h->cull = nullptr;
       h->cull_state = -1;
     } else {
-      double d2 = 0.0;
-      for (int k = 0; k < 3; ++k) {
-        const double e = h->domain[3 + k] - h->domain[k];
-        d2 += e * e;
-      }
       int32_t bad = 0;
       ProfRange pr("sdf_cull_build", s);
-      AXSQ_TRY(cull_build(h->bvh, h->tris, h->cells, std::sqrt(d2), h->cull, &bad, s));
+      AXSQ_TRY(cull_build(h->bvh, h->tris, h->cells, cs, diag, h->cull, &bad, s));
       h->cull_state = bad ? -1 : 1;
     }
   }
@@ -2727,7 +2756,21 @@ int sdf_eval_launch(const axsq_sdf* h, const double* x, const double* y, const d
   const bool cells = h->cells;  // quad cells: FP64 nodes, two records per leaf
   const bool mixed = (fp_mode == AXSQ_FP32_TRAVERSAL) && !cells;
   const CullNode* cull = nullptr;
-  if (!stats && cull_wanted(h, nq)) AXSQ_TRY(sdf_cull_nodes(const_cast<axsq_sdf*>(h), s, &cull));
+  CullSpace cs{};
+  double diag = 0.0;
+  for (int k = 0; k < 3; ++k) {
+    const double e = h->domain[3 + k] - h->domain[k];
+    diag += e * e;
+    cs.o[k] = 0.5 * (h->domain[k] + h->domain[3 + k]);
+  }
+  diag = std::sqrt(diag);
+  axsq_sdf* hm = const_cast<axsq_sdf*>(h);
+  if (!stats && cull_wanted(h, diag, nq, !hm->evaluated.exchange(true))) {
+    int e2 = 0;
+    (void)std::frexp(diag, &e2);  // diag in [2^(e2 - 1), 2^e2)
+    cs.scale = std::ldexp(1.0, 1 - e2);
+    AXSQ_TRY(sdf_cull_nodes(hm, cs, diag, s, &cull));
+  }
   if (h->sort_queries && nq > 4096) {
     AXSQ_TRY(ws.k0.ensure(sizeof(uint32_t) * nq));
     AXSQ_TRY(ws.v0.ensure(sizeof(uint32_t) * nq));
@@ -2754,25 +2797,29 @@ int sdf_eval_launch(const axsq_sdf* h, const double* x, const double* y, const d
   const uint64_t qkey[5] = {(uint64_t)(uintptr_t)x, (uint64_t)(uintptr_t)y,
                             (uint64_t)(uintptr_t)z, (uint64_t)stride, (uint64_t)nq};
   if (!cull) return sdf_eval_reference(h, a, false, qkey, mixed, stats, s);
-  axsq_sdf* hm = const_cast<axsq_sdf*>(h);
-  AXSQ_TRY(ws.cull_list.ensure(sizeof(int32_t) * 2 * (size_t)nq));
+  AXSQ_TRY(ws.cull_list.ensure(sizeof(int32_t) * 3 * (size_t)nq));
   AXSQ_TRY(ws.cnt.ensure(sizeof(uint32_t) * 4));
   a.redo = ws.cull_list.as<int32_t>();
   a.nredo = ws.cnt.as<uint32_t>();
   AXSQ_TRY(fill_i32(reinterpret_cast<int32_t*>(a.nredo), 0, 3, s));
   CullArgs c{};
   c.nodes = cull;
-  double d2 = 0.0;
+  c.cs = cs;
   for (int k = 0; k < 3; ++k) {
-    const double e = h->domain[3 + k] - h->domain[k];
-    d2 += e * e;
     c.cmax = std::max(c.cmax, (float)std::max(std::fabs(h->domain[k]),
                                               std::fabs(h->domain[3 + k])) * 1.00001f);
   }
-  c.reach2 = kCullReach * kCullReach * d2;
+  c.reach2 = kCullReach * kCullReach * diag * diag;
   c.longq = a.redo + nq;
+  c.longd = reinterpret_cast<float*>(c.longq + nq);
   c.nlong = a.nredo + 1;
   c.ticket = a.nredo + 2;
+  // A small batch ends with its longest lane walk, so it hands on early; a
+  // large one pays for what it hands on. 40,000 queries on 20,480 / 2.1M
+  // triangles, 128 steps 0.30 / 0.61 ms, 256 0.40 / 0.62, 512 0.57 / 0.82;
+  // 250,000: 0.43 / 1.60, 0.50 / 1.02, 0.66 / 1.20; 1.5M: 1.2 / 7.6, 1.03 /
+  // 3.8, 1.17 / 3.2.
+  c.steps = nq <= 65536 ? 128 : nq <= 786432 ? 256 : 512;
   ProfRange p1(mixed ? "sdf_eval_fp32_cull" : "sdf_eval_fp64_cull", s);
   // one lane per query, then one wave per long walk; a small batch one wave
   // per query at once
