@@ -31,7 +31,8 @@ struct BuildParams {
   double bounds[6];
   double minc[3];
   double inv[3];
-  int32_t quirky;  // some leaf box has a coordinate with min -0.0 and max +0.0 (or the reverse)
+  int32_t quirky;  // bit 0: some leaf box has a coordinate with min -0.0 and max +0.0 (or the
+                   // reverse); bit 1: some valid box has a NaN coordinate
   int32_t pad;
 };
 
@@ -58,8 +59,7 @@ __device__ __forceinline__ void invalid_box(double b[6], double big = kDblMax) {
 }
 
 // Per-block partial of k_transform: min/max of the block's valid scaled boxes
-// (6 doubles), then 1.0 if one of its boxes has a coordinate whose min and
-// max are equal zeros of opposite signs (else 0.0), then padding.
+// (6 doubles), then BuildParams::quirky's bits of its boxes, then padding.
 constexpr int kPartStride = 8;
 
 // A coordinate whose min and max compare equal but differ in their bits
@@ -112,9 +112,10 @@ __global__ __launch_bounds__(kBlock) void k_transform(const void* __restrict__ i
     store_box(out + 6 * i, b);
     if (box_valid(b))
       for (int k = 0; k < 6; ++k) acc[k] = b[k];
-    quirky = box_signed_zero_pair(b);
+    quirky = box_signed_zero_pair(b) ? 1 : 0;
+    for (int k = 0; k < 6; ++k) quirky |= __builtin_isnan(b[k]) ? 2 : 0;
   }
-  quirky = __syncthreads_or(quirky);
+  quirky = (__syncthreads_or(quirky & 1) ? 1 : 0) | (__syncthreads_or(quirky & 2) ? 2 : 0);
   for (int k = 0; k < 6; ++k) s_red[k][threadIdx.x] = acc[k];
   __syncthreads();
   for (int off = kBlock / 2; off > 0; off >>= 1) {
@@ -131,7 +132,7 @@ __global__ __launch_bounds__(kBlock) void k_transform(const void* __restrict__ i
   if (threadIdx.x == 0) {
     double* p = partials + kPartStride * (int64_t)blockIdx.x;
     for (int k = 0; k < 6; ++k) p[k] = s_red[k][0];
-    p[6] = quirky ? 1.0 : 0.0;
+    p[6] = (double)quirky;
     p[7] = 0.0;
   }
 }
@@ -142,7 +143,7 @@ __global__ __launch_bounds__(kBlock) void k_transform(const void* __restrict__ i
 // tree (f32: extent and 1 / extent rounded to float, the zero test's
 // threshold 1e-8 as a float). Run by a whole 1024-thread workgroup, which
 // finds the partials' min/max in one fixed order; thread 0 returns the
-// parameters (and whether any partial flags a signed-zero pair).
+// parameters (and the partials' quirky bits).
 __device__ void finish_params(const double* __restrict__ partials, int64_t nparts,
                               const double* __restrict__ boxes, int64_t n, int f32,
                               double (*s_red)[1024], BuildParams& out, int& quirky) {
@@ -158,9 +159,9 @@ __device__ void finish_params(const double* __restrict__ partials, int64_t npart
       const double b = pp[3 + k];
       if (b > acc[3 + k]) acc[3 + k] = b;
     }
-    q |= (pp[6] != 0.0) ? 1 : 0;
+    q |= (int)pp[6];
   }
-  quirky = __syncthreads_or(q);
+  quirky = (__syncthreads_or(q & 1) ? 1 : 0) | (__syncthreads_or(q & 2) ? 2 : 0);
   for (int k = 0; k < 6; ++k) s_red[k][t] = acc[k];
   __syncthreads();
   for (int off = 512; off > 0; off >>= 1) {
@@ -241,8 +242,8 @@ __global__ __launch_bounds__(kBlock) void k_mcodes(const double* __restrict__ bo
 }
 
 // Small builds: the bounds and constants (every workgroup finds the same
-// ones from the transform's partials; workgroup 0 writes them to host_out,
-// pinned host memory), then the
+// ones from the transform's partials; workgroup 0 writes them to prm and to
+// host_out, pinned host memory), then the
 // code of box i = 1024 * workgroup + thread, and the sort's first digit
 // histogram: workgroup g is sort tile g, so its counts go straight to
 // hist0[g * 256 + digit].
@@ -250,6 +251,7 @@ __global__ __launch_bounds__(1024) void k_mcodes_small(const double* __restrict_
                                                         int64_t nparts,
                                                         const double* __restrict__ boxes,
                                                         int64_t n, int dims, int f32,
+                                                        BuildParams* __restrict__ prm,
                                                         BuildParams* __restrict__ host_out,
                                                         uint32_t* __restrict__ keys,
                                                         uint32_t* __restrict__ vals,
@@ -267,6 +269,7 @@ __global__ __launch_bounds__(1024) void k_mcodes_small(const double* __restrict_
     if (blockIdx.x == 0) {
       p.quirky = quirky;
       p.pad = 0;
+      *prm = p;
       *host_out = p;
     }
     for (int d = 0; d < 3; ++d) {
@@ -715,6 +718,13 @@ __global__ __launch_bounds__(kRefitThreads) void k_refit_span(
 __device__ __forceinline__ float f_down(double x) { return __double2float_rd(x); }
 __device__ __forceinline__ float f_up(double x) { return __double2float_ru(x); }
 
+// The compact nodes of the searches (NULL: none), placed by the build's bounds.
+struct FindOut {
+  FindNode* nodes;
+  const BuildParams* prm;
+  int dims;
+};
+
 // emit_bvh_parents, LinearBVH.hpp:225-264, into 128-byte nodes (child links
 // are node indices, not doubled offsets) and, for mixed precision, 64-byte
 // FP32 nodes whose min corners round down and max corners round up. lc / rc:
@@ -723,7 +733,7 @@ __device__ __forceinline__ void emit_node(int32_t i, int32_t lc, int32_t rc, con
                                           const double rb[6], int32_t lo, int32_t hi,
                                           int32_t mid, Node64* __restrict__ nodes,
                                           Node32* __restrict__ nodes32,
-                                          int4* __restrict__ ranges32) {
+                                          int4* __restrict__ ranges32, const FindOut& fo) {
   Node64 nd;
   for (int k = 0; k < 6; ++k) {
     nd.l[k] = lb[k];
@@ -752,6 +762,11 @@ __device__ __forceinline__ void emit_node(int32_t i, int32_t lc, int32_t rc, con
     nodes32[i] = h;
     ranges32[i] = make_int4(lo, hi, mid, 0);
   }
+  if (fo.nodes) {
+    FindSpace fs;
+    (void)find_space(fo.prm->bounds, fs);
+    fo.nodes[i] = make_find_node(fs, fo.dims, nd.l, nd.r, nd.flags, lc, rc);
+  }
 }
 
 __global__ __launch_bounds__(kBlock) void k_emit(const double* __restrict__ leaf_boxes,
@@ -762,7 +777,7 @@ __global__ __launch_bounds__(kBlock) void k_emit(const double* __restrict__ leaf
                                                   const int32_t* __restrict__ range,
                                                   Node64* __restrict__ nodes,
                                                   Node32* __restrict__ nodes32,
-                                                  int4* __restrict__ ranges32,
+                                                  int4* __restrict__ ranges32, FindOut fo,
                                                   int32_t* __restrict__ status) {
   const int32_t i = (int32_t)(blockIdx.x * blockDim.x + threadIdx.x);
   if (i == 0) *status = 0;  // the tree's error flag starts clear
@@ -782,7 +797,7 @@ __global__ __launch_bounds__(kBlock) void k_emit(const double* __restrict__ leaf
     load_box(inner_boxes + 6 * (int64_t)rc, rb);
   }
   emit_node(i, lc, rc, lb, rb, range[3 * i], range[3 * i + 1], range[3 * i + 2], nodes, nodes32,
-            ranges32);
+            ranges32, fo);
 }
 
 constexpr int kSegLeaves = 512;  // leaves per workgroup of k_seg_local
@@ -804,8 +819,8 @@ __global__ __launch_bounds__(2 * kSegLeaves) void k_seg_local(
     int32_t* __restrict__ rchild, int32_t* __restrict__ parents, int32_t* __restrict__ range,
     const double* __restrict__ leaf_boxes, int64_t n, int64_t P, int levels,
     double* __restrict__ seg, Node64* __restrict__ nodes, Node32* __restrict__ nodes32,
-    int4* __restrict__ ranges32, int32_t* __restrict__ status, int32_t* __restrict__ deferred,
-    int32_t* __restrict__ ndeferred) {
+    int4* __restrict__ ranges32, FindOut fo, int32_t* __restrict__ status,
+    int32_t* __restrict__ deferred, int32_t* __restrict__ ndeferred) {
   __shared__ double s_box[6][2 * kSegLeaves];
   __shared__ int32_t s_rng[3][kSegLeaves];
   __shared__ int32_t s_ndef;
@@ -910,7 +925,7 @@ __global__ __launch_bounds__(2 * kSegLeaves) void k_seg_local(
   if (side == 0) {
     const int32_t lc = (lo == split) ? -(split + 1) : split;
     const int32_t rc = (hi == split + 1) ? -(split + 2) : split + 1;
-    emit_node((int32_t)k, lc, rc, bx, rb, lo, hi, split, nodes, nodes32, ranges32);
+    emit_node((int32_t)k, lc, rc, bx, rb, lo, hi, split, nodes, nodes32, ranges32, fo);
   }
 }
 
@@ -938,7 +953,7 @@ __global__ __launch_bounds__(kBlock) void k_emit_seg(
     const double* __restrict__ leaf_boxes, const double* __restrict__ seg, int64_t P,
     const int32_t* __restrict__ range, const int32_t* __restrict__ deferred,
     const int32_t* __restrict__ ndeferred, int64_t nlists, Node64* __restrict__ nodes,
-    Node32* __restrict__ nodes32, int4* __restrict__ ranges32) {
+    Node32* __restrict__ nodes32, int4* __restrict__ ranges32, FindOut fo) {
   constexpr int kHalf = kWaveLanes / 2;
   const int lane = threadIdx.x % kWaveLanes;
   const int half = lane / kHalf, hl = lane % kHalf;
@@ -1019,7 +1034,7 @@ __global__ __launch_bounds__(kBlock) void k_emit_seg(
     if (lane == 0) {
       const int32_t lc = (lo == split) ? -(split + 1) : split;
       const int32_t rc = (hi == split + 1) ? -(split + 2) : split + 1;
-      emit_node(i, lc, rc, bx, rb, lo, hi, split, nodes, nodes32, ranges32);
+      emit_node(i, lc, rc, bx, rb, lo, hi, split, nodes, nodes32, ranges32, fo);
     }
   }
 }
@@ -1102,6 +1117,7 @@ void bvh_release(axsq_bvh* b) {
   hipFree(b->nodes);
   hipFree(b->nodes32);
   hipFree(b->ranges32);
+  hipFree(b->fnodes);
   hipFree(b->leaf_boxes);
   hipFree(b->leaf_ids);
   hipFree(b->mcodes);
@@ -1110,6 +1126,7 @@ void bvh_release(axsq_bvh* b) {
   b->nodes = nullptr;
   b->nodes32 = nullptr;
   b->ranges32 = nullptr;
+  b->fnodes = nullptr;
   b->leaf_boxes = nullptr;
   b->leaf_ids = nullptr;
   b->mcodes = nullptr;
@@ -1155,13 +1172,15 @@ int bvh_build_into(axsq_bvh* b, const double* boxes, int64_t n_in, double scale,
   Workspace& ws = workspace();
 
   // (re)allocate the persistent arrays when the size changes
-  if (b->n != n || (fp_mode == AXSQ_FP32_TRAVERSAL && !b->nodes32) || !b->nodes) {
+  if (b->n != n || (fp_mode == AXSQ_FP32_TRAVERSAL && !b->nodes32) || !b->nodes ||
+      (b->searched && !b->fnodes)) {
     bvh_release(b);
     AXSQ_TRY(dmalloc(&b->nodes, (size_t)inner));
     if (fp_mode == AXSQ_FP32_TRAVERSAL) {
       AXSQ_TRY(dmalloc(&b->nodes32, (size_t)inner));
       AXSQ_TRY(dmalloc(&b->ranges32, (size_t)inner));
     }
+    if (b->searched) AXSQ_TRY(dmalloc(&b->fnodes, (size_t)inner));
     AXSQ_TRY(dmalloc(&b->leaf_boxes, 6 * (size_t)n));
     AXSQ_TRY(dmalloc(&b->leaf_ids, (size_t)n));
     AXSQ_TRY(dmalloc(&b->mcodes, (size_t)n));
@@ -1228,6 +1247,8 @@ int bvh_build_into(axsq_bvh* b, const double* boxes, int64_t n_in, double scale,
   int32_t* ndef = deferred + nseg * kSegLeaves;                      // a list and its length
   Node32* n32 = fp_mode == AXSQ_FP32_TRAVERSAL ? b->nodes32 : nullptr;
 
+  const FindOut fo{b->searched ? b->fnodes : nullptr, prm, dims};
+
   // the exact climb: refit tiers, then the nodes (counters cleared by the caller)
   auto climb_and_emit = [&]() -> int {
     k_refit_chunks<<<grid_for(n), kBlock, 0, s>>>(b->leaf_boxes, inner, lch, rch, par, rng, ib,
@@ -1242,7 +1263,7 @@ int bvh_build_into(axsq_bvh* b, const double* boxes, int64_t n_in, double scale,
       AXSQ_CHECK_HIP(hipGetLastError());
     }
     k_emit<<<grid_for(inner), kBlock, 0, s>>>(b->leaf_boxes, ib, inner, lch, rch, rng, b->nodes,
-                                              n32, b->ranges32, b->status);
+                                              n32, b->ranges32, fo, b->status);
     AXSQ_CHECK_HIP(hipGetLastError());
     return AXSQ_OK;
   };
@@ -1276,7 +1297,7 @@ int bvh_build_into(axsq_bvh* b, const double* boxes, int64_t n_in, double scale,
                                                                partials, hists + 256 * hs,
                                                                nhist - 256 * hs);
       AXSQ_CHECK_HIP(hipGetLastError());
-      k_mcodes_small<<<nkb, 1024, 0, q>>>(partials, nparts, scaled, n, dims, f32 ? 1 : 0,
+      k_mcodes_small<<<nkb, 1024, 0, q>>>(partials, nparts, scaled, n, dims, f32 ? 1 : 0, prm,
                                           host_out, keys, vals, hists);
       AXSQ_CHECK_HIP(hipGetLastError());
       AXSQ_TRY(radix_sort_small_build(keys, vals, ws.k1.as<uint32_t>(), ws.v1.as<uint32_t>(), n,
@@ -1284,10 +1305,10 @@ int bvh_build_into(axsq_bvh* b, const double* boxes, int64_t n_in, double scale,
                                       q));
       k_seg_local<<<(unsigned)nseg, 2 * kSegLeaves, 0, q>>>(
           b->mcodes, inner, lch, rch, par, rng, b->leaf_boxes, n, P, levels, seg, b->nodes, n32,
-          b->ranges32, b->status, deferred, ndef);
+          b->ranges32, fo, b->status, deferred, ndef);
       if (nseg > 1) {  // one workgroup of k_seg_local holds every node
         k_emit_seg<<<2048, kBlock, 0, q>>>(b->leaf_boxes, seg, P, rng, deferred, ndef, nseg,
-                                           b->nodes, n32, b->ranges32);
+                                           b->nodes, n32, b->ranges32, fo);
         AXSQ_CHECK_HIP(hipGetLastError());
       }
       AXSQ_CHECK_HIP(hipGetLastError());
@@ -1300,6 +1321,7 @@ int bvh_build_into(axsq_bvh* b, const double* boxes, int64_t n_in, double scale,
         (uint64_t)(uintptr_t)(f32 ? (const void*)boxes_f32 : (const void*)boxes),
         (uint64_t)n_in, (uint64_t)dims, f32 ? 1u : 0u, (uint64_t)__builtin_bit_cast(uint64_t, scale),
         (uint64_t)(uintptr_t)n32, (uint64_t)(uintptr_t)b->nodes, (uint64_t)(uintptr_t)b->ranges32,
+        (uint64_t)(uintptr_t)fo.nodes,
         (uint64_t)(uintptr_t)b->leaf_boxes, (uint64_t)(uintptr_t)b->leaf_ids,
         (uint64_t)(uintptr_t)b->mcodes, (uint64_t)(uintptr_t)b->status,
         (uint64_t)(uintptr_t)base, (uint64_t)(uintptr_t)hists, (uint64_t)(uintptr_t)keys,
@@ -1359,7 +1381,9 @@ int bvh_build_into(axsq_bvh* b, const double* boxes, int64_t n_in, double scale,
   const BuildParams& hp = *static_cast<const BuildParams*>(b->host_params);
   AXSQ_CHECK_HIP(hipStreamSynchronize(s));
   for (int k = 0; k < 6; ++k) b->bounds[k] = hp.bounds[k];
-  if (small && hp.quirky) {
+  FindSpace fs;
+  b->find_ok = b->searched && !(hp.quirky & 2) && find_space(b->bounds, fs);
+  if (small && (hp.quirky & 1)) {
     // a leaf box with a signed-zero pair: unions may depend on the grouping,
     // so the boxes come from the climb, in the SEQ order
     AXSQ_TRY(fill_i32(cnt, 0, inner, s));

@@ -194,17 +194,6 @@ __device__ __forceinline__ float unordered(uint32_t k) {
   return __uint_as_float((k & 0x80000000u) ? (k & 0x7fffffffu) : ~k);
 }
 
-// lo and hi as halves rounded outward (halves are sign and magnitude, so the
-// next one down or up is one off in its bits).
-__device__ __forceinline__ uint32_t half_range(float lo, float hi) {
-  uint16_t l = __half_as_ushort(__float2half_rn(lo)), h = __half_as_ushort(__float2half_rn(hi));
-  if (__half2float(__ushort_as_half(l)) > lo)
-    l = (l & 0x8000u) ? l + 1 : (l == 0 ? 0x8001u : l - 1);
-  if (__half2float(__ushort_as_half(h)) < hi)
-    h = (h & 0x8000u) ? (h == 0x8000u ? 1 : h - 1) : h + 1;
-  return (uint32_t)l | ((uint32_t)h << 16);
-}
-
 __device__ __forceinline__ void store_extents(CullNode* __restrict__ n, const Extents& l,
                                               const Extents& r, int32_t flags) {
   constexpr uint32_t kNone = 0xfc007c00u;  // an invalid child: from +inf to -inf

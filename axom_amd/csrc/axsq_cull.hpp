@@ -43,9 +43,8 @@
 // relative 2^-18.
 #pragma once
 
-#include <hip/hip_fp16.h>
-
 #include "axsq_device.hpp"
+#include "axsq_find.hpp"  // halves
 
 namespace axsq {
 

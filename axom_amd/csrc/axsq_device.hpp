@@ -435,11 +435,10 @@ __device__ __forceinline__ double tri_angle(const double* T, int idx) {
 }
 
 // intersect_ray_bbox_test per axis, primal/operators/detail/intersect_ray_impl.hpp:150-187,
-// with utilities::max/min (core/utilities/Utilities.hpp:80-96).
-__device__ __forceinline__ bool ray_slab(double x0, double n, double bmin, double bmax,
-                                         double& tmin, double& tmax, double eps) {
+// with utilities::max/min (core/utilities/Utilities.hpp:80-96). invn = 1.0 / n.
+__device__ __forceinline__ bool ray_slab(double x0, double n, double invn, double bmin,
+                                         double bmax, double& tmin, double& tmax, double eps) {
   if (near_eq(n, 0.0, eps)) return !((x0 < bmin) || (x0 > bmax));
-  const double invn = 1.0 / n;
   double t1 = (bmin - x0) * invn;
   double t2 = (bmax - x0) * invn;
   if (t1 > t2) {
@@ -452,13 +451,15 @@ __device__ __forceinline__ bool ray_slab(double x0, double n, double bmin, doubl
   return !(tmin > tmax);
 }
 
-// intersect_ray(Ray, Box, ip, EPS), intersect_ray_impl.hpp:321-351
-__device__ __forceinline__ bool ray_box(const double r[6], const double b[6], double eps) {
+// intersect_ray(Ray, Box, ip, EPS), intersect_ray_impl.hpp:321-351, with the
+// directions' inverses, which a walk computes once.
+__device__ __forceinline__ bool ray_box(const double r[6], const double inv[3], const double b[6],
+                                        double eps) {
   double tmin = 2.2250738585072014e-308;  // DBL_MIN: a ray, not a line
   double tmax = kDblMax;
-  bool hit = ray_slab(r[0], r[3], b[0], b[3], tmin, tmax, eps);
-  hit = hit && ray_slab(r[1], r[4], b[1], b[4], tmin, tmax, eps);
-  hit = hit && ray_slab(r[2], r[5], b[2], b[5], tmin, tmax, eps);
+  bool hit = ray_slab(r[0], r[3], inv[0], b[0], b[3], tmin, tmax, eps);
+  hit = hit && ray_slab(r[1], r[4], inv[1], b[1], b[4], tmin, tmax, eps);
+  hit = hit && ray_slab(r[2], r[5], inv[2], b[2], b[5], tmin, tmax, eps);
   return hit;
 }
 

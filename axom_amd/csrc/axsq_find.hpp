@@ -1,0 +1,193 @@
+// axsq_find.hpp -- compact nodes for the point and box searches.
+//
+// Those searches are bound by the bytes a visit reads: the lanes of a wave are
+// at different nodes, the vector L1 returns 16 bytes of one lane a cycle, and
+// a visit of the 128-byte FP64 node takes seven such reads (its FP32 form
+// four). This node takes three: both child boxes as halves, rounded outward,
+// relative to a float centre and scaled to the node's own size.
+//
+// Exactness. A candidate is a leaf whose FP64 box passes the FP64 test: a box
+// contains its children's boxes bit for bit, so a leaf that passes is reached
+// whatever its ancestors' tests. The walk here reaches every leaf whose
+// outward box passes, in the same order (left before right), and takes it at
+// once where the query is inside by more than all rounding could give
+// (kFindSure of the node's size), and after the FP64 test otherwise. So ids,
+// counts and order are those of the FP64 walk.
+//
+// Rounding. Query coordinates are taken relative to the root box's centre,
+// times a power of two (FindSpace), and split into two floats; a node's t is
+// their difference to its centre, times its scale s, in two fused steps, so
+// that it is off by at most 2^-22 near the box's faces, and by s 2^-46 from
+// the split. The build widens the extents by 2^-20 + s 2^-44. Boxes down to
+// about 2^-36 of the root box keep their own resolution.
+#pragma once
+
+#include <hip/hip_fp16.h>
+#include <math.h>
+
+#include "axsq_device.hpp"
+
+namespace axsq {
+
+// Coordinates of the searches: (x - o) * scale, the root box's longest side
+// between 1 and 2. ok: finite and in range; else the FP64 nodes are walked.
+struct FindSpace {
+  double o[3];
+  double scale;
+};
+
+__host__ __device__ inline bool find_space(const double b[6], FindSpace& fs) {
+  double ext = 0.0;
+  bool ok = true;
+  for (int d = 0; d < 3; ++d) {
+    const double e = b[3 + d] - b[d];
+    ok = ok && b[d] >= -1e100 && b[3 + d] <= 1e100 && e >= 0.0;
+    if (e > ext) ext = e;
+    fs.o[d] = 0.5 * (b[d] + b[3 + d]);
+  }
+  fs.scale = 1.0;
+  if (ext > 0.0) {
+    int e2 = 0;
+    (void)frexp(ext, &e2);
+    ok = ok && e2 > -330;
+    fs.scale = ldexp(1.0, 1 - (e2 > -330 ? e2 : -330));
+  }
+  return ok;
+}
+
+// Child boxes along x, y, z: l[d] / r[d] are halves lo | hi << 16 of
+// (X - c) * s, X in the search's coordinates, cs = -c * s. Links: an inner
+// node's index, or a leaf position with bit 31 and, where the node's scale
+// lets a test be sure, bit 30 set.
+struct __attribute__((aligned(16))) FindNode {
+  float cs[3];
+  float s;
+  uint32_t l[3], r[3];
+  uint32_t lc, rc;
+};
+static_assert(sizeof(FindNode) == 48, "FindNode is three 16-byte loads");
+
+constexpr uint32_t kFindLeaf = 0x80000000u, kFindSureBit = 0x40000000u;
+constexpr uint32_t kFindPos = 0x3fffffffu;
+constexpr uint32_t kFindEnd = kFindLeaf | kFindPos;  // no leaf has that position
+constexpr uint32_t kFindNone = 0xfc007c00u;  // an invalid child's range, from +inf to -inf
+// Inside by this much of the node's scale is inside the FP64 box: the halves
+// are off by 2^-10 at most, everything else by 2^-12.
+constexpr float kFindSure = 0.00195313f;  // 2^-9
+
+// Halves rounded outward (sign and magnitude, so the next one down or up is
+// one off in its bits).
+__device__ __forceinline__ uint32_t half_range(float lo, float hi) {
+  uint16_t l = __half_as_ushort(__float2half_rn(lo)), h = __half_as_ushort(__float2half_rn(hi));
+  if (__half2float(__ushort_as_half(l)) > lo)
+    l = (l & 0x8000u) ? l + 1 : (l == 0 ? 0x8001u : l - 1);
+  if (__half2float(__ushort_as_half(h)) < hi)
+    h = (h & 0x8000u) ? (h == 0x8000u ? 1 : h - 1) : h + 1;
+  return (uint32_t)l | ((uint32_t)h << 16);
+}
+
+// lo - t and t - hi with the halves taken as they are (v_fma_mix_f32: one
+// instruction, no conversion).
+__device__ __forceinline__ float half_lo_minus(uint32_t ext, float t) {
+  float r;
+  asm("v_fma_mix_f32 %0, %1, 1.0, -%2 op_sel_hi:[1,0,0]" : "=v"(r) : "v"(ext), "v"(t));
+  return r;
+}
+__device__ __forceinline__ float half_minus_hi(uint32_t ext, float t) {
+  float r;
+  asm("v_fma_mix_f32 %0, -%1, 1.0, %2 op_sel:[1,0,0] op_sel_hi:[1,0,0]"
+      : "=v"(r)
+      : "v"(ext), "v"(t));
+  return r;
+}
+
+// The node of children l, r (valid by `flags` bits 0 and 1) with links lc, rc
+// (inner index or -(leaf + 1)). dims 2: the z range never decides.
+__device__ __forceinline__ FindNode make_find_node(const FindSpace& fs, int dims,
+                                                   const double l[6], const double r[6],
+                                                   int32_t flags, int32_t lc, int32_t rc) {
+  FindNode n;
+  float c[3];
+  double X[2][6], m = 0.0;
+  for (int d = 0; d < 6; ++d) {
+    X[0][d] = (l[d] - fs.o[d % 3]) * fs.scale;
+    X[1][d] = (r[d] - fs.o[d % 3]) * fs.scale;
+  }
+  for (int d = 0; d < 3; ++d) {
+    const double lo = (flags & 1) ? ((flags & 2) ? fmin(X[0][d], X[1][d]) : X[0][d]) : X[1][d];
+    const double hi = (flags & 1) ? ((flags & 2) ? fmax(X[0][3 + d], X[1][3 + d]) : X[0][3 + d])
+                                  : X[1][3 + d];
+    c[d] = (flags & 3) ? (float)(0.5 * (lo + hi)) : 0.0f;
+    if ((flags & 3) && d < dims) m = fmax(m, fmax(fabs(lo - c[d]), fabs(hi - c[d])));
+  }
+  int e2 = -59;
+  if (m > 0.0) (void)frexp(m, &e2);
+  e2 = e2 < -59 ? -59 : e2 > 3 ? 3 : e2;
+  const double s = ldexp(1.0, 1 - e2);  // extents below 2
+  const double margin = 9.5367431640625e-07 + s * 5.684341886080802e-14;  // 2^-20 + s 2^-44
+  n.s = (float)s;
+  for (int d = 0; d < 3; ++d) {
+    n.cs[d] = (float)(-(double)c[d] * s);
+    for (int k = 0; k < 2; ++k) {
+      uint32_t e = kFindNone;
+      if (flags & (1 << k)) {
+        const double lo = d < dims ? (X[k][d] - (double)c[d]) * s - margin : -2.0;
+        const double hi = d < dims ? (X[k][3 + d] - (double)c[d]) * s + margin : 2.0;
+        e = half_range((float)(lo - fabs(lo) * 1e-7), (float)(hi + fabs(hi) * 1e-7));
+      }
+      if (k == 0)
+        n.l[d] = e;
+      else
+        n.r[d] = e;
+    }
+  }
+  const uint32_t sure = s <= 1073741824.0 ? kFindSureBit : 0u;  // 2^30
+  n.lc = lc >= 0 ? (uint32_t)lc : (kFindLeaf | sure | (uint32_t)(-lc - 1));
+  n.rc = rc >= 0 ? (uint32_t)rc : (kFindLeaf | sure | (uint32_t)(-rc - 1));
+  return n;
+}
+
+// A query's two corners in the search's coordinates, as float pairs (a
+// point's are equal). Far coordinates are clamped: outside every box either
+// way.
+template <bool BOX>
+struct FindQuery {
+  float lh[3], ll[3], hh[BOX ? 3 : 1], hl[BOX ? 3 : 1];
+  __device__ __forceinline__ static void split(double x, float& h, float& l) {
+    x = x > 1e30 ? 1e30 : x < -1e30 ? -1e30 : x;  // a NaN stays
+    h = (float)x;
+    l = (float)(x - (double)h);
+  }
+  __device__ __forceinline__ void init(const FindSpace& fs, const double* prim) {
+    for (int d = 0; d < 3; ++d) {
+      split((prim[d] - fs.o[d]) * fs.scale, lh[d], ll[d]);
+      if constexpr (BOX) split((prim[3 + d] - fs.o[d]) * fs.scale, hh[d], hl[d]);
+    }
+  }
+};
+
+// A visit: the largest signed distance of the query beyond a face of each
+// child box, in the node's scale (positive: outside). A point's NaN
+// coordinate drops out of the maximum: contains() passes it.
+template <bool BOX, int DIMS>
+__device__ __forceinline__ void find_visit(const FindNode* __restrict__ nodes, uint32_t cur,
+                                           const FindQuery<BOX>& q, float& gl, float& gr,
+                                           uint32_t& lc, uint32_t& rc) {
+  const float4* p = reinterpret_cast<const float4*>(nodes + cur);
+  const float4 f0 = p[0];
+  const uint4 g0 = reinterpret_cast<const uint4*>(p)[1], g1 = reinterpret_cast<const uint4*>(p)[2];
+  const float cs[3] = {f0.x, f0.y, f0.z};
+  const uint32_t el[3] = {g0.x, g0.y, g0.z}, er[3] = {g0.w, g1.x, g1.y};
+  gl = gr = -INFINITY;
+#pragma unroll
+  for (int d = 0; d < DIMS; ++d) {
+    const float tl = fmaf(q.ll[d], f0.w, fmaf(q.lh[d], f0.w, cs[d]));
+    const float th = BOX ? fmaf(q.hl[d], f0.w, fmaf(q.hh[d], f0.w, cs[d])) : tl;
+    gl = fmaxf(fmaxf(half_lo_minus(el[d], th), half_minus_hi(el[d], tl)), gl);
+    gr = fmaxf(fmaxf(half_lo_minus(er[d], th), half_minus_hi(er[d], tl)), gr);
+  }
+  lc = g1.z;
+  rc = g1.w;
+}
+
+}  // namespace axsq

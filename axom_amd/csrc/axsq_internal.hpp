@@ -12,6 +12,7 @@
 #include "axsq.h"
 #include "axsq_cull.hpp"
 #include "axsq_device.hpp"
+#include "axsq_find.hpp"
 
 namespace axsq {
 
@@ -163,6 +164,9 @@ struct axsq_bvh {
   int4* ranges32 = nullptr;         // with nodes32: each node's leaf range and split
                                     // {lo, hi, mid, 0}, so an FP32 walk reads 16 B, not
                                     // the FP64 node's 128-B line
+  axsq::FindNode* fnodes = nullptr; // n-1 compact nodes of the point and box searches
+  bool searched = true;             // built with them (not the tree inside an axsq_sdf)
+  bool find_ok = false;             // and they hold: finite boxes within find_space's range
   double* leaf_boxes = nullptr;     // n scaled leaf boxes in leaf order (AoS)
   int32_t* leaf_ids = nullptr;      // n: leaf position -> original id
   uint32_t* mcodes = nullptr;       // n sorted Morton codes
@@ -268,6 +272,7 @@ int find_launch(const axsq_bvh* b, int kind, int mode, const void* x, const void
                 const int32_t* fill_cnt, const int32_t* offsets, int32_t* cands, int32_t* stash,
                 int kstash, int32_t* stash_cnt, int32_t* over, uint32_t* nover, hipStream_t s);
 // The fill for queries with at most kstash candidates, from the kept ids.
-int stash_copy_launch(const int32_t* stash, int kstash, const int32_t* stash_cnt,
-                      const int32_t* offsets, int64_t nq, int32_t* cands, hipStream_t s);
+int stash_copy_launch(const axsq_bvh* b, const int32_t* stash, int kstash,
+                      const int32_t* stash_cnt, const int32_t* offsets, int64_t nq,
+                      int32_t* cands, hipStream_t s);
 }  // namespace axsq

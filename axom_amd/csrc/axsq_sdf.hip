@@ -565,18 +565,12 @@ struct CullVisit {
   bool in_l, in_r, right;
 };
 
-// Squared distance from t to a child's extents. The subtractions take the
-// halves as they are (v_fma_mix_f32: one instruction, no conversion).
+// Squared distance from t to a child's extents.
 __device__ __forceinline__ float cull_key(const uint32_t ext[3], const float t[3]) {
   float g[3];
 #pragma unroll
   for (int d = 0; d < 3; ++d) {
-    float lo, hi;
-    asm("v_fma_mix_f32 %0, %1, 1.0, -%2 op_sel_hi:[1,0,0]" : "=v"(lo) : "v"(ext[d]), "v"(t[d]));
-    asm("v_fma_mix_f32 %0, -%1, 1.0, %2 op_sel:[1,0,0] op_sel_hi:[1,0,0]"
-        : "=v"(hi)
-        : "v"(ext[d]), "v"(t[d]));
-    g[d] = fmaxf(fmaxf(lo, hi), 0.0f);
+    g[d] = fmaxf(fmaxf(half_lo_minus(ext[d], t[d]), half_minus_hi(ext[d], t[d])), 0.0f);
   }
   return fmaf(g[0], g[0], fmaf(g[1], g[1], g[2] * g[2]));
 }
@@ -2357,6 +2351,7 @@ int sdf_setup(axsq_sdf* h, hipStream_t s) {
     k_tri_boxes<<<grid_for(nt), kBlock, 0, s>>>(h->vx, h->vy, h->vz, h->conn, nt, boxes);
   hipError_t e = hipGetLastError();
   int rc = (e == hipSuccess) ? AXSQ_OK : AXSQ_ERR_HIP;
+  h->bvh->searched = false;
   if (rc == AXSQ_OK) rc = bvh_build_into(h->bvh, boxes, nt, 1.000123, h->fp_mode, s);
   hipFree(boxes);
   if (e != hipSuccess) set_error("k_tri_boxes: %s", hipGetErrorString(e));

@@ -1,0 +1,147 @@
+"""The point and box searches on the compact nodes (halves, scaled per node)
+give the oracle's lists, order included, over the forms a search takes: 2-D and
+3-D, double and float trees, two-array and interleaved points, both calls
+(one-call and count-then-fill), and the inputs where a rounded box could decide
+differently: queries on the faces of the scaled boxes and one step either side,
+scenes far from the origin, boxes of very different sizes, flat and invalid
+boxes, and coordinates that are not finite. Results are integers: no tolerance.
+"""
+import ctypes
+
+import numpy as np
+import pytest
+
+torch = pytest.importorskip("torch")
+
+from axom_amd import _lib as L  # noqa: E402
+from axom_amd import spin  # noqa: E402
+from oracle import oracle as orc  # noqa: E402
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+
+
+def _t(a):
+    return torch.as_tensor(np.ascontiguousarray(a), device=DEV)
+
+
+def _scene(name, n, nd, rng):
+    """(n, 2 nd) boxes: min, max."""
+    c = rng.random((n, nd))
+    h = rng.uniform(0.0005, 0.03, (n, nd))
+    if name == "far":  # boxes of 2^-20 of their distance to the origin
+        c = 1.0e6 + c
+    elif name == "scales":  # sizes and distances over twelve decades
+        s = 10.0 ** rng.uniform(-12, 0, (n, 1))
+        c, h = 0.5 + (c - 0.5) * s, h * s
+    elif name == "tiny":
+        c, h = c * 1e-90, h * 1e-90
+    elif name == "huge":  # past the range of the compact nodes
+        c, h = c * 1e120, h * 1e120
+    elif name == "flat":
+        h[rng.random(n) < 0.5, rng.integers(nd)] = 0.0
+        h[rng.random(n) < 0.2] = 0.0
+    elif name == "same":
+        c[:], h[:] = 0.5, 0.01
+    b = np.concatenate([c - h, c + h], 1)
+    if name == "invalid":
+        b[::7, 0], b[::7, nd] = b[::7, nd].copy(), b[::7, 0].copy()
+        b[::11] = [np.finfo(np.float64).max / 8] * nd + [-np.finfo(np.float64).max / 8] * nd
+        b[n - 1] = b[max(1, n - 2)]
+    elif name == "nan":
+        b[n // 2, 0] = np.nan
+    return b
+
+
+def _queries(kind, nq, nd, boxes, leaf_boxes, dtype, rng):
+    ok = np.isfinite(boxes).all(1) & (boxes[:, :nd] <= boxes[:, nd:]).all(1)
+    b = boxes[ok] if ok.any() else boxes
+    lo, hi = b[:, :nd].min(0), b[:, nd:].max(0)
+    p = lo + (hi - lo) * rng.uniform(-0.05, 1.05, (nq, nd))
+    # on the faces of the leaves' scaled boxes, and one step either side
+    k = nq // 2
+    f = leaf_boxes[rng.integers(leaf_boxes.shape[0], size=k)].reshape(k, 2, nd)
+    u = rng.random((k, nd))
+    q = f[:, 0] + (f[:, 1] - f[:, 0]) * u
+    ax, side = rng.integers(nd, size=k), rng.integers(2, size=k)
+    face = f[np.arange(k), side, ax].astype(dtype)
+    step = rng.integers(-1, 2, size=k)
+    face = np.where(step < 0, np.nextafter(face, dtype(-np.inf)),
+                    np.where(step > 0, np.nextafter(face, dtype(np.inf)), face))
+    q[np.arange(k), ax] = face
+    p[:k] = q
+    p[k] = np.inf
+    p[k + 1, 0] = -np.inf
+    p[k + 2, 0] = np.nan
+    p[k + 3] = np.nan
+    if kind == "points":
+        return p.astype(dtype)
+    h = (hi - lo) * rng.uniform(0.0, 0.02, (nq, nd)) * (rng.random((nq, 1)) < 0.7)
+    q = np.concatenate([p - h, p + h], 1)
+    q[k + 4, 0], q[k + 4, nd] = hi[0], lo[0]  # an inverted query
+    q[k + 5, nd] = np.nan
+    q[k + 6, :nd], q[k + 6, nd:] = -np.inf, np.inf
+    return q.astype(dtype)
+
+
+def _find(g, kind, prims, nq):
+    off = torch.empty(nq, dtype=torch.int32, device=DEV)
+    cnt = torch.empty_like(off)
+    f = {"points": g.findPoints, "boxes": g.findBoundingBoxes}[kind]
+    cand = f(off, cnt, nq, prims)
+    return off.cpu().numpy(), cnt.cpu().numpy(), cand.cpu().numpy()
+
+
+@pytest.mark.parametrize("scene", ["plain", "far", "scales", "tiny", "huge", "flat", "same",
+                                   "invalid", "nan"])
+@pytest.mark.parametrize("nd,dtype", [(3, np.float64), (2, np.float64), (3, np.float32),
+                                      (2, np.float32)])
+@pytest.mark.parametrize("n", [2, 3, 65, 4097])
+def test_find_on_compact_nodes(scene, nd, dtype, n):
+    rng = np.random.default_rng([n, nd, sorted(["plain", "far", "scales", "tiny", "huge", "flat",
+                                                "same", "invalid", "nan"]).index(scene)])
+    if dtype is np.float32 and scene in ("tiny", "huge"):
+        pytest.skip("outside the float range")
+    with np.errstate(over="ignore"):
+        boxes = _scene(scene, n, nd, rng).astype(dtype)
+    kw = dict(FloatType=torch.float32) if dtype is np.float32 else {}
+    g = spin.BVH(NDIMS=nd, scaleFactor=1.000123, **kw)
+    g.initialize(_t(boxes))
+    o = orc.OracleBVH(boxes, 1.000123, ndims=nd, dtype=dtype)
+    oe = o.export()
+    leaf = oe["nodes"][oe["children"] < 0]
+    if leaf.shape[1] == 6 and nd == 2:
+        leaf = leaf[:, [0, 1, 3, 4]]
+    good = np.isfinite(leaf).all(1)
+    nq = 331
+    for kind in ("points", "boxes"):
+        q = _queries(kind, nq, nd, boxes.astype(np.float64), leaf[good], dtype, rng)
+        ooff, ocnt, ocand = o.find(kind, q)
+        off, cnt, cand = _find(g, kind, _t(q), nq)
+        assert np.array_equal(cnt, ocnt), (kind, np.flatnonzero(cnt != ocnt)[:5])
+        assert np.array_equal(off, ooff) and np.array_equal(cand, ocand), kind
+        if kind == "points":  # separate coordinate arrays
+            off, cnt, cand = _find(g, kind, tuple(_t(q[:, d]) for d in range(nd)), nq)
+            assert np.array_equal(cnt, ocnt) and np.array_equal(cand, ocand)
+
+
+def test_count_then_fill_on_compact_nodes():
+    """The two-call search: the fill walks again and writes the counted lists."""
+    rng = np.random.default_rng(5)
+    boxes = _scene("plain", 20_011, 3, rng)
+    g, o = spin.BVH(_t(boxes)), orc.OracleBVH(boxes, 1.000123)
+    q = np.concatenate([boxes[:777, :3], boxes[:777, 3:]], 1)
+    ooff, ocnt, ocand = o.find("boxes", q)
+    t = _t(q)
+    n = q.shape[0]
+    off = torch.empty(n, dtype=torch.int32, device=DEV)
+    cnt = torch.empty_like(off)
+    tot = ctypes.c_int64()
+    args = (ctypes.c_void_p(t.data_ptr()), None, None, 6, n, g._tol)
+    L.check(L.lib().axsq_bvh_find_count(g._h, L.QUERY_BOXES, *args[:5], g._tol, spin._ptr(off),
+                                        spin._ptr(cnt), ctypes.byref(tot), None))
+    assert tot.value == ocand.size and np.array_equal(cnt.cpu().numpy(), ocnt)
+    cand = torch.empty(tot.value, dtype=torch.int32, device=DEV)
+    L.check(L.lib().axsq_bvh_find_fill(g._h, L.QUERY_BOXES, *args[:5], g._tol, spin._ptr(off),
+                                       spin._ptr(cnt), spin._ptr(cand), None))
+    assert np.array_equal(cand.cpu().numpy(), ocand)
