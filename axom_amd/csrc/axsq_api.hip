@@ -590,7 +590,7 @@ static int find_fill_kept(const axsq_bvh* b, int kind, const void* x, const void
                           const int32_t* offsets, const int32_t* counts, int32_t* cands,
                           int64_t nover, int kstash, hipStream_t s) {
   Workspace& ws = workspace();
-  AXSQ_TRY(stash_copy_launch(b, ws.find_stash.as<int32_t>(), kstash, ws.find_cnt.as<int32_t>(),
+  AXSQ_TRY(stash_copy_launch(b, kind, ws.find_stash.as<int32_t>(), kstash, ws.find_cnt.as<int32_t>(),
                              offsets, nq, cands, s));
   if (nover > 0)
     AXSQ_TRY(find_launch(b, kind, 2, x, y, z, stride, nover, tol, nullptr, counts, offsets,
@@ -724,7 +724,7 @@ int axsq_bvh_find_into_noalloc(const axsq_bvh* b, int kind, const double* x, con
   }
   *total = tn[0];
   if (*total == 0 || *total > capacity) return AXSQ_OK;  // too small: nothing written
-  AXSQ_TRY(stash_copy_launch(b, kept, kstash, kept_cnt, offsets, nq, candidates, s));
+  AXSQ_TRY(stash_copy_launch(b, kind, kept, kstash, kept_cnt, offsets, nq, candidates, s));
   const int64_t nover = (int64_t)(uint32_t)tn[1];
   if (nover > 0)
     AXSQ_TRY(find_launch(b, kind, 2, x, y, z, stride, nover, tol, nullptr, counts, offsets,

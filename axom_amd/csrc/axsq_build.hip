@@ -1172,11 +1172,13 @@ int bvh_build_into(axsq_bvh* b, const double* boxes, int64_t n_in, double scale,
   Workspace& ws = workspace();
 
   // (re)allocate the persistent arrays when the size changes
-  if (b->n != n || (fp_mode == AXSQ_FP32_TRAVERSAL && !b->nodes32) || !b->nodes ||
+  // the FP32 nodes are the distance walk's; a searched tree has the compact ones
+  const bool want32 = fp_mode == AXSQ_FP32_TRAVERSAL && !b->searched;
+  if (b->n != n || (want32 && !b->nodes32) || !b->nodes ||
       (b->searched && !b->fnodes)) {
     bvh_release(b);
     AXSQ_TRY(dmalloc(&b->nodes, (size_t)inner));
-    if (fp_mode == AXSQ_FP32_TRAVERSAL) {
+    if (want32) {
       AXSQ_TRY(dmalloc(&b->nodes32, (size_t)inner));
       AXSQ_TRY(dmalloc(&b->ranges32, (size_t)inner));
     }
@@ -1245,7 +1247,7 @@ int bvh_build_into(axsq_bvh* b, const double* boxes, int64_t n_in, double scale,
   double* seg = reinterpret_cast<double*>(base + off_seg);
   int32_t* deferred = reinterpret_cast<int32_t*>(base + off_def);  // per k_seg_local workgroup:
   int32_t* ndef = deferred + nseg * kSegLeaves;                      // a list and its length
-  Node32* n32 = fp_mode == AXSQ_FP32_TRAVERSAL ? b->nodes32 : nullptr;
+  Node32* n32 = want32 ? b->nodes32 : nullptr;
 
   const FindOut fo{b->searched ? b->fnodes : nullptr, prm, dims};
 

@@ -1,4 +1,4 @@
-// axsq_find.hpp -- compact nodes for the point and box searches.
+// axsq_find.hpp -- compact nodes for the searches.
 //
 // Those searches are bound by the bytes a visit reads: the lanes of a wave are
 // at different nodes, the vector L1 returns 16 bytes of one lane a cycle, and
@@ -74,6 +74,7 @@ constexpr uint32_t kFindNone = 0xfc007c00u;  // an invalid child's range, from +
 // Inside by this much of the node's scale is inside the FP64 box: the halves
 // are off by 2^-10 at most, everything else by 2^-12.
 constexpr float kFindSure = 0.00195313f;  // 2^-9
+constexpr float kFindFar = 3e38f;  // beyond every far end of a ray's interval
 
 // Halves rounded outward (sign and magnitude, so the next one down or up is
 // one off in its bits).
@@ -186,6 +187,65 @@ __device__ __forceinline__ void find_visit(const FindNode* __restrict__ nodes, u
     gl = fmaxf(fmaxf(half_lo_minus(el[d], th), half_minus_hi(el[d], tl)), gl);
     gr = fmaxf(fmaxf(half_lo_minus(er[d], th), half_minus_hi(er[d], tl)), gr);
   }
+  lc = g1.z;
+  rc = g1.w;
+}
+
+// A ray on the compact nodes. The slab test (FP64, or float in a float tree) of
+// a box inside a node's outward box passes only if this one does: in the node's
+// coordinates, with the direction over its largest component, each axis gives
+// the interval (lo - t) inv .. (hi - t) inv, widened by 2^-20 (|t| + 2) |inv|, at
+// least twice its rounding and the exact test's together; the intervals must
+// meet at or beyond the origin. An axis whose direction the reference takes as
+// zero (inv = 0 here) only tests lo <= t <= hi. The widening also covers a far
+// origin's split (2^-48 of it). init returns false for a ray outside the range
+// in which neither test overflows or underflows (t up to 2^80, inv to 2^40).
+struct FindRay {
+  float h[3], l[3];  // the origin as float pairs
+  float inv[3];      // largest |direction| / direction; 0: taken as zero
+  __device__ __forceinline__ bool init(const FindSpace& fs, const double* ray, double tol,
+                                       bool f32) {
+    const double m = fmax(fmax(fabs(ray[3]), fabs(ray[4])), fabs(ray[5]));
+    const double big = f32 ? 1e15 : 1e100;
+    bool ok = !f32 || (fs.scale <= 1e15 && fs.scale >= 1e-15);
+    for (int d = 0; d < 3; ++d) {
+      const double x = (ray[d] - fs.o[d]) * fs.scale, n = fabs(ray[3 + d]);
+      FindQuery<false>::split(x, h[d], l[d]);
+      const bool flat = f32 ? fabsf((float)ray[3 + d]) <= (float)tol : near_eq(ray[3 + d], 0.0, tol);
+      inv[d] = flat ? 0.0f : (float)(m / ray[3 + d]);
+      ok = ok && fabs(x) <= 1048576.0 && fabs(ray[d]) <= big && fabs(fs.o[d]) <= big && n <= big &&
+           (flat || (n * big >= 1.0 && m <= n * 1.099511627776e12));
+    }
+    return ok;
+  }
+};
+
+template <int DIMS>
+__device__ __forceinline__ void find_visit_ray(const FindNode* __restrict__ nodes, uint32_t cur,
+                                               const FindRay& q, bool& in_l, bool& in_r,
+                                               uint32_t& lc, uint32_t& rc) {
+  const float4* p = reinterpret_cast<const float4*>(nodes + cur);
+  const float4 f0 = p[0];
+  const uint4 g0 = reinterpret_cast<const uint4*>(p)[1], g1 = reinterpret_cast<const uint4*>(p)[2];
+  const float cs[3] = {f0.x, f0.y, f0.z};
+  const uint32_t el[3] = {g0.x, g0.y, g0.z}, er[3] = {g0.w, g1.x, g1.y};
+  float nl = 0.0f, nr = 0.0f, fl = INFINITY, fr = INFINITY;  // near and far ends
+#pragma unroll
+  for (int d = 0; d < DIMS; ++d) {
+    const bool flat = q.inv[d] == 0.0f;
+    const float ia = flat ? 1.0f : q.inv[d], ib = flat ? -1.0f : q.inv[d];
+    const float t = fmaf(q.l[d], f0.w, fmaf(q.h[d], f0.w, cs[d]));
+    const float e = fmaf(fabsf(t), 9.5367432e-7f, 1.9073487e-6f) * fabsf(ia);
+    const float a = half_lo_minus(el[d], t) * ia, b = -(half_minus_hi(el[d], t) * ib);
+    const float c = half_lo_minus(er[d], t) * ia, g = -(half_minus_hi(er[d], t) * ib);
+    // flat: a, b are the distances outside, and only their sign counts
+    nl = fmaxf(nl, flat ? (fmaxf(a, b) > e ? INFINITY : 0.0f) : fminf(a, b) - e);
+    nr = fmaxf(nr, flat ? (fmaxf(c, g) > e ? INFINITY : 0.0f) : fminf(c, g) - e);
+    fl = fminf(fl, flat ? kFindFar : fmaxf(a, b) + e);
+    fr = fminf(fr, flat ? kFindFar : fmaxf(c, g) + e);
+  }
+  in_l = !(nl > fl) && el[0] != kFindNone;
+  in_r = !(nr > fr) && er[0] != kFindNone;
   lc = g1.z;
   rc = g1.w;
 }

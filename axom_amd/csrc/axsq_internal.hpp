@@ -272,7 +272,7 @@ int find_launch(const axsq_bvh* b, int kind, int mode, const void* x, const void
                 const int32_t* fill_cnt, const int32_t* offsets, int32_t* cands, int32_t* stash,
                 int kstash, int32_t* stash_cnt, int32_t* over, uint32_t* nover, hipStream_t s);
 // The fill for queries with at most kstash candidates, from the kept ids.
-int stash_copy_launch(const axsq_bvh* b, const int32_t* stash, int kstash,
+int stash_copy_launch(const axsq_bvh* b, int kind, const int32_t* stash, int kstash,
                       const int32_t* stash_cnt, const int32_t* offsets, int64_t nq,
                       int32_t* cands, hipStream_t s);
 }  // namespace axsq

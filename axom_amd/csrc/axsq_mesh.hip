@@ -588,7 +588,7 @@ extern "C" int axsq_mesh_candidates(const double* ix, const double* iy, const do
     AXSQ_TRY(out.alloc(&pf, total));
     AXSQ_TRY(out.alloc(&ps, total));
     // the pair list (:440-458): query cell, then its candidates in order
-    AXSQ_TRY(stash_copy_launch(b, ws.find_stash.as<int32_t>(), kstash, ws.find_cnt.as<int32_t>(),
+    AXSQ_TRY(stash_copy_launch(b, AXSQ_QUERY_BOXES, ws.find_stash.as<int32_t>(), kstash, ws.find_cnt.as<int32_t>(),
                                offsets, nq, ps, s));
     if (n_over > 0)
       AXSQ_TRY(find_launch(b, AXSQ_QUERY_BOXES, 2, qbox, nullptr, nullptr, 6, n_over, tol,

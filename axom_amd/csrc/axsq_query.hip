@@ -15,8 +15,8 @@
 //
 // Points and boxes walk the compact nodes of axsq_find.hpp in either traversal
 // form (k_find_compact), unless the tree's coordinates are out of their range or
-// visits are counted (k_find, on the FP64 nodes); rays walk the FP64 nodes. Lists
-// and order are the same in all.
+// visits are counted (k_find, on the FP64 nodes); rays do too, a wave for several
+// rays (k_ray_count) or for one (k_ray_fill). Lists and order are the same in all.
 #include "axsq_internal.hpp"
 #include "axsq_traverse.hpp"
 
@@ -275,11 +275,244 @@ __global__ __launch_bounds__(kBlock) void k_find_compact(FindArgs a) {
   if (!FILL && a.stash) list_over(a, live && count > a.kstash, i);
 }
 
+// Orders a wave's LDS accesses: each wave below has its own block and LDS.
+__device__ __forceinline__ void wave_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+}
+
+__device__ __forceinline__ int lanes_below(uint64_t m) {
+  return (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32),
+                                        __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
+}
+
+// One visit for a ray: on the compact node, or, for a ray outside their range
+// (ok false), the exact test on the FP64 node.
+template <int DIMS>
+__device__ __forceinline__ void ray_visit(const FindArgs& a, uint32_t node, const FindRay& q,
+                                          bool ok, const double* prim, const double* inv,
+                                          bool& in_l, bool& in_r, uint32_t& lc, uint32_t& rc) {
+  find_visit_ray<DIMS>(a.fnodes, node, q, in_l, in_r, lc, rc);
+  if (!ok) {
+    double l[6], r[6];
+    int32_t l2, r2, flags;
+    load_node(a.nodes, (int32_t)node, l, r, l2, r2, flags);
+    in_l = (flags & 1) && pred64<AXSQ_QUERY_RAYS>(prim, inv, a.tol, l, a.f32, a.dims);
+    in_r = (flags & 2) && pred64<AXSQ_QUERY_RAYS>(prim, inv, a.tol, r, a.f32, a.dims);
+  }
+}
+
+__device__ __forceinline__ bool ray_leaf(const FindArgs& a, int32_t pos, const double* prim,
+                                         const double* inv) {
+  double lb[6];
+  load_leaf_box(a.leaf_boxes, pos, lb);
+  return valid6(lb) && pred64<AXSQ_QUERY_RAYS>(prim, inv, a.tol, lb, a.f32, a.dims);
+}
+
+// The count pass for rays. A ray's walk is long (132 visits among 100,000
+// boxes), of very different lengths, and serial, so one lane per ray leaves
+// most lanes waiting for the wave's longest walk and the chip for the longest
+// of all. Here a wave holds `rays` rays and a list of (ray, node) entries still
+// to visit, and each step its 64 lanes visit the last 64, whatever their rays;
+// reached leaves go to a second list, tested 64 at a time on their FP64 boxes.
+// A ray's leaves so come in any order; their positions are the walk's order,
+// which k_stash_copy restores. The list cannot overflow: a step takes at most
+// as many entries as leave 64 free, each adds at most one net, and near the end
+// one entry at a time walks depth first, which a tree of depth 64 fits.
+// 100,000 rays, 100,000 boxes: 965 us one lane per ray on the FP64 nodes, 662 on
+// the compact ones, 129 here.
+constexpr int kPoolRays = 32;
+template <int DIMS>
+__global__ __launch_bounds__(kWaveLanes) void k_ray_count(FindArgs a, int rays) {
+  constexpr int kItems = 512, kLeaves = 192, kFree = kStack;
+  __shared__ uint32_t s_node[kItems], s_leaf[kLeaves];
+  __shared__ uint8_t s_who[kItems], s_leaf_who[kLeaves];
+  __shared__ double s_prim[9][kPoolRays];  // origin, direction, 1 / direction
+  __shared__ float s_q[3 * DIMS][kPoolRays];
+  __shared__ int32_t s_count[kPoolRays], s_ok[kPoolRays];
+  const int lane = (int)threadIdx.x;
+  const int64_t i = (int64_t)blockIdx.x * rays + lane;
+  const bool mine = lane < rays && i < a.nq;
+  if (mine) {
+    double prim[6];
+    load_prim<AXSQ_QUERY_RAYS>(a, i, prim);
+    FindRay q;
+    s_ok[lane] = q.init(a.space, prim, a.tol, a.f32);
+    for (int d = 0; d < 6; ++d) s_prim[d][lane] = prim[d];
+    for (int d = 0; d < 3; ++d) s_prim[6 + d][lane] = 1.0 / prim[3 + d];
+    for (int d = 0; d < DIMS; ++d) {
+      s_q[3 * d][lane] = q.h[d];
+      s_q[3 * d + 1][lane] = q.l[d];
+      s_q[3 * d + 2][lane] = q.inv[d];
+    }
+    s_count[lane] = 0;
+    s_node[lane] = 0;
+    s_who[lane] = (uint8_t)lane;
+  }
+  int n = __popcll(__ballot(mine)), nl = 0;  // entries, leaves
+  const int64_t limit = (int64_t)n * a.ninner;
+  int64_t visits = 0;
+  wave_sync();
+  for (;;) {
+    if (nl >= kWaveLanes || (n == 0 && nl > 0)) {
+      const int m = nl < kWaveLanes ? nl : kWaveLanes;
+      nl -= m;
+      if (lane < m) {
+        const int who = s_leaf_who[nl + lane];
+        const int32_t pos = (int32_t)(s_leaf[nl + lane] & kFindPos);
+        double prim[6], inv[3];
+        for (int d = 0; d < 6; ++d) prim[d] = s_prim[d][who];
+        for (int d = 0; d < 3; ++d) inv[d] = s_prim[6 + d][who];
+        if (ray_leaf(a, pos, prim, inv)) {
+          const int32_t c = atomicAdd(&s_count[who], 1);
+          if (a.stash && c < a.kstash)
+            a.stash[((int64_t)blockIdx.x * rays + who) * a.kstash + c] = pos;
+        }
+      }
+      wave_sync();
+      continue;
+    }
+    if (n == 0) break;
+    const int spare = kItems - kFree - n;
+    const int k = min(min(n, kWaveLanes), max(spare, 1));
+    visits += k;
+    if (visits > limit || n >= kItems) {  // only a malformed tree
+      if (lane == 0) atomicOr(a.status, kStatusStack);
+      break;
+    }
+    n -= k;
+    bool in_l = false, in_r = false;
+    uint32_t lc = 0, rc = 0;
+    int who = 0;
+    if (lane < k) {
+      const uint32_t node = s_node[n + lane];
+      who = s_who[n + lane];
+      FindRay q;
+      for (int d = 0; d < DIMS; ++d) {
+        q.h[d] = s_q[3 * d][who];
+        q.l[d] = s_q[3 * d + 1][who];
+        q.inv[d] = s_q[3 * d + 2][who];
+      }
+      const bool ok = s_ok[who];
+      double prim[6], inv[3];
+      if (!ok) {
+        for (int d = 0; d < 6; ++d) prim[d] = s_prim[d][who];
+        for (int d = 0; d < 3; ++d) inv[d] = s_prim[6 + d][who];
+      }
+      ray_visit<DIMS>(a, node, q, ok, prim, inv, in_l, in_r, lc, rc);
+    }
+    wave_sync();  // the entries are read before their places are written
+    auto put = [&](bool in, uint32_t code, bool leaves) {
+      const bool p = in && ((code & kFindLeaf) != 0) == leaves;
+      const uint64_t m = __ballot(p);
+      if (leaves) {
+        if (p) {
+          s_leaf[nl + lanes_below(m)] = code;
+          s_leaf_who[nl + lanes_below(m)] = (uint8_t)who;
+        }
+        nl += __popcll(m);
+      } else {
+        if (p) {
+          s_node[n + lanes_below(m)] = code;
+          s_who[n + lanes_below(m)] = (uint8_t)who;
+        }
+        n += __popcll(m);
+      }
+    };
+    put(in_r, rc, false);
+    put(in_l, lc, false);
+    put(in_r, rc, true);
+    put(in_l, lc, true);
+    wave_sync();
+  }
+  const int32_t c = mine ? s_count[lane] : 0;
+  if (mine) {
+    a.counts[i] = c;
+    if (a.stash) a.stash_cnt[i] = c;
+  }
+  if (a.stash) list_over(a, mine && c > a.kstash, i);
+}
+
+// The fill pass for rays, in order: a wave per ray holds the pending nodes and
+// leaves as a list, the leftmost last; each step takes the last 64, puts each
+// node's reached children in its place and writes out the leaves that no node
+// is left of. The list is bounded as in k_ray_count.
+// 20,000 boxes in the plane, 50,000 rays of 134 candidates, the whole search:
+// 3,790 us with a lane per ray on the FP64 nodes, 540 here.
+template <int MODE, int DIMS>
+__global__ __launch_bounds__(kWaveLanes) void k_ray_fill(FindArgs a) {
+  constexpr int kItems = 512, kFree = kStack;
+  __shared__ uint32_t s_item[kItems];
+  const int lane = (int)threadIdx.x;
+  for (int64_t j = blockIdx.x; j < a.nq; j += gridDim.x) {
+    const int64_t i = (MODE == kFillListed) ? (int64_t)a.over[j] : j;
+    double prim[6], inv[3];
+    load_prim<AXSQ_QUERY_RAYS>(a, i, prim);
+    for (int d = 0; d < 3; ++d) inv[d] = 1.0 / prim[3 + d];
+    FindRay q;
+    const bool ok = q.init(a.space, prim, a.tol, a.f32);
+    const int32_t offset = a.offsets[i], room = a.fill_cnt[i];
+    int32_t count = 0, visits = 0;
+    int n = 1;
+    bool bad = false;
+    wave_sync();
+    if (lane == 0) s_item[0] = 0;
+    wave_sync();
+    while (n > 0) {
+      const int k = min(min(n, kWaveLanes), max(kItems - kFree - n, 1));
+      const uint32_t item = lane < k ? s_item[n - 1 - lane] : 0u;
+      const bool node = lane < k && !(item & kFindLeaf);
+      const uint64_t nodes = __ballot(node);
+      const int lead = nodes ? __ffsll((unsigned long long)nodes) - 1 : k;  // leading leaves
+      if (lead > 0) {
+        const int32_t pos = (int32_t)(item & kFindPos);
+        const bool take = lane < lead && ray_leaf(a, pos, prim, inv);
+        const uint64_t m = __ballot(take);
+        const int32_t c = count + lanes_below(m);
+        if (take && c < room) a.cands[offset + c] = a.leaf_ids[pos];
+        count += __popcll(m);
+      }
+      visits += __popcll(nodes);
+      if (visits > a.ninner || n >= kItems) {  // only a malformed tree
+        bad = true;
+        break;
+      }
+      uint32_t first = item, second = item;
+      bool one = lane >= lead && lane < k, two = false;
+      if (node) {
+        bool in_l, in_r;
+        uint32_t lc, rc;
+        ray_visit<DIMS>(a, item, q, ok, prim, inv, in_l, in_r, lc, rc);
+        first = in_l ? lc : rc;
+        second = rc;
+        one = in_l || in_r;
+        two = in_l && in_r;
+      }
+      const uint64_t m1 = __ballot(one), m2 = __ballot(two);
+      n += __popcll(m1) + __popcll(m2) - k;
+      const int at = n - 1 - lanes_below(m1) - lanes_below(m2);
+      wave_sync();  // the entries are read before their places are written
+      if (one) s_item[at] = first;
+      if (two) s_item[at - 1] = second;
+      wave_sync();
+    }
+    if (lane == 0 && bad) atomicOr(a.status, kStatusStack);
+    if (lane == 0 && count != room) atomicOr(a.status, kStatusFillMismatch);
+  }
+}
+
+// Queries of one wave of the copy: 64, or 16 where it also puts them in order,
+// which takes a step per id (100,000 rays: 55 us at 64, 23 at 16).
+template <bool ANY_ORDER>
+constexpr int copy_queries() { return ANY_ORDER ? 16 : 64; }
+
 // The fill pass for queries with at most kstash (<= 64) candidates: the ids of
-// the leaf positions the count pass kept, at offsets[i]. A wave whose queries have at most 4 ids
-// each copies one query per lane; otherwise it copies its 64 queries' ids one
+// the leaf positions the count pass kept, at offsets[i]; in order of position
+// (ANY_ORDER: a ray's are kept as its wave met them). A wave whose queries have at most 4 ids
+// each copies one query per lane; otherwise it copies its queries' ids one
 // query at a time, lane l taking id l, so each load and store is one
 // contiguous run, with eight queries' loads issued before their stores.
+template <bool ANY_ORDER>
 __global__ __launch_bounds__(kBlock) void k_stash_copy(const int32_t* __restrict__ stash,
                                                         int kstash,
                                                         const int32_t* __restrict__ stash_cnt,
@@ -287,31 +520,51 @@ __global__ __launch_bounds__(kBlock) void k_stash_copy(const int32_t* __restrict
                                                         const int32_t* __restrict__ leaf_ids,
                                                         int64_t nq, int32_t* __restrict__ cands) {
   const int lane = (int)__lane_id();
-  const int64_t base = (int64_t)blockIdx.x * blockDim.x + threadIdx.x - lane;  // the wave's first
+  constexpr int Q = copy_queries<ANY_ORDER>();
+  const int64_t base =
+      ((int64_t)blockIdx.x * blockDim.x + threadIdx.x - lane) / kWaveLanes * Q;  // the wave's first
   if (base >= nq) return;  // the whole wave
   const int64_t mine = base + lane;
-  const int32_t c_me = (mine < nq) ? stash_cnt[mine] : 0;
-  const int32_t o_me = (mine < nq) ? offsets[mine] : 0;
+  const bool has = lane < Q && mine < nq;
+  const int32_t c_me = has ? stash_cnt[mine] : 0;
+  const int32_t o_me = has ? offsets[mine] : 0;
   if (__ballot(c_me > 4 && c_me <= kstash) == 0) {  // few ids everywhere: a lane per query
     if (c_me <= kstash)
-      for (int32_t k = 0; k < c_me; ++k) cands[o_me + k] = leaf_ids[stash[mine * kstash + k]];
+      for (int32_t k = 0; k < c_me; ++k) {
+        const int32_t pos = stash[mine * kstash + k];
+        int32_t at = k;
+        if (ANY_ORDER) {
+          at = 0;
+          for (int32_t t = 0; t < c_me; ++t) at += stash[mine * kstash + t] < pos;
+        }
+        cands[o_me + at] = leaf_ids[pos];
+      }
     return;
   }
-  for (int j0 = 0; j0 < 64; j0 += 8) {
-    int32_t v[8], cc[8], oo[8];
+  for (int j0 = 0; j0 < Q; j0 += 8) {
+    int32_t v[8], cc[8], oo[8], at[8];
 #pragma unroll
     for (int u = 0; u < 8; ++u) {
       cc[u] = __shfl(c_me, j0 + u);
       oo[u] = __shfl(o_me, j0 + u);
       const bool take = cc[u] <= kstash && lane < cc[u];
       v[u] = take ? stash[(base + j0 + u) * kstash + lane] : 0;
+      at[u] = lane;
+    }
+    if (ANY_ORDER) {
+#pragma unroll
+      for (int u = 0; u < 8; ++u) {
+        const int c = cc[u] <= kstash ? __builtin_amdgcn_readfirstlane(cc[u]) : 0;
+        at[u] = 0;
+        for (int t = 0; t < c; ++t) at[u] += __builtin_amdgcn_readlane(v[u], t) < v[u];
+      }
     }
 #pragma unroll
     for (int u = 0; u < 8; ++u)
       if (cc[u] <= kstash && lane < cc[u]) v[u] = leaf_ids[v[u]];
 #pragma unroll
     for (int u = 0; u < 8; ++u)
-      if (cc[u] <= kstash && lane < cc[u]) cands[oo[u] + lane] = v[u];
+      if (cc[u] <= kstash && lane < cc[u]) cands[oo[u] + at[u]] = v[u];
   }
 }
 
@@ -319,7 +572,26 @@ template <int MODE>
 hipError_t launch_mode(int kind, bool compact, const FindArgs& a, hipStream_t s) {
   const unsigned g = grid_for(a.nq);
   if (kind == AXSQ_QUERY_RAYS) {
-    k_find<AXSQ_QUERY_RAYS, MODE><<<g, kBlock, 0, s>>>(a);
+    if (!compact) {
+      k_find<AXSQ_QUERY_RAYS, MODE><<<g, kBlock, 0, s>>>(a);
+    } else if constexpr (MODE == kCountPass) {
+      // few rays: fewer a wave, to fill the chip's 5,120 waves of this kernel
+      // (10,000 rays at 2 / 8 / 32 a wave: 191 / 201 / 262 us; 100,000 at 8 / 16 /
+      // 32: 289 / 299 / 284)
+      int rays = 1;
+      while (rays < kPoolRays && a.nq > (int64_t)rays * 5120) rays *= 2;
+      const unsigned gr = (unsigned)((a.nq + rays - 1) / rays);
+      if (a.dims == 2)
+        k_ray_count<2><<<gr, kWaveLanes, 0, s>>>(a, rays);
+      else
+        k_ray_count<3><<<gr, kWaveLanes, 0, s>>>(a, rays);
+    } else {
+      const unsigned gr = (unsigned)std::min<int64_t>(a.nq, int64_t(1) << 20);
+      if (a.dims == 2)
+        k_ray_fill<MODE, 2><<<gr, kWaveLanes, 0, s>>>(a);
+      else
+        k_ray_fill<MODE, 3><<<gr, kWaveLanes, 0, s>>>(a);
+    }
   } else if (kind == AXSQ_QUERY_POINTS) {
     if (!compact)
       k_find<AXSQ_QUERY_POINTS, MODE><<<g, kBlock, 0, s>>>(a);
@@ -385,13 +657,18 @@ int find_launch(const axsq_bvh* b, int kind, int mode, const void* x, const void
   return AXSQ_OK;
 }
 
-int stash_copy_launch(const axsq_bvh* b, const int32_t* stash, int kstash,
+int stash_copy_launch(const axsq_bvh* b, int kind, const int32_t* stash, int kstash,
                       const int32_t* stash_cnt, const int32_t* offsets, int64_t nq,
                       int32_t* cands, hipStream_t s) {
   if (nq <= 0) return AXSQ_OK;
   ProfRange pr("bvh_find_copy", s);
-  k_stash_copy<<<grid_for(nq), kBlock, 0, s>>>(stash, kstash, stash_cnt, offsets, b->leaf_ids, nq,
-                                              cands);
+  if (kind == AXSQ_QUERY_RAYS && b->find_ok)
+    k_stash_copy<true><<<grid_for((nq + copy_queries<true>() - 1) / copy_queries<true>() * 64),
+                         kBlock, 0, s>>>(stash, kstash, stash_cnt, offsets, b->leaf_ids, nq,
+                                         cands);
+  else
+    k_stash_copy<false><<<grid_for(nq), kBlock, 0, s>>>(stash, kstash, stash_cnt, offsets,
+                                                        b->leaf_ids, nq, cands);
   AXSQ_CHECK_HIP(hipGetLastError());
   return AXSQ_OK;
 }

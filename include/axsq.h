@@ -41,8 +41,9 @@ extern "C" {
 #define AXSQ_ERR_STATE (-5)
 
 /* Precision of the tree traversal. AXSQ_FP64 is the reference's plain form;
- * AXSQ_FP32_TRAVERSAL walks FP32 nodes whose boxes are rounded outward and
- * finishes every leaf test in FP64. */
+ * AXSQ_FP32_TRAVERSAL walks nodes whose boxes are rounded outward and finishes
+ * every leaf test in FP64. Candidate searches give the same lists in both, and
+ * walk outward-rounded compact nodes in both. */
 #define AXSQ_FP64 0
 #define AXSQ_FP32_TRAVERSAL 1
 
@@ -83,7 +84,7 @@ int axsq_release_workspace(void);
  * -> LinearBVH::buildImpl (src/axom/spin/policy/LinearBVH.hpp:193-269)
  * -> build_radix_tree (src/axom/spin/internal/linear_bvh/build_radix_tree.hpp:579-611).
  * scale: BVH::setScaleFactor (BVH.hpp:269, default 1.000123).
- * fp_mode: AXSQ_FP64, or AXSQ_FP32_TRAVERSAL to also emit FP32 nodes.
+ * fp_mode: AXSQ_FP64 or AXSQ_FP32_TRAVERSAL.
  * n may be 0 or 1 (padded to 2 leaves with an invalid box, BVH.hpp:441-464). */
 int axsq_bvh_build(axsq_bvh** out, const double* boxes, int64_t n, double scale,
                    int fp_mode, void* stream);

@@ -1,10 +1,11 @@
-"""The point and box searches on the compact nodes (halves, scaled per node)
+"""The point, box and ray searches on the compact nodes (halves, scaled per node)
 give the oracle's lists, order included, over the forms a search takes: 2-D and
 3-D, double and float trees, two-array and interleaved points, both calls
 (one-call and count-then-fill), and the inputs where a rounded box could decide
 differently: queries on the faces of the scaled boxes and one step either side,
 scenes far from the origin, boxes of very different sizes, flat and invalid
-boxes, and coordinates that are not finite. Results are integers: no tolerance.
+boxes, rays along axes, through corners, from far away and of extreme lengths,
+and coordinates that are not finite. Results are integers: no tolerance.
 """
 import ctypes
 
@@ -84,10 +85,48 @@ def _queries(kind, nq, nd, boxes, leaf_boxes, dtype, rng):
     return q.astype(dtype)
 
 
+def _rays(nq, nd, boxes, leaf_boxes, dtype, rng):
+    ok = np.isfinite(boxes).all(1) & (boxes[:, :nd] <= boxes[:, nd:]).all(1)
+    b = boxes[ok] if ok.any() else boxes
+    lo, hi = b[:, :nd].min(0), b[:, nd:].max(0)
+    ext = (hi - lo).max()
+    o = lo + (hi - lo) * rng.uniform(-0.2, 1.2, (nq, nd))
+    d = rng.normal(size=(nq, nd))
+    f = leaf_boxes[rng.integers(leaf_boxes.shape[0], size=nq)].reshape(nq, 2, nd)
+    corner = f[np.arange(nq)[:, None], rng.integers(2, size=(nq, nd)), np.arange(nd)[None]]
+    k = np.arange(nq) % 12
+    m = k == 1  # along an axis, in a face's plane or a step from it
+    ax = rng.integers(nd, size=nq)
+    d[m] = 0.0
+    d[m, ax[m]] = np.where(rng.random(m.sum()) < 0.5, 1.0, -1.0)
+    o[m] = np.where(np.arange(nd)[None] == ax[m, None], o[m], corner[m])
+    m = k == 2  # one axis taken as zero, the others not
+    d[m, ax[m]] = rng.choice([0.0, 1e-17, -1e-17, 1e-9, -3e-8], m.sum())
+    o[m, ax[m]] = corner[m, ax[m]]
+    m = (k == 3) | (k == 4)  # at a corner
+    d[m] = corner[m] - o[m]
+    m = k == 5  # from far away, at a corner
+    o[m] = o[m] + 10.0 ** rng.uniform(0, 9, (m.sum(), 1)) * ext * d[m]
+    d[m] = corner[m] - o[m]
+    m = k == 6  # from a corner
+    o[m] = corner[m]
+    d /= np.maximum(np.linalg.norm(d, axis=1, keepdims=True), 1e-300)
+    m = k == 7  # not unit
+    d[m] *= 10.0 ** rng.uniform(-25, 25, (m.sum(), 1))
+    m = k == 8
+    bad = rng.choice([np.nan, np.inf, -np.inf, 0.0, 1e-310], (m.sum(), 2 * nd))
+    q = np.concatenate([o, d], 1)
+    q[m] = np.where(rng.random(bad.shape) < 0.4, bad, q[m])
+    q[8] = np.nan
+    q[20, nd:] = 0.0
+    with np.errstate(over="ignore"):
+        return q.astype(dtype)
+
+
 def _find(g, kind, prims, nq):
     off = torch.empty(nq, dtype=torch.int32, device=DEV)
     cnt = torch.empty_like(off)
-    f = {"points": g.findPoints, "boxes": g.findBoundingBoxes}[kind]
+    f = {"points": g.findPoints, "boxes": g.findBoundingBoxes, "rays": g.findRays}[kind]
     cand = f(off, cnt, nq, prims)
     return off.cpu().numpy(), cnt.cpu().numpy(), cand.cpu().numpy()
 
@@ -123,25 +162,36 @@ def test_find_on_compact_nodes(scene, nd, dtype, n):
         if kind == "points":  # separate coordinate arrays
             off, cnt, cand = _find(g, kind, tuple(_t(q[:, d]) for d in range(nd)), nq)
             assert np.array_equal(cnt, ocnt) and np.array_equal(cand, ocand)
+    for nq in (31, 5000):
+        q = _rays(nq, nd, boxes.astype(np.float64), leaf[good], dtype, rng)
+        ooff, ocnt, ocand = o.find("rays", q)
+        off, cnt, cand = _find(g, "rays", _t(q), nq)
+        assert np.array_equal(cnt, ocnt), ("rays", nq, np.flatnonzero(cnt != ocnt)[:5])
+        assert np.array_equal(off, ooff) and np.array_equal(cand, ocand), ("rays", nq)
 
 
-def test_count_then_fill_on_compact_nodes():
+@pytest.mark.parametrize("kind", ["boxes", "rays"])
+def test_count_then_fill_on_compact_nodes(kind):
     """The two-call search: the fill walks again and writes the counted lists."""
     rng = np.random.default_rng(5)
     boxes = _scene("plain", 20_011, 3, rng)
     g, o = spin.BVH(_t(boxes)), orc.OracleBVH(boxes, 1.000123)
-    q = np.concatenate([boxes[:777, :3], boxes[:777, 3:]], 1)
-    ooff, ocnt, ocand = o.find("boxes", q)
+    q = boxes[:777]
+    if kind == "rays":
+        e = o.export()
+        q = _rays(777, 3, boxes, e["nodes"][e["children"] < 0], np.float64, rng)
+    code = {"boxes": L.QUERY_BOXES, "rays": L.QUERY_RAYS}[kind]
+    ooff, ocnt, ocand = o.find(kind, q)
     t = _t(q)
     n = q.shape[0]
     off = torch.empty(n, dtype=torch.int32, device=DEV)
     cnt = torch.empty_like(off)
     tot = ctypes.c_int64()
     args = (ctypes.c_void_p(t.data_ptr()), None, None, 6, n, g._tol)
-    L.check(L.lib().axsq_bvh_find_count(g._h, L.QUERY_BOXES, *args[:5], g._tol, spin._ptr(off),
+    L.check(L.lib().axsq_bvh_find_count(g._h, code, *args[:5], g._tol, spin._ptr(off),
                                         spin._ptr(cnt), ctypes.byref(tot), None))
     assert tot.value == ocand.size and np.array_equal(cnt.cpu().numpy(), ocnt)
     cand = torch.empty(tot.value, dtype=torch.int32, device=DEV)
-    L.check(L.lib().axsq_bvh_find_fill(g._h, L.QUERY_BOXES, *args[:5], g._tol, spin._ptr(off),
+    L.check(L.lib().axsq_bvh_find_fill(g._h, code, *args[:5], g._tol, spin._ptr(off),
                                        spin._ptr(cnt), spin._ptr(cand), None))
     assert np.array_equal(cand.cpu().numpy(), ocand)
