@@ -496,8 +496,6 @@ __device__ __forceinline__ SegBox seg_shfl_down(const SegBox& v, int off) {
   return o;
 }
 
-constexpr int kWaveLanes = 64;
-
 // propagate_aabbs, build_radix_tree.hpp:505-576: every leaf thread climbs
 // towards the root; at each node the first thread to arrive stops and the
 // second unions the two child boxes and goes on. Here the climb is split by

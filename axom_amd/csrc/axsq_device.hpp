@@ -13,6 +13,7 @@ namespace axsq {
 
 constexpr int32_t kBarrier = -2000000000;  // bvh_traverse.hpp:80
 constexpr int kStack = 64;                 // bvh_traverse.hpp:79
+constexpr int kWaveLanes = 64;
 constexpr double kDblMax = 1.7976931348623157e308;
 
 struct Box {

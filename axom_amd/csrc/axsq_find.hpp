@@ -191,6 +191,17 @@ __device__ __forceinline__ void find_visit(const FindNode* __restrict__ nodes, u
   rc = g1.w;
 }
 
+// Orders a wave's LDS accesses among its lanes (blocks of one wave).
+__device__ __forceinline__ void wave_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+}
+
+__device__ __forceinline__ int lanes_below(uint64_t m) {
+  return (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32),
+                                        __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
+}
+
 // A ray on the compact nodes. The slab test (FP64, or float in a float tree) of
 // a box inside a node's outward box passes only if this one does: in the node's
 // coordinates, with the direction over its largest component, each axis gives
@@ -248,6 +259,132 @@ __device__ __forceinline__ void find_visit_ray(const FindNode* __restrict__ node
   in_r = !(nr > fr) && er[0] != kFindNone;
   lc = g1.z;
   rc = g1.w;
+}
+
+// Several queries' walks by one wave, in any order: a list of (query, node)
+// entries still to visit, of which each step's 64 lanes take the last 64,
+// whatever their queries, and a list of reached leaves, taken 64 at a time.
+// visit(node, query, in_l, in_r, lc, rc) and leaf(leaf position, query). The
+// list cannot overflow: a step takes at most as many entries as leave kFree
+// free, each adds at most one net, and near the end one entry at a time walks
+// depth first, which a tree of kStack levels fits. False: a malformed tree.
+struct FindPool {
+  static constexpr int kItems = 512, kLeaves = 192, kFree = kStack;
+  uint32_t node[kItems], leaf[kLeaves];
+  uint8_t who[kItems], leaf_who[kLeaves];
+};
+
+// `mine`: this lane's query takes part (query = lane).
+template <class Visit, class Leaf>
+__device__ __forceinline__ bool find_pooled(FindPool& l, bool mine, int32_t ninner, Visit&& visit,
+                                            Leaf&& take) {
+  const int lane = (int)__lane_id();
+  const uint64_t has = __ballot(mine);
+  if (mine) {
+    l.node[lanes_below(has)] = 0;
+    l.who[lanes_below(has)] = (uint8_t)lane;
+  }
+  int n = __popcll(has), nl = 0;  // entries, leaves
+  const int64_t limit = (int64_t)n * ninner;
+  int64_t visits = 0;
+  wave_sync();
+  for (;;) {
+    if (nl >= kWaveLanes || (n == 0 && nl > 0)) {
+      const int m = nl < kWaveLanes ? nl : kWaveLanes;
+      nl -= m;
+      if (lane < m) take((int32_t)(l.leaf[nl + lane] & kFindPos), (int)l.leaf_who[nl + lane]);
+      wave_sync();
+      continue;
+    }
+    if (n == 0) return true;
+    const int k = min(min(n, kWaveLanes), max(FindPool::kItems - FindPool::kFree - n, 1));
+    visits += k;
+    if (visits > limit || n >= FindPool::kItems) return false;
+    n -= k;
+    bool in_l = false, in_r = false;
+    uint32_t lc = 0, rc = 0;
+    int who = 0;
+    if (lane < k) {
+      who = l.who[n + lane];
+      visit(l.node[n + lane], who, in_l, in_r, lc, rc);
+    }
+    wave_sync();  // the entries are read before their places are written
+    auto put = [&](bool in, uint32_t code, bool leaves) {
+      const bool t = in && ((code & kFindLeaf) != 0) == leaves;
+      const uint64_t m = __ballot(t);
+      if (leaves) {
+        if (t) {
+          l.leaf[nl + lanes_below(m)] = code;
+          l.leaf_who[nl + lanes_below(m)] = (uint8_t)who;
+        }
+        nl += __popcll(m);
+      } else {
+        if (t) {
+          l.node[n + lanes_below(m)] = code;
+          l.who[n + lanes_below(m)] = (uint8_t)who;
+        }
+        n += __popcll(m);
+      }
+    };
+    put(in_r, rc, false);
+    put(in_l, lc, false);
+    put(in_r, rc, true);
+    put(in_l, lc, true);
+    wave_sync();
+  }
+}
+
+// One query's walk by a wave, in the walk's order: the pending nodes and
+// leaves as a list, the leftmost last; each step takes the last 64, puts each
+// node's reached children in its place and hands out the leaves that no node is
+// left of. test(leaf position) is asked of those, hit(rank, leaf position)
+// called for the ones that pass; returns their number, -1 for a malformed
+// tree. The list is bounded as above.
+constexpr int kOrderedItems = 512;
+template <class Visit, class Test, class Hit>
+__device__ __forceinline__ int32_t find_ordered(uint32_t* items, int32_t ninner, Visit&& visit,
+                                                Test&& test, Hit&& hit) {
+  const int lane = (int)__lane_id();
+  int32_t count = 0, visits = 0;
+  int n = 1;
+  wave_sync();
+  if (lane == 0) items[0] = 0;
+  wave_sync();
+  while (n > 0) {
+    const int k = min(min(n, kWaveLanes), max(kOrderedItems - kStack - n, 1));
+    const uint32_t item = lane < k ? items[n - 1 - lane] : 0u;
+    const bool node = lane < k && !(item & kFindLeaf);
+    const uint64_t nodes = __ballot(node);
+    const int lead = nodes ? __ffsll((unsigned long long)nodes) - 1 : k;  // leading leaves
+    if (lead > 0) {
+      const int32_t pos = (int32_t)(item & kFindPos);
+      const bool pass = lane < lead && test(pos);
+      const uint64_t m = __ballot(pass);
+      if (pass) hit(count + lanes_below(m), pos);
+      count += __popcll(m);
+    }
+    visits += __popcll(nodes);
+    if (visits > ninner || n >= kOrderedItems) return -1;
+    uint32_t first = item, second = item;
+    bool one = lane >= lead && lane < k, two = false;
+    if (node) {
+      bool in_l, in_r;
+      uint32_t lc, rc;
+      visit(item, in_l, in_r, lc, rc);
+      first = in_l ? lc : rc;
+      second = rc;
+      one = in_l || in_r;
+      two = in_l && in_r;
+    }
+    const uint64_t m1 = __ballot(one), m2 = __ballot(two);
+    n += __popcll(m1) + __popcll(m2) - k;
+    const int at = n - 1 - lanes_below(m1) - lanes_below(m2);
+    wave_sync();  // the entries are read before their places are written
+    if (one) items[at] = first;
+    if (two) items[at - 1] = second;
+    wave_sync();
+  }
+  return count;
 }
 
 }  // namespace axsq

@@ -6,10 +6,10 @@
 // for every box (count, scan, fill of all candidates), keeps the pairs i < j
 // and tests them. Here the triangle test is the traversal's leaf action
 // (the custom leaf action of quest/examples/quest_bvh_two_pass.cpp:144-232):
-// one lane per triangle walks the tree with its box and tests each reached
-// triangle j > i on the spot, keeping the first kPairSlots hits. A scan of the
-// hit counts places every triangle's pairs; triangles with more hits walk
-// again to write them all. The candidate lists are never stored. The output
+// triangle i's box walks the tree and each reached triangle j > i is tested on
+// the spot, keeping kPairSlots hits of i. A scan of the hit counts places every
+// triangle's pairs; triangles with more hits walk again to write them all. The
+// candidate lists are never stored. The output
 // order is the sequential path's: pairs grouped by the first triangle, the
 // second in the first's BVH traversal order; degenerate indices ascending.
 #include <hip/hip_runtime.h>
@@ -34,6 +34,7 @@ __global__ __launch_bounds__(kBlock) void k_tri_setup(const double* __restrict__
                                                       double* __restrict__ tri,
                                                       double* __restrict__ boxes,
                                                       int32_t* __restrict__ degen,
+                                                      int32_t* __restrict__ npair,
                                                       int32_t* __restrict__ status) {
   const int64_t c = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (c >= n) return;
@@ -60,6 +61,7 @@ __global__ __launch_bounds__(kBlock) void k_tri_setup(const double* __restrict__
   degen[c] = near_eq(0.5 * sqrt(dot3(nrm[0], nrm[1], nrm[2], nrm[0], nrm[1], nrm[2])), 0.0, 1.0e-12)
                  ? 1
                  : 0;
+  npair[c] = 0;
   for (int k = 0; k < 9; ++k) tri[9 * c + k] = t[k];
   for (int k = 0; k < 6; ++k) boxes[6 * c + k] = b[k];
 }
@@ -78,16 +80,19 @@ struct IsectArgs {
   int64_t n;
   double eps;
   int32_t* npair;  // hits per triangle
-  int32_t* slots;  // kPairSlots per triangle
+  int32_t* slots;  // kPairSlots per triangle: the hits' leaf positions
   const int32_t* poff;
   int32_t* first;
   int32_t* second;
+  int32_t* more;    // triangles with more hits than slots, and their number
+  uint32_t* nmore;
   int32_t* status;
 };
 
 // One walk of triangle i's box through the tree (BoundingBox::intersectsWith,
-// BVH.hpp:558-560, as findBoundingBoxes tests it) that calls hit(j) for each
-// reached triangle j > i that intersects triangle i (boundary excluded).
+// BVH.hpp:558-560, as findBoundingBoxes tests it) that calls hit(j, j's leaf
+// position) for each reached triangle j > i that intersects triangle i (boundary
+// excluded).
 template <class Hit>
 __device__ __forceinline__ void isect_walk(const IsectArgs& a, int64_t i, lds_i32* stk, Hit&& hit) {
   double prim[6];
@@ -108,140 +113,181 @@ __device__ __forceinline__ void isect_walk(const IsectArgs& a, int64_t i, lds_i3
         const double* tj = a.tri + 9 * (int64_t)j;
         if (tri_tri_intersect(a0, a1, a2, load_v3(tj), load_v3(tj + 3), load_v3(tj + 6), false,
                               a.eps))
-          hit(j);
+          hit(j, pos);
       });
   if (v < 0) atomicOr(a.status, 1);
 }
 
-// Walk 1: count every triangle's hits, keep the first kPairSlots. Lane p of the
-// launch takes the triangle at leaf position p, so that a wave's 64 boxes are
-// neighbours in the tree (in mesh order they can be anywhere). On the compact
-// nodes the walk visits while few lanes wait at a leaf, as in k_sdf_cull: a
-// leaf step is a triangle test, which costs every lane of the wave its
-// instructions.
-// 2.6M triangles, two crossing noisy spheres: 4.1 ms in mesh order on the FP64
-// nodes, 3.4 here.
-template <bool COMPACT>
+// Whether triangle f's corner box meets the scaled box of triangle s, at leaf
+// position sp, and the triangles intersect.
+__device__ __forceinline__ bool isect_test(const IsectArgs& a, int32_t f, int32_t s, int32_t sp) {
+  const double* u = a.boxes + 6 * (int64_t)f;
+  const double* b = a.leaf_boxes + 6 * (int64_t)sp;
+  if (!((u[3] >= b[0] && u[0] <= b[3]) && (u[4] >= b[1] && u[1] <= b[4]) &&
+        (u[5] >= b[2] && u[2] <= b[5])))
+    return false;
+  const double* ti = a.tri + 9 * (int64_t)f;
+  const double* tj = a.tri + 9 * (int64_t)s;
+  return tri_tri_intersect(load_v3(ti), load_v3(ti + 3), load_v3(ti + 6), load_v3(tj),
+                           load_v3(tj + 3), load_v3(tj + 6), false, a.eps);
+}
+
+// Walk 1 where the compact nodes cannot serve: a lane per triangle.
 __global__ __launch_bounds__(kBlock) void k_isect_count(IsectArgs a) {
-  __shared__ int32_t s_stack[COMPACT ? 16 * kBlock : stack_lds_words(kBlock)];
+  __shared__ int32_t s_stack[stack_lds_words(kBlock)];
   const int64_t p = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (p >= a.n) return;
   const int64_t i = a.n > 1 ? (int64_t)a.leaf_ids[p] : 0;
   int32_t c = 0;
-  auto hit = [&](int32_t j) {
-    if (c < kPairSlots) a.slots[kPairSlots * i + c] = j;
+  isect_walk(a, i, lane_stack_base(s_stack), [&](int32_t, int32_t pos) {
+    if (c < kPairSlots) a.slots[kPairSlots * i + c] = pos;
     ++c;
-  };
-  if constexpr (!COMPACT) {
-    isect_walk(a, i, lane_stack_base(s_stack), hit);
-  } else {
-    constexpr int kRing = 16;
-    typedef __attribute__((address_space(3))) uint32_t lds_u32;
-    lds_u32* ring = (lds_u32*)(reinterpret_cast<uint32_t*>(s_stack) +
-                               (threadIdx.x / kWaveLanes) * (kRing * kWaveLanes) +
-                               threadIdx.x % kWaveLanes);
-    uint32_t deep[kStack];
-    double prim[6];
-    for (int k = 0; k < 6; ++k) prim[k] = a.boxes[6 * i + k];
-    FindQuery<true> q;
-    q.init(a.space, prim);
-    const double* ti = a.tri + 9 * i;
-    const V3 a0 = load_v3(ti), a1 = load_v3(ti + 3), a2 = load_v3(ti + 6);
-    uint32_t cur = 0;
-    int32_t sp = -1, base = 0, visits = 0;
-    bool bad = false;
-    for (int k = 0; k < 6; ++k)  // a NaN box overlaps nothing
-      if (__builtin_isnan(prim[k])) cur = kFindEnd;
-    auto pop = [&]() {
-      if (sp < 0) {
-        cur = kFindEnd;
-        return;
-      }
-      if (sp < base)
-        cur = deep[--base];
-      else
-        cur = ring[(sp & (kRing - 1)) * kWaveLanes];
-      --sp;
-    };
-    for (;;) {
-      uint64_t want_leaf;
-      for (;;) {
-        const uint64_t want_node = __ballot(!(cur & kFindLeaf));
-        want_leaf = __ballot((cur & kFindLeaf) && cur != kFindEnd);
-        const int n_node = __popcll(want_node), n_leaf = __popcll(want_leaf);
-        if (n_node == 0 || 2 * n_leaf >= n_node + n_leaf) break;
-        if (!(cur & kFindLeaf)) {
-          float gl, gr;
-          uint32_t lc, rc;
-          find_visit<true, 3>(a.fnodes, cur, q, gl, gr, lc, rc);
-          const bool in_l = !(gl > 0.0f), in_r = !(gr > 0.0f);
-          if (!(gl < -kFindSure)) lc &= ~(lc & kFindLeaf ? kFindSureBit : 0u);
-          if (!(gr < -kFindSure)) rc &= ~(rc & kFindLeaf ? kFindSureBit : 0u);
-          cur = in_l ? lc : rc;
-          if (in_l && in_r) {
-            ++sp;
-            if (sp - base >= kRing) {
-              deep[base] = ring[(base & (kRing - 1)) * kWaveLanes];
-              ++base;
-            }
-            if (sp < kStack) ring[(sp & (kRing - 1)) * kWaveLanes] = rc;
-          } else if (!in_l && !in_r) {
-            pop();
-          }
-          if (++visits > a.ninner || sp >= kStack) {  // only a malformed tree
-            bad = true;
-            cur = kFindEnd;
-          }
-        }
-      }
-      if (want_leaf == 0) break;
-      if ((cur & kFindLeaf) && cur != kFindEnd) {
-        const int32_t pos = (int32_t)(cur & kFindPos);
-        const int32_t j = a.leaf_ids[pos];
-        bool take = (int64_t)j > i && (int64_t)j < a.n;
-        if (take && !(cur & kFindSureBit)) {
-          const double* b = a.leaf_boxes + 6 * (int64_t)pos;
-          take = (prim[3] >= b[0] && prim[0] <= b[3]) && (prim[4] >= b[1] && prim[1] <= b[4]) &&
-                 (prim[5] >= b[2] && prim[2] <= b[5]);
-        }
-        if (take) {
-          const double* tj = a.tri + 9 * (int64_t)j;
-          if (tri_tri_intersect(a0, a1, a2, load_v3(tj), load_v3(tj + 3), load_v3(tj + 6), false,
-                                a.eps))
-            hit(j);
-        }
-        pop();
-      }
-    }
-    if (bad) atomicOr(a.status, 1);
-  }
+  });
   a.npair[i] = c;
 }
 
-// Write the pairs at the scanned offsets; triangles with more hits than
-// slots walk again (the walk is deterministic, so the same hits come in the
-// same order).
+// Walk 1: count every triangle's hits, keep kPairSlots of them in any order.
+// A wave takes the triangles at `tris` neighbouring leaf positions and works
+// on (triangle, node) entries as k_ray_count does on rays: 64 visits a step,
+// then 64 triangle tests a step, where a lane per triangle left lanes idle in
+// both (a test is some hundred FP64 instructions, and a wave at a time had few).
+// Each pair is met once, from its lower leaf position p: a left child whose
+// positions end at or before p is skipped (the link of a left child is the last
+// position of its range). Its smaller triangle index is then the first of the
+// pair, the other the second, and the reference's box test, the first's corner
+// box against the second's scaled one, is done as it is; the walk's query box
+// contains both boxes of p, widened by 4 units in the last place of its largest
+// coordinate, which covers a scaled box that rounding left inside its corner box.
+// 2.6M triangles, two crossing noisy spheres: 4.1 ms with a lane per triangle
+// in mesh order on the FP64 nodes, 3.4 in leaf order on the compact ones, 1.04
+// here.
+constexpr int kPoolTris = 64;
+__global__ __launch_bounds__(kWaveLanes) void k_isect_pool(IsectArgs a, int tris) {
+  __shared__ FindPool s_pool;
+  __shared__ float s_q[12][kPoolTris];
+  __shared__ int32_t s_id[kPoolTris];
+  const int lane = (int)threadIdx.x;
+  const int64_t p0 = (int64_t)blockIdx.x * tris;
+  int32_t id = -1;
+  if (lane < tris && p0 + lane < a.n) {
+    id = a.leaf_ids[p0 + lane];
+    if ((int64_t)id >= a.n) id = -1;  // the padding of a single triangle's tree
+  }
+  if (id >= 0) {
+    const double* sb = a.leaf_boxes + 6 * (p0 + lane);
+    const double* b = a.boxes + 6 * (int64_t)id;
+    double prim[6];
+    for (int d = 0; d < 3; ++d) {
+      const double lo = b[d] < sb[d] ? b[d] : sb[d], hi = b[3 + d] > sb[3 + d] ? b[3 + d] : sb[3 + d];
+      const double w = 1e-15 * fmax(fabs(lo), fabs(hi));
+      prim[d] = lo - w;
+      prim[3 + d] = hi + w;
+    }
+    FindQuery<true> q;
+    q.init(a.space, prim);
+    for (int d = 0; d < 3; ++d) {
+      s_q[4 * d][lane] = q.lh[d];
+      s_q[4 * d + 1][lane] = q.ll[d];
+      s_q[4 * d + 2][lane] = q.hh[d];
+      s_q[4 * d + 3][lane] = q.hl[d];
+    }
+    s_id[lane] = id;
+  }
+  const bool done = find_pooled(
+      s_pool, id >= 0, a.ninner,
+      [&](uint32_t node, int who, bool& in_l, bool& in_r, uint32_t& lc, uint32_t& rc) {
+        FindQuery<true> q;
+        for (int d = 0; d < 3; ++d) {
+          q.lh[d] = s_q[4 * d][who];
+          q.ll[d] = s_q[4 * d + 1][who];
+          q.hh[d] = s_q[4 * d + 2][who];
+          q.hl[d] = s_q[4 * d + 3][who];
+        }
+        float gl, gr;
+        find_visit<true, 3>(a.fnodes, node, q, gl, gr, lc, rc);
+        const int32_t p = (int32_t)p0 + who;
+        in_l = !(gl > 0.0f) && (int32_t)(lc & kFindPos) > p;
+        in_r = !(gr > 0.0f) && !((rc & kFindLeaf) && (int32_t)(rc & kFindPos) <= p);
+      },
+      [&](int32_t q, int who) {
+        const int32_t p = (int32_t)p0 + who, ip = s_id[who], iq = a.leaf_ids[q];
+        const int32_t f = ip < iq ? ip : iq, s = ip < iq ? iq : ip, sp = ip < iq ? q : p;
+        if ((int64_t)s < a.n && isect_test(a, f, s, sp)) {
+          const int32_t c = atomicAdd(a.npair + f, 1);
+          if (c < kPairSlots) a.slots[kPairSlots * (int64_t)f + c] = sp;
+        }
+      });
+  if (!done && lane == 0) atomicOr(a.status, 1);
+}
+
+// Write the pairs at the scanned offsets, the kept hits in leaf order, the
+// walk's; triangles with more hits than slots are listed.
 __global__ __launch_bounds__(kBlock) void k_isect_emit(IsectArgs a) {
-  __shared__ int32_t s_stack[stack_lds_words(kBlock)];
   const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   const int32_t c = (i < a.n) ? a.npair[i] : 0;
-  if (c == 0) return;  // (no block-wide barrier follows)
-  const int32_t o = a.poff[i];
-  if (c <= kPairSlots) {
-    for (int32_t k = 0; k < c; ++k) {
-      a.first[o + k] = (int32_t)i;
-      a.second[o + k] = a.slots[kPairSlots * i + k];
-    }
+  if (c == 0) return;
+  if (c > kPairSlots) {
+    a.more[atomicAdd(a.nmore, 1u)] = (int32_t)i;
     return;
   }
-  int32_t m = 0;
-  isect_walk(a, i, lane_stack_base(s_stack), [&](int32_t j) {
-    if (m < c) {
-      a.first[o + m] = (int32_t)i;
-      a.second[o + m] = j;
-    }
-    ++m;
-  });
+  const int32_t o = a.poff[i];
+  const int32_t* slot = a.slots + kPairSlots * i;
+  for (int32_t k = 0; k < c; ++k) {
+    const int32_t pos = slot[k];
+    int32_t at = o;
+    for (int32_t t = 0; t < c; ++t) at += slot[t] < pos;
+    a.first[at] = (int32_t)i;
+    a.second[at] = a.leaf_ids[pos];
+  }
+}
+
+// The listed triangles walk again and write every hit in the walk's order: a
+// wave per triangle (find_ordered), since a few have very many (a lane each on
+// the FP64 nodes took 277 us at the size above, a wave each 36).
+__global__ __launch_bounds__(kWaveLanes) void k_isect_more(IsectArgs a) {
+  __shared__ uint32_t s_item[kOrderedItems];
+  const uint32_t n = *a.nmore;
+  for (uint32_t e = blockIdx.x; e < n; e += gridDim.x) {
+    const int32_t i = a.more[e], o = a.poff[i], c = a.npair[i];
+    FindQuery<true> q;
+    q.init(a.space, a.boxes + 6 * (int64_t)i);
+    const int32_t m = find_ordered(
+        s_item, a.ninner,
+        [&](uint32_t node, bool& in_l, bool& in_r, uint32_t& lc, uint32_t& rc) {
+          float gl, gr;
+          find_visit<true, 3>(a.fnodes, node, q, gl, gr, lc, rc);
+          in_l = !(gl > 0.0f);
+          in_r = !(gr > 0.0f);
+        },
+        [&](int32_t pos) {
+          const int32_t j = a.leaf_ids[pos];
+          return j > i && (int64_t)j < a.n && isect_test(a, i, j, pos);
+        },
+        [&](int32_t k, int32_t pos) {
+          if (k >= c) return;
+          a.first[o + k] = i;
+          a.second[o + k] = a.leaf_ids[pos];
+        });
+    if (m < 0 && threadIdx.x == 0) atomicOr(a.status, 1);
+  }
+}
+
+// The same a lane per triangle, where the compact nodes cannot serve.
+__global__ __launch_bounds__(kBlock) void k_isect_more_lane(IsectArgs a) {
+  __shared__ int32_t s_stack[stack_lds_words(kBlock)];
+  const uint32_t n = *a.nmore;
+  for (uint32_t e = blockIdx.x * blockDim.x + threadIdx.x; e < n; e += gridDim.x * blockDim.x) {
+    const int64_t i = a.more[e];
+    const int32_t o = a.poff[i], c = a.npair[i];
+    int32_t m = 0;
+    isect_walk(a, i, lane_stack_base(s_stack), [&](int32_t j, int32_t) {
+      if (m < c) {
+        a.first[o + m] = (int32_t)i;
+        a.second[o + m] = j;
+      }
+      ++m;
+    });
+  }
 }
 
 __global__ __launch_bounds__(kBlock) void k_flag_emit(const int32_t* __restrict__ flag,
@@ -383,7 +429,7 @@ extern "C" int axsq_mesh_self_intersections(const double* x, const double* y, co
     Workspace& ws = workspace();
     AXSQ_TRY(ws.mesh_tri.ensure(sizeof(double) * 9 * n));
     AXSQ_TRY(ws.mesh_box.ensure(sizeof(double) * 6 * n));
-    AXSQ_TRY(ws.mesh_int.ensure(sizeof(int32_t) * (4 * n + 2) + 2 * sizeof(int64_t) + 64));
+    AXSQ_TRY(ws.mesh_int.ensure(sizeof(int32_t) * (5 * n + 2) + 2 * sizeof(int64_t) + 64));
     AXSQ_TRY(ws.mesh_slots.ensure(sizeof(int32_t) * kPairSlots * n));
     double* tri = ws.mesh_tri.as<double>();
     double* boxes = ws.mesh_box.as<double>();
@@ -392,12 +438,13 @@ extern "C" int axsq_mesh_self_intersections(const double* x, const double* y, co
     int32_t* degoff = degf + n;
     int32_t* npair = degoff + n;
     int32_t* poff = npair + n;
-    int32_t* status = poff + n;
-    AXSQ_TRY(fill_i32(status, 0, 1, s));
+    int32_t* more = poff + n;
+    int32_t* status = more + n;  // and the length of `more`
+    AXSQ_TRY(fill_i32(status, 0, 2, s));
     {
       ProfRange pr("mesh_isect_setup", s);
       k_tri_setup<<<grid_for(n), kBlock, 0, s>>>(x, y, z, tris, n, nverts, tri, boxes, degf,
-                                                 status);
+                                                 npair, status);
       AXSQ_CHECK_HIP(hipGetLastError());
     }
     int32_t st = 0;
@@ -433,13 +480,20 @@ extern "C" int axsq_mesh_self_intersections(const double* x, const double* y, co
     a.npair = npair;
     a.slots = ws.mesh_slots.as<int32_t>();
     a.poff = poff;
+    a.more = more;
+    a.nmore = reinterpret_cast<uint32_t*>(status + 1);
     a.status = b->status;
+    const bool compact = b->find_ok && find_space(b->bounds, a.space);
     {
       ProfRange pr("mesh_isect_walk", s);
-      if (b->find_ok && find_space(b->bounds, a.space))
-        k_isect_count<true><<<grid_for(n), kBlock, 0, s>>>(a);
-      else
-        k_isect_count<false><<<grid_for(n), kBlock, 0, s>>>(a);
+      if (compact) {
+        // fewer triangles a wave where there are few, to fill the chip
+        int tris = 8;
+        while (tris < kPoolTris && n > (int64_t)tris * 4096) tris *= 2;
+        k_isect_pool<<<(unsigned)((n + tris - 1) / tris), kWaveLanes, 0, s>>>(a, tris);
+      } else {
+        k_isect_count<<<grid_for(n), kBlock, 0, s>>>(a);
+      }
       AXSQ_CHECK_HIP(hipGetLastError());
     }
     AXSQ_TRY(scan_exclusive_i32(npair, poff, n, tot, ws, s));
@@ -463,6 +517,11 @@ extern "C" int axsq_mesh_self_intersections(const double* x, const double* y, co
     {
       ProfRange pr("mesh_isect_emit", s);
       k_isect_emit<<<grid_for(n), kBlock, 0, s>>>(a);
+      AXSQ_CHECK_HIP(hipGetLastError());
+      if (compact)
+        k_isect_more<<<(unsigned)std::min<int64_t>(n, 8192), kWaveLanes, 0, s>>>(a);
+      else
+        k_isect_more_lane<<<std::min(grid_for(n), 1024u), kBlock, 0, s>>>(a);
       AXSQ_CHECK_HIP(hipGetLastError());
       k_flag_emit<<<grid_for(n), kBlock, 0, s>>>(degf, degoff, n, pd);
       AXSQ_CHECK_HIP(hipGetLastError());
@@ -588,8 +647,8 @@ extern "C" int axsq_mesh_candidates(const double* ix, const double* iy, const do
     AXSQ_TRY(out.alloc(&pf, total));
     AXSQ_TRY(out.alloc(&ps, total));
     // the pair list (:440-458): query cell, then its candidates in order
-    AXSQ_TRY(stash_copy_launch(b, AXSQ_QUERY_BOXES, ws.find_stash.as<int32_t>(), kstash, ws.find_cnt.as<int32_t>(),
-                               offsets, nq, ps, s));
+    AXSQ_TRY(stash_copy_launch(b, AXSQ_QUERY_BOXES, ws.find_stash.as<int32_t>(), kstash,
+                               ws.find_cnt.as<int32_t>(), offsets, nq, ps, s));
     if (n_over > 0)
       AXSQ_TRY(find_launch(b, AXSQ_QUERY_BOXES, 2, qbox, nullptr, nullptr, 6, n_over, tol,
                            nullptr, counts, offsets, ps, nullptr, 0, nullptr,

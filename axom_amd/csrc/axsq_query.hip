@@ -275,17 +275,6 @@ __global__ __launch_bounds__(kBlock) void k_find_compact(FindArgs a) {
   if (!FILL && a.stash) list_over(a, live && count > a.kstash, i);
 }
 
-// Orders a wave's LDS accesses: each wave below has its own block and LDS.
-__device__ __forceinline__ void wave_sync() {
-  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-}
-
-__device__ __forceinline__ int lanes_below(uint64_t m) {
-  return (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32),
-                                        __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
-}
-
 // One visit for a ray: on the compact node, or, for a ray outside their range
 // (ok false), the exact test on the FP64 node.
 template <int DIMS>
@@ -312,21 +301,15 @@ __device__ __forceinline__ bool ray_leaf(const FindArgs& a, int32_t pos, const d
 // The count pass for rays. A ray's walk is long (132 visits among 100,000
 // boxes), of very different lengths, and serial, so one lane per ray leaves
 // most lanes waiting for the wave's longest walk and the chip for the longest
-// of all. Here a wave holds `rays` rays and a list of (ray, node) entries still
-// to visit, and each step its 64 lanes visit the last 64, whatever their rays;
-// reached leaves go to a second list, tested 64 at a time on their FP64 boxes.
-// A ray's leaves so come in any order; their positions are the walk's order,
-// which k_stash_copy restores. The list cannot overflow: a step takes at most
-// as many entries as leave 64 free, each adds at most one net, and near the end
-// one entry at a time walks depth first, which a tree of depth 64 fits.
+// of all. Here a wave walks for `rays` rays together (find_pooled). A ray's
+// leaves so come in any order; their positions are the walk's order, which
+// k_stash_copy restores.
 // 100,000 rays, 100,000 boxes: 965 us one lane per ray on the FP64 nodes, 662 on
 // the compact ones, 129 here.
 constexpr int kPoolRays = 32;
 template <int DIMS>
 __global__ __launch_bounds__(kWaveLanes) void k_ray_count(FindArgs a, int rays) {
-  constexpr int kItems = 512, kLeaves = 192, kFree = kStack;
-  __shared__ uint32_t s_node[kItems], s_leaf[kLeaves];
-  __shared__ uint8_t s_who[kItems], s_leaf_who[kLeaves];
+  __shared__ FindPool s_pool;
   __shared__ double s_prim[9][kPoolRays];  // origin, direction, 1 / direction
   __shared__ float s_q[3 * DIMS][kPoolRays];
   __shared__ int32_t s_count[kPoolRays], s_ok[kPoolRays];
@@ -346,85 +329,35 @@ __global__ __launch_bounds__(kWaveLanes) void k_ray_count(FindArgs a, int rays) 
       s_q[3 * d + 2][lane] = q.inv[d];
     }
     s_count[lane] = 0;
-    s_node[lane] = 0;
-    s_who[lane] = (uint8_t)lane;
   }
-  int n = __popcll(__ballot(mine)), nl = 0;  // entries, leaves
-  const int64_t limit = (int64_t)n * a.ninner;
-  int64_t visits = 0;
-  wave_sync();
-  for (;;) {
-    if (nl >= kWaveLanes || (n == 0 && nl > 0)) {
-      const int m = nl < kWaveLanes ? nl : kWaveLanes;
-      nl -= m;
-      if (lane < m) {
-        const int who = s_leaf_who[nl + lane];
-        const int32_t pos = (int32_t)(s_leaf[nl + lane] & kFindPos);
+  const bool done = find_pooled(
+      s_pool, mine, a.ninner,
+      [&](uint32_t node, int who, bool& in_l, bool& in_r, uint32_t& lc, uint32_t& rc) {
+        FindRay q;
+        for (int d = 0; d < DIMS; ++d) {
+          q.h[d] = s_q[3 * d][who];
+          q.l[d] = s_q[3 * d + 1][who];
+          q.inv[d] = s_q[3 * d + 2][who];
+        }
+        const bool ok = s_ok[who];
+        double prim[6], inv[3];
+        if (!ok) {
+          for (int d = 0; d < 6; ++d) prim[d] = s_prim[d][who];
+          for (int d = 0; d < 3; ++d) inv[d] = s_prim[6 + d][who];
+        }
+        ray_visit<DIMS>(a, node, q, ok, prim, inv, in_l, in_r, lc, rc);
+      },
+      [&](int32_t pos, int who) {
         double prim[6], inv[3];
         for (int d = 0; d < 6; ++d) prim[d] = s_prim[d][who];
         for (int d = 0; d < 3; ++d) inv[d] = s_prim[6 + d][who];
-        if (ray_leaf(a, pos, prim, inv)) {
-          const int32_t c = atomicAdd(&s_count[who], 1);
-          if (a.stash && c < a.kstash)
-            a.stash[((int64_t)blockIdx.x * rays + who) * a.kstash + c] = pos;
-        }
-      }
-      wave_sync();
-      continue;
-    }
-    if (n == 0) break;
-    const int spare = kItems - kFree - n;
-    const int k = min(min(n, kWaveLanes), max(spare, 1));
-    visits += k;
-    if (visits > limit || n >= kItems) {  // only a malformed tree
-      if (lane == 0) atomicOr(a.status, kStatusStack);
-      break;
-    }
-    n -= k;
-    bool in_l = false, in_r = false;
-    uint32_t lc = 0, rc = 0;
-    int who = 0;
-    if (lane < k) {
-      const uint32_t node = s_node[n + lane];
-      who = s_who[n + lane];
-      FindRay q;
-      for (int d = 0; d < DIMS; ++d) {
-        q.h[d] = s_q[3 * d][who];
-        q.l[d] = s_q[3 * d + 1][who];
-        q.inv[d] = s_q[3 * d + 2][who];
-      }
-      const bool ok = s_ok[who];
-      double prim[6], inv[3];
-      if (!ok) {
-        for (int d = 0; d < 6; ++d) prim[d] = s_prim[d][who];
-        for (int d = 0; d < 3; ++d) inv[d] = s_prim[6 + d][who];
-      }
-      ray_visit<DIMS>(a, node, q, ok, prim, inv, in_l, in_r, lc, rc);
-    }
-    wave_sync();  // the entries are read before their places are written
-    auto put = [&](bool in, uint32_t code, bool leaves) {
-      const bool p = in && ((code & kFindLeaf) != 0) == leaves;
-      const uint64_t m = __ballot(p);
-      if (leaves) {
-        if (p) {
-          s_leaf[nl + lanes_below(m)] = code;
-          s_leaf_who[nl + lanes_below(m)] = (uint8_t)who;
-        }
-        nl += __popcll(m);
-      } else {
-        if (p) {
-          s_node[n + lanes_below(m)] = code;
-          s_who[n + lanes_below(m)] = (uint8_t)who;
-        }
-        n += __popcll(m);
-      }
-    };
-    put(in_r, rc, false);
-    put(in_l, lc, false);
-    put(in_r, rc, true);
-    put(in_l, lc, true);
-    wave_sync();
-  }
+        if (!ray_leaf(a, pos, prim, inv)) return;
+        const int32_t c = atomicAdd(&s_count[who], 1);
+        if (a.stash && c < a.kstash)
+          a.stash[((int64_t)blockIdx.x * rays + who) * a.kstash + c] = pos;
+      });
+  if (!done && lane == 0) atomicOr(a.status, kStatusStack);
+  wave_sync();
   const int32_t c = mine ? s_count[lane] : 0;
   if (mine) {
     a.counts[i] = c;
@@ -433,16 +366,12 @@ __global__ __launch_bounds__(kWaveLanes) void k_ray_count(FindArgs a, int rays) 
   if (a.stash) list_over(a, mine && c > a.kstash, i);
 }
 
-// The fill pass for rays, in order: a wave per ray holds the pending nodes and
-// leaves as a list, the leftmost last; each step takes the last 64, puts each
-// node's reached children in its place and writes out the leaves that no node
-// is left of. The list is bounded as in k_ray_count.
+// The fill pass for rays: a wave per ray (find_ordered).
 // 20,000 boxes in the plane, 50,000 rays of 134 candidates, the whole search:
-// 3,790 us with a lane per ray on the FP64 nodes, 540 here.
+// 3,790 us with a lane per ray on the FP64 nodes, 500 here.
 template <int MODE, int DIMS>
 __global__ __launch_bounds__(kWaveLanes) void k_ray_fill(FindArgs a) {
-  constexpr int kItems = 512, kFree = kStack;
-  __shared__ uint32_t s_item[kItems];
+  __shared__ uint32_t s_item[kOrderedItems];
   const int lane = (int)threadIdx.x;
   for (int64_t j = blockIdx.x; j < a.nq; j += gridDim.x) {
     const int64_t i = (MODE == kFillListed) ? (int64_t)a.over[j] : j;
@@ -452,51 +381,16 @@ __global__ __launch_bounds__(kWaveLanes) void k_ray_fill(FindArgs a) {
     FindRay q;
     const bool ok = q.init(a.space, prim, a.tol, a.f32);
     const int32_t offset = a.offsets[i], room = a.fill_cnt[i];
-    int32_t count = 0, visits = 0;
-    int n = 1;
-    bool bad = false;
-    wave_sync();
-    if (lane == 0) s_item[0] = 0;
-    wave_sync();
-    while (n > 0) {
-      const int k = min(min(n, kWaveLanes), max(kItems - kFree - n, 1));
-      const uint32_t item = lane < k ? s_item[n - 1 - lane] : 0u;
-      const bool node = lane < k && !(item & kFindLeaf);
-      const uint64_t nodes = __ballot(node);
-      const int lead = nodes ? __ffsll((unsigned long long)nodes) - 1 : k;  // leading leaves
-      if (lead > 0) {
-        const int32_t pos = (int32_t)(item & kFindPos);
-        const bool take = lane < lead && ray_leaf(a, pos, prim, inv);
-        const uint64_t m = __ballot(take);
-        const int32_t c = count + lanes_below(m);
-        if (take && c < room) a.cands[offset + c] = a.leaf_ids[pos];
-        count += __popcll(m);
-      }
-      visits += __popcll(nodes);
-      if (visits > a.ninner || n >= kItems) {  // only a malformed tree
-        bad = true;
-        break;
-      }
-      uint32_t first = item, second = item;
-      bool one = lane >= lead && lane < k, two = false;
-      if (node) {
-        bool in_l, in_r;
-        uint32_t lc, rc;
-        ray_visit<DIMS>(a, item, q, ok, prim, inv, in_l, in_r, lc, rc);
-        first = in_l ? lc : rc;
-        second = rc;
-        one = in_l || in_r;
-        two = in_l && in_r;
-      }
-      const uint64_t m1 = __ballot(one), m2 = __ballot(two);
-      n += __popcll(m1) + __popcll(m2) - k;
-      const int at = n - 1 - lanes_below(m1) - lanes_below(m2);
-      wave_sync();  // the entries are read before their places are written
-      if (one) s_item[at] = first;
-      if (two) s_item[at - 1] = second;
-      wave_sync();
-    }
-    if (lane == 0 && bad) atomicOr(a.status, kStatusStack);
+    const int32_t count = find_ordered(
+        s_item, a.ninner,
+        [&](uint32_t node, bool& in_l, bool& in_r, uint32_t& lc, uint32_t& rc) {
+          ray_visit<DIMS>(a, node, q, ok, prim, inv, in_l, in_r, lc, rc);
+        },
+        [&](int32_t pos) { return ray_leaf(a, pos, prim, inv); },
+        [&](int32_t c, int32_t pos) {
+          if (c < room) a.cands[offset + c] = a.leaf_ids[pos];
+        });
+    if (lane == 0 && count < 0) atomicOr(a.status, kStatusStack);
     if (lane == 0 && count != room) atomicOr(a.status, kStatusFillMismatch);
   }
 }

@@ -61,7 +61,6 @@ __device__ __forceinline__ bool valid6(const T b[6]) {
 #define AXSQ_LDS_STACK 32
 #endif
 constexpr int kLdsStack = AXSQ_LDS_STACK;
-constexpr int kWaveLanes = 64;
 
 // LDS-qualified word: accesses compile to ds_read/ds_write, not flat ops.
 typedef __attribute__((address_space(3))) int32_t lds_i32;

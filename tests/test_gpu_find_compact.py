@@ -15,7 +15,7 @@ import pytest
 torch = pytest.importorskip("torch")
 
 from axom_amd import _lib as L  # noqa: E402
-from axom_amd import spin  # noqa: E402
+from axom_amd import quest, spin  # noqa: E402
 from oracle import oracle as orc  # noqa: E402
 
 pytestmark = pytest.mark.gpu
@@ -195,3 +195,30 @@ def test_count_then_fill_on_compact_nodes(kind):
     L.check(L.lib().axsq_bvh_find_fill(g._h, code, *args[:5], g._tol, spin._ptr(off),
                                        spin._ptr(cnt), spin._ptr(cand), None))
     assert np.array_equal(cand.cpu().numpy(), ocand)
+
+
+@pytest.mark.parametrize("scene", ["plain", "far", "flat", "sizes", "huge"])
+@pytest.mark.parametrize("n", [3, 63, 64, 65, 513, 6000])
+def test_self_intersections_on_compact_nodes(scene, n):
+    """Pairs met once, from their lower leaf, are the reference's pairs: soups
+    whose triangles hit more others than are kept, lie in a plane (boxes without
+    extent), are far from the origin (boxes thin by units in the last place) or
+    differ in size by six decades; a huge one takes the general walk."""
+    rng = np.random.default_rng(n)
+    size = (0.4 / n) ** (1 / 3)
+    s = 10.0 ** rng.uniform(-6, 0, (n, 1, 1)) if scene == "sizes" else 1.0
+    v = rng.uniform(-1, 1, (n, 1, 3)) + s * rng.normal(0, size, (n, 3, 3))
+    if scene == "flat":
+        v[: n // 2, :, 2] = 0.25
+        v[n // 2 :, :, 0] = np.round(v[n // 2 :, :, 0], 1)
+    elif scene == "far":
+        v = v + 2.0**24
+        v[:, :, 0] = 2.0**24 + rng.integers(0, 3, (n, 3)) * 2.0**-28
+    elif scene == "huge":
+        v = v * 1e120
+    t = np.arange(3 * n, dtype=np.int32).reshape(n, 3)
+    v = np.ascontiguousarray(v.reshape(-1, 3))
+    pairs, degen = quest.findTriMeshIntersectionsBVH(_t(v), _t(t))
+    want, want_degen = orc.mesh_self_intersections(v, t)
+    assert np.array_equal(pairs.cpu().numpy().reshape(-1, 2), want.reshape(-1, 2))
+    assert np.array_equal(degen.cpu().numpy(), want_degen)
