@@ -37,6 +37,8 @@ class AxsqError(RuntimeError):
         self.code = code
 
 
+ALLOC_FN = ctypes.CFUNCTYPE(_vp, _vp, _i64)
+
 _SIGS = {
     "axsq_last_error": (ctypes.c_char_p, []),
     "axsq_version": (_i32, []),
@@ -101,6 +103,12 @@ _SIGS = {
     "axsq_sdf_last_suspended": (_i32, [_vp, ctypes.POINTER(_i64)]),
     "axsq_sdf_last_early": (_i32, [_vp, ctypes.POINTER(_i64)]),
     "axsq_tri_tri_intersect": (_i32, [_vp, _vp, _i64, _i32, _dbl, _vp, _vp]),
+    "axsq_mesh_self_intersections_alloc": (_i32, [
+        _vp, _vp, _vp, _i64, _vp, _i64, _dbl, ALLOC_FN, _vp, ctypes.POINTER(_vp),
+        ctypes.POINTER(_i64), ctypes.POINTER(_vp), ctypes.POINTER(_i64), _vp]),
+    "axsq_mesh_candidates_alloc": (_i32, [
+        _vp, _vp, _vp, _i64, _vp, _i64, _vp, _vp, _vp, _i64, _vp, _i64, _i32, ALLOC_FN, _vp,
+        ctypes.POINTER(_vp), ctypes.POINTER(_i64), _vp]),
     "axsq_mesh_candidates": (_i32, [_vp, _vp, _vp, _i64, _vp, _i64, _vp, _vp, _vp, _i64, _vp,
                                     _i64, _i32, ctypes.POINTER(_vp), ctypes.POINTER(_vp),
                                     ctypes.POINTER(_i64), _vp]),

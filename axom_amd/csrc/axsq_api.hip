@@ -23,7 +23,8 @@ int sdf_setup(axsq_sdf* h, hipStream_t s);
 int sdf_build_v2t(axsq_sdf* h, hipStream_t s);
 int sdf_eval_launch(const axsq_sdf* h, const double* x, const double* y, const double* z,
                     int64_t stride, int64_t nq, int fp_mode, double* dist, double* cp,
-                    double* normal, int32_t* elem, bool stats, hipStream_t s);
+                    double* normal, int32_t* elem, bool stats, hipStream_t s,
+                    bool* done);
 int sdf_backward_launch(const axsq_sdf* h, const double* x, const double* y, const double* z,
                         int64_t stride, int64_t nq, const double* dist, const int32_t* elem,
                         const float* gout, double* grad_q, double* grad_v, hipStream_t s);
@@ -87,6 +88,10 @@ void Workspace::release() {
   find_over.release();
   find_n.release();
   one.release();
+  cull_n.release();
+  find_n_zero = cull_n_zero = false;
+  if (host_words) hipHostFree(host_words);
+  host_words = nullptr;
   if (mesh_bvh) {
     axsq_bvh_destroy(mesh_bvh);
     mesh_bvh = nullptr;
@@ -161,32 +166,85 @@ void prof_flush() {
   g_pending.swap(keep);
 }
 
-// Waits for the stream, folds profiling ranges, and turns a traversal stack
-// overflow flagged by a kernel into an error code.
-static int finish(int32_t* status, hipStream_t s) {
+__global__ void k_read_back(ReadBack r, int64_t* __restrict__ out) {
+  for (int k = 0; k < 2; ++k) {
+    out[k] = r.total[k] ? *r.total[k] : 0;
+    out[3 + k] = r.status[k] ? *r.status[k] : 0;
+    if (r.status[k]) *r.status[k] = 0;
+  }
+  out[2] = r.list ? (int64_t)*r.list : 0;
+  for (int k = 0; k < r.nlist; ++k) r.list[k] = 0;
+}
+
+int read_back(const ReadBack& r, ReadValues* v, hipStream_t s) {
+  Workspace& ws = workspace();
+  if (!ws.host_words) {
+    void* p = nullptr;
+    if (hipHostMalloc(&p, sizeof(int64_t) * kReadWords, hipHostMallocDefault) != hipSuccess) {
+      set_error("host allocation of %zu bytes failed", sizeof(int64_t) * kReadWords);
+      return AXSQ_ERR_NOMEM;
+    }
+    ws.host_words = static_cast<int64_t*>(p);
+  }
+  void* dev = nullptr;
+  AXSQ_CHECK_HIP(hipHostGetDevicePointer(&dev, ws.host_words, 0));
+  k_read_back<<<1, 1, 0, s>>>(r, static_cast<int64_t*>(dev));
+  AXSQ_CHECK_HIP(hipGetLastError());
   AXSQ_CHECK_HIP(hipStreamSynchronize(s));
   prof_flush();
+  const int64_t* w = ws.host_words;
+  v->total[0] = w[0];
+  v->total[1] = w[1];
+  v->list = w[2];
+  v->status[0] = (int32_t)w[3];
+  v->status[1] = (int32_t)w[4];
+  return AXSQ_OK;
+}
+
+int status_error(int32_t status) {
+  if (status & kStatusStack) {
+    set_error("traversal stopped: stack deeper than %d entries or malformed tree", kStack);
+    return AXSQ_ERR_STACK_OVERFLOW;
+  }
+  if (status & kStatusFillMismatch) {
+    set_error("candidate fill: the search found another number of candidates than the "
+              "counts give for some query (queries, tolerance or tree changed since the "
+              "count); no id was written past a query's count");
+    return AXSQ_ERR_INVALID_ARG;
+  }
   if (status) {
-    int32_t h = 0;
-    AXSQ_CHECK_HIP(hipMemcpy(&h, status, sizeof(int32_t), hipMemcpyDeviceToHost));
-    if (h) {
-      int32_t z = 0;
-      AXSQ_CHECK_HIP(hipMemcpy(status, &z, sizeof(int32_t), hipMemcpyHostToDevice));
-      if (h & kStatusStack) {
-        set_error("traversal stopped: stack deeper than %d entries or malformed tree", kStack);
-        return AXSQ_ERR_STACK_OVERFLOW;
-      }
-      if (h & kStatusFillMismatch) {
-        set_error("candidate fill: the search found another number of candidates than the "
-                  "counts give for some query (queries, tolerance or tree changed since the "
-                  "count); no id was written past a query's count");
-        return AXSQ_ERR_INVALID_ARG;
-      }
-      set_error("element id out of range in the adjoint input");
-      return AXSQ_ERR_INVALID_ARG;
-    }
+    set_error("element id out of range in the adjoint input");
+    return AXSQ_ERR_INVALID_ARG;
   }
   return AXSQ_OK;
+}
+
+// Waits for the stream, folds profiling ranges, and turns what a kernel
+// flagged in the status word into an error code.
+static int finish(int32_t* status, hipStream_t s) {
+  if (!status) {
+    AXSQ_CHECK_HIP(hipStreamSynchronize(s));
+    prof_flush();
+    return AXSQ_OK;
+  }
+  ReadBack r;
+  r.status[0] = status;
+  ReadValues v;
+  AXSQ_TRY(read_back(r, &v, s));
+  return status_error(v.status[0]);
+}
+
+// The same for a call that allocates nothing.
+static int finish_noalloc(int32_t* status, hipStream_t s) {
+  AXSQ_CHECK_HIP(hipStreamSynchronize(s));
+  prof_flush();
+  int32_t h = 0;
+  AXSQ_CHECK_HIP(hipMemcpy(&h, status, sizeof(int32_t), hipMemcpyDeviceToHost));
+  if (h) {
+    int32_t z = 0;
+    AXSQ_CHECK_HIP(hipMemcpy(status, &z, sizeof(int32_t), hipMemcpyHostToDevice));
+  }
+  return status_error(h);
 }
 
 static bool valid_kind(int k) {
@@ -498,11 +556,13 @@ static int find_count_impl(const axsq_bvh* b, int kind, const void* x, const voi
     AXSQ_TRY(ws.find_cnt.ensure(sizeof(int32_t) * (size_t)nq));
     AXSQ_TRY(ws.find_over.ensure(sizeof(int32_t) * (size_t)nq));
   }
+  if (!ws.find_n.p) ws.find_n_zero = false;
   AXSQ_TRY(ws.find_n.ensure(sizeof(int64_t) * 2));
   // find_n: [0] the scanned total (int64), [1] the listed queries (uint32)
   int64_t* tot_dev = ws.find_n.as<int64_t>();
   uint32_t* nover = reinterpret_cast<uint32_t*>(tot_dev + 1);
-  AXSQ_TRY(fill_i32(reinterpret_cast<int32_t*>(nover), 0, 1, s));
+  if (!ws.find_n_zero) AXSQ_TRY(fill_i32(reinterpret_cast<int32_t*>(nover), 0, 1, s));
+  ws.find_n_zero = false;
   if (b->stats) AXSQ_TRY(fill_i32(reinterpret_cast<int32_t*>(b->find_visits), 0, 2, s));
   AXSQ_TRY(find_launch(b, kind, 0, x, y, z, stride, nq, tol, counts, nullptr, nullptr, nullptr,
                        keep ? ws.find_stash.as<int32_t>() : nullptr, kstash,
@@ -512,21 +572,27 @@ static int find_count_impl(const axsq_bvh* b, int kind, const void* x, const voi
     ProfRange ps("bvh_find_scan", s);
     AXSQ_TRY(scan_exclusive_i32(counts, offsets, nq, tot_dev, ws, s));
   }
-  int64_t tn[2] = {0, 0};
-  AXSQ_CHECK_HIP(hipMemcpyAsync(tn, tot_dev, sizeof(tn), hipMemcpyDeviceToHost, s));
-  AXSQ_TRY(finish(b->status, s));
+  ReadBack r;
+  r.total[0] = tot_dev;
+  r.list = nover;
+  r.nlist = 1;
+  r.status[0] = b->status;
+  ReadValues v;
+  AXSQ_TRY(read_back(r, &v, s));
+  ws.find_n_zero = true;
+  AXSQ_TRY(status_error(v.status[0]));
   if (b->stats) {
-    unsigned long long v = 0;
-    AXSQ_CHECK_HIP(hipMemcpy(&v, b->find_visits, sizeof(v), hipMemcpyDeviceToHost));
-    const_cast<axsq_bvh*>(b)->last_visits = (int64_t)v;
+    unsigned long long n = 0;
+    AXSQ_CHECK_HIP(hipMemcpy(&n, b->find_visits, sizeof(n), hipMemcpyDeviceToHost));
+    const_cast<axsq_bvh*>(b)->last_visits = (int64_t)n;
   }
-  const int64_t t = tn[0];
+  const int64_t t = v.total[0];
   if (t > 0x7fffffffll) {
     set_error("candidate total %lld exceeds the int32 index range", (long long)t);
     return AXSQ_ERR_INVALID_ARG;
   }
   *total = t;
-  if (nover_out) *nover_out = (int64_t)(uint32_t)tn[1];
+  if (nover_out) *nover_out = v.list;
   if (kstash_out) *kstash_out = kstash;
   return AXSQ_OK;
 }
@@ -590,12 +656,12 @@ static int find_fill_kept(const axsq_bvh* b, int kind, const void* x, const void
                           const int32_t* offsets, const int32_t* counts, int32_t* cands,
                           int64_t nover, int kstash, hipStream_t s) {
   Workspace& ws = workspace();
-  AXSQ_TRY(stash_copy_launch(b, kind, ws.find_stash.as<int32_t>(), kstash, ws.find_cnt.as<int32_t>(),
+  AXSQ_TRY(stash_copy_launch(b, kind, false, ws.find_stash.as<int32_t>(), kstash, ws.find_cnt.as<int32_t>(),
                              offsets, nq, cands, s));
   if (nover > 0)
     AXSQ_TRY(find_launch(b, kind, 2, x, y, z, stride, nover, tol, nullptr, counts, offsets,
                          cands, nullptr, 0, nullptr, ws.find_over.as<int32_t>(), nullptr, s));
-  return finish(b->status, s);
+  return finish(nover > 0 ? b->status : nullptr, s);  // the copy flags nothing
 }
 
 static int check_find_outputs(const char* name, int64_t nq, const int32_t* offsets,
@@ -717,19 +783,19 @@ int axsq_bvh_find_into_noalloc(const axsq_bvh* b, int kind, const double* x, con
   AXSQ_TRY(scan_exclusive_i32_into(counts, offsets, nq, sums, tot_dev, s));
   int64_t tn[2] = {0, 0};
   AXSQ_CHECK_HIP(hipMemcpyAsync(tn, tot_dev, sizeof(tn), hipMemcpyDeviceToHost, s));
-  AXSQ_TRY(finish(b->status, s));
+  AXSQ_TRY(finish_noalloc(b->status, s));
   if (tn[0] > 0x7fffffffll) {
     set_error("candidate total %lld exceeds the int32 index range", (long long)tn[0]);
     return AXSQ_ERR_INVALID_ARG;
   }
   *total = tn[0];
   if (*total == 0 || *total > capacity) return AXSQ_OK;  // too small: nothing written
-  AXSQ_TRY(stash_copy_launch(b, kind, kept, kstash, kept_cnt, offsets, nq, candidates, s));
+  AXSQ_TRY(stash_copy_launch(b, kind, false, kept, kstash, kept_cnt, offsets, nq, candidates, s));
   const int64_t nover = (int64_t)(uint32_t)tn[1];
   if (nover > 0)
     AXSQ_TRY(find_launch(b, kind, 2, x, y, z, stride, nover, tol, nullptr, counts, offsets,
                          candidates, nullptr, 0, nullptr, over, nullptr, s));
-  return finish(b->status, s);
+  return finish_noalloc(b->status, s);
 }
 
 }  // extern "C"
@@ -1125,8 +1191,10 @@ int axsq_sdf_eval(const axsq_sdf* h, const double* x, const double* y, const dou
   hipStream_t s = (hipStream_t)stream;
   const bool stats = h->stats && fp_mode == AXSQ_FP64;
   if (stats) AXSQ_TRY(fill_i32(reinterpret_cast<int32_t*>(h->stats_dev), 0, 4, s));
-  AXSQ_TRY(sdf_eval_launch(h, x, y, z, stride, nq, fp_mode, dist, cp, normal, elem, stats, s));
-  AXSQ_TRY(finish(h->bvh->status, s));
+  bool done = false;
+  AXSQ_TRY(sdf_eval_launch(h, x, y, z, stride, nq, fp_mode, dist, cp, normal, elem, stats, s,
+                           &done));
+  if (!done) AXSQ_TRY(finish(h->bvh->status, s));
   if (stats) {
     int64_t st[2];
     AXSQ_CHECK_HIP(hipMemcpy(st, h->stats_dev, sizeof(st), hipMemcpyDeviceToHost));

@@ -82,8 +82,9 @@ struct IsectArgs {
   int32_t* npair;  // hits per triangle
   int32_t* slots;  // kPairSlots per triangle: the hits' leaf positions
   const int32_t* poff;
-  int32_t* first;
+  int32_t* first;  // entry k of a pair's member at `step` * k
   int32_t* second;
+  int step;
   int32_t* more;    // triangles with more hits than slots, and their number
   uint32_t* nmore;
   int32_t* status;
@@ -236,8 +237,8 @@ __global__ __launch_bounds__(kBlock) void k_isect_emit(IsectArgs a) {
     const int32_t pos = slot[k];
     int32_t at = o;
     for (int32_t t = 0; t < c; ++t) at += slot[t] < pos;
-    a.first[at] = (int32_t)i;
-    a.second[at] = a.leaf_ids[pos];
+    a.first[(int64_t)a.step * at] = (int32_t)i;
+    a.second[(int64_t)a.step * at] = a.leaf_ids[pos];
   }
 }
 
@@ -265,8 +266,8 @@ __global__ __launch_bounds__(kWaveLanes) void k_isect_more(IsectArgs a) {
         },
         [&](int32_t k, int32_t pos) {
           if (k >= c) return;
-          a.first[o + k] = i;
-          a.second[o + k] = a.leaf_ids[pos];
+          a.first[(int64_t)a.step * (o + k)] = i;
+          a.second[(int64_t)a.step * (o + k)] = a.leaf_ids[pos];
         });
     if (m < 0 && threadIdx.x == 0) atomicOr(a.status, 1);
   }
@@ -282,8 +283,8 @@ __global__ __launch_bounds__(kBlock) void k_isect_more_lane(IsectArgs a) {
     int32_t m = 0;
     isect_walk(a, i, lane_stack_base(s_stack), [&](int32_t j, int32_t) {
       if (m < c) {
-        a.first[o + m] = (int32_t)i;
-        a.second[o + m] = j;
+        a.first[(int64_t)a.step * (o + m)] = (int32_t)i;
+        a.second[(int64_t)a.step * (o + m)] = j;
       }
       ++m;
     });
@@ -357,10 +358,18 @@ __global__ __launch_bounds__(kBlock) void k_expand_first(const int32_t* __restri
 
 struct Scratch {
   std::vector<void*> ptrs;
+  axsq_alloc_fn fn = nullptr;  // the caller's, whose blocks stay its own
+  void* ctx = nullptr;
   template <class T>
   int alloc(T** p, int64_t count) {
     *p = nullptr;
     const size_t bytes = sizeof(T) * (size_t)(count > 0 ? count : 1);
+    if (fn) {
+      *p = static_cast<T*>(fn(ctx, (int64_t)bytes));
+      if (*p) return AXSQ_OK;
+      set_error("the caller's allocator gave no %zu bytes", bytes);
+      return AXSQ_ERR_NOMEM;
+    }
     if (hipMalloc((void**)p, bytes) != hipSuccess) {
       *p = nullptr;
       set_error("device allocation of %zu bytes failed", bytes);
@@ -400,17 +409,23 @@ extern "C" int axsq_tri_tri_intersect(const double* t1, const double* t2, int64_
   return AXSQ_OK;
 }
 
-extern "C" int axsq_mesh_self_intersections(const double* x, const double* y, const double* z,
-                                            int64_t nverts, const int32_t* tris, int64_t ntris,
-                                            double threshold, int32_t** first, int32_t** second,
-                                            int64_t* npairs, int32_t** degenerate,
-                                            int64_t* ndegen, void* stream) {
+namespace {
+// first / second: an array each; pairs: one array of (first, second) records
+// and `degenerate`, from the caller's allocator.
+int self_intersections(const double* x, const double* y, const double* z, int64_t nverts,
+                       const int32_t* tris, int64_t ntris, double threshold, int32_t** first,
+                       int32_t** second, int32_t** pairs, int64_t* npairs, int32_t** degenerate,
+                       int64_t* ndegen, axsq_alloc_fn alloc, void* ctx, void* stream) {
   clear_error();
-  if (!first || !second || !npairs || !degenerate || !ndegen) {
+  if (!((first && second) || pairs) || !npairs || !degenerate || !ndegen) {
     set_error("axsq_mesh_self_intersections: NULL output");
     return AXSQ_ERR_INVALID_ARG;
   }
-  *first = *second = *degenerate = nullptr;
+  if (pairs)
+    *pairs = nullptr;
+  else
+    *first = *second = nullptr;
+  *degenerate = nullptr;
   *npairs = *ndegen = 0;
   if (ntris < 0 || nverts < 0 || ntris > 0x3fffffffll || nverts > 0x7fffffffll ||
       (ntris > 0 && (!x || !y || !z || !tris || nverts < 1))) {
@@ -419,11 +434,20 @@ extern "C" int axsq_mesh_self_intersections(const double* x, const double* y, co
   }
   hipStream_t s = (hipStream_t)stream;
   Scratch out;  // the caller's arrays until they are handed over
+  out.fn = alloc;
+  out.ctx = ctx;
   int32_t *pf = nullptr, *ps = nullptr, *pd = nullptr;
+  // pairs: the second member of a record after the first
+  auto alloc_out = [&](int64_t np, int64_t nd) -> int {
+    AXSQ_TRY(out.alloc(&pf, pairs ? 2 * np : np));
+    if (pairs)
+      ps = pf + 1;
+    else
+      AXSQ_TRY(out.alloc(&ps, np));
+    return out.alloc(&pd, nd);
+  };
   if (ntris == 0) {
-    AXSQ_TRY(out.alloc(&pf, 1));
-    AXSQ_TRY(out.alloc(&ps, 1));
-    AXSQ_TRY(out.alloc(&pd, 1));
+    AXSQ_TRY(alloc_out(0, 0));
   } else {
     const int64_t n = ntris;
     Workspace& ws = workspace();
@@ -446,14 +470,6 @@ extern "C" int axsq_mesh_self_intersections(const double* x, const double* y, co
       k_tri_setup<<<grid_for(n), kBlock, 0, s>>>(x, y, z, tris, n, nverts, tri, boxes, degf,
                                                  npair, status);
       AXSQ_CHECK_HIP(hipGetLastError());
-    }
-    int32_t st = 0;
-    AXSQ_CHECK_HIP(hipMemcpyAsync(&st, status, sizeof(int32_t), hipMemcpyDeviceToHost, s));
-    AXSQ_CHECK_HIP(hipStreamSynchronize(s));
-    if (st) {
-      set_error("axsq_mesh_self_intersections: connectivity refers to a vertex outside [0, %lld)",
-                (long long)nverts);
-      return AXSQ_ERR_INVALID_ARG;
     }
     // the BVH over the corner boxes, default scale (MeshTester_detail.hpp:322-338)
     if (!ws.mesh_bvh) {
@@ -498,20 +514,22 @@ extern "C" int axsq_mesh_self_intersections(const double* x, const double* y, co
     }
     AXSQ_TRY(scan_exclusive_i32(npair, poff, n, tot, ws, s));
     AXSQ_TRY(scan_exclusive_i32(degf, degoff, n, tot + 1, ws, s));
-    int64_t totals[2] = {0, 0};
-    int32_t walk_status = 0;
-    AXSQ_CHECK_HIP(hipMemcpyAsync(totals, tot, 2 * sizeof(int64_t), hipMemcpyDeviceToHost, s));
-    AXSQ_CHECK_HIP(
-        hipMemcpyAsync(&walk_status, b->status, sizeof(int32_t), hipMemcpyDeviceToHost, s));
-    AXSQ_CHECK_HIP(hipStreamSynchronize(s));
-    if (walk_status) {
-      AXSQ_TRY(fill_i32(b->status, 0, 1, s));
-      set_error("traversal stopped: stack deeper than %d entries or malformed tree", kStack);
-      return AXSQ_ERR_STACK_OVERFLOW;
+    ReadBack r;
+    r.total[0] = tot;
+    r.total[1] = tot + 1;
+    r.status[0] = b->status;
+    r.status[1] = status;
+    ReadValues v;
+    AXSQ_TRY(read_back(r, &v, s));
+    if (v.status[1]) {  // such a vertex was taken as vertex 0 up to here
+      set_error("axsq_mesh_self_intersections: connectivity refers to a vertex outside [0, %lld)",
+                (long long)nverts);
+      return AXSQ_ERR_INVALID_ARG;
     }
-    AXSQ_TRY(out.alloc(&pf, totals[0]));
-    AXSQ_TRY(out.alloc(&ps, totals[0]));
-    AXSQ_TRY(out.alloc(&pd, totals[1]));
+    AXSQ_TRY(status_error(v.status[0]));
+    const int64_t* totals = v.total;
+    AXSQ_TRY(alloc_out(totals[0], totals[1]));
+    a.step = pairs ? 2 : 1;
     a.first = pf;
     a.second = ps;
     {
@@ -534,24 +552,31 @@ extern "C" int axsq_mesh_self_intersections(const double* x, const double* y, co
   out.keep(pf);
   out.keep(ps);
   out.keep(pd);
-  *first = pf;
-  *second = ps;
+  if (pairs) {
+    *pairs = pf;
+  } else {
+    *first = pf;
+    *second = ps;
+  }
   *degenerate = pd;
   return AXSQ_OK;
 }
 
-extern "C" int axsq_mesh_candidates(const double* ix, const double* iy, const double* iz,
-                                    int64_t inverts, const int32_t* icells, int64_t nicells,
-                                    const double* qx, const double* qy, const double* qz,
-                                    int64_t qnverts, const int32_t* qcells, int64_t nqcells,
-                                    int nodes_per_cell, int32_t** first, int32_t** second,
-                                    int64_t* npairs, void* stream) {
+// As above: first / second or pairs.
+int mesh_candidates(const double* ix, const double* iy, const double* iz, int64_t inverts,
+                    const int32_t* icells, int64_t nicells, const double* qx, const double* qy,
+                    const double* qz, int64_t qnverts, const int32_t* qcells, int64_t nqcells,
+                    int nodes_per_cell, int32_t** first, int32_t** second, int32_t** pairs,
+                    int64_t* npairs, axsq_alloc_fn alloc, void* ctx, void* stream) {
   clear_error();
-  if (!first || !second || !npairs) {
+  if (!((first && second) || pairs) || !npairs) {
     set_error("axsq_mesh_candidates: NULL output");
     return AXSQ_ERR_INVALID_ARG;
   }
-  *first = *second = nullptr;
+  if (pairs)
+    *pairs = nullptr;
+  else
+    *first = *second = nullptr;
   *npairs = 0;
   if (nodes_per_cell < 1 || nodes_per_cell > 8) {
     set_error("axsq_mesh_candidates: nodes_per_cell %d outside [1, 8]", nodes_per_cell);
@@ -566,11 +591,13 @@ extern "C" int axsq_mesh_candidates(const double* ix, const double* iy, const do
   }
   hipStream_t s = (hipStream_t)stream;
   Scratch out;
-  int32_t *pf = nullptr, *ps = nullptr;
+  out.fn = alloc;
+  out.ctx = ctx;
+  int32_t *pf = nullptr, *ps = nullptr;  // pairs: pf alone, of records
   int64_t total = 0;
   if (nicells == 0 || nqcells == 0) {
-    AXSQ_TRY(out.alloc(&pf, 1));
-    AXSQ_TRY(out.alloc(&ps, 1));
+    AXSQ_TRY(out.alloc(&pf, 0));
+    if (!pairs) AXSQ_TRY(out.alloc(&ps, 0));
   } else {
     const int64_t ni = nicells, nq = nqcells;
     Workspace& ws = workspace();
@@ -591,13 +618,6 @@ extern "C" int axsq_mesh_candidates(const double* ix, const double* iy, const do
     k_cell_boxes_n<<<grid_for(nq), kBlock, 0, s>>>(qx, qy, qz, qnverts, qcells, nq,
                                                    nodes_per_cell, qbox, status);
     AXSQ_CHECK_HIP(hipGetLastError());
-    int32_t st = 0;
-    AXSQ_CHECK_HIP(hipMemcpyAsync(&st, status, sizeof(int32_t), hipMemcpyDeviceToHost, s));
-    AXSQ_CHECK_HIP(hipStreamSynchronize(s));
-    if (st) {
-      set_error("axsq_mesh_candidates: a cell refers to a vertex outside its mesh");
-      return AXSQ_ERR_INVALID_ARG;
-    }
     // the BVH over the insert mesh's boxes, default scale
     // (quest_candidates_example.cpp:420-423)
     if (!ws.mesh_bvh) {
@@ -617,51 +637,114 @@ extern "C" int axsq_mesh_candidates(const double* ix, const double* iy, const do
     AXSQ_TRY(ws.find_stash.ensure(sizeof(int32_t) * kstash * (size_t)nq));
     AXSQ_TRY(ws.find_cnt.ensure(sizeof(int32_t) * (size_t)nq));
     AXSQ_TRY(ws.find_over.ensure(sizeof(int32_t) * (size_t)nq));
-    AXSQ_TRY(ws.find_n.ensure(sizeof(int64_t) * 2));
-    uint32_t* nover = reinterpret_cast<uint32_t*>(ws.find_n.as<int64_t>());
-    AXSQ_TRY(fill_i32(reinterpret_cast<int32_t*>(nover), 0, 1, s));
+    if (!ws.find_n.p) ws.find_n_zero = false;
+    AXSQ_TRY(ws.find_n.ensure(sizeof(int64_t) * 2));  // the list's length as in find_count_impl
+    uint32_t* nover = reinterpret_cast<uint32_t*>(ws.find_n.as<int64_t>() + 1);
+    if (!ws.find_n_zero) AXSQ_TRY(fill_i32(reinterpret_cast<int32_t*>(nover), 0, 1, s));
+    ws.find_n_zero = false;
     const double tol = 2.220446049250313e-16;  // BVH default tolerance (unused by boxes)
     AXSQ_TRY(find_launch(b, AXSQ_QUERY_BOXES, 0, qbox, nullptr, nullptr, 6, nq, tol, counts,
                          nullptr, nullptr, nullptr, ws.find_stash.as<int32_t>(), kstash,
                          ws.find_cnt.as<int32_t>(), ws.find_over.as<int32_t>(), nover, s));
     AXSQ_TRY(scan_exclusive_i32(counts, offsets, nq, tot, ws, s));
-    int64_t tn[2] = {0, 0};
-    int32_t walk_status = 0;
-    AXSQ_CHECK_HIP(hipMemcpyAsync(&tn[0], tot, sizeof(int64_t), hipMemcpyDeviceToHost, s));
-    AXSQ_CHECK_HIP(hipMemcpyAsync(&tn[1], nover, sizeof(uint32_t), hipMemcpyDeviceToHost, s));
-    AXSQ_CHECK_HIP(
-        hipMemcpyAsync(&walk_status, b->status, sizeof(int32_t), hipMemcpyDeviceToHost, s));
-    AXSQ_CHECK_HIP(hipStreamSynchronize(s));
-    if (walk_status) {
-      AXSQ_TRY(fill_i32(b->status, 0, 1, s));
-      set_error("traversal stopped: stack deeper than %d entries or malformed tree", kStack);
-      return AXSQ_ERR_STACK_OVERFLOW;
+    ReadBack r;
+    r.total[0] = tot;
+    r.list = nover;
+    r.nlist = 1;
+    r.status[0] = b->status;
+    r.status[1] = status;
+    ReadValues v;
+    AXSQ_TRY(read_back(r, &v, s));
+    ws.find_n_zero = true;
+    if (v.status[1]) {
+      set_error("axsq_mesh_candidates: a cell refers to a vertex outside its mesh");
+      return AXSQ_ERR_INVALID_ARG;
     }
-    total = tn[0];
+    AXSQ_TRY(status_error(v.status[0]));
+    total = v.total[0];
     if (total > 0x7fffffffll) {
       set_error("axsq_mesh_candidates: %lld candidate pairs exceed the int32 index range",
                 (long long)total);
       return AXSQ_ERR_INVALID_ARG;
     }
-    const int64_t n_over = (int64_t)(uint32_t)tn[1];
-    AXSQ_TRY(out.alloc(&pf, total));
-    AXSQ_TRY(out.alloc(&ps, total));
+    AXSQ_TRY(out.alloc(&pf, pairs ? 2 * total : total));
+    if (!pairs) AXSQ_TRY(out.alloc(&ps, total));
     // the pair list (:440-458): query cell, then its candidates in order
-    AXSQ_TRY(stash_copy_launch(b, AXSQ_QUERY_BOXES, ws.find_stash.as<int32_t>(), kstash,
-                               ws.find_cnt.as<int32_t>(), offsets, nq, ps, s));
-    if (n_over > 0)
-      AXSQ_TRY(find_launch(b, AXSQ_QUERY_BOXES, 2, qbox, nullptr, nullptr, 6, n_over, tol,
-                           nullptr, counts, offsets, ps, nullptr, 0, nullptr,
-                           ws.find_over.as<int32_t>(), nullptr, s));
-    k_expand_first<<<grid_for(nq), kBlock, 0, s>>>(offsets, counts, nq, pf);
-    AXSQ_CHECK_HIP(hipGetLastError());
+    int32_t* const ids = pairs ? pf : ps;
+    AXSQ_TRY(stash_copy_launch(b, AXSQ_QUERY_BOXES, pairs != nullptr,
+                               ws.find_stash.as<int32_t>(), kstash, ws.find_cnt.as<int32_t>(),
+                               offsets, nq, ids, s));
+    if (v.list > 0)
+      AXSQ_TRY(find_launch(b, AXSQ_QUERY_BOXES, 2, qbox, nullptr, nullptr, 6, v.list, tol,
+                           nullptr, counts, offsets, ids, nullptr, 0, nullptr,
+                           ws.find_over.as<int32_t>(), nullptr, s, pairs != nullptr));
+    if (!pairs) {
+      k_expand_first<<<grid_for(nq), kBlock, 0, s>>>(offsets, counts, nq, pf);
+      AXSQ_CHECK_HIP(hipGetLastError());
+    }
     AXSQ_CHECK_HIP(hipStreamSynchronize(s));
     prof_flush();
   }
   out.keep(pf);
   out.keep(ps);
-  *first = pf;
-  *second = ps;
+  if (pairs) {
+    *pairs = pf;
+  } else {
+    *first = pf;
+    *second = ps;
+  }
   *npairs = total;
   return AXSQ_OK;
+}
+}  // namespace
+
+extern "C" int axsq_mesh_self_intersections(const double* x, const double* y, const double* z,
+                                            int64_t nverts, const int32_t* tris, int64_t ntris,
+                                            double threshold, int32_t** first, int32_t** second,
+                                            int64_t* npairs, int32_t** degenerate,
+                                            int64_t* ndegen, void* stream) {
+  return self_intersections(x, y, z, nverts, tris, ntris, threshold, first, second, nullptr,
+                            npairs, degenerate, ndegen, nullptr, nullptr, stream);
+}
+
+extern "C" int axsq_mesh_self_intersections_alloc(const double* x, const double* y,
+                                                  const double* z, int64_t nverts,
+                                                  const int32_t* tris, int64_t ntris,
+                                                  double threshold, axsq_alloc_fn alloc,
+                                                  void* ctx, int32_t** pairs, int64_t* npairs,
+                                                  int32_t** degenerate, int64_t* ndegen,
+                                                  void* stream) {
+  if (!alloc || !pairs) {
+    set_error("axsq_mesh_self_intersections_alloc: NULL allocator or output");
+    return AXSQ_ERR_INVALID_ARG;
+  }
+  return self_intersections(x, y, z, nverts, tris, ntris, threshold, nullptr, nullptr, pairs,
+                            npairs, degenerate, ndegen, alloc, ctx, stream);
+}
+
+extern "C" int axsq_mesh_candidates(const double* ix, const double* iy, const double* iz,
+                                    int64_t inverts, const int32_t* icells, int64_t nicells,
+                                    const double* qx, const double* qy, const double* qz,
+                                    int64_t qnverts, const int32_t* qcells, int64_t nqcells,
+                                    int nodes_per_cell, int32_t** first, int32_t** second,
+                                    int64_t* npairs, void* stream) {
+  return mesh_candidates(ix, iy, iz, inverts, icells, nicells, qx, qy, qz, qnverts, qcells,
+                         nqcells, nodes_per_cell, first, second, nullptr, npairs, nullptr,
+                         nullptr, stream);
+}
+
+extern "C" int axsq_mesh_candidates_alloc(const double* ix, const double* iy, const double* iz,
+                                          int64_t inverts, const int32_t* icells,
+                                          int64_t nicells, const double* qx, const double* qy,
+                                          const double* qz, int64_t qnverts,
+                                          const int32_t* qcells, int64_t nqcells,
+                                          int nodes_per_cell, axsq_alloc_fn alloc, void* ctx,
+                                          int32_t** pairs, int64_t* npairs, void* stream) {
+  if (!alloc || !pairs) {
+    set_error("axsq_mesh_candidates_alloc: NULL allocator or output");
+    return AXSQ_ERR_INVALID_ARG;
+  }
+  return mesh_candidates(ix, iy, iz, inverts, icells, nicells, qx, qy, qz, qnverts, qcells,
+                         nqcells, nodes_per_cell, nullptr, nullptr, pairs, npairs, alloc, ctx,
+                         stream);
 }

@@ -43,6 +43,7 @@ struct FindArgs {
   const int32_t* fill_cnt;   // fill: each query's room, the counts its count pass wrote
   const int32_t* offsets;
   int32_t* cands;
+  int pairs;  // fill: cands takes (query, id) records
   int32_t* status;
   int32_t* stash;      // count pass: kstash leaf positions per query (or NULL)
   int kstash;
@@ -110,6 +111,14 @@ __device__ __forceinline__ void load_prim(const FindArgs& a, int64_t i, double p
   }
 }
 
+// Candidate k of the whole search: query i's id.
+__device__ __forceinline__ void put_cand(const FindArgs& a, int64_t k, int64_t i, int32_t id) {
+  if (a.pairs)
+    reinterpret_cast<int2*>(a.cands)[k] = make_int2((int32_t)i, id);
+  else
+    a.cands[k] = id;
+}
+
 // The end of a count pass: lists the queries with more than kstash ids, one
 // list slot per wave.
 __device__ __forceinline__ void list_over(const FindArgs& a, bool more, int64_t i) {
@@ -145,7 +154,7 @@ __global__ __launch_bounds__(kBlock) void k_find(FindArgs a) {
     int32_t* const stash = (!FILL && a.stash) ? a.stash + i * a.kstash : nullptr;
     auto emit = [&](int32_t pos) {
       if (FILL) {
-        if (count < room) a.cands[offset + count] = a.leaf_ids[pos];
+        if (count < room) put_cand(a, (int64_t)offset + count, i, a.leaf_ids[pos]);
       } else {
         if (stash && count < a.kstash) stash[count] = pos;
       }
@@ -211,7 +220,7 @@ __global__ __launch_bounds__(kBlock) void k_find_compact(FindArgs a) {
         if (!(valid6(lb) && pred64<KIND>(prim, nullptr, a.tol, lb))) return;
       }
       if (FILL) {
-        if (count < room) a.cands[offset + count] = a.leaf_ids[pos];
+        if (count < room) put_cand(a, (int64_t)offset + count, i, a.leaf_ids[pos]);
       } else {
         if (stash && count < a.kstash) stash[count] = pos;
       }
@@ -406,7 +415,7 @@ constexpr int copy_queries() { return ANY_ORDER ? 16 : 64; }
 // each copies one query per lane; otherwise it copies its queries' ids one
 // query at a time, lane l taking id l, so each load and store is one
 // contiguous run, with eight queries' loads issued before their stores.
-template <bool ANY_ORDER>
+template <bool ANY_ORDER, bool PAIRS>
 __global__ __launch_bounds__(kBlock) void k_stash_copy(const int32_t* __restrict__ stash,
                                                         int kstash,
                                                         const int32_t* __restrict__ stash_cnt,
@@ -415,6 +424,12 @@ __global__ __launch_bounds__(kBlock) void k_stash_copy(const int32_t* __restrict
                                                         int64_t nq, int32_t* __restrict__ cands) {
   const int lane = (int)__lane_id();
   constexpr int Q = copy_queries<ANY_ORDER>();
+  auto put = [&](int32_t k, int64_t i, int32_t id) {
+    if (PAIRS)
+      reinterpret_cast<int2*>(cands)[k] = make_int2((int32_t)i, id);
+    else
+      cands[k] = id;
+  };
   const int64_t base =
       ((int64_t)blockIdx.x * blockDim.x + threadIdx.x - lane) / kWaveLanes * Q;  // the wave's first
   if (base >= nq) return;  // the whole wave
@@ -431,7 +446,7 @@ __global__ __launch_bounds__(kBlock) void k_stash_copy(const int32_t* __restrict
           at = 0;
           for (int32_t t = 0; t < c_me; ++t) at += stash[mine * kstash + t] < pos;
         }
-        cands[o_me + at] = leaf_ids[pos];
+        put(o_me + at, mine, leaf_ids[pos]);
       }
     return;
   }
@@ -458,7 +473,7 @@ __global__ __launch_bounds__(kBlock) void k_stash_copy(const int32_t* __restrict
       if (cc[u] <= kstash && lane < cc[u]) v[u] = leaf_ids[v[u]];
 #pragma unroll
     for (int u = 0; u < 8; ++u)
-      if (cc[u] <= kstash && lane < cc[u]) cands[oo[u] + at[u]] = v[u];
+      if (cc[u] <= kstash && lane < cc[u]) put(oo[u] + at[u], base + j0 + u, v[u]);
   }
 }
 
@@ -511,7 +526,8 @@ hipError_t launch_mode(int kind, bool compact, const FindArgs& a, hipStream_t s)
 int find_launch(const axsq_bvh* b, int kind, int mode, const void* x, const void* y,
                 const void* z, int64_t stride, int64_t nq, double tol, int32_t* counts,
                 const int32_t* fill_cnt, const int32_t* offsets, int32_t* cands, int32_t* stash,
-                int kstash, int32_t* stash_cnt, int32_t* over, uint32_t* nover, hipStream_t s) {
+                int kstash, int32_t* stash_cnt, int32_t* over, uint32_t* nover, hipStream_t s,
+                bool pairs) {
   FindArgs a;
   a.nodes = b->nodes;
   a.fnodes = b->fnodes;
@@ -530,6 +546,7 @@ int find_launch(const axsq_bvh* b, int kind, int mode, const void* x, const void
   a.fill_cnt = fill_cnt;
   a.offsets = offsets;
   a.cands = cands;
+  a.pairs = pairs;
   a.status = b->status;
   a.stash = stash;
   a.kstash = kstash;
@@ -551,18 +568,17 @@ int find_launch(const axsq_bvh* b, int kind, int mode, const void* x, const void
   return AXSQ_OK;
 }
 
-int stash_copy_launch(const axsq_bvh* b, int kind, const int32_t* stash, int kstash,
+int stash_copy_launch(const axsq_bvh* b, int kind, bool pairs, const int32_t* stash, int kstash,
                       const int32_t* stash_cnt, const int32_t* offsets, int64_t nq,
                       int32_t* cands, hipStream_t s) {
   if (nq <= 0) return AXSQ_OK;
   ProfRange pr("bvh_find_copy", s);
-  if (kind == AXSQ_QUERY_RAYS && b->find_ok)
-    k_stash_copy<true><<<grid_for((nq + copy_queries<true>() - 1) / copy_queries<true>() * 64),
-                         kBlock, 0, s>>>(stash, kstash, stash_cnt, offsets, b->leaf_ids, nq,
-                                         cands);
-  else
-    k_stash_copy<false><<<grid_for(nq), kBlock, 0, s>>>(stash, kstash, stash_cnt, offsets,
-                                                        b->leaf_ids, nq, cands);
+  const bool any = kind == AXSQ_QUERY_RAYS && b->find_ok;
+  const int64_t q = any ? copy_queries<true>() : copy_queries<false>();
+  auto* const copy = any ? (pairs ? k_stash_copy<true, true> : k_stash_copy<true, false>)
+                         : (pairs ? k_stash_copy<false, true> : k_stash_copy<false, false>);
+  copy<<<grid_for((nq + q - 1) / q * kWaveLanes), kBlock, 0, s>>>(stash, kstash, stash_cnt,
+                                                                  offsets, b->leaf_ids, nq, cands);
   AXSQ_CHECK_HIP(hipGetLastError());
   return AXSQ_OK;
 }

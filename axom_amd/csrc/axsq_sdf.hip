@@ -2722,7 +2722,7 @@ static int sdf_cull_nodes(axsq_sdf* h, const CullSpace& cs, double diag, hipStre
 
 int sdf_eval_launch(const axsq_sdf* h, const double* x, const double* y, const double* z,
                     int64_t stride, int64_t nq, int fp_mode, double* dist, double* cp,
-                    double* normal, int32_t* elem, bool stats, hipStream_t s) {
+                    double* normal, int32_t* elem, bool stats, hipStream_t s, bool* done) {
   Workspace& ws = workspace();
   const axsq_bvh* b = h->bvh;
   SdfArgs a{};
@@ -2793,10 +2793,12 @@ int sdf_eval_launch(const axsq_sdf* h, const double* x, const double* y, const d
                             (uint64_t)(uintptr_t)z, (uint64_t)stride, (uint64_t)nq};
   if (!cull) return sdf_eval_reference(h, a, false, qkey, mixed, stats, s);
   AXSQ_TRY(ws.cull_list.ensure(sizeof(int32_t) * 3 * (size_t)nq));
-  AXSQ_TRY(ws.cnt.ensure(sizeof(uint32_t) * 4));
+  if (!ws.cull_n.p) ws.cull_n_zero = false;
+  AXSQ_TRY(ws.cull_n.ensure(sizeof(uint32_t) * 4));
   a.redo = ws.cull_list.as<int32_t>();
-  a.nredo = ws.cnt.as<uint32_t>();
-  AXSQ_TRY(fill_i32(reinterpret_cast<int32_t*>(a.nredo), 0, 3, s));
+  a.nredo = ws.cull_n.as<uint32_t>();
+  if (!ws.cull_n_zero) AXSQ_TRY(fill_i32(reinterpret_cast<int32_t*>(a.nredo), 0, 3, s));
+  ws.cull_n_zero = false;
   CullArgs c{};
   c.nodes = cull;
   c.cs = cs;
@@ -2834,12 +2836,21 @@ int sdf_eval_launch(const axsq_sdf* h, const double* x, const double* y, const d
   }
   AXSQ_CHECK_HIP(hipGetLastError());
   p1.stop();
-  uint32_t listed = 0;
-  AXSQ_CHECK_HIP(hipMemcpyAsync(&listed, a.nredo, sizeof(listed), hipMemcpyDeviceToHost, s));
-  AXSQ_CHECK_HIP(hipStreamSynchronize(s));
+  pr.stop();
+  ReadBack r;
+  r.list = a.nredo;
+  r.nlist = 3;
+  r.status[0] = b->status;
+  ReadValues v;
+  AXSQ_TRY(read_back(r, &v, s));
+  ws.cull_n_zero = true;
   hm->last_suspended = 0;
   hm->last_early = 0;
-  if (listed == 0) return AXSQ_OK;
+  *done = true;
+  AXSQ_TRY(status_error(v.status[0]));
+  if (v.list == 0) return AXSQ_OK;
+  *done = false;
+  const int64_t listed = v.list;
   a.order = reinterpret_cast<const uint32_t*>(ws.cull_list.p);
   a.npos = std::min<int64_t>(listed, nq);
   return sdf_eval_reference(h, a, true, qkey, mixed, false, s);

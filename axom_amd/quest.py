@@ -283,27 +283,25 @@ def signed_distance_finalize():
 
 
 # ---- mesh tester ---------------------------------------------------------------
-class _DeviceArray:
-    """A library-owned device int32 array seen through __cuda_array_interface__."""
+class _Int32Blocks:
+    """The blocks a call asks for, as int32 tensors of the current stream."""
 
-    def __init__(self, ptr, n):
-        self.__cuda_array_interface__ = {"shape": (n,), "typestr": "<i4",
-                                         "data": (ptr, False), "version": 2}
+    def __init__(self, device):
+        blocks, errors = [], []  # not through self: a cycle would keep the blocks
 
+        def alloc(_, nbytes):
+            try:
+                blocks.append(torch.empty(nbytes // 4, dtype=torch.int32, device=device))
+                return blocks[-1].data_ptr()
+            except Exception as e:  # raised by check()
+                errors.append(e)
+                return None
+        self.blocks, self._errors, self.fn = blocks, errors, L.ALLOC_FN(alloc)
 
-def _take_int32(ptr, n, device):
-    """Copies a library-allocated device int32 array into a torch tensor and
-    releases the library's copy."""
-    try:
-        if n == 0:
-            return torch.empty(0, dtype=torch.int32, device=device)
-        view = torch.as_tensor(_DeviceArray(ptr, n), device=device)
-        out = view.clone()
-        torch.cuda.current_stream(device).synchronize()
-        return out
-    finally:
-        if ptr:
-            L.lib().axsq_free(ctypes.c_void_p(ptr))
+    def check(self, rc):
+        if self._errors:
+            raise self._errors[0]
+        L.check(rc)
 
 
 def findTriMeshIntersectionsBVH(vertices, triangles, intersectionThreshold=1e-8):
@@ -316,17 +314,15 @@ def findTriMeshIntersectionsBVH(vertices, triangles, intersectionThreshold=1e-8)
     sequential order, and the degenerate triangles' indices, ascending."""
     x, y, z = _soa(vertices)
     t = _dev(triangles, torch.int32, "triangles", 3)
-    pf, ps, pd = ctypes.c_void_p(), ctypes.c_void_p(), ctypes.c_void_p()
+    out = _Int32Blocks(x.device)
+    pp, pd = ctypes.c_void_p(), ctypes.c_void_p()
     npairs, ndeg = ctypes.c_int64(), ctypes.c_int64()
-    L.check(L.lib().axsq_mesh_self_intersections(
+    out.check(L.lib().axsq_mesh_self_intersections_alloc(
         _ptr(x), _ptr(y), _ptr(z), x.shape[0], _ptr(t), t.shape[0], float(intersectionThreshold),
-        ctypes.byref(pf), ctypes.byref(ps), ctypes.byref(npairs), ctypes.byref(pd),
+        out.fn, None, ctypes.byref(pp), ctypes.byref(npairs), ctypes.byref(pd),
         ctypes.byref(ndeg), stream_ptr()))
-    first = _take_int32(pf.value, npairs.value, x.device)
-    second = _take_int32(ps.value, npairs.value, x.device)
-    degen = _take_int32(pd.value, ndeg.value, x.device)
-    return torch.stack([first, second], dim=1), degen
-
+    pairs, degen = out.blocks
+    return pairs[:2 * npairs.value].view(npairs.value, 2), degen[:ndeg.value]
 
 
 def findCandidatesBVH(insertVertices, insertCells, queryVertices, queryCells):
@@ -345,12 +341,10 @@ def findCandidatesBVH(insertVertices, insertCells, queryVertices, queryCells):
     qc = _dev(queryCells, torch.int32, "queryCells")
     if ic.dim() != 2 or qc.dim() != 2 or ic.shape[1] != qc.shape[1]:
         raise ValueError("cells must be (C,k) tensors with the same k for both meshes")
-    pf, ps = ctypes.c_void_p(), ctypes.c_void_p()
-    npairs = ctypes.c_int64()
-    L.check(L.lib().axsq_mesh_candidates(
+    out = _Int32Blocks(ix.device)
+    pp, npairs = ctypes.c_void_p(), ctypes.c_int64()
+    out.check(L.lib().axsq_mesh_candidates_alloc(
         _ptr(ix), _ptr(iy), _ptr(iz), ix.shape[0], _ptr(ic), ic.shape[0],
         _ptr(qx), _ptr(qy), _ptr(qz), qx.shape[0], _ptr(qc), qc.shape[0], int(ic.shape[1]),
-        ctypes.byref(pf), ctypes.byref(ps), ctypes.byref(npairs), stream_ptr()))
-    first = _take_int32(pf.value, npairs.value, ix.device)
-    second = _take_int32(ps.value, npairs.value, ix.device)
-    return torch.stack([first, second], dim=1)
+        out.fn, None, ctypes.byref(pp), ctypes.byref(npairs), stream_ptr()))
+    return out.blocks[0][:2 * npairs.value].view(npairs.value, 2)

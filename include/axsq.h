@@ -405,6 +405,20 @@ int axsq_mesh_self_intersections(const double* x, const double* y, const double*
                                  int64_t* npairs, int32_t** degenerate, int64_t* ndegen,
                                  void* stream);
 
+/* The caller's device memory for a call's results: at least `bytes` bytes that
+ * the call's stream may use, aligned to 8, or NULL, which ends the call with
+ * AXSQ_ERR_NOMEM. Called at most twice, on the calling thread. The block is the
+ * caller's whether or not the call then succeeds. */
+typedef void* (*axsq_alloc_fn)(void* ctx, int64_t bytes);
+
+/* axsq_mesh_self_intersections with the results in the caller's memory: the
+ * first block *pairs, *npairs records (first, second), the second *degenerate. */
+int axsq_mesh_self_intersections_alloc(const double* x, const double* y, const double* z,
+                                       int64_t nverts, const int32_t* tris, int64_t ntris,
+                                       double threshold, axsq_alloc_fn alloc, void* ctx,
+                                       int32_t** pairs, int64_t* npairs, int32_t** degenerate,
+                                       int64_t* ndegen, void* stream);
+
 /* Candidate pairs between two meshes of cells with nodes_per_cell nodes each
  * (hexahedra: 8): findCandidatesBVH of src/axom/quest/examples/
  * quest_candidates_example.cpp:397-495. Each cell's bounding box
@@ -421,6 +435,15 @@ int axsq_mesh_candidates(const double* ix, const double* iy, const double* iz, i
                          const double* qy, const double* qz, int64_t qnverts,
                          const int32_t* qcells, int64_t nqcells, int nodes_per_cell,
                          int32_t** first, int32_t** second, int64_t* npairs, void* stream);
+
+/* axsq_mesh_candidates with the result in the caller's memory: *pairs, *npairs
+ * records (first, second). */
+int axsq_mesh_candidates_alloc(const double* ix, const double* iy, const double* iz,
+                               int64_t inverts, const int32_t* icells, int64_t nicells,
+                               const double* qx, const double* qy, const double* qz,
+                               int64_t qnverts, const int32_t* qcells, int64_t nqcells,
+                               int nodes_per_cell, axsq_alloc_fn alloc, void* ctx,
+                               int32_t** pairs, int64_t* npairs, void* stream);
 
 #ifdef __cplusplus
 }

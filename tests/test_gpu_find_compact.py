@@ -222,3 +222,44 @@ def test_self_intersections_on_compact_nodes(scene, n):
     want, want_degen = orc.mesh_self_intersections(v, t)
     assert np.array_equal(pairs.cpu().numpy().reshape(-1, 2), want.reshape(-1, 2))
     assert np.array_equal(degen.cpu().numpy(), want_degen)
+
+
+def test_pair_lists_in_arrays_of_their_own_and_in_the_callers_memory():
+    """Both forms of the two pair searches give the same lists; an allocator
+    that gives nothing ends the call with an error and no result."""
+    rng = np.random.default_rng(9)
+    n = 700
+    v = rng.uniform(-1, 1, (n, 1, 3)) + rng.normal(0, 0.08, (n, 3, 3))
+    x, y, z = (_t(v.reshape(-1, 3)[:, d]) for d in range(3))
+    t = _t(np.arange(3 * n, dtype=np.int32).reshape(n, 3))
+    vp = ctypes.c_void_p
+
+    def take(ptr, count):
+        out = torch.empty(count, dtype=torch.int32, device=DEV)
+        hip = ctypes.CDLL("libamdhip64.so")
+        assert hip.hipMemcpy(vp(out.data_ptr()), ptr, ctypes.c_size_t(4 * count), 3) == 0
+        L.check(L.lib().axsq_free(ptr))
+        return out.cpu().numpy()
+
+    pairs, degen = quest.findTriMeshIntersectionsBVH((x, y, z), t)
+    a, b, d, np_, nd = vp(), vp(), vp(), ctypes.c_int64(), ctypes.c_int64()
+    mesh = (spin._ptr(x), spin._ptr(y), spin._ptr(z), 3 * n, spin._ptr(t), n)
+    L.check(L.lib().axsq_mesh_self_intersections(
+        *mesh, 1e-8, ctypes.byref(a), ctypes.byref(b), ctypes.byref(np_), ctypes.byref(d),
+        ctypes.byref(nd), None))
+    assert np_.value == pairs.shape[0] > 0 and nd.value == degen.numel()
+    assert np.array_equal(np.stack([take(a, np_.value), take(b, np_.value)], 1),
+                          pairs.cpu().numpy())
+    L.check(L.lib().axsq_free(d))
+
+    pairs = quest.findCandidatesBVH((x, y, z), t, (x, y, z), t)
+    L.check(L.lib().axsq_mesh_candidates(*mesh, *mesh, 3, ctypes.byref(a), ctypes.byref(b),
+                                         ctypes.byref(np_), None))
+    assert np_.value == pairs.shape[0] > n
+    assert np.array_equal(np.stack([take(a, np_.value), take(b, np_.value)], 1),
+                          pairs.cpu().numpy())
+
+    none = L.ALLOC_FN(lambda ctx, nbytes: None)
+    rc = L.lib().axsq_mesh_candidates_alloc(*mesh, *mesh, 3, none, None, ctypes.byref(a),
+                                            ctypes.byref(np_), None)
+    assert rc == L.ERRORS_BY_NAME["AXSQ_ERR_NOMEM"] and not a.value and np_.value == 0
