@@ -1,14 +1,9 @@
 // axsq_prims.hip -- scan and stable radix sort for gfx950 (wave64).
 //
-// Radix sort: least-significant-digit first, 8-bit digits; per pass a tile
-// histogram, an exclusive scan of the digit-major histogram and a stable
-// scatter. With at most 256 tiles the scatter does the scan itself (two
-// kernels per pass instead of five), and inputs of at most 262,144 keys use
-// tiles of 1,024 keys instead of 4,096. Inside a tile of 256 threads x ITEMS
-// keys, keys are ranked in global order: sub-tile k covers
-// [base + 256k, base + 256k + 256) and each 64-lane wave finds the lanes that
-// share its digit with 8 ballots, so equal keys keep their input order and the
-// result equals a stable sort.
+// Radix sort: least-significant-digit first, digits of up to 8 bits; per pass
+// a tile histogram, a scan over the tiles and a stable scatter. Inputs of at
+// most 262,144 keys use tiles of 1,024 keys instead of 4,096 and the scatter
+// does the scan itself (two kernels per pass).
 #include <stdarg.h>
 #include <stdio.h>
 
@@ -147,64 +142,108 @@ __global__ __launch_bounds__(kBlock) void k_scan_tiles(const T* __restrict__ in,
 
 // ---- radix sort -------------------------------------------------------------
 // ITEMS keys per thread make a tile of kBlock * ITEMS keys per workgroup. The
-// histogram is digit-major (hist[digit * nblocks + tile], the order the scan
-// needs) or, for a scatter that sums it itself, tile-major
-// (hist[tile * 256 + digit], so that those sums read it coalesced).
+// histogram is digit-major (hist[digit * nblocks + tile]: a scan over the
+// tiles reads rows) or, for a scatter that sums it itself, tile-major
+// (hist[tile * 256 + digit]).
 template <int ITEMS, bool TILE_MAJOR>
 __global__ __launch_bounds__(kBlock) void k_radix_hist(const uint32_t* __restrict__ keys,
                                                         int64_t n, int shift, int nbits,
                                                         uint32_t* __restrict__ hist,
                                                         int64_t nblocks) {
+  static_assert(kBlock == 256, "a digit per thread");
   __shared__ uint32_t s_h[256];
   s_h[threadIdx.x] = 0;
   __syncthreads();
   const uint32_t mask = (1u << nbits) - 1u;
   const int64_t base = (int64_t)blockIdx.x * (kBlock * ITEMS);
+  uint32_t kk[ITEMS];
 #pragma unroll
   for (int k = 0; k < ITEMS; ++k) {
     const int64_t i = base + k * kBlock + threadIdx.x;
-    if (i < n) atomicAdd(&s_h[(keys[i] >> shift) & mask], 1u);
+    kk[k] = i < n ? (keys[i] >> shift) & mask : 0u;
   }
+#pragma unroll
+  for (int k = 0; k < ITEMS; ++k)
+    if (base + k * kBlock + threadIdx.x < n) atomicAdd(&s_h[kk[k]], 1u);
   __syncthreads();
   if (TILE_MAJOR)
     hist[(int64_t)blockIdx.x * 256 + threadIdx.x] = s_h[threadIdx.x];
-  else
+  else if (threadIdx.x <= mask)
     hist[(int64_t)threadIdx.x * nblocks + blockIdx.x] = s_h[threadIdx.x];
 }
 
-// Stable scatter of one digit. The output position of digit d's first key in
-// this tile is either read from the exclusively scanned digit-major
-// histogram (SCANNED) or, when there are few tiles, found here from the raw
-// tile-major histogram: the keys of smaller digits everywhere plus the keys of
-// digit d in earlier tiles (16 loads in flight per thread). All of the tile's keys are loaded before the ranking loop so
-// that their latencies overlap.
+// One block per digit: its row of tile counts to exclusive sums, in place, and
+// the row's total.
+__global__ __launch_bounds__(kBlock) void k_radix_rows(uint32_t* __restrict__ hist,
+                                                       int64_t nblocks,
+                                                       uint32_t* __restrict__ totals) {
+  __shared__ uint32_t s_w[kWavesPerBlock];
+  uint32_t* row = hist + (int64_t)blockIdx.x * nblocks;
+  uint32_t run = 0;
+  for (int64_t b0 = 0; b0 < nblocks; b0 += kBlock * 4) {
+    uint32_t v[4], sum = 0;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      const int64_t b = b0 + 4 * (int64_t)threadIdx.x + k;
+      v[k] = b < nblocks ? row[b] : 0u;
+      sum += v[k];
+    }
+    uint32_t all;
+    uint32_t at = run + block_exclusive<uint32_t>(sum, s_w, &all);
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      const int64_t b = b0 + 4 * (int64_t)threadIdx.x + k;
+      if (b < nblocks) row[b] = at;
+      at += v[k];
+    }
+    run += all;
+  }
+  if (threadIdx.x == 0) totals[blockIdx.x] = run;
+}
+
+// Stable scatter of one digit. Each wave ranks its ITEMS * 64 consecutive keys
+// by itself (the lanes that share a digit by ballots, the earlier ones by a
+// counter per digit), one barrier orders the waves, and the tile is put in
+// digit order in LDS, so that it is written as one run per digit: ranking the
+// block 256 keys at a time took three barriers each and wrote every key where
+// it fell. Where a digit's first key of the tile goes is the keys of smaller
+// digits everywhere plus its own in earlier tiles: from the scanned rows and
+// their totals (SCANNED), or, where there are few tiles, summed here from the
+// raw tile-major histogram (16 loads in flight per thread).
+// 4M keys, a pass of histogram, scan and scatter with 8-bit digits: 70 us before
+// (45 the scatter), 42 now (26), of 13 that reading and writing takes; 6-bit
+// digits 38.
 template <int ITEMS, bool SCANNED>
 __global__ __launch_bounds__(kBlock) void k_radix_scatter(
     const uint32_t* __restrict__ keys, const uint32_t* __restrict__ vals, int64_t n, int shift,
-    int nbits, const uint32_t* __restrict__ hist, int64_t nblocks,
-    uint32_t* __restrict__ keys_out, uint32_t* __restrict__ vals_out,
-    uint32_t* __restrict__ next_hist = nullptr, int next_shift = 0, int next_nbits = 0) {
-  __shared__ uint32_t s_base[256];
-  __shared__ uint32_t s_wcnt[kWavesPerBlock][256];
+    int nbits, const uint32_t* __restrict__ hist, const uint32_t* __restrict__ totals,
+    int64_t nblocks, uint32_t* __restrict__ keys_out, uint32_t* __restrict__ vals_out) {
+  constexpr int TILE = kBlock * ITEMS;
+  __shared__ uint32_t s_cnt[kWavesPerBlock][256];  // counts, then where a wave's digit starts
+  __shared__ uint32_t s_first[256];                // output position less the place in the tile
+  __shared__ uint32_t s_key[TILE], s_val[TILE];
   __shared__ uint32_t s_w[kWavesPerBlock];
-  const int t = threadIdx.x;
-  const int wid = t / kWave;
+  const int t = threadIdx.x, wid = t / kWave, lane = (int)__lane_id();
   const uint64_t lt = lanemask_lt();
   const uint32_t mask = (1u << nbits) - 1u;
-  const int64_t base = (int64_t)blockIdx.x * (kBlock * ITEMS);
+  const int64_t base = (int64_t)blockIdx.x * TILE;
+  const int m = n - base < TILE ? (int)(n - base) : TILE;
   uint32_t kk[ITEMS], vv[ITEMS];
 #pragma unroll
   for (int k = 0; k < ITEMS; ++k) {
-    const int64_t i = base + k * kBlock + t;
-    kk[k] = (i < n) ? keys[i] : 0u;
-    vv[k] = (i < n) ? vals[i] : 0u;
+    const int j = (wid * ITEMS + k) * kWave + lane;
+    kk[k] = j < m ? keys[base + j] : 0u;
+    vv[k] = j < m ? vals[base + j] : 0u;
   }
+  uint32_t tot = 0, pre = 0;  // of digit t
   if constexpr (SCANNED) {
-    s_base[t] = hist[(int64_t)t * nblocks + blockIdx.x];
+    if (t <= mask) {
+      tot = totals[t];
+      pre = hist[(int64_t)t * nblocks + blockIdx.x];
+    }
   } else {
     const uint32_t* h = hist + t;
     const int64_t me = blockIdx.x;
-    uint32_t pre = 0, tot = 0;
     int64_t b = 0;
     for (; b + 16 <= nblocks; b += 16) {
       uint32_t x[16];
@@ -221,46 +260,53 @@ __global__ __launch_bounds__(kBlock) void k_radix_scatter(
       tot += x;
       pre += (b < me) ? x : 0u;
     }
-    s_base[t] = block_exclusive<uint32_t>(tot, s_w, nullptr) + pre;
   }
 #pragma unroll
-  for (int w = 0; w < kWavesPerBlock; ++w) s_wcnt[w][t] = 0;
-  __syncthreads();
+  for (int w = 0; w < kWavesPerBlock; ++w) s_cnt[w][t] = 0;
+  const uint32_t out = block_exclusive<uint32_t>(tot, s_w, nullptr) + pre;  // (and a barrier)
+  uint32_t rank[ITEMS];
 #pragma unroll
   for (int k = 0; k < ITEMS; ++k) {
-    const int64_t i = base + k * kBlock + t;
-    const bool valid = i < n;
-    const uint32_t key = kk[k], val = vv[k];
-    const uint32_t d = valid ? (key >> shift) & mask : 0u;
+    const bool valid = (wid * ITEMS + k) * kWave + lane < m;
+    const uint32_t d = (kk[k] >> shift) & mask;
     uint64_t peers = __ballot(valid);
     for (int b = 0; b < nbits; ++b) {
       const bool bit = (d >> b) & 1u;
       const uint64_t bb = __ballot(valid && bit);
       peers &= bit ? bb : ~bb;
     }
-    const uint32_t rank = (uint32_t)__popcll(peers & lt);
-    const bool leader = valid && ((peers & lt) == 0);
-    if (leader) s_wcnt[wid][d] = (uint32_t)__popcll(peers);
-    __syncthreads();
-    if (valid) {
-      uint32_t pos = s_base[d] + rank;
-      for (int w = 0; w < wid; ++w) pos += s_wcnt[w][d];
-      keys_out[pos] = key;
-      vals_out[pos] = val;
-      if (next_hist)  // the next pass's tile histogram, tiles of kBlock * ITEMS keys
-        atomicAdd(&next_hist[(int64_t)(pos / (kBlock * ITEMS)) * 256 +
-                             ((key >> next_shift) & ((1u << next_nbits) - 1u))],
-                  1u);
-    }
-    __syncthreads();
-    uint32_t add = 0;
+    const uint32_t before = valid ? s_cnt[wid][d] : 0u;
+    wave_sync();
+    rank[k] = before + (uint32_t)__popcll(peers & lt);
+    if (valid && (peers & lt) == 0) s_cnt[wid][d] = before + (uint32_t)__popcll(peers);
+    wave_sync();
+  }
+  __syncthreads();
+  uint32_t cnt = 0;
 #pragma unroll
-    for (int w = 0; w < kWavesPerBlock; ++w) {
-      add += s_wcnt[w][t];
-      s_wcnt[w][t] = 0;
-    }
-    s_base[t] += add;
-    __syncthreads();
+  for (int w = 0; w < kWavesPerBlock; ++w) {
+    const uint32_t c = s_cnt[w][t];
+    s_cnt[w][t] = cnt;
+    cnt += c;
+  }
+  const uint32_t place = block_exclusive<uint32_t>(cnt, s_w, nullptr);
+#pragma unroll
+  for (int w = 0; w < kWavesPerBlock; ++w) s_cnt[w][t] += place;
+  s_first[t] = out - place;
+  __syncthreads();
+#pragma unroll
+  for (int k = 0; k < ITEMS; ++k) {
+    if ((wid * ITEMS + k) * kWave + lane >= m) continue;
+    const uint32_t at = s_cnt[wid][(kk[k] >> shift) & mask] + rank[k];
+    s_key[at] = kk[k];
+    s_val[at] = vv[k];
+  }
+  __syncthreads();
+  for (int j = t; j < m; j += kBlock) {
+    const uint32_t key = s_key[j];
+    const uint32_t at = s_first[(key >> shift) & mask] + (uint32_t)j;
+    keys_out[at] = key;
+    vals_out[at] = s_val[j];
   }
 }
 
@@ -441,48 +487,36 @@ int radix_sort_pairs(uint32_t* keys, uint32_t* vals, uint32_t* keys_alt, uint32_
     set_error("radix sort: %lld keys exceed the int32 position range", (long long)n);
     return AXSQ_ERR_INVALID_ARG;
   }
-  // Small inputs take 1,024-key tiles, so that more workgroups share the work;
-  // with at most kFewTiles tiles the scatter scans the histogram itself.
-  constexpr int64_t kFewTiles = 256;
-  const bool small = n <= kFewTiles * kBlock * 4;
+  // Small inputs take 1,024-key tiles, so that more workgroups share the work,
+  // at most 256 of them, whose histogram the scatter sums itself. The passes
+  // share the bits evenly: fewer digits make longer runs (17 bits in two digits
+  // of 9 and 8 took 115 us for 4M keys, in three of 6, 6 and 5 112).
+  const bool small = n <= 256 * kBlock * 4;
   const int64_t tile = small ? kBlock * 4 : kTile;
   const int64_t nb = (n + tile - 1) / tile;
-  const bool few = nb <= kFewTiles;
-  const int64_t nh = 256 * nb;
-  AXSQ_TRY(ws.hist.ensure(sizeof(uint32_t) * (size_t)nh));
+  const int passes = (bits + 7) / 8;
+  AXSQ_TRY(ws.hist.ensure(sizeof(uint32_t) * (size_t)(256 * (nb + 1))));
   uint32_t* hist = ws.hist.as<uint32_t>();
-  AXSQ_TRY(ws.misc.ensure(sizeof(int64_t) * 2));
+  uint32_t* totals = hist + 256 * nb;
   uint32_t *ki = keys, *vi = vals, *ko = keys_alt, *vo = vals_alt;
-  for (int shift = 0; shift < bits; shift += 8) {
-    const int nbits = (bits - shift < 8) ? bits - shift : 8;
+  const unsigned g = (unsigned)nb;
+  for (int pass = 0, shift = 0; pass < passes; ++pass) {
+    const int left = passes - pass;
+    const int nbits = (bits - shift + left - 1) / left;
     if (small) {
-      k_radix_hist<4, true><<<(unsigned)nb, kBlock, 0, s>>>(ki, n, shift, nbits, hist, nb);
-      AXSQ_CHECK_HIP(hipGetLastError());
-      k_radix_scatter<4, false><<<(unsigned)nb, kBlock, 0, s>>>(ki, vi, n, shift, nbits, hist,
-                                                                  nb, ko, vo);
+      k_radix_hist<4, true><<<g, kBlock, 0, s>>>(ki, n, shift, nbits, hist, nb);
+      k_radix_scatter<4, false><<<g, kBlock, 0, s>>>(ki, vi, n, shift, nbits, hist, totals, nb,
+                                                     ko, vo);
     } else {
-      if (few)
-        k_radix_hist<kItems, true><<<(unsigned)nb, kBlock, 0, s>>>(ki, n, shift, nbits, hist, nb);
-      else
-        k_radix_hist<kItems, false><<<(unsigned)nb, kBlock, 0, s>>>(ki, n, shift, nbits, hist, nb);
-      AXSQ_CHECK_HIP(hipGetLastError());
-      if (few) {
-        k_radix_scatter<kItems, false><<<(unsigned)nb, kBlock, 0, s>>>(ki, vi, n, shift, nbits,
-                                                                       hist, nb, ko, vo);
-      } else {
-        AXSQ_TRY(scan_exclusive_i32((const int32_t*)hist, (int32_t*)hist, nh,
-                                    ws.misc.as<int64_t>(), ws, s));
-        k_radix_scatter<kItems, true><<<(unsigned)nb, kBlock, 0, s>>>(ki, vi, n, shift, nbits,
-                                                                      hist, nb, ko, vo);
-      }
+      k_radix_hist<kItems, false><<<g, kBlock, 0, s>>>(ki, n, shift, nbits, hist, nb);
+      k_radix_rows<<<1u << nbits, kBlock, 0, s>>>(hist, nb, totals);
+      k_radix_scatter<kItems, true><<<g, kBlock, 0, s>>>(ki, vi, n, shift, nbits, hist, totals,
+                                                         nb, ko, vo);
     }
     AXSQ_CHECK_HIP(hipGetLastError());
-    uint32_t* t = ki;
-    ki = ko;
-    ko = t;
-    t = vi;
-    vi = vo;
-    vo = t;
+    shift += nbits;
+    std::swap(ki, ko);
+    std::swap(vi, vo);
   }
   *keys_out = ki;
   *vals_out = vi;

@@ -1808,13 +1808,14 @@ __global__ __launch_bounds__(kBlock) void k_susp_keys(const SdfSuspended* __rest
   vals[j] = (uint32_t)j;
 }
 
-// Morton code of each query in the mesh's bounding box (ordering only).
+// Morton code of each query in the mesh's bounding box, less its lowest `drop`
+// bits (ordering only).
 __global__ __launch_bounds__(kBlock) void k_query_codes(const double* __restrict__ qx,
                                                          const double* __restrict__ qy,
                                                          const double* __restrict__ qz,
                                                          int64_t qs, int64_t nq, double lo0,
                                                          double lo1, double lo2, double s0,
-                                                         double s1, double s2,
+                                                         double s1, double s2, int drop,
                                                          uint32_t* __restrict__ keys,
                                                          uint32_t* __restrict__ vals) {
   const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -1822,7 +1823,7 @@ __global__ __launch_bounds__(kBlock) void k_query_codes(const double* __restrict
   const double c[3] = {qx[i * qs], qy[i * qs], qz[i * qs]};
   const double minc[3] = {lo0, lo1, lo2};
   const double inv[3] = {s0, s1, s2};
-  keys[i] = morton_of(c, minc, inv);
+  keys[i] = morton_of(c, minc, inv) >> drop;
   vals[i] = (uint32_t)i;
 }
 
@@ -2766,7 +2767,8 @@ int sdf_eval_launch(const axsq_sdf* h, const double* x, const double* y, const d
     cs.scale = std::ldexp(1.0, 1 - e2);
     AXSQ_TRY(sdf_cull_nodes(hm, cs, diag, s, &cull));
   }
-  if (h->sort_queries && nq > 4096) {
+  // a wave per query (below) needs no order: 5,000 queries 103 us sorted, 75 not
+  if (h->sort_queries && nq > (cull ? kCoopQueries : 4096)) {
     AXSQ_TRY(ws.k0.ensure(sizeof(uint32_t) * nq));
     AXSQ_TRY(ws.v0.ensure(sizeof(uint32_t) * nq));
     AXSQ_TRY(ws.k1.ensure(sizeof(uint32_t) * nq));
@@ -2776,15 +2778,21 @@ int sdf_eval_launch(const axsq_sdf* h, const double* x, const double* y, const d
       const double ext = h->domain[3 + d] - h->domain[d];
       inv[d] = ext > 0.0 ? 1.0 / ext : 0.0;
     }
+    // As many bits as bring a wave's 64 queries together also where they lie
+    // along a surface, which crosses about 3 * 4^b of the 8^b cells of b bits an
+    // axis, and no more: each 8 are a pass. 16 bits for up to 262,144 queries (50
+    // a cell), 21 above (80 for 4M). The whole call with 16 / 21 / 30 bits: 60,000
+    // near a surface 270 / 280 / 301 us, 1M 820 / 825 / 854, 4M 5885 / 5670 / 5688.
+    const int bits = nq <= 262144 ? 16 : 21;
     ProfRange pq("sdf_query_order", s);
     k_query_codes<<<grid_for(nq), kBlock, 0, s>>>(x, y, z, stride, nq, h->domain[0],
                                                   h->domain[1], h->domain[2], inv[0], inv[1],
-                                                  inv[2], ws.k0.as<uint32_t>(),
+                                                  inv[2], 30 - bits, ws.k0.as<uint32_t>(),
                                                   ws.v0.as<uint32_t>());
     AXSQ_CHECK_HIP(hipGetLastError());
     uint32_t *sk, *sv;
     AXSQ_TRY(radix_sort_pairs(ws.k0.as<uint32_t>(), ws.v0.as<uint32_t>(), ws.k1.as<uint32_t>(),
-                              ws.v1.as<uint32_t>(), nq, 30, ws, s, &sk, &sv));
+                              ws.v1.as<uint32_t>(), nq, bits, ws, s, &sk, &sv));
     pq.stop();
     a.order = sv;
   }
@@ -2816,7 +2824,9 @@ int sdf_eval_launch(const axsq_sdf* h, const double* x, const double* y, const d
   // triangles, 128 steps 0.30 / 0.61 ms, 256 0.40 / 0.62, 512 0.57 / 0.82;
   // 250,000: 0.43 / 1.60, 0.50 / 1.02, 0.66 / 1.20; 1.5M: 1.2 / 7.6, 1.03 /
   // 3.8, 1.17 / 3.2.
-  c.steps = nq <= 65536 ? 128 : nq <= 786432 ? 256 : 512;
+  // At most 65,536: 30,011 on 20,480 triangles 0.224 / 0.208 / 0.232 with 64, 96
+  // and 128 steps, 60,000 on 327,680 0.354 / 0.261 / 0.270.
+  c.steps = nq <= 65536 ? 96 : nq <= 786432 ? 256 : 512;
   ProfRange p1(mixed ? "sdf_eval_fp32_cull" : "sdf_eval_fp64_cull", s);
   // one lane per query, then one wave per long walk; a small batch one wave
   // per query at once
