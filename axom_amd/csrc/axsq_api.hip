@@ -1118,6 +1118,7 @@ int axsq_sdf_destroy(axsq_sdf* h) {
   hipFree(h->skip);
   hipFree(h->wsteps);
   hipFree(h->cull);
+  hipFree(h->cull_norms);
   if (h->early_done) hipEventDestroy(h->early_done);
   hipFree(h->v2t_start);
   hipFree(h->v2t_end);

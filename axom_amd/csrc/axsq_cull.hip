@@ -115,13 +115,15 @@ __device__ __forceinline__ float tri_tau(const double T[9], double reach) {
   return (float)(tau * 1.000001);
 }
 
-// Per leaf: tau, and the running sum of normals within its block of 256.
+// Per leaf: tau, its triangles' NormRec, and the running sum of normals within
+// its block of 256.
 template <bool CELLS>
 __global__ __launch_bounds__(kBlock) void k_cull_leaf(const TriRec* __restrict__ tris, int64_t n,
                                                        double reach, double tau_max, double scale,
                                                        float* __restrict__ tau,
                                                        double* __restrict__ pre,
                                                        double* __restrict__ totals,
+                                                       NormRec* __restrict__ norms,
                                                        int32_t* __restrict__ ctl) {
   __shared__ double s_w[kBlock / kCullWave][3];
   const int64_t pos = (int64_t)blockIdx.x * kBlock + threadIdx.x;
@@ -136,6 +138,11 @@ __global__ __launch_bounds__(kBlock) void k_cull_leaf(const TriRec* __restrict__
       t = (te < 0.0f || t < 0.0f) ? -1.0f : fmaxf(t, te);
       tri_normal(T, m);
       for (int d = 0; d < 3; ++d) nr[d] += m[d];
+      NormRec r;
+      unit3(m, r.un);
+      const bool flat = tri_degenerate(m);
+      for (int k = 0; k < 3; ++k) r.angle[k] = flat ? -1.0 : tri_angle(T, k);
+      norms[CELLS ? 2 * pos + e : pos] = r;
     }
     if (!(t >= 0.0f && t <= tau_max)) {
       atomicOr(&ctl[0], 1);
@@ -470,7 +477,7 @@ __global__ __launch_bounds__(kBlock) void k_cull_large_end(const Node64* __restr
 
 template <bool CELLS>
 int build(const axsq_bvh* b, const TriRec* tris, const CullSpace& cs, double diag, CullNode* out,
-          Workspace& ws, int32_t* bad, hipStream_t s) {
+          NormRec* norms, Workspace& ws, int32_t* bad, hipStream_t s) {
   const int64_t n = b->n;
   const int32_t ninner = (int32_t)(n - 1);
   const int64_t nb = grid_for(n);
@@ -494,7 +501,7 @@ int build(const axsq_bvh* b, const TriRec* tris, const CullSpace& cs, double dia
   AXSQ_TRY(fill_i32(ctl, 0, 4, s));
   k_cull_leaf<CELLS><<<(unsigned)nb, kBlock, 0, s>>>(tris, n, kCullReach * diag,
                                                      diag * (1.0 / 1024.0), cs.scale, tau, pre, totals,
-                                                     ctl);
+                                                     norms, ctl);
   AXSQ_CHECK_HIP(hipGetLastError());
   k_cull_scan<<<1, 1024, 0, s>>>(totals, nb);
   AXSQ_CHECK_HIP(hipGetLastError());
@@ -523,10 +530,10 @@ int build(const axsq_bvh* b, const TriRec* tris, const CullSpace& cs, double dia
 }  // namespace
 
 int cull_build(const axsq_bvh* b, const TriRec* tris, bool cells, const CullSpace& cs, double diag,
-               CullNode* out, int32_t* bad, hipStream_t s) {
+               CullNode* out, NormRec* norms, int32_t* bad, hipStream_t s) {
   Workspace& ws = workspace();
-  return cells ? build<true>(b, tris, cs, diag, out, ws, bad, s)
-               : build<false>(b, tris, cs, diag, out, ws, bad, s);
+  return cells ? build<true>(b, tris, cs, diag, out, norms, ws, bad, s)
+               : build<false>(b, tris, cs, diag, out, norms, ws, bad, s);
 }
 
 }  // namespace axsq

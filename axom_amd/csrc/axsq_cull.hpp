@@ -68,6 +68,18 @@ struct __attribute__((aligned(16))) CullNode {
 };
 static_assert(sizeof(CullNode) == 80, "CullNode is five 16-byte loads");
 
+// A triangle's part of a pseudo-normal sum: its unit normal and its angle at
+// each corner, or -1 where a degenerate triangle adds nothing. Computed once a
+// mesh by normal_term's own operations, so the sums are the same: a query on a
+// vertex adds about six terms of some 600 FP64 instructions each (square roots,
+// divisions, an arc cosine). The walk of 4M queries on 81,920 triangles: 3.77 ms
+// without the table, 3.59 with it.
+struct __attribute__((aligned(16))) NormRec {
+  double un[3];
+  double angle[3];
+};
+static_assert(sizeof(NormRec) == 48, "NormRec is three 16-byte loads");
+
 // Queries farther than this many mesh diagonals from the mesh's farthest
 // corner go to the reference walk: tau is computed for that distance.
 constexpr double kCullReach = 4.0;

@@ -435,6 +435,11 @@ __device__ __forceinline__ double tri_angle(const double* T, int idx) {
   return acos(dp);
 }
 
+// Triangle::degenerate (Triangle.hpp:104-109,327-330) from the triangle's normal.
+__device__ __forceinline__ bool tri_degenerate(const double n[3]) {
+  return near_eq(0.5 * sqrt(dot3(n[0], n[1], n[2], n[0], n[1], n[2])), 0.0, 1.0e-12);
+}
+
 // intersect_ray_bbox_test per axis, primal/operators/detail/intersect_ray_impl.hpp:150-187,
 // with utilities::max/min (core/utilities/Utilities.hpp:80-96). invn = 1.0 / n.
 __device__ __forceinline__ bool ray_slab(double x0, double n, double invn, double bmin,

@@ -266,6 +266,7 @@ struct axsq_sdf {
   // oriented child boxes of the culled walk (axsq_cull.hpp), one per inner
   // node: 0 not built for the current vertices, 1 built, -1 not usable
   axsq::CullNode* cull = nullptr;
+  axsq::NormRec* cull_norms = nullptr;  // with cull: one per triangle record
   int cull_state = 0;
   std::atomic<bool> evaluated{false};  // since the vertices were set
   std::mutex cull_mu;       // held while a call builds them
@@ -284,7 +285,7 @@ void bvh_release(axsq_bvh* b);
 // coordinates, diag: the mesh's diagonal) into out, n - 1 records; *bad is set
 // when they must not be used. Returns after the stream has run them.
 int cull_build(const axsq_bvh* b, const TriRec* tris, bool cells, const CullSpace& cs, double diag,
-               CullNode* out, int32_t* bad, hipStream_t s);
+               CullNode* out, NormRec* norms, int32_t* bad, hipStream_t s);
 // n 2-D boxes (4 doubles) -> 3-D boxes with z range [0, 0] (6 doubles)
 int widen_boxes2d(const double* boxes2d, int64_t n, double* out, hipStream_t s);
 // Candidate search launches (axsq_query.hip). mode 0: count pass (keeping the

@@ -138,8 +138,7 @@ __device__ __forceinline__ void normal_term(const double T[9], int code, double 
     return;
   }
   c[0] = c[1] = c[2] = 0.0;
-  const double area = 0.5 * sqrt(dot3(n[0], n[1], n[2], n[0], n[1], n[2]));
-  if (!near_eq(area, 0.0, 1.0e-12)) {
+  if (!tri_degenerate(n)) {
     const double alpha = tri_angle(T, code);
     unit3(n, un);
     c[0] = un[0] * alpha;
@@ -221,6 +220,19 @@ __device__ __forceinline__ void add_terms(double sn[3], const TriRec* __restrict
     sn[1] += c[1];
     sn[2] += c[2];
   }
+}
+
+// The term of list entry e from the table (normal_term's values).
+__device__ __forceinline__ void table_term(const NormRec* __restrict__ norms, uint32_t e,
+                                           double c[3]) {
+  const double2* p = reinterpret_cast<const double2*>(norms + (e >> 2));
+  const double2 r0 = p[0], r1 = p[1], r2 = p[2];
+  const int code = (int)(e & 3u);
+  const double al = code == 0 ? r1.y : code == 1 ? r2.x : r2.y;
+  const bool edge = code == 3, none = !edge && al < 0.0;
+  c[0] = edge ? r0.x : none ? 0.0 : r0.x * al;
+  c[1] = edge ? r0.y : none ? 0.0 : r0.y * al;
+  c[2] = edge ? r1.x : none ? 0.0 : r1.x * al;
 }
 
 // Surface normal (getSurfaceNormal, SignedDistance.hpp:741-749), sign
@@ -506,6 +518,7 @@ constexpr int64_t kCoopWaves = 4096;  // waves that share the long walks
 
 struct CullArgs {
   const CullNode* nodes;
+  const NormRec* norms;
   CullSpace cs;    // mesh coordinates
   double reach2;   // squared reach: queries farther from the mesh are listed
   float cmax;      // largest coordinate of the mesh's box, by magnitude
@@ -750,7 +763,11 @@ __global__ __launch_bounds__(kWaveLanes) AXSQ_CULL_WAVES_ATTR void k_sdf_cull(Sd
     a.redo[atomicAdd(a.nredo, 1u)] = (int32_t)i;  // one slot per query
     return;
   }
-  add_terms(m.sn, a.tris, terms, 1, nterms);
+  for (int32_t j = 0; j < nterms; ++j) {
+    double t[3];
+    table_term(c.norms, (uint32_t)terms[j], t);
+    for (int d = 0; d < 3; ++d) m.sn[d] += t[d];
+  }
   sdf_finish(a, i, q, m, cn);
 }
 
@@ -1057,12 +1074,7 @@ __global__ __launch_bounds__(kWaveLanes) void k_sdf_coop(SdfArgs a, CullArgs c, 
       // the recorded terms, one lane each, added in their order
       __syncthreads();
       double t[3] = {0.0, 0.0, 0.0};
-      if (lane < nterms) {
-        const uint32_t e = (uint32_t)s_terms[lane];
-        double T[9];
-        load_tri(a.tris, (int32_t)(e >> 2), T);
-        normal_term(T, (int)(e & 3u), t);
-      }
+      if (lane < nterms) table_term(c.norms, (uint32_t)s_terms[lane], t);
       for (int32_t l = 0; l < nterms; ++l)
         for (int d = 0; d < 3; ++d) m.sn[d] += lane_get(t[d], l);
       if (lane == 0) sdf_finish(a, i, q, m, cn);
@@ -2706,14 +2718,19 @@ static int sdf_cull_nodes(axsq_sdf* h, const CullSpace& cs, double diag, hipStre
   std::lock_guard<std::mutex> lock(h->cull_mu);
   if (h->cull_state == 0) {
     const size_t n = (size_t)(h->bvh->n - 1);
-    if (!h->cull && hipMalloc((void**)&h->cull, sizeof(CullNode) * n) != hipSuccess) {
+    const size_t nrec = (n + 1) * (h->cells ? 2 : 1);
+    if (!h->cull && (hipMalloc((void**)&h->cull, sizeof(CullNode) * n) != hipSuccess ||
+                     hipMalloc((void**)&h->cull_norms, sizeof(NormRec) * nrec) != hipSuccess)) {
       (void)hipGetLastError();
+      (void)hipFree(h->cull);
       h->cull = nullptr;
+      h->cull_norms = nullptr;
       h->cull_state = -1;
     } else {
       int32_t bad = 0;
       ProfRange pr("sdf_cull_build", s);
-      AXSQ_TRY(cull_build(h->bvh, h->tris, h->cells, cs, diag, h->cull, &bad, s));
+      AXSQ_TRY(cull_build(h->bvh, h->tris, h->cells, cs, diag, h->cull, h->cull_norms, &bad,
+                          s));
       h->cull_state = bad ? -1 : 1;
     }
   }
@@ -2809,6 +2826,7 @@ int sdf_eval_launch(const axsq_sdf* h, const double* x, const double* y, const d
   ws.cull_n_zero = false;
   CullArgs c{};
   c.nodes = cull;
+  c.norms = h->cull_norms;
   c.cs = cs;
   for (int k = 0; k < 3; ++k) {
     c.cmax = std::max(c.cmax, (float)std::max(std::fabs(h->domain[k]),
