@@ -2161,38 +2161,52 @@ __global__ __launch_bounds__(kBlock) void k_copy_u32(const uint32_t* __restrict_
 }
 
 // ---- adjoint -----------------------------------------------------------------
-// Sort keys of the adjoint: the winning triangle, or nt for a query without
-// one (elem -1), which sorts after every triangle; any other id outside
-// [0, nt) sets bit kStatusElem of *status and also takes key nt.
-__global__ __launch_bounds__(kBlock) void k_elem_keys(const int32_t* __restrict__ elem, int64_t nq,
-                                                       int64_t nt, uint32_t* __restrict__ keys,
-                                                       uint32_t* __restrict__ vals,
-                                                       int32_t* __restrict__ status) {
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= nq) return;
-  const int32_t e = elem[i];
-  const bool in_range = e >= 0 && (int64_t)e < nt;
-  if (!in_range && e != -1) atomicOr(status, kStatusElem);
-  keys[i] = in_range ? (uint32_t)e : (uint32_t)nt;
-  vals[i] = (uint32_t)i;
+// The triangles' corners by element, one record each for k_bwd_query's gathers.
+__global__ __launch_bounds__(kBlock) void k_bwd_corners(
+    const double* __restrict__ vx, const double* __restrict__ vy, const double* __restrict__ vz,
+    const int32_t* __restrict__ conn, int64_t nt, TriRec* __restrict__ corners) {
+  const int64_t c = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (c >= nt) return;
+  TriRec r;
+  for (int k = 0; k < 3; ++k) {
+    const int32_t v = conn[3 * c + k];
+    r.v[3 * k] = vx[v];
+    r.v[3 * k + 1] = vy[v];
+    r.v[3 * k + 2] = vz[v];
+  }
+  r.id = (int32_t)c;
+  r.pad = 0;
+  corners[c] = r;
 }
 
-// One lane per query, in element order (position p of the sorted list): the
-// query gradient, and the closest point's barycentric weights w and the
-// scaled direction d that the per-triangle sums read (terms[6p .. 6p + 5]).
+// One lane per query, in query order: the query gradient, and the closest
+// point's barycentric weights w and the scaled direction d that the
+// per-triangle sums read (terms[6i .. 6i + 5]). What a query reads and writes
+// of its own (116 bytes) is one run per wave this way; in element order each
+// was a line of its own. The triangle is a gather, from a table that stays in
+// cache or is read once a query. With vertex gradients (terms given), the sort
+// keys: the triangle, or nt for a query without one (elem -1), after every
+// triangle; any other id outside [0, nt) sets bit kStatusElem of *status and
+// also takes key nt.
+// 4M queries, 81,920 triangles: 324 us in element order, 165; 8M and 1.3M: 670,
+// 328.
 __global__ __launch_bounds__(kBlock) void k_bwd_query(
-    const double* __restrict__ vx, const double* __restrict__ vy, const double* __restrict__ vz,
-    const int32_t* __restrict__ conn, int64_t nt, const uint32_t* __restrict__ keys,
-    const uint32_t* __restrict__ qidx, int64_t nq, const double* __restrict__ qx,
-    const double* __restrict__ qy, const double* __restrict__ qz, int64_t qs,
-    const double* __restrict__ dist, const float* __restrict__ gout, double* __restrict__ grad_q,
-    double* __restrict__ terms) {
-  const int64_t p = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (p >= nq) return;
-  const int64_t c = (int64_t)keys[p];
-  if (c >= nt) {  // no closest triangle: the distance is constant in the query
+    const TriRec* __restrict__ corners, int64_t nt, const int32_t* __restrict__ elem,
+    int64_t nq, const double* __restrict__ qx, const double* __restrict__ qy,
+    const double* __restrict__ qz, int64_t qs, const double* __restrict__ dist,
+    const float* __restrict__ gout, double* __restrict__ grad_q, double* __restrict__ terms,
+    uint32_t* __restrict__ keys, uint32_t* __restrict__ vals, int32_t* __restrict__ status) {
+  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= nq) return;
+  const int64_t c = (int64_t)elem[i];
+  const bool in_range = c >= 0 && c < nt;
+  if (terms) {
+    keys[i] = in_range ? (uint32_t)c : (uint32_t)nt;
+    vals[i] = (uint32_t)i;
+  }
+  if (!in_range) {  // no closest triangle: the distance is constant in the query
+    if (c != -1) atomicOr(status, kStatusElem);
     if (grad_q) {
-      const int64_t i = (int64_t)qidx[p];
       grad_q[3 * i] = 0.0;
       grad_q[3 * i + 1] = 0.0;
       grad_q[3 * i + 2] = 0.0;
@@ -2200,13 +2214,7 @@ __global__ __launch_bounds__(kBlock) void k_bwd_query(
     return;
   }
   double T[9];
-  for (int k = 0; k < 3; ++k) {
-    const int32_t v = conn[3 * c + k];
-    T[3 * k] = vx[v];
-    T[3 * k + 1] = vy[v];
-    T[3 * k + 2] = vz[v];
-  }
-  const int64_t i = (int64_t)qidx[p];
+  load_tri(corners, (int32_t)c, T);
   const double P[3] = {qx[i * qs], qy[i * qs], qz[i * qs]};
   double cp[3], w[3];
   closest_point<true>(P, T, 1e-12, cp, w);
@@ -2234,53 +2242,61 @@ __global__ __launch_bounds__(kBlock) void k_bwd_query(
     grad_q[3 * i + 1] = d1;
     grad_q[3 * i + 2] = d2;
   }
-  double* t = terms + 6 * p;
-  t[0] = w[0];
-  t[1] = w[1];
-  t[2] = w[2];
-  t[3] = d0;
-  t[4] = d1;
-  t[5] = d2;
+  if (!terms) return;
+  double2* t = reinterpret_cast<double2*>(terms + 6 * i);
+  t[0] = make_double2(w[0], w[1]);
+  t[1] = make_double2(w[2], d0);
+  t[2] = make_double2(d1, d2);
 }
 
-// One wave per triangle: the per-corner partial sums (9 doubles per
-// triangle) over its queries in ascending index order, from k_bwd_query's
-// terms. The lanes load 64 queries' terms at a time and form their products;
-// lane k < 9 then adds component k in query order. The sums are the
-// one-lane sequential sums, bit for bit, while a triangle reached by many
-// queries (hundreds, where queries share a vertex's normal cone) costs a few
-// coalesced loads instead of a chain of hundreds.
+// The per-corner partial sums (9 doubles per triangle) over its queries in
+// ascending index order, from k_bwd_query's terms: the one-lane sequential
+// sums, bit for bit. A wave takes TRIS triangles, whose queries are one run of
+// the sorted list: the lanes gather 64 queries' terms at a time and form their
+// products, and lane 9 t + k adds component k of triangle t. A triangle reached
+// by many queries (hundreds, where queries share a vertex's normal cone) costs
+// a few gathers, one reached by few shares one with its neighbours.
+// 4M queries on 81,920, 8M on 1.3M and 1M on 327,680 triangles (49, 6 and 3 a
+// triangle): 112 / 417 / 74 us with one triangle a wave, 180 / 222 / 32 with
+// seven, 150 / 461 / 53 with 16 lanes a triangle that load for themselves. So
+// seven below 16 queries a triangle, one above.
 constexpr int kBwdWave = 64;
+template <int TRIS>
 __global__ __launch_bounds__(kBwdWave) void k_bwd_tri(int64_t nt,
                                                        const int32_t* __restrict__ seg_start,
                                                        const int32_t* __restrict__ seg_end,
+                                                       const uint32_t* __restrict__ qidx,
                                                        const double* __restrict__ terms,
                                                        double* __restrict__ part) {
   __shared__ double s_pr[9][kBwdWave];
-  const int64_t c = blockIdx.x;
-  const int lane = (int)threadIdx.x;
-  if (c >= nt) return;
-  const int32_t b = seg_start[c], e = seg_end[c];
-  double acc = 0.0;  // lane k < 9: component k (corner k / 3, axis k % 3)
-  for (int32_t base = b; base < e; base += kBwdWave) {
+  const int lane = (int)threadIdx.x, k = lane % 9;
+  const int64_t c = (int64_t)blockIdx.x * TRIS + lane / 9;
+  const bool mine = lane < 9 * TRIS && c < nt;
+  const int32_t b = mine ? seg_start[c] : 0, e = mine ? seg_end[c] : 0;
+  // the run: from the first to the last of those that have queries
+  const uint64_t some = __ballot(e > b);
+  const int32_t lo = some ? __shfl(b, __builtin_ctzll(some)) : 0;
+  const int32_t hi = some ? __shfl(e, 63 - __builtin_clzll(some)) : 0;
+  double acc = 0.0;
+  for (int32_t base = lo; base < hi; base += kBwdWave) {
     const int32_t p = base + lane;
-    if (p < e) {
-      const double* t = terms + 6 * (int64_t)p;
-      const double w[3] = {t[0], t[1], t[2]};
-      const double d0 = t[3], d1 = t[4], d2 = t[5];
-      for (int k = 0; k < 3; ++k) {
-        s_pr[3 * k][lane] = -(w[k] * d0);
-        s_pr[3 * k + 1][lane] = -(w[k] * d1);
-        s_pr[3 * k + 2][lane] = -(w[k] * d2);
+    if (p < hi) {
+      const double2* t = reinterpret_cast<const double2*>(terms + 6 * (int64_t)qidx[p]);
+      const double2 t0 = t[0], t1 = t[1], t2 = t[2];
+      const double w[3] = {t0.x, t0.y, t1.x};
+      const double d0 = t1.y, d1 = t2.x, d2 = t2.y;
+      for (int j = 0; j < 3; ++j) {
+        s_pr[3 * j][lane] = -(w[j] * d0);
+        s_pr[3 * j + 1][lane] = -(w[j] * d1);
+        s_pr[3 * j + 2][lane] = -(w[j] * d2);
       }
     }
     __syncthreads();
-    const int32_t m = (e - base < kBwdWave) ? e - base : kBwdWave;
-    if (lane < 9)
-      for (int32_t l = 0; l < m; ++l) acc += s_pr[lane][l];
+    const int32_t last = min(e - base, kBwdWave);
+    for (int32_t l = max(b - base, 0); l < last; ++l) acc += s_pr[k][l];
     __syncthreads();
   }
-  if (lane < 9) part[9 * c + lane] = acc;
+  if (mine) part[9 * c + k] = acc;
 }
 
 // One lane per vertex: sum of its incident corner partials, ascending triangle.
@@ -2889,35 +2905,48 @@ int sdf_backward_launch(const axsq_sdf* h, const double* x, const double* y, con
                         const float* gout, double* grad_q, double* grad_v, hipStream_t s) {
   Workspace& ws = workspace();
   const int64_t nt = h->ntris;
-  AXSQ_TRY(ws.k0.ensure(sizeof(uint32_t) * nq));
-  AXSQ_TRY(ws.v0.ensure(sizeof(uint32_t) * nq));
-  AXSQ_TRY(ws.k1.ensure(sizeof(uint32_t) * nq));
-  AXSQ_TRY(ws.v1.ensure(sizeof(uint32_t) * nq));
-  // segments of the nt triangles and of key nt (queries without a triangle;
-  // 2*(nt+1) int32), partials (9*nt doubles), per-query terms (6*nq doubles)
-  const size_t seg_bytes = (sizeof(int32_t) * 2 * (nt + 1) + 255) & ~size_t(255);
-  const size_t part_bytes = sizeof(double) * 9 * nt;
-  AXSQ_TRY(ws.flag.ensure(seg_bytes + part_bytes + sizeof(double) * 6 * nq));
-  int32_t* seg_start = ws.flag.as<int32_t>();
+  // corners (nt records) and, for the vertices' gradients: segments of the nt
+  // triangles and of key nt (queries without a triangle; 2*(nt+1) int32),
+  // partials (9*nt doubles), per-query terms (6*nq doubles)
+  auto up = [](size_t b) { return (b + 255) & ~size_t(255); };
+  const size_t corner_bytes = up(sizeof(TriRec) * nt);
+  const size_t seg_bytes = up(sizeof(int32_t) * 2 * (nt + 1));
+  const size_t part_bytes = up(sizeof(double) * 9 * nt);
+  AXSQ_TRY(ws.flag.ensure(corner_bytes +
+                          (grad_v ? seg_bytes + part_bytes + sizeof(double) * 6 * nq : 0)));
+  char* const base = ws.flag.as<char>();
+  TriRec* corners = reinterpret_cast<TriRec*>(base);
+  int32_t* seg_start = reinterpret_cast<int32_t*>(base + corner_bytes);
   int32_t* seg_end = seg_start + nt + 1;
-  double* part = reinterpret_cast<double*>(ws.flag.as<char>() + seg_bytes);
-  double* terms = reinterpret_cast<double*>(ws.flag.as<char>() + seg_bytes + part_bytes);
+  double* part = reinterpret_cast<double*>(base + corner_bytes + seg_bytes);
+  double* terms = reinterpret_cast<double*>(base + corner_bytes + seg_bytes + part_bytes);
+  if (grad_v) {
+    AXSQ_TRY(ws.k0.ensure(sizeof(uint32_t) * nq));
+    AXSQ_TRY(ws.v0.ensure(sizeof(uint32_t) * nq));
+    AXSQ_TRY(ws.k1.ensure(sizeof(uint32_t) * nq));
+    AXSQ_TRY(ws.v1.ensure(sizeof(uint32_t) * nq));
+  }
   ProfRange pr("sdf_backward", s);
-  k_elem_keys<<<grid_for(nq), kBlock, 0, s>>>(elem, nq, nt, ws.k0.as<uint32_t>(),
-                                              ws.v0.as<uint32_t>(), h->bvh->status);
+  k_bwd_corners<<<grid_for(nt), kBlock, 0, s>>>(h->vx, h->vy, h->vz, h->conn, nt, corners);
   AXSQ_CHECK_HIP(hipGetLastError());
-  uint32_t *sk, *sv;
-  AXSQ_TRY(radix_sort_pairs(ws.k0.as<uint32_t>(), ws.v0.as<uint32_t>(), ws.k1.as<uint32_t>(),
-                            ws.v1.as<uint32_t>(), nq, bits_for((uint64_t)nt), ws, s, &sk, &sv));
-  AXSQ_TRY(fill_i32(seg_start, 0, 2 * (nt + 1), s));
-  k_segments<<<grid_for(nq), kBlock, 0, s>>>(sk, nq, nt + 1, seg_start, seg_end, h->bvh->status);
-  AXSQ_CHECK_HIP(hipGetLastError());
-  k_bwd_query<<<grid_for(nq), kBlock, 0, s>>>(h->vx, h->vy, h->vz, h->conn, nt, sk, sv, nq, x, y,
-                                              z, stride, dist, gout, grad_q, terms);
-  AXSQ_CHECK_HIP(hipGetLastError());
-  k_bwd_tri<<<(unsigned)nt, kBwdWave, 0, s>>>(nt, seg_start, seg_end, terms, part);
+  k_bwd_query<<<grid_for(nq), kBlock, 0, s>>>(
+      corners, nt, elem, nq, x, y, z, stride, dist, gout, grad_q, grad_v ? terms : nullptr,
+      ws.k0.as<uint32_t>(), ws.v0.as<uint32_t>(), h->bvh->status);
   AXSQ_CHECK_HIP(hipGetLastError());
   if (grad_v) {
+    uint32_t *sk, *sv;
+    AXSQ_TRY(radix_sort_pairs(ws.k0.as<uint32_t>(), ws.v0.as<uint32_t>(), ws.k1.as<uint32_t>(),
+                              ws.v1.as<uint32_t>(), nq, bits_for((uint64_t)nt), ws, s, &sk,
+                              &sv));
+    AXSQ_TRY(fill_i32(seg_start, 0, 2 * (nt + 1), s));
+    k_segments<<<grid_for(nq), kBlock, 0, s>>>(sk, nq, nt + 1, seg_start, seg_end,
+                                               h->bvh->status);
+    AXSQ_CHECK_HIP(hipGetLastError());
+    if (nq < 16 * nt)
+      k_bwd_tri<7><<<grid_for(nt, 7), kBwdWave, 0, s>>>(nt, seg_start, seg_end, sv, terms, part);
+    else
+      k_bwd_tri<1><<<(unsigned)nt, kBwdWave, 0, s>>>(nt, seg_start, seg_end, sv, terms, part);
+    AXSQ_CHECK_HIP(hipGetLastError());
     k_bwd_vert<<<grid_for(h->nverts), kBlock, 0, s>>>(h->v2t_start, h->v2t_end, h->v2t_slot,
                                                       h->nverts, part, grad_v);
     AXSQ_CHECK_HIP(hipGetLastError());

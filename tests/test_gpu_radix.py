@@ -53,3 +53,35 @@ def test_queries_of_a_triangle_in_order(nq):
     i = torch.as_tensor(order, device=DEV)
     gq3, gv3 = s.backward(q[i].contiguous(), d[i].contiguous(), elem[i].contiguous(), gout)
     assert torch.equal(gq3, gq[i]) and torch.equal(gv3, gv)
+
+
+@pytest.mark.parametrize("few", [True, False])
+def test_adjoint_sums_of_short_and_long_segments(few):
+    """Vertex gradients are the sequential sums over each triangle's queries,
+    with no query, a few, and a wave's batch of 64 more or less, over triangles
+    that share a wave or not; without the vertices' part the
+    query gradients are the same, and an id out of range is refused either way."""
+    v, t = synth.icosphere(2)
+    nt = t.shape[0]
+    # 320 triangles: below and above 16 queries a triangle on average
+    counts = [0, 0, 1, 8, 9, 63, 64, 65, 95, 97, 128, 129, 1000] + [3 if few else 20] * (nt - 15)
+    counts += [0, 0]
+    rng = np.random.default_rng(3)
+    elem = rng.permutation(np.repeat(np.arange(nt), counts)).astype(np.int32)
+    nq = elem.size
+    tri = v[t[elem]]
+    w = rng.dirichlet(np.ones(3), nq)
+    p = np.einsum("ij,ijk->ik", w, tri) * rng.uniform(1.05, 1.5, (nq, 1))
+    s = quest.SignedDistance(_t(v), _t(t))
+    q, e = _t(p), _t(elem)
+    d = torch.ones(nq, dtype=torch.float64, device=DEV)
+    gout = _t(rng.normal(size=nq).astype(np.float32))
+    gq, gv = s.backward(q, d, e, gout)
+    only_q, none = s.backward(q, d, e, gout, want_vertices=False)
+    assert none is None and torch.equal(only_q, gq)
+    ogq, ogv = orc.OracleSDF(v, t).backward(p, d.cpu().numpy(), elem, gout.cpu().numpy())
+    assert np.array_equal(gq.cpu().numpy(), ogq) and np.array_equal(gv.cpu().numpy(), ogv)
+    e[5] = nt
+    for wv in (True, False):
+        with pytest.raises(RuntimeError):
+            s.backward(q, d, e, gout, want_vertices=wv)
