@@ -763,7 +763,8 @@ __device__ __forceinline__ void emit_node(int32_t i, int32_t lc, int32_t rc, con
   if (fo.nodes) {
     FindSpace fs;
     (void)find_space(fo.prm->bounds, fs);
-    fo.nodes[i] = make_find_node(fs, fo.dims, nd.l, nd.r, nd.flags, lc, rc);
+    store_find_node(fo.nodes, i, fo.dims,
+                    make_find_node(fs, fo.dims, nd.l, nd.r, nd.flags, lc, rc));
   }
 }
 

@@ -300,7 +300,7 @@ int find_launch(const axsq_bvh* b, int kind, int mode, const void* x, const void
                 int kstash, int32_t* stash_cnt, int32_t* over, uint32_t* nover, hipStream_t s,
                 bool pairs = false);
 // The fill for queries with at most kstash candidates, from the kept ids.
-// pairs: cands takes (query, id) records.
+// pairs (points and boxes): cands takes (query, id) records.
 int stash_copy_launch(const axsq_bvh* b, int kind, bool pairs, const int32_t* stash, int kstash,
                       const int32_t* stash_cnt, const int32_t* offsets, int64_t nq,
                       int32_t* cands, hipStream_t s);

@@ -186,7 +186,7 @@ __global__ __launch_bounds__(kBlock) void k_find(FindArgs a) {
 // the kept ids are leaf positions (the copy looks the ids up), so no load
 // stands in a visit's way. The ring of pending children is k_sdf_cull's.
 // 1M points into 100,000 boxes, 3-D / 2-D (18.9 / 48.5 visits each): 329 / 1,060
-// us with the FP64 nodes and the vote schedule, 168 / 641 here.
+// us with the FP64 nodes and the vote schedule, 168 / 532 here.
 template <int KIND, int MODE, int DIMS>
 __global__ __launch_bounds__(kBlock) void k_find_compact(FindArgs a) {
   constexpr bool FILL = MODE != kCountPass;
@@ -312,7 +312,7 @@ __device__ __forceinline__ bool ray_leaf(const FindArgs& a, int32_t pos, const d
 // most lanes waiting for the wave's longest walk and the chip for the longest
 // of all. Here a wave walks for `rays` rays together (find_pooled). A ray's
 // leaves so come in any order; their positions are the walk's order, which
-// k_stash_copy restores.
+// k_stash_order restores.
 // 100,000 rays, 100,000 boxes: 965 us one lane per ray on the FP64 nodes, 662 on
 // the compact ones, 129 here.
 constexpr int kPoolRays = 32;
@@ -404,53 +404,85 @@ __global__ __launch_bounds__(kWaveLanes) void k_ray_fill(FindArgs a) {
   }
 }
 
-// Queries of one wave of the copy: 64, or 16 where it also puts them in order,
-// which takes a step per id (100,000 rays: 55 us at 64, 23 at 16).
-template <bool ANY_ORDER>
-constexpr int copy_queries() { return ANY_ORDER ? 16 : 64; }
-
 // The fill pass for queries with at most kstash (<= 64) candidates: the ids of
-// the leaf positions the count pass kept, at offsets[i]; in order of position
-// (ANY_ORDER: a ray's are kept as its wave met them). A wave whose queries have at most 4 ids
-// each copies one query per lane; otherwise it copies its queries' ids one
-// query at a time, lane l taking id l, so each load and store is one
-// contiguous run, with eight queries' loads issued before their stores.
-template <bool ANY_ORDER, bool PAIRS>
+// the leaf positions the count pass kept, at offsets[i]. The ids of a wave's 64
+// queries are one run of the output, which its lanes take 64 at a time, each
+// finding its query among the 64 offsets; four such steps' loads are in flight
+// at once. Where no query has more than 4 ids a lane copies its own.
+// 1M queries of 12 ids: 84 us with a query at a time over the wave, 48 here.
+template <bool PAIRS>
 __global__ __launch_bounds__(kBlock) void k_stash_copy(const int32_t* __restrict__ stash,
                                                         int kstash,
                                                         const int32_t* __restrict__ stash_cnt,
                                                         const int32_t* __restrict__ offsets,
                                                         const int32_t* __restrict__ leaf_ids,
                                                         int64_t nq, int32_t* __restrict__ cands) {
+  __shared__ int32_t s_off[kBlock];
   const int lane = (int)__lane_id();
-  constexpr int Q = copy_queries<ANY_ORDER>();
+  int32_t* off = s_off + (threadIdx.x - lane);
+  const int64_t base = (int64_t)blockIdx.x * blockDim.x + threadIdx.x - lane;  // the wave's first
+  if (base >= nq) return;  // the whole wave
   auto put = [&](int32_t k, int64_t i, int32_t id) {
     if (PAIRS)
       reinterpret_cast<int2*>(cands)[k] = make_int2((int32_t)i, id);
     else
       cands[k] = id;
   };
-  const int64_t base =
-      ((int64_t)blockIdx.x * blockDim.x + threadIdx.x - lane) / kWaveLanes * Q;  // the wave's first
-  if (base >= nq) return;  // the whole wave
   const int64_t mine = base + lane;
-  const bool has = lane < Q && mine < nq;
-  const int32_t c_me = has ? stash_cnt[mine] : 0;
-  const int32_t o_me = has ? offsets[mine] : 0;
-  if (__ballot(c_me > 4 && c_me <= kstash) == 0) {  // few ids everywhere: a lane per query
-    if (c_me <= kstash)
-      for (int32_t k = 0; k < c_me; ++k) {
-        const int32_t pos = stash[mine * kstash + k];
-        int32_t at = k;
-        if (ANY_ORDER) {
-          at = 0;
-          for (int32_t t = 0; t < c_me; ++t) at += stash[mine * kstash + t] < pos;
-        }
-        put(o_me + at, mine, leaf_ids[pos]);
-      }
+  const int32_t c = (mine < nq) ? stash_cnt[mine] : 0;
+  const int32_t o = (mine < nq) ? offsets[mine] : 0x7fffffff;
+  if (__ballot(c > 4 && c <= kstash) == 0) {  // few ids everywhere
+    if (c <= kstash)
+      for (int32_t k = 0; k < c; ++k) put(o + k, mine, leaf_ids[stash[mine * kstash + k]]);
     return;
   }
-  for (int j0 = 0; j0 < Q; j0 += 8) {
+  off[lane] = o;
+  wave_sync();
+  const int last = (int)min(nq - base, (int64_t)kWaveLanes) - 1;
+  const int32_t lo = __shfl(o, 0), hi = __shfl(o, last) + __shfl(c, last);
+  const uint64_t listed = __ballot(c > kstash);  // searched again
+  for (int32_t j0 = lo + lane; j0 - lane < hi; j0 += 4 * kWaveLanes) {
+    int32_t id[4];
+    int q[4];
+    bool take[4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      const int32_t j = j0 + u * kWaveLanes;
+      q[u] = 0;  // the last query whose ids start at or before j
+#pragma unroll
+      for (int step = kWaveLanes / 2; step > 0; step >>= 1)
+        if (off[q[u] + step] <= j) q[u] += step;
+      take[u] = j < hi && !((listed >> q[u]) & 1);
+      id[u] = take[u] ? stash[(base + q[u]) * kstash + (j - off[q[u]])] : 0;
+    }
+#pragma unroll
+    for (int u = 0; u < 4; ++u)
+      if (take[u]) id[u] = leaf_ids[id[u]];
+#pragma unroll
+    for (int u = 0; u < 4; ++u)
+      if (take[u]) put(j0 + u * kWaveLanes, base + q[u], id[u]);
+  }
+}
+
+// The same for rays, whose positions were kept in any order: in order of
+// position. A wave takes 16 rays, one after the other, lane l placing id l by
+// the number of smaller ones (100,000 rays: 55 us with 64 rays a wave, 23 with 16).
+constexpr int kCopyRays = 16;
+__global__ __launch_bounds__(kBlock) void k_stash_order(const int32_t* __restrict__ stash,
+                                                         int kstash,
+                                                         const int32_t* __restrict__ stash_cnt,
+                                                         const int32_t* __restrict__ offsets,
+                                                         const int32_t* __restrict__ leaf_ids,
+                                                         int64_t nq, int32_t* __restrict__ cands) {
+  const int lane = (int)__lane_id();
+  const int64_t base =
+      ((int64_t)blockIdx.x * blockDim.x + threadIdx.x - lane) / kWaveLanes * kCopyRays;
+  if (base >= nq) return;  // the whole wave
+  const int64_t mine = base + lane;
+  const bool has = lane < kCopyRays && mine < nq;
+  const int32_t c_me = has ? stash_cnt[mine] : 0;
+  const int32_t o_me = has ? offsets[mine] : 0;
+  for (int j0 = 0; j0 < kCopyRays; j0 += 8) {
     int32_t v[8], cc[8], oo[8], at[8];
 #pragma unroll
     for (int u = 0; u < 8; ++u) {
@@ -458,22 +490,19 @@ __global__ __launch_bounds__(kBlock) void k_stash_copy(const int32_t* __restrict
       oo[u] = __shfl(o_me, j0 + u);
       const bool take = cc[u] <= kstash && lane < cc[u];
       v[u] = take ? stash[(base + j0 + u) * kstash + lane] : 0;
-      at[u] = lane;
     }
-    if (ANY_ORDER) {
 #pragma unroll
-      for (int u = 0; u < 8; ++u) {
-        const int c = cc[u] <= kstash ? __builtin_amdgcn_readfirstlane(cc[u]) : 0;
-        at[u] = 0;
-        for (int t = 0; t < c; ++t) at[u] += __builtin_amdgcn_readlane(v[u], t) < v[u];
-      }
+    for (int u = 0; u < 8; ++u) {
+      const int c = cc[u] <= kstash ? __builtin_amdgcn_readfirstlane(cc[u]) : 0;
+      at[u] = 0;
+      for (int t = 0; t < c; ++t) at[u] += __builtin_amdgcn_readlane(v[u], t) < v[u];
     }
 #pragma unroll
     for (int u = 0; u < 8; ++u)
       if (cc[u] <= kstash && lane < cc[u]) v[u] = leaf_ids[v[u]];
 #pragma unroll
     for (int u = 0; u < 8; ++u)
-      if (cc[u] <= kstash && lane < cc[u]) put(oo[u] + at[u], base + j0 + u, v[u]);
+      if (cc[u] <= kstash && lane < cc[u]) cands[oo[u] + at[u]] = v[u];
   }
 }
 
@@ -573,12 +602,14 @@ int stash_copy_launch(const axsq_bvh* b, int kind, bool pairs, const int32_t* st
                       int32_t* cands, hipStream_t s) {
   if (nq <= 0) return AXSQ_OK;
   ProfRange pr("bvh_find_copy", s);
-  const bool any = kind == AXSQ_QUERY_RAYS && b->find_ok;
-  const int64_t q = any ? copy_queries<true>() : copy_queries<false>();
-  auto* const copy = any ? (pairs ? k_stash_copy<true, true> : k_stash_copy<true, false>)
-                         : (pairs ? k_stash_copy<false, true> : k_stash_copy<false, false>);
-  copy<<<grid_for((nq + q - 1) / q * kWaveLanes), kBlock, 0, s>>>(stash, kstash, stash_cnt,
-                                                                  offsets, b->leaf_ids, nq, cands);
+  if (kind == AXSQ_QUERY_RAYS && b->find_ok) {
+    k_stash_order<<<grid_for((nq + kCopyRays - 1) / kCopyRays * kWaveLanes), kBlock, 0, s>>>(
+        stash, kstash, stash_cnt, offsets, b->leaf_ids, nq, cands);
+  } else {
+    auto* const copy = pairs ? k_stash_copy<true> : k_stash_copy<false>;
+    copy<<<grid_for(nq), kBlock, 0, s>>>(stash, kstash, stash_cnt, offsets, b->leaf_ids, nq,
+                                         cands);
+  }
   AXSQ_CHECK_HIP(hipGetLastError());
   return AXSQ_OK;
 }
