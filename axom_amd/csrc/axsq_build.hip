@@ -8,16 +8,20 @@
 //   k_mcodes      30-bit Morton code of each scaled-box centroid
 //   radix sort    stable LSD sort of (code, id)
 //   k_reorder     scaled leaf boxes in leaf (sorted) order
-//   k_karras      Karras 2012 hierarchy over the sorted codes
+//   k_seg_local   Karras 2012 hierarchy over the sorted codes by wide searches,
+//                 beside a balanced segment tree over each 512 leaves in LDS,
+//                 whose unions give the child boxes of every node inside
+//                 those leaves; nodes out (128-byte FP64; FP32 or the
+//                 searches' compact ones as the tree needs)
+//   k_emit_seg    the few nodes that reach across
+// Up to kSmallSortMax boxes bounds, codes and the sort's first histogram are one
+// kernel (k_mcodes_small), the sort's last pass writes the leaves in tree order,
+// and the whole is one graph. Trees of kSegMax leaves or more, and those with a
+// signed-zero box, whose unions depend on the grouping, take the climb instead:
+//   k_karras      the hierarchy
 //   k_refit_*     bottom-up boxes; the second thread to reach a node goes on
 //                 (hand-offs kept inside workgroups by tiers of leaf spans)
-//   k_emit        128-byte FP64 nodes (+ 64-byte FP32 nodes, rounded outward)
-// Up to kSmallSortMax boxes the same tree takes eight launches: k_transform;
-// k_mcodes_small (bounds + codes + the sort's first histogram); the sort's
-// passes, the last writing the leaves in tree order; k_seg_local (the
-// hierarchy by wide searches beside a balanced segment tree over each 512
-// leaves in LDS, whose unions give the child boxes of every node inside
-// those leaves); k_emit_seg (the few nodes that reach across) -- no climb.
+//   k_emit        the nodes
 
 #include <mutex>
 
@@ -143,10 +147,10 @@ __global__ __launch_bounds__(kBlock) void k_transform(const void* __restrict__ i
 // tree (f32: extent and 1 / extent rounded to float, the zero test's
 // threshold 1e-8 as a float). Run by a whole 1024-thread workgroup, which
 // finds the partials' min/max in one fixed order; thread 0 returns the
-// parameters (and the partials' quirky bits).
+// parameters.
 __device__ void finish_params(const double* __restrict__ partials, int64_t nparts,
                               const double* __restrict__ boxes, int64_t n, int f32,
-                              double (*s_red)[1024], BuildParams& out, int& quirky) {
+                              double (*s_red)[1024], BuildParams& out) {
   const int t = threadIdx.x;
   double acc[6];
   invalid_box(acc);
@@ -161,7 +165,7 @@ __device__ void finish_params(const double* __restrict__ partials, int64_t npart
     }
     q |= (int)pp[6];
   }
-  quirky = (__syncthreads_or(q & 1) ? 1 : 0) | (__syncthreads_or(q & 2) ? 2 : 0);
+  const int quirky = (__syncthreads_or(q & 1) ? 1 : 0) | (__syncthreads_or(q & 2) ? 2 : 0);
   for (int k = 0; k < 6; ++k) s_red[k][t] = acc[k];
   __syncthreads();
   for (int off = 512; off > 0; off >>= 1) {
@@ -180,6 +184,8 @@ __device__ void finish_params(const double* __restrict__ partials, int64_t npart
     for (int k = 0; k < 6; ++k) b[k] = s_red[k][0];
     if (!box_valid(b)) load_box(boxes + 6 * (n - 1), b);
     for (int k = 0; k < 6; ++k) out.bounds[k] = b[k];
+    out.quirky = quirky;
+    out.pad = 0;
     for (int d = 0; d < 3; ++d) {
       out.minc[d] = b[d];
       if (f32) {
@@ -200,11 +206,8 @@ __global__ __launch_bounds__(1024) void k_bounds(const double* __restrict__ part
                                                   BuildParams* __restrict__ host_out, int f32) {
   __shared__ double s_red[6][1024];
   BuildParams p;
-  int quirky;
-  finish_params(partials, nparts, boxes, n, f32, s_red, p, quirky);
+  finish_params(partials, nparts, boxes, n, f32, s_red, p);
   if (threadIdx.x == 0) {
-    p.quirky = quirky;
-    p.pad = 0;
     *prm = p;
     *host_out = p;
   }
@@ -263,12 +266,9 @@ __global__ __launch_bounds__(1024) void k_mcodes_small(const double* __restrict_
   const int t = threadIdx.x;
   if (t < 256) s_h[t] = 0u;
   BuildParams p;
-  int quirky;
-  finish_params(partials, nparts, boxes, n, f32, s_red, p, quirky);
+  finish_params(partials, nparts, boxes, n, f32, s_red, p);
   if (t == 0) {
     if (blockIdx.x == 0) {
-      p.quirky = quirky;
-      p.pad = 0;
       *prm = p;
       *host_out = p;
     }
@@ -358,18 +358,15 @@ __device__ __forceinline__ void karras_node(const uint32_t* __restrict__ mc, int
   if (i == 0) parents[0] = -1;
 }
 
-// The same node with several loads in flight per step, for trees of at most
-// kSmallSortMax leaves. delta(i, i + x * d) does not increase with x, so the
+// The same node with several loads in flight per step, for trees of fewer than
+// kSegMax leaves. delta(i, i + x * d) does not increase with x, so the
 // range end and the split are the last positions that pass their tests: the
 // reference's doubling search and binary searches find exactly those (the
 // split search's float-rounded steps are exact below 2^24), and so do
 // 8-way searches that test 7 positions at a time.
 __device__ __forceinline__ void karras_node_wide(const uint32_t* __restrict__ mc, int32_t inner,
-                                                 int32_t i, int32_t* __restrict__ lchild,
-                                                 int32_t* __restrict__ rchild,
-                                                 int32_t* __restrict__ parents,
-                                                 int32_t* __restrict__ range, int32_t& lo_out,
-                                                 int32_t& hi_out, int32_t& split_out) {
+                                                 int32_t i, int32_t& lo_out, int32_t& hi_out,
+                                                 int32_t& split_out) {
   const uint32_t ci = mc[i];
   auto delta = [&](int32_t b) -> int32_t {  // karras_delta(i, b)
     const bool oor = (b < 0 || b > inner);
@@ -407,7 +404,8 @@ __device__ __forceinline__ void karras_node_wide(const uint32_t* __restrict__ mc
   const int32_t dp = delta(i + 1), dm = delta(i - 1);
   const int32_t d = (dp - dm) < 0 ? -1 : 1;
   const int32_t dmin = d > 0 ? dm : dp;
-  // doubling search: the first lmax = 2^k (k >= 1) that fails, all probes at once
+  // doubling search: the first lmax = 2^k (k >= 1) that fails, all probes up to
+  // 2^18 at once (few nodes reach farther)
   int32_t lmax = 1 << 19;
   {
     int32_t v[18];
@@ -417,33 +415,15 @@ __device__ __forceinline__ void karras_node_wide(const uint32_t* __restrict__ mc
     for (int k = 18; k >= 1; --k)
       if (!(v[k - 1] > dmin)) lmax = 1 << k;
   }
+  if (lmax == 1 << 19)
+    while (delta(i + lmax * d) > dmin) lmax *= 2;  // ends past the tree, below 2^25
   const int32_t l = last_pass(lmax >= 4 ? lmax / 2 : 0, lmax - 1, d, dmin);
   const int32_t j = i + l * d;
   const int32_t dnode = delta(j);
   const int32_t s = last_pass(0, l - 1, d, dnode);
   const int32_t split = i + s * d + (d < 0 ? d : 0);
-  const int32_t lo = (i < j) ? i : j;
-  const int32_t hi = (i < j) ? j : i;
-  range[3 * i] = lo;
-  range[3 * i + 1] = hi;
-  range[3 * i + 2] = split;
-  if (lo == split) {
-    parents[split + inner] = i;
-    lchild[i] = split + inner;
-  } else {
-    parents[split] = i;
-    lchild[i] = split;
-  }
-  if (hi == split + 1) {
-    parents[split + inner + 1] = i;
-    rchild[i] = split + inner + 1;
-  } else {
-    parents[split + 1] = i;
-    rchild[i] = split + 1;
-  }
-  if (i == 0) parents[0] = -1;
-  lo_out = lo;
-  hi_out = hi;
+  lo_out = (i < j) ? i : j;
+  hi_out = (i < j) ? j : i;
   split_out = split;
 }
 
@@ -462,7 +442,7 @@ __global__ __launch_bounds__(kBlock) void k_karras(const uint32_t* __restrict__ 
   karras_node(mc, inner, i, lchild, rchild, parents, range);
 }
 
-// ---- box unions over leaf ranges (small builds) ------------------------------
+// ---- box unions over leaf ranges (trees below kSegMax leaves) ------------------------------
 // BoundingBox::addBox is associative over boxes without a signed-zero pair
 // (box_signed_zero_pair), so the box of a run of leaves can be put together
 // from any split of the run into consecutive pieces, combined left to right
@@ -799,10 +779,15 @@ __global__ __launch_bounds__(kBlock) void k_emit(const double* __restrict__ leaf
             ranges32, fo);
 }
 
+// Trees of fewer leaves take segment trees, whose scratch is 48 bytes a leaf
+// (rounded up to a power of two) and whose searches are exact below 2^24.
+// Hierarchy and boxes of 2.6M leaves: 590 us with the climb, 475; a
+// build of 500,000 boxes 314 us, 250.
+constexpr int64_t kSegMax = int64_t(1) << 24;
 constexpr int kSegLeaves = 512;  // leaves per workgroup of k_seg_local
 constexpr int kSegLog = 9;
 
-// Small builds, one 1,024-thread workgroup per 512 leaves and inner nodes
+// One 1,024-thread workgroup per 512 leaves and inner nodes
 // (base = 512 * workgroup). Its first 512 threads find the hierarchy's nodes
 // base .. base + 511 (karras_node_wide) while the other 512 put together the
 // segment tree of its leaves in LDS (local node u in [1, 512) at level l covers leaves
@@ -814,8 +799,7 @@ constexpr int kSegLog = 9;
 // are listed for k_emit_seg, kSegLeaves slots per workgroup
 // (deferred[512 * workgroup + j], their number in ndeferred[workgroup]).
 __global__ __launch_bounds__(2 * kSegLeaves) void k_seg_local(
-    const uint32_t* __restrict__ mc, int32_t inner, int32_t* __restrict__ lchild,
-    int32_t* __restrict__ rchild, int32_t* __restrict__ parents, int32_t* __restrict__ range,
+    const uint32_t* __restrict__ mc, int32_t inner, int32_t* __restrict__ range,
     const double* __restrict__ leaf_boxes, int64_t n, int64_t P, int levels,
     double* __restrict__ seg, Node64* __restrict__ nodes, Node32* __restrict__ nodes32,
     int4* __restrict__ ranges32, FindOut fo, int32_t* __restrict__ status,
@@ -837,7 +821,7 @@ __global__ __launch_bounds__(2 * kSegLeaves) void k_seg_local(
     const int64_t kn = base + t;
     int32_t nlo = 0, nhi = 0, nsp = 0;
     if (kn < inner)
-      karras_node_wide(mc, inner, (int32_t)kn, lchild, rchild, parents, range, nlo, nhi, nsp);
+      karras_node_wide(mc, inner, (int32_t)kn, nlo, nhi, nsp);
     s_rng[0][t] = nlo;
     s_rng[1][t] = nhi;
     s_rng[2][t] = nsp;
@@ -879,7 +863,12 @@ __global__ __launch_bounds__(2 * kSegLeaves) void k_seg_local(
   const int side = t & 1;
   const int32_t lo = s_rng[0][t >> 1], hi = s_rng[1][t >> 1], split = s_rng[2][t >> 1];
   const bool mine = k < inner && lo >= base && hi < base + kSegLeaves;
-  if (side == 0 && k < inner && !mine) deferred[base + atomicAdd(&s_ndef, 1)] = (int32_t)k;
+  if (side == 0 && k < inner && !mine) {
+    deferred[base + atomicAdd(&s_ndef, 1)] = (int32_t)k;
+    range[3 * k] = lo;
+    range[3 * k + 1] = hi;
+    range[3 * k + 2] = split;
+  }
   __syncthreads();
   if (t == 0) ndeferred[blockIdx.x] = s_ndef;
   if (!mine) return;  // both threads of a pair leave together
@@ -944,10 +933,10 @@ __device__ __forceinline__ SegBox half_wave_union(SegBox v) {
 // lists), its two halves on the two children at once. A child's leaf range
 // [a, b] is the pieces the bottom-up walk takes below level 9 (left side
 // ascending, right side descending; at most 9 each) and the run of level-9
-// nodes between them. Lane j of a half takes the j-th left piece, the j-th
-// right piece from the right end and up to 16 consecutive level-9 nodes of
-// the run (loaded 8 at a time); three order-keeping unions over the half
-// then give left ++ run ++ right.
+// nodes between them. The lanes of a half hold them in that order, the run (up
+// to 512 nodes for 262,144 leaves, loaded 4 at a time) spread over the lanes in
+// the middle, and one order-keeping union over the half gives the box; a long
+// run takes all lanes and a union of its own.
 __global__ __launch_bounds__(kBlock) void k_emit_seg(
     const double* __restrict__ leaf_boxes, const double* __restrict__ seg, int64_t P,
     const int32_t* __restrict__ range, const int32_t* __restrict__ deferred,
@@ -989,34 +978,52 @@ __global__ __launch_bounds__(kBlock) void k_emit_seg(
       }
       if (r & 1) {
         --r;
-        if (nr - 1 - cr == hl) xr = r;
+        if (nr - 1 - cr == hl - (kHalf - kSegLog)) xr = r;
         ++cr;
       }
       l >>= 1;
       r >>= 1;
     }
-    const int64_t per_lane = (m1 - m0 + kHalf - 1) / kHalf;  // at most 16
-    const int64_t j0 = m0 + per_lane * hl, j1 = (j0 + per_lane < m1) ? j0 + per_lane : m1;
-    SegBox L, M, R, mb[8];
-    L.empty = xl < 0;
-    R.empty = xr < 0;
-    if (xl >= 0) piece(xl, L);
-    if (xr >= 0) piece(xr, R);
-    M.empty = true;
-    for (int64_t jb = j0; jb < j1; jb += 8) {
+    // lanes 0 .. 8 hold the left pieces, 9 .. 22 take the run, 23 .. 31 hold the
+    // right pieces, all in leaf order
+    SegBox v, mb[4];
+    v.empty = true;
+    auto run = [&](int64_t j0, int64_t j1) {  // the run's nodes [j0, j1) in order
+      for (int64_t jb = j0; jb < j1; jb += 4) {
 #pragma unroll
-      for (int u = 0; u < 8; ++u)
-        if (jb + u < j1) piece(jb + u, mb[u]);
+        for (int u = 0; u < 4; ++u)
+          if (jb + u < j1) piece(jb + u, mb[u]);
 #pragma unroll
-      for (int u = 0; u < 8; ++u)
-        if (jb + u < j1) seg_combine(M, mb[u]);
+        for (int u = 0; u < 4; ++u)
+          if (jb + u < j1) seg_combine(v, mb[u]);
+      }
+    };
+    constexpr int kRun = kHalf - 2 * kSegLog;
+    if (__ballot(m1 - m0 > 8 * kRun) == 0) {
+      if (xl >= 0) piece(xl, v);
+      if (xr >= 0) piece(xr, v);
+      const int64_t per_lane = (m1 - m0 + kRun - 1) / kRun;
+      if (hl >= kSegLog && hl < kSegLog + kRun) {
+        const int64_t j0 = m0 + per_lane * (hl - kSegLog);
+        run(j0, (j0 + per_lane < m1) ? j0 + per_lane : m1);
+      }
+      v = half_wave_union(v);
+    } else {  // a long run: all lanes on it, then the pieces
+      const int64_t per_lane = (m1 - m0 + kHalf - 1) / kHalf;
+      const int64_t j0 = m0 + per_lane * hl;
+      run(j0, (j0 + per_lane < m1) ? j0 + per_lane : m1);
+      const SegBox M = half_wave_union(v);
+      SegBox L, R;
+      L.empty = xl < 0;
+      R.empty = xr < 0;
+      if (xl >= 0) piece(xl, L);
+      if (xr >= 0) piece(xr, R);
+      v = half_wave_union(L);
+      R = half_wave_union(R);
+      seg_combine(v, M);
+      seg_combine(v, R);
     }
-    L = half_wave_union(L);
-    M = half_wave_union(M);
-    R = half_wave_union(R);
-    seg_combine(L, M);
-    seg_combine(L, R);
-    for (int c = 0; c < 6; ++c) out[c] = L.b[c];
+    for (int c = 0; c < 6; ++c) out[c] = v.b[c];
   };
   for (int64_t q = q0; q < nd; q += per) {
     const int32_t i = deferred[g * kSegLeaves + q];
@@ -1200,8 +1207,8 @@ int bvh_build_into(axsq_bvh* b, const double* boxes, int64_t n_in, double scale,
   AXSQ_TRY(ws.v0.ensure(sizeof(uint32_t) * n));
   AXSQ_TRY(ws.k1.ensure(sizeof(uint32_t) * n));
   AXSQ_TRY(ws.v1.ensure(sizeof(uint32_t) * n));
-  // inputs of up to kSmallSortMax boxes take the segment-tree path
-  const bool small = n <= kSmallSortMax;
+  const bool small = n <= kSmallSortMax;  // the small sort
+  const bool segs = n < kSegMax;          // boxes by segment trees, not the climb
   int64_t P = 2;
   int levels = 1;
   while (P < n) {
@@ -1226,8 +1233,8 @@ int bvh_build_into(axsq_bvh* b, const double* boxes, int64_t n_in, double scale,
   const size_t off_seg =
       (off_ex + sizeof(int32_t) * (nchunks + 1 + nchunks * kBlock + n) + 255) & ~size_t(255);
   const int64_t nseg = (n + kSegLeaves - 1) / kSegLeaves;  // workgroups of k_seg_local
-  const size_t off_def = off_seg + (small ? sizeof(double) * 6 * (size_t)P : 0);
-  const size_t total = off_def + (small ? sizeof(int32_t) * (size_t)nseg * (kSegLeaves + 1) : 0);
+  const size_t off_def = off_seg + (segs ? sizeof(double) * 6 * (size_t)P : 0);
+  const size_t total = off_def + (segs ? sizeof(int32_t) * (size_t)nseg * (kSegLeaves + 1) : 0);
   AXSQ_TRY(ws.flag.ensure(total));
   char* base = ws.flag.as<char>();
   double* scaled = reinterpret_cast<double*>(base);
@@ -1250,8 +1257,28 @@ int bvh_build_into(axsq_bvh* b, const double* boxes, int64_t n_in, double scale,
 
   const FindOut fo{b->searched ? b->fnodes : nullptr, prm, dims};
 
-  // the exact climb: refit tiers, then the nodes (counters cleared by the caller)
+  // the hierarchy and child boxes from the sorted leaves: segment trees
+  auto seg_nodes = [&](hipStream_t q) -> int {
+    k_seg_local<<<(unsigned)nseg, 2 * kSegLeaves, 0, q>>>(b->mcodes, inner, rng, b->leaf_boxes, n,
+                                                          P, levels, seg, b->nodes, n32,
+                                                          b->ranges32, fo, b->status, deferred,
+                                                          ndef);
+    AXSQ_CHECK_HIP(hipGetLastError());
+    if (nseg > 1) {  // one workgroup of k_seg_local holds every node
+      // at least a wave per workgroup of k_seg_local
+      const unsigned g = (unsigned)std::max<int64_t>(2048, (nseg + 3) / 4);
+      k_emit_seg<<<g, kBlock, 0, q>>>(b->leaf_boxes, seg, P, rng, deferred, ndef, nseg, b->nodes,
+                                      n32, b->ranges32, fo);
+      AXSQ_CHECK_HIP(hipGetLastError());
+    }
+    return AXSQ_OK;
+  };
+
+  // the exact climb: hierarchy, refit tiers, then the nodes
   auto climb_and_emit = [&]() -> int {
+    k_karras<<<grid_for(inner), kBlock, 0, s>>>(b->mcodes, inner, lch, rch, par, rng, cnt, inner,
+                                                n_ex1, 1);
+    AXSQ_CHECK_HIP(hipGetLastError());
     k_refit_chunks<<<grid_for(n), kBlock, 0, s>>>(b->leaf_boxes, inner, lch, rch, par, rng, ib,
                                                   ex0, n_ex0);
     AXSQ_CHECK_HIP(hipGetLastError());
@@ -1304,15 +1331,7 @@ int bvh_build_into(axsq_bvh* b, const double* boxes, int64_t n_in, double scale,
       AXSQ_TRY(radix_sort_small_build(keys, vals, ws.k1.as<uint32_t>(), ws.v1.as<uint32_t>(), n,
                                       bits, hists, scaled, b->leaf_boxes, b->mcodes, b->leaf_ids,
                                       q));
-      k_seg_local<<<(unsigned)nseg, 2 * kSegLeaves, 0, q>>>(
-          b->mcodes, inner, lch, rch, par, rng, b->leaf_boxes, n, P, levels, seg, b->nodes, n32,
-          b->ranges32, fo, b->status, deferred, ndef);
-      if (nseg > 1) {  // one workgroup of k_seg_local holds every node
-        k_emit_seg<<<2048, kBlock, 0, q>>>(b->leaf_boxes, seg, P, rng, deferred, ndef, nseg,
-                                           b->nodes, n32, b->ranges32, fo);
-        AXSQ_CHECK_HIP(hipGetLastError());
-      }
-      AXSQ_CHECK_HIP(hipGetLastError());
+      AXSQ_TRY(seg_nodes(q));
       return AXSQ_OK;
     };
     // the launches as one HIP graph, captured on a stream of our own and
@@ -1373,10 +1392,7 @@ int bvh_build_into(axsq_bvh* b, const double* boxes, int64_t n_in, double scale,
     k_reorder<<<grid_for(n), kBlock, 0, s>>>(scaled, sv, sk, n, b->leaf_boxes, b->leaf_ids,
                                              b->mcodes);
     AXSQ_CHECK_HIP(hipGetLastError());
-    k_karras<<<grid_for(inner), kBlock, 0, s>>>(b->mcodes, inner, lch, rch, par, rng, cnt, inner,
-                                                n_ex1, 1);
-    AXSQ_CHECK_HIP(hipGetLastError());
-    AXSQ_TRY(climb_and_emit());
+    AXSQ_TRY(segs ? seg_nodes(s) : climb_and_emit());
   }
   pr.stop();
   const BuildParams& hp = *static_cast<const BuildParams*>(b->host_params);
@@ -1384,11 +1400,9 @@ int bvh_build_into(axsq_bvh* b, const double* boxes, int64_t n_in, double scale,
   for (int k = 0; k < 6; ++k) b->bounds[k] = hp.bounds[k];
   FindSpace fs;
   b->find_ok = b->searched && !(hp.quirky & 2) && find_space(b->bounds, fs);
-  if (small && (hp.quirky & 1)) {
+  if (segs && (hp.quirky & 1)) {
     // a leaf box with a signed-zero pair: unions may depend on the grouping,
     // so the boxes come from the climb, in the SEQ order
-    AXSQ_TRY(fill_i32(cnt, 0, inner, s));
-    AXSQ_TRY(fill_i32(n_ex1, 0, 1, s));
     AXSQ_TRY(climb_and_emit());
     AXSQ_CHECK_HIP(hipStreamSynchronize(s));
   }
