@@ -23,31 +23,55 @@ namespace {
 
 __device__ __forceinline__ V3 load_v3(const double* p) { return {p[0], p[1], p[2]}; }
 
-// Triangle corners (9 doubles, A B C), the corner box (BoundingBox{A, B, C},
+// The vertices as 32-byte records, for k_tri_setup's gathers: three arrays of
+// coordinates cost a line each.
+__global__ __launch_bounds__(kBlock) void k_pack_verts(const double* __restrict__ x,
+                                                       const double* __restrict__ y,
+                                                       const double* __restrict__ z, int64_t n,
+                                                       double2* __restrict__ out) {
+  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= n) return;
+  out[2 * i] = make_double2(x[i], y[i]);
+  out[2 * i + 1] = make_double2(z[i], 0.0);
+}
+
+// Triangle corners (A B C, TriRec), the corner box (BoundingBox{A, B, C},
 // compute_bounding_box.hpp:110-114, BoundingBox.hpp:405-422,464-482) and the
-// degenerate flag (Triangle::degenerate, Triangle.hpp:104-109,327-330).
+// degenerate flag (Triangle::degenerate, Triangle.hpp:104-109,327-330). verts:
+// k_pack_verts' records, or NULL.
+// 2.6M triangles of 1.3M vertices: 247 us from the three arrays, 186 with the
+// records (15 of it making them).
 __global__ __launch_bounds__(kBlock) void k_tri_setup(const double* __restrict__ x,
                                                       const double* __restrict__ y,
                                                       const double* __restrict__ z,
+                                                      const double2* __restrict__ verts,
                                                       const int32_t* __restrict__ conn,
                                                       int64_t n, int64_t nverts,
-                                                      double* __restrict__ tri,
+                                                      TriRec* __restrict__ tri,
                                                       double* __restrict__ boxes,
                                                       int32_t* __restrict__ degen,
                                                       int32_t* __restrict__ npair,
                                                       int32_t* __restrict__ status) {
   const int64_t c = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (c >= n) return;
-  double t[9];
+  TriRec r;
+  double* t = r.v;
   for (int k = 0; k < 3; ++k) {
     int32_t v = conn[3 * c + k];
     if (v < 0 || v >= nverts) {
       atomicOr(status, 2);
       v = 0;
     }
-    t[3 * k] = x[v];
-    t[3 * k + 1] = y[v];
-    t[3 * k + 2] = z[v];
+    if (verts) {
+      const double2 a = verts[2 * (int64_t)v], b = verts[2 * (int64_t)v + 1];
+      t[3 * k] = a.x;
+      t[3 * k + 1] = a.y;
+      t[3 * k + 2] = b.x;
+    } else {
+      t[3 * k] = x[v];
+      t[3 * k + 1] = y[v];
+      t[3 * k + 2] = z[v];
+    }
   }
   double b[6] = {t[0], t[1], t[2], t[0], t[1], t[2]};
   for (int corner = 1; corner < 3; ++corner)
@@ -58,12 +82,13 @@ __global__ __launch_bounds__(kBlock) void k_tri_setup(const double* __restrict__
     }
   double nrm[3];
   tri_normal(t, nrm);
-  degen[c] = near_eq(0.5 * sqrt(dot3(nrm[0], nrm[1], nrm[2], nrm[0], nrm[1], nrm[2])), 0.0, 1.0e-12)
-                 ? 1
-                 : 0;
+  degen[c] = tri_degenerate(nrm) ? 1 : 0;
   npair[c] = 0;
-  for (int k = 0; k < 9; ++k) tri[9 * c + k] = t[k];
-  for (int k = 0; k < 6; ++k) boxes[6 * c + k] = b[k];
+  r.id = (int32_t)c;
+  r.pad = 0;
+  tri[c] = r;
+  double2* o = reinterpret_cast<double2*>(boxes + 6 * c);
+  for (int k = 0; k < 3; ++k) o[k] = make_double2(b[2 * k], b[2 * k + 1]);
 }
 
 constexpr int kPairSlots = 4;  // hits kept per triangle by the first walk
@@ -75,7 +100,7 @@ struct IsectArgs {
   int32_t ninner;
   const int32_t* leaf_ids;
   const double* leaf_boxes;
-  const double* tri;    // 9 doubles per triangle
+  const TriRec* tri;    // per triangle
   const double* boxes;  // 6 doubles per triangle (the unscaled corner box)
   int64_t n;
   double eps;
@@ -98,7 +123,7 @@ template <class Hit>
 __device__ __forceinline__ void isect_walk(const IsectArgs& a, int64_t i, lds_i32* stk, Hit&& hit) {
   double prim[6];
   for (int k = 0; k < 6; ++k) prim[k] = a.boxes[6 * i + k];
-  const double* ti = a.tri + 9 * i;
+  const double* ti = a.tri[i].v;
   const V3 a0 = load_v3(ti), a1 = load_v3(ti + 3), a2 = load_v3(ti + 6);
   auto no_pref = [](const auto*, const auto*) { return false; };
   const int32_t v = traverse_voted<Node64, double>(
@@ -111,7 +136,7 @@ __device__ __forceinline__ void isect_walk(const IsectArgs& a, int64_t i, lds_i3
       [&](int32_t pos) {
         const int32_t j = a.leaf_ids[pos];
         if ((int64_t)j <= i || (int64_t)j >= a.n) return;
-        const double* tj = a.tri + 9 * (int64_t)j;
+        const double* tj = a.tri[j].v;
         if (tri_tri_intersect(a0, a1, a2, load_v3(tj), load_v3(tj + 3), load_v3(tj + 6), false,
                               a.eps))
           hit(j, pos);
@@ -122,15 +147,22 @@ __device__ __forceinline__ void isect_walk(const IsectArgs& a, int64_t i, lds_i3
 // Whether triangle f's corner box meets the scaled box of triangle s, at leaf
 // position sp, and the triangles intersect.
 __device__ __forceinline__ bool isect_test(const IsectArgs& a, int32_t f, int32_t s, int32_t sp) {
-  const double* u = a.boxes + 6 * (int64_t)f;
-  const double* b = a.leaf_boxes + 6 * (int64_t)sp;
-  if (!((u[3] >= b[0] && u[0] <= b[3]) && (u[4] >= b[1] && u[1] <= b[4]) &&
-        (u[5] >= b[2] && u[2] <= b[5])))
+  // 16-byte loads: the vector L1 returns one lane's a cycle, whatever they hold
+  const double2* u = reinterpret_cast<const double2*>(a.boxes + 6 * (int64_t)f);
+  const double2* b = reinterpret_cast<const double2*>(a.leaf_boxes + 6 * (int64_t)sp);
+  const double2 u0 = u[0], u1 = u[1], u2 = u[2], b0 = b[0], b1 = b[1], b2 = b[2];
+  if (!((u1.y >= b0.x && u0.x <= b1.y) && (u2.x >= b0.y && u0.y <= b2.x) &&
+        (u2.y >= b1.x && u1.x <= b2.y)))
     return false;
-  const double* ti = a.tri + 9 * (int64_t)f;
-  const double* tj = a.tri + 9 * (int64_t)s;
-  return tri_tri_intersect(load_v3(ti), load_v3(ti + 3), load_v3(ti + 6), load_v3(tj),
-                           load_v3(tj + 3), load_v3(tj + 6), false, a.eps);
+  V3 p[2][3];
+  for (int k = 0; k < 2; ++k) {
+    const double2* t = reinterpret_cast<const double2*>(a.tri + (k ? s : f));
+    const double2 t0 = t[0], t1 = t[1], t2 = t[2], t3 = t[3];
+    p[k][0] = {t0.x, t0.y, t1.x};
+    p[k][1] = {t1.y, t2.x, t2.y};
+    p[k][2] = {t3.x, t3.y, reinterpret_cast<const double*>(t)[8]};
+  }
+  return tri_tri_intersect(p[0][0], p[0][1], p[0][2], p[1][0], p[1][1], p[1][2], false, a.eps);
 }
 
 // Walk 1 where the compact nodes cannot serve: a lane per triangle.
@@ -160,8 +192,8 @@ __global__ __launch_bounds__(kBlock) void k_isect_count(IsectArgs a) {
 // contains both boxes of p, widened by 4 units in the last place of its largest
 // coordinate, which covers a scaled box that rounding left inside its corner box.
 // 2.6M triangles, two crossing noisy spheres: 4.1 ms with a lane per triangle
-// in mesh order on the FP64 nodes, 3.4 in leaf order on the compact ones, 1.04
-// here.
+// in mesh order on the FP64 nodes, 3.4 in leaf order on the compact ones, 0.90
+// here (1.04 with the tests' loads 8 bytes wide).
 constexpr int kPoolTris = 64;
 __global__ __launch_bounds__(kWaveLanes) void k_isect_pool(IsectArgs a, int tris) {
   __shared__ FindPool s_pool;
@@ -451,11 +483,14 @@ int self_intersections(const double* x, const double* y, const double* z, int64_
   } else {
     const int64_t n = ntris;
     Workspace& ws = workspace();
-    AXSQ_TRY(ws.mesh_tri.ensure(sizeof(double) * 9 * n));
+    // records of the vertices where the three arrays outgrow an XCD's L2 (4 MB)
+    const bool pack = nverts >= 131072;
+    AXSQ_TRY(ws.mesh_tri.ensure(sizeof(TriRec) * n + (pack ? 32 * (size_t)nverts : 0)));
     AXSQ_TRY(ws.mesh_box.ensure(sizeof(double) * 6 * n));
     AXSQ_TRY(ws.mesh_int.ensure(sizeof(int32_t) * (5 * n + 2) + 2 * sizeof(int64_t) + 64));
     AXSQ_TRY(ws.mesh_slots.ensure(sizeof(int32_t) * kPairSlots * n));
-    double* tri = ws.mesh_tri.as<double>();
+    TriRec* tri = ws.mesh_tri.as<TriRec>();
+    double2* verts = pack ? reinterpret_cast<double2*>(tri + n) : nullptr;
     double* boxes = ws.mesh_box.as<double>();
     int64_t* tot = reinterpret_cast<int64_t*>(ws.mesh_int.as<char>());
     int32_t* degf = reinterpret_cast<int32_t*>(tot + 2);
@@ -467,7 +502,11 @@ int self_intersections(const double* x, const double* y, const double* z, int64_
     AXSQ_TRY(fill_i32(status, 0, 2, s));
     {
       ProfRange pr("mesh_isect_setup", s);
-      k_tri_setup<<<grid_for(n), kBlock, 0, s>>>(x, y, z, tris, n, nverts, tri, boxes, degf,
+      if (pack) {
+        k_pack_verts<<<grid_for(nverts), kBlock, 0, s>>>(x, y, z, nverts, verts);
+        AXSQ_CHECK_HIP(hipGetLastError());
+      }
+      k_tri_setup<<<grid_for(n), kBlock, 0, s>>>(x, y, z, verts, tris, n, nverts, tri, boxes, degf,
                                                  npair, status);
       AXSQ_CHECK_HIP(hipGetLastError());
     }
