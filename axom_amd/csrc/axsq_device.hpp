@@ -14,6 +14,16 @@ namespace axsq {
 constexpr int32_t kBarrier = -2000000000;  // bvh_traverse.hpp:80
 constexpr int kStack = 64;                 // bvh_traverse.hpp:79
 constexpr int kWaveLanes = 64;
+// Workgroups go to the 8 XCDs in turn, each with an L2 of its own. The place of
+// workgroup b of n where runs of CHUNK neighbours go to one XCD.
+template <unsigned CHUNK>
+__device__ __forceinline__ unsigned xcd_block(unsigned b, unsigned n) {
+  const unsigned group = 8 * CHUNK;
+  const unsigned g0 = b / group * group;
+  if (g0 + group > n) return b;  // the last, partial group
+  const unsigned r = b - g0;
+  return g0 + (r % 8) * CHUNK + r / 8;
+}
 constexpr double kDblMax = 1.7976931348623157e308;
 
 struct Box {

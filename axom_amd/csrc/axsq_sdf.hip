@@ -510,6 +510,13 @@ __global__ __launch_bounds__(kSdfBlock) AXSQ_SDF_WAVES_ATTR void k_sdf_eval(SdfA
 #define AXSQ_CULL_VOTE_PCT 35
 #endif
 constexpr int kCullLds = AXSQ_CULL_LDS;
+// Waves in a row that go to one XCD: neighbours in the query order read the
+// same nodes, from one L2 instead of eight. In turn / runs of 16 / 64 / 256 /
+// 1,024: 4M queries on 2.1M triangles 7.37 / 7.22 / 7.15 / 7.23 / 7.54 ms a call, 8M
+// on 1.3M (an iteration) 16.5 / 16.2 / 16.2 / 16.1 / 16.3, 4M on 81,920 (with
+// adjoint; its nodes fit any L2) 4.15 / 4.15 / 4.17 / 4.19 / 4.39: the longer the
+// run, the less even the XCDs' shares.
+constexpr unsigned kCullRun = 64;
 // Batches walked one wave per query from the start: 10,000 queries on 5,120 /
 // 2.1M triangles 0.19 / 0.34 ms, a lane per query first 0.26 / 0.44; 20,000
 // 0.26 / 0.49 and 0.26 / 0.52; 40,000 0.40 / 0.81 and 0.26 / 0.61.
@@ -650,7 +657,7 @@ template <bool MIXED, bool CELLS>
 __global__ __launch_bounds__(kWaveLanes) AXSQ_CULL_WAVES_ATTR void k_sdf_cull(SdfArgs a, CullArgs c) {
   __shared__ uint64_t s_ring[kCullLds * kWaveLanes];
   const int lane = (int)threadIdx.x;
-  const int64_t t = (int64_t)blockIdx.x * kWaveLanes + lane;
+  const int64_t t = (int64_t)xcd_block<kCullRun>(blockIdx.x, gridDim.x) * kWaveLanes + lane;
   if (t >= a.npos) return;
   const int64_t i = a.order ? (int64_t)a.order[t] : t;
   lds_u64* ring = (lds_u64*)(s_ring + lane);
@@ -2854,13 +2861,14 @@ int sdf_eval_launch(const axsq_sdf* h, const double* x, const double* y, const d
   c.nlong = a.nredo + 1;
   c.ticket = a.nredo + 2;
   // A small batch ends with its longest lane walk, so it hands on early; a
-  // large one pays for what it hands on. 40,000 queries on 20,480 / 2.1M
-  // triangles, 128 steps 0.30 / 0.61 ms, 256 0.40 / 0.62, 512 0.57 / 0.82;
-  // 250,000: 0.43 / 1.60, 0.50 / 1.02, 0.66 / 1.20; 1.5M: 1.2 / 7.6, 1.03 /
-  // 3.8, 1.17 / 3.2.
-  // At most 65,536: 30,011 on 20,480 triangles 0.224 / 0.208 / 0.232 with 64, 96
-  // and 128 steps, 60,000 on 327,680 0.354 / 0.261 / 0.270.
-  c.steps = nq <= 65536 ? 96 : nq <= 786432 ? 256 : 512;
+  // large one pays for what it hands on, and more where the tree is large and
+  // walks are long. With 64 / 96 / 128 steps 30,011 queries on 20,480 triangles
+  // took 0.224 / 0.208 / 0.232 ms, 60,000 on 327,680 0.354 / 0.261 / 0.270; with
+  // 128 / 256 / 512 250,000 on 20,480 0.43 / 0.50 / 0.66 and on 2.1M 1.60 / 1.02 /
+  // 1.20; with 256 / 384 / 512 1M on 81,920 1.25 / 1.28 / 1.35, on 327,680 1.66 /
+  // 1.61 / 1.70, on 2.1M 2.59 / 2.34 / 2.35, 4M on 2.1M 8.3 / 6.8 / 6.5.
+  const bool large = b->n > (int64_t(1) << 18);
+  c.steps = nq <= 65536 ? 96 : nq <= 786432 ? 256 : nq <= 1572864 ? (large ? 384 : 256) : 512;
   ProfRange p1(mixed ? "sdf_eval_fp32_cull" : "sdf_eval_fp64_cull", s);
   // one lane per query, then one wave per long walk; a small batch one wave
   // per query at once
