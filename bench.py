@@ -11,18 +11,21 @@ gradient) over all queries, inputs resident in HBM.
   fp32_traversal   the same step with FP32 traversal (FP64 finish), and its
                    error against the FP64 result
   roofline         dominant kernel (FP64 SDF forward) timed with HIP events on
-                   its stream; algorithmic bytes per query
-                   = 24 (query) + 8 (distance) + 24 (closest point) + 4 (element)
-                   + V*104 (inner-node visits: 2 x 48 B boxes + 2 x 4 B links)
-                   + L*84 (leaf checks: 3 x 24 B vertices + 3 x 4 B indices),
-                   V, L = mean visits / leaf checks of the reference traversal
-                   (the FP64 kernel follows it exactly; counted on the GPU);
-                   traffic = HBM bytes per launch from the committed counter runs
+                   its stream against the bytes no form of it can do without:
+                   24 (query) + 8 (distance) + 24 (closest point) + 4 (element)
+                   per query, and once per launch 72 B per triangle (three
+                   vertices). The walk is bound by the return path of the
+                   vector L1, so its fraction of the HBM peak is low; traffic =
+                   HBM bytes per launch from the committed counter runs. The
+                   mean visits and leaf checks are those of the reference
+                   traversal (counted on the GPU by the walk that follows it);
+                   the culled walk behind the timing makes fewer
   bvh_build        BVH build Mprims/s over the 81,920 triangles and over the
                    100,000 boxes of the findPoints workload
   find_points      100,000 boxes / 1,000,000 points: findPoints queries/s (FP64
-                   and FP32 traversal), the count pass's roofline (24 B point +
-                   8 B offset and count + 4 B per candidate + V x 104 B)
+                   and FP32 traversal), the search pass's roofline (24 B point +
+                   8 B offset and count + 4 B per candidate, and 48 B per box
+                   once)
   configs          the three larger workloads at their full sizes: torus
                    (2,097,152 triangles, 16M queries, forward), wavy L7
                    icosphere (1M queries, forward + adjoint), L8 shape fit (8M
@@ -124,23 +127,27 @@ def prof_reader(L, _lib):
     return prof
 
 
-def sdf_roofline(kernel, ms, vbar, lbar, node_bytes, nq):
-    """Roofline of one signed-distance forward launch over nq queries: 24 B
-    query + 8 B distance + 24 B closest point + 4 B element + V node visits x
-    node_bytes (104 FP64 / 56 FP32) + L leaf checks x 84 B."""
-    bpq = 24 + 8 + 24 + 4 + node_bytes * vbar + 84.0 * lbar
-    ach = bpq * nq / (ms / 1e3) / 1e9
+def hbm_roofline(kernel, ms, nbytes):
+    """One launch of `kernel` against the HBM peak, over the bytes it cannot do
+    without (each input read once, each output written once)."""
+    ach = nbytes / (ms / 1e3) / 1e9
     return {"bound": "hbm", "achieved": ach, "peak": HBM_PEAK_GBS, "unit": "GB/s",
             "frac": ach / HBM_PEAK_GBS, "kernel": kernel, "avg_launch_ms": ms,
-            "bytes_per_query": bpq, "mean_inner_visits": vbar, "mean_leaf_checks": lbar}
+            "bytes_per_launch": nbytes}
+
+
+def sdf_roofline(ms, vbar, lbar, nq, ntris, per_query):
+    """hbm_roofline of a signed-distance forward: per_query bytes a query and
+    72 B a triangle; vbar / lbar are the reference traversal's counts."""
+    return dict(hbm_roofline("k_sdf_cull", ms, per_query * nq + 72 * ntris),
+                reference_inner_visits=vbar, reference_leaf_checks=lbar)
 
 
 def sdf_config(torch, dev, L, _lib, v, t, q, g, steps, want_bwd, cpu_threads, cpu_sample,
                label):
     """Signed distance over one mesh and query set: FP64 and FP32-traversal
     forward (+ adjoint when want_bwd), ms per step, queries/s, the forward's
-    roofline with the reference traversal's V and L (counted by the FP64
-    kernel), the FP32 form's max / RMS relative error and sign mismatches
+    roofline and the reference traversal's visits and leaf checks, the FP32 form's max / RMS relative error and sign mismatches
     against FP64; with cpu_threads, the oracle on a bounded sample."""
     from axom_amd import quest
     vd, td, qd = (torch.as_tensor(a, device=dev) for a in (v, t, q))
@@ -179,10 +186,9 @@ def sdf_config(torch, dev, L, _lib, v, t, q, g, steps, want_bwd, cpu_threads, cp
     visits, leaves = sdf.lastStats()
     sdf.enableStats(False)
     vbar, lbar = visits / nq, leaves / nq
-    out["fp64"]["roofline"] = sdf_roofline("k_sdf_eval<FP64>", out["fp64"]["sdf_eval_ms"], vbar,
-                                           lbar, 104.0, nq)
-    out["fp32"]["roofline"] = sdf_roofline("k_sdf_eval<FP32 traversal>",
-                                           out["fp32"]["sdf_eval_ms"], vbar, lbar, 56.0, nq)
+    for mode in ("fp64", "fp32"):  # 24 B query, 8 B distance, 4 B element
+        out[mode]["roofline"] = sdf_roofline(out[mode]["sdf_eval_ms"], vbar, lbar, nq,
+                                             t.shape[0], 36)
     rel = (res["fp32"] - res["fp64"]).abs() / res["fp64"].abs().clamp_min(1e-300)
     out["fp32"]["max_rel_err_vs_fp64"] = float(rel.max())
     out["fp32"]["rms_rel_err_vs_fp64"] = float(torch.sqrt((rel * rel).mean()))
@@ -255,9 +261,9 @@ def shapefit_config(torch, dev, v, t, q, target, cpu_threads, label, iterations=
 
 def find_points_config(torch, dev, L, _lib, boxes, pts, cpu_threads, reps=10):
     """BVH build over the boxes and findPoints over the points (FP64 and FP32
-    traversal), with the count pass's roofline: 24 B point + 8 B offset and
-    count + 4 B per candidate + V inner-node visits x 104 B, V counted by the
-    FP64 count pass (the reference walk's own visits)."""
+    traversal), with the search pass's roofline: 24 B point + 8 B offset and
+    count + 4 B per candidate, and 48 B per box once; the visits are the
+    reference walk's."""
     from axom_amd import spin
     prof = prof_reader(L, _lib)
     sync_time = sync_timer(torch)
@@ -290,16 +296,13 @@ def find_points_config(torch, dev, L, _lib, boxes, pts, cpu_threads, reps=10):
     bvh.findPoints(off, cnt, n, p)
     vbar = bvh.lastStats() / n
     bvh.enableStats(False)
-    bpq = 24 + 8 + 4.0 * cand.numel() / n + 104.0 * vbar
-    ach = bpq * n / (t_count / 1e3) / 1e9
-    out["roofline"] = {"bound": "hbm", "achieved": ach, "peak": HBM_PEAK_GBS, "unit": "GB/s",
-                       "frac": ach / HBM_PEAK_GBS, "kernel": "k_find<points, count>",
-                       "avg_launch_ms": t_count, "bytes_per_query": bpq,
-                       "mean_inner_visits": vbar,
-                       "other_kernels_ms": {"scan": prof("bvh_find_scan"),
-                                            "copy": prof("bvh_find_copy"),
-                                            "fill": prof("bvh_find_fill")},
-                       "fill_launches_per_call": prof.launches("bvh_find_fill") / calls}
+    out["roofline"] = dict(
+        hbm_roofline("k_find_compact<points>", t_count,
+                     32 * n + 4 * cand.numel() + 48 * boxes.shape[0]),
+        reference_inner_visits=vbar,
+        other_kernels_ms={"scan": prof("bvh_find_scan"), "copy": prof("bvh_find_copy"),
+                          "fill": prof("bvh_find_fill")},
+        fill_launches_per_call=prof.launches("bvh_find_fill") / calls)
     bvh32 = spin.BVH(bx, fp_mode="fp32")
     off32, cnt32 = torch.empty_like(off), torch.empty_like(cnt)
     tq32 = sync_time(lambda: res.__setitem__("c32", bvh32.findPoints(off32, cnt32, n, p)), reps)
@@ -545,8 +548,7 @@ def main():
     log("timing FP64 forward+backward")
     el64 = timed("fp64", args.steps, args.warmup)
     n_eval, ms_eval = prof("sdf_eval_fp64")
-    n_p1, ms_p1 = prof("sdf_eval_fp64_pass1")
-    n_p2, ms_p2 = prof("sdf_eval_fp64_pass2")
+    n_cull, ms_cull = prof("sdf_eval_fp64_cull")
     n_bwd, ms_bwd = prof("sdf_backward")
     n_ord, ms_ord = prof("sdf_query_order")
     d64 = dist.clone()
@@ -561,31 +563,24 @@ def main():
                                "SignedDistance forward (dist, cp, elem) + adjoint" % nq,
                    "queries": nq, "triangles": int(t.shape[0]), "parallelism": "single GPU"},
         "kernels_ms_per_step": {"sdf_eval_fp64": ms_eval / max(n_eval, 1),
-                                "sdf_eval_fp64_pass1": ms_p1 / max(n_p1, 1),
-                                "sdf_eval_fp64_pass2": ms_p2 / max(n_p2, 1),
+                                "sdf_eval_fp64_cull": ms_cull / max(n_cull, 1),
                                 "sdf_query_order": ms_ord / max(n_ord, 1),
                                 "sdf_backward": ms_bwd / max(n_bwd, 1)},
         "second_pass_walks": sdf.lastSuspended(),
         "host": host,
     }
 
-    # roofline of the dominant kernel: visits / leaf checks of the traversal
+    # roofline of the dominant kernel; the counts are the reference traversal's
     sdf.enableStats(True)
     sdf.computeDistances(nq, qd, outSgnDist=dist, outClosestPts=cp, outElem=elem, fp_mode="fp64")
     visits, leaves = sdf.lastStats()
     sdf.enableStats(False)
     vbar, lbar = visits / nq, leaves / nq
-    bytes_per_query = 24 + 8 + 24 + 4 + 104.0 * vbar + 84.0 * lbar
-    t_eval = ms_eval / max(n_eval, 1) / 1000.0
-    achieved = bytes_per_query * nq / t_eval / 1e9
     traffic = None
     if os.path.exists(PROFILE_TRAFFIC):
         traffic = json.load(open(PROFILE_TRAFFIC)).get("hbm_bytes_per_launch")
-    out["roofline"] = {"bound": "hbm", "achieved": achieved, "peak": HBM_PEAK_GBS, "unit": "GB/s",
-                       "frac": achieved / HBM_PEAK_GBS, "traffic": traffic,
-                       "kernel": "k_sdf_eval<FP64>", "avg_launch_ms": t_eval * 1e3,
-                       "bytes_per_query": bytes_per_query, "mean_inner_visits": vbar,
-                       "mean_leaf_checks": lbar}
+    out["roofline"] = dict(sdf_roofline(ms_eval / max(n_eval, 1), vbar, lbar, nq, t.shape[0], 60),
+                           traffic=traffic)
 
     if not args.no_extras:
         log("timing FP32-traversal forward+backward")
