@@ -263,3 +263,21 @@ def test_pair_lists_in_arrays_of_their_own_and_in_the_callers_memory():
     rc = L.lib().axsq_mesh_candidates_alloc(*mesh, *mesh, 3, none, None, ctypes.byref(a),
                                             ctypes.byref(np_), None)
     assert rc == L.ERRORS_BY_NAME["AXSQ_ERR_NOMEM"] and not a.value and np_.value == 0
+
+
+@pytest.mark.parametrize("nverts", [131071, 131072, 131073])
+def test_self_intersections_either_side_of_packed_vertices(nverts):
+    """From 131,072 vertices on the triangles are read through packed records."""
+    rng = np.random.default_rng(nverts)
+    n = 4001
+    v = rng.random((nverts, 3))
+    ids = rng.choice(nverts - 1, size=3 * n, replace=False).astype(np.int32)
+    ids[-1] = nverts - 1
+    t = ids.reshape(n, 3)
+    v[t[:, 1:]] = v[t[:, :1]] + rng.normal(0.0, 0.03, (n, 2, 3))
+    t[7, 1] = t[7, 0]  # no area
+    pairs, degen = quest.findTriMeshIntersectionsBVH(_t(v), _t(t))
+    opairs, odegen = orc.mesh_self_intersections(v, t, nthreads=8)
+    assert opairs.shape[0] > 100 and odegen.tolist() == [7]
+    assert np.array_equal(pairs.cpu().numpy(), opairs)
+    assert np.array_equal(degen.cpu().numpy(), odegen)
