@@ -543,6 +543,7 @@ struct CullQuery {
   float scale;   // mesh coordinates per unit
   float slack;   // added to the running distance
   float a0, a1;  // order plane: decided beyond a0 + a1 / |D|
+  float qm;      // FP32 form: largest coordinate of the mesh's boxes and the query
   float thr;     // box keys above it are left out
   bool ok;       // finite and within reach
   template <bool MIXED>
@@ -566,10 +567,31 @@ struct CullQuery {
     slack = 1.01e-6f * scale + R * 1.9073486e-6f + qmax * 8.8817842e-16f;
     // a query at most a0 + a1 / |D| from a node's order plane reads the boxes:
     // FP64 right_first is decided to 2^-49 R^2 / |D| and the plane's float form
-    // to 2^-20 R; the FP32 form also rounds coordinates (2^-23 of qmax)
+    // to 2^-20 R; the FP32 form's own decision is near_plane's
     a0 = (MIXED ? R + qmax : R) * 1.9073486e-6f;
-    a1 = MIXED ? (R + qmax) * R * 9.5367432e-7f : R * R * 1.7763568e-15f;
+    a1 = MIXED ? 0.0f : R * R * 1.7763568e-15f;
+    qm = qmax * 1.001f;  // the boxes are scaled by 1.000123
     thr = 3.402823466e38f;
+  }
+  // Whether float rounding could decide which child of a node is nearer, sd
+  // from its order plane, t its projections. The FP32 form compares float
+  // distances to the float boxes' centroids: a centroid less the query is off
+  // by 2^-22 of the coordinates (qm) an axis and 2^-24 of itself, the squares by
+  // 5 2^-24 of themselves, so with both centroids within r the comparison
+  // (2 |D| sd) is decided beyond (3.47 r qm + 1.28 r^2) 2^-22 / |D|. Taking for r
+  // the distance at this node and not to the mesh's farthest corner spares near
+  // queries the FP32 boxes at most nodes of the tree's lower half: 4M queries on
+  // 2.1M triangles 7.2 -> 6.7 ms, 8M on 1.3M (an iteration) 16.3 -> 15.8.
+  template <bool MIXED>
+  __device__ __forceinline__ bool near_plane(float sd, const float t[3], float inv_d) const {
+    if constexpr (MIXED) {
+      const float tt = fmaf(t[0], t[0], fmaf(t[1], t[1], t[2] * t[2]));
+      const float r = fmaf(__builtin_amdgcn_sqrtf(tt), 1.00001f,
+                           fmaf(0.50001f, __builtin_amdgcn_rcpf(inv_d), a0));
+      return !(fabsf(sd) > fmaf((r + qm) * r * 9.5367432e-7f, inv_d, a0));
+    } else {
+      return !(fabsf(sd) > fmaf(a1, inv_d, a0));
+    }
   }
   __device__ __forceinline__ void bound(double sq) {
     const float r = fmaf(sqrtf((float)sq) * 1.0000003f, scale, slack);
@@ -615,7 +637,7 @@ __device__ __forceinline__ CullVisit cull_visit(const SdfArgs& a, const CullArgs
   v.in_r = v.kr <= k.thr;
   const float sd = fmaf(f2.y, t[0], f2.z * t[1]);
   v.right = v.in_r && (sd > 0.0f || !v.in_l);
-  if (v.in_l && v.in_r && !(fabsf(sd) > fmaf(k.a1, f2.w, k.a0))) {
+  if (v.in_l && v.in_r && k.near_plane<MIXED>(sd, t, f2.w)) {
     int32_t l2, r2, flags;
     if constexpr (MIXED) {
       float lb[6], rb[6];

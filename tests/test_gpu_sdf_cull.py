@@ -114,6 +114,30 @@ def test_scaled_and_shifted_meshes(scale, shift):
         _check(v * scale + shift, t, q[:n] * scale + shift)
 
 
+@pytest.mark.parametrize("nq", [12_000, 20_000])
+@pytest.mark.parametrize("level,scale,shift", [(2, 1.0, 0.0), (5, 1.0, 0.0), (5, 1.0, 50.0),
+                                               (5, 30.0, 1e5), (6, 0.01, 0.0)])
+def test_fp32_order_is_the_reference_walks(monkeypatch, level, scale, shift, nq):
+    """With FP32 traversal the first of several tied triangles wins, in the order
+    of float comparisons: the reference walk's own outputs, bit for bit, where
+    queries tie (vertices, edges, points over them) near, far and in between."""
+    v, t, _ = synth.workload2(nq=1, level=level)
+    rng = np.random.default_rng(nq + level)
+    n = nq // 4
+    f = t[rng.integers(0, t.shape[0], n)]
+    mid = 0.5 * (v[f[:, 0]] + v[f[:, 1]])
+    off = 1.0 + 10.0 ** rng.uniform(-6, 0.3, (n, 1))
+    q = np.concatenate([v[f[:, 0]], mid, v[f[:, 1]] * off, mid * off])
+    v, q = v * scale + shift, q * scale + shift
+    g = _eval(quest.SignedDistance(_t(v), _t(t), fp_mode="fp32"), q, "fp32")
+    monkeypatch.setenv("AXSQ_SDF_BUDGET", "65536")  # the reference walk, on FP32 nodes alone
+    sdf = quest.SignedDistance(_t(v), _t(t), fp_mode="fp32")
+    r = _eval(sdf, q, "fp32")
+    assert sdf.lastSuspended() == 0
+    for k in ("dist", "cp", "elem", "normal"):
+        assert np.array_equal(g[k], r[k]), k
+
+
 def test_sliver_and_repeated_corners():
     """Triangles with equal corners keep the boxes; a sliver without a useful
     closest-point tolerance sends the mesh to the reference walk."""
