@@ -263,10 +263,12 @@ __global__ __launch_bounds__(kBlock) void k_cull_nodes(CullSpace cs,
       u[d] = D[d] - tw * w[d];
       ul += u[d] * u[d];
     }
-    if (ul > 1e-6 * dl && ul > 0.0 && ul < 1e300) {
+    const bool split = ul > 1e-12 * dl && ul > 0.0 && ul < 1e300;
+    if (split) {
       const double iu = 1.0 / sqrt(ul);
       for (int d = 0; d < 3; ++d) u[d] *= iu;
-    } else {  // any tangent: the axis least along w, made orthogonal
+    } else {  // any tangent: the axis least along w, made orthogonal; no order
+              // plane, D has a third component in this frame
       const int k = fabs(w[0]) <= fabs(w[1]) ? (fabs(w[0]) <= fabs(w[2]) ? 0 : 2)
                                              : (fabs(w[1]) <= fabs(w[2]) ? 1 : 2);
       const double wk = k == 0 ? w[0] : k == 1 ? w[1] : w[2];
@@ -279,7 +281,7 @@ __global__ __launch_bounds__(kBlock) void k_cull_nodes(CullSpace cs,
       for (int d = 0; d < 3; ++d) u[d] *= iu;
     }
     const double dlen = sqrt(dl), idl = dl > 0.0 ? 1.0 / dlen : 0.0;
-    const bool plane = idl > 0.0 && idl < 1e30;
+    const bool plane = split && idl > 0.0 && idl < 1e30;
     double a = 0.0, bb = 0.0;
     float xm[3];
     const float zero[3] = {0.0f, 0.0f, 0.0f};

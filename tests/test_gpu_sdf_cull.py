@@ -138,6 +138,21 @@ def test_fp32_order_is_the_reference_walks(monkeypatch, level, scale, shift, nq)
         assert np.array_equal(g[k], r[k]), k
 
 
+@pytest.mark.parametrize("dy", [5e-4, 1e-5, 1e-8, 0.0])
+def test_children_split_along_the_normal(dy):
+    """Two triangles stacked along their mean normal, their centroids a little
+    apart sideways, too: queries beside them, at one distance from both, see the
+    nearer centroid by that sideways part alone."""
+    v = np.array([[0, 1, 0], [1, 1, 0], [0.5, 0, 0],
+                  [0, 1, 1], [1, 1, 1], [0.5, -2 * dy, 1 + 0.25 * dy]])
+    t = np.array([[0, 1, 2], [3, 4, 5]], np.int32)
+    rng = np.random.default_rng(3)
+    q = np.stack([rng.uniform(0.1, 0.9, 20_000), rng.uniform(1.1, 3.0, 20_000),
+                  np.full(20_000, 0.5)], 1)
+    for n in (20_000, 500):
+        _check(v, t, q[:n], watertight=False)
+
+
 def test_sliver_and_repeated_corners():
     """Triangles with equal corners keep the boxes; a sliver without a useful
     closest-point tolerance sends the mesh to the reference walk."""
