@@ -49,13 +49,14 @@ struct Extents {
   }
 };
 
-// The share of a vertex at x; tau in mesh coordinates. Projections are
-// rounded to under 2^-21 of the sum of |x|, about the diagonal's 1 to 2.
+// The share of a vertex at x; tau in mesh coordinates. A projection is off by
+// 2^-24 |x| (x itself) and 4 2^-24 |p| (axsq_cull.hpp), t - e by 2^-24 |t| more.
 __device__ __forceinline__ void add_vertex(const CullNode& n, const float x[3], float tau,
                                            Extents& out) {
   float t[3];
   cull_project(n.w, n.u, n.m, x, t);
-  out.add(t, fmaf(fabsf(x[0]) + fabsf(x[1]) + fabsf(x[2]) + 1.0f, 4.76837158e-7f, tau));
+  const float e = fmaf(fabsf(t[0]) + fabsf(t[1]) + fabsf(t[2]), 3.3e-7f, tau);
+  out.add(t, fmaf(fabsf(x[0]) + fabsf(x[1]) + fabsf(x[2]), 6.6e-8f, e));
 }
 
 // Adds leaf pos's triangle records to the extents.
@@ -283,16 +284,13 @@ __global__ __launch_bounds__(kBlock) void k_cull_nodes(CullSpace cs,
     const double dlen = sqrt(dl), idl = dl > 0.0 ? 1.0 / dlen : 0.0;
     const bool plane = split && idl > 0.0 && idl < 1e30;
     double a = 0.0, bb = 0.0;
-    float xm[3];
-    const float zero[3] = {0.0f, 0.0f, 0.0f};
     for (int d = 0; d < 3; ++d) {
       n.w[d] = (float)w[d];
       n.u[d] = (float)u[d];
-      xm[d] = (float)((0.5 * (cl[d] + cr[d]) - cs.o[d]) * cs.scale);
+      n.m[d] = (float)((0.5 * (cl[d] + cr[d]) - cs.o[d]) * cs.scale);
       a += D[d] * idl * w[d];
       bb += D[d] * idl * u[d];
     }
-    cull_project(n.w, n.u, zero, xm, n.m);
     n.a = plane ? (float)a : 0.0f;
     n.b = plane ? (float)bb : 0.0f;
     n.inv_d = plane ? (float)(idl / cs.scale * 1.000001) : INFINITY;

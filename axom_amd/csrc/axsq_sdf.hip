@@ -563,8 +563,8 @@ struct CullQuery {
       qmax = fmaxf(qmax, fabsf((float)q[d]));
     }
     qmax *= scale;
-    // 1e-6: ties (checkCandidate); 2^-19 R: projections; 2^-50 qmax: q - o
-    slack = 1.01e-6f * scale + R * 1.9073486e-6f + qmax * 8.8817842e-16f;
+    // 1e-6: ties (checkCandidate); 1.1 2^-21 R: projections; 2^-50 qmax: q - o
+    slack = 1.01e-6f * scale + R * 5.25e-7f + qmax * 8.8817842e-16f;
     // a query at most a0 + a1 / |D| from a node's order plane reads the boxes:
     // FP64 right_first is decided to 2^-49 R^2 / |D| and the plane's float form
     // to 2^-20 R; the FP32 form's own decision is near_plane's
