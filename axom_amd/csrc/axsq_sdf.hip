@@ -2884,13 +2884,18 @@ int sdf_eval_launch(const axsq_sdf* h, const double* x, const double* y, const d
   c.ticket = a.nredo + 2;
   // A small batch ends with its longest lane walk, so it hands on early; a
   // large one pays for what it hands on, and more where the tree is large and
-  // walks are long. With 64 / 96 / 128 steps 30,011 queries on 20,480 triangles
-  // took 0.224 / 0.208 / 0.232 ms, 60,000 on 327,680 0.354 / 0.261 / 0.270; with
-  // 128 / 256 / 512 250,000 on 20,480 0.43 / 0.50 / 0.66 and on 2.1M 1.60 / 1.02 /
-  // 1.20; with 256 / 384 / 512 1M on 81,920 1.25 / 1.28 / 1.35, on 327,680 1.66 /
-  // 1.61 / 1.70, on 2.1M 2.59 / 2.34 / 2.35, 4M on 2.1M 8.3 / 6.8 / 6.5.
-  const bool large = b->n > (int64_t(1) << 18);
-  c.steps = nq <= 65536 ? 96 : nq <= 786432 ? 256 : nq <= 1572864 ? (large ? 384 : 256) : 512;
+  // walks are long. Microseconds a call with 96 / 128 / 192 / 256 / 320 steps, on
+  // 20,480, 81,920 and 2.1M triangles:
+  //   30,000 queries: 203 219 267 309 349, 301 297 361 430 472, 639 647 615 601 634
+  //   64,000: 302 257 292 336 379, 567 433 391 443 499, 1045 1021 851 744 727
+  //   180,000: 466 333 350 384 426, 1143 641 468 514 552, 2419 2251 1601 1164 1028
+  // with 256 / 384 / 512 1M on 81,920 1250 / 1280 / 1350, on 327,680 1660 / 1610 /
+  // 1700, on 2.1M 2590 / 2340 / 2350, 4M on 2.1M 8300 / 6800 / 6500.
+  const int size = b->n <= (int64_t(1) << 15) ? 0 : b->n <= (int64_t(1) << 18) ? 1 : 2;
+  static constexpr int32_t kSteps[5][3] = {
+      {96, 128, 128}, {128, 192, 256}, {192, 256, 320}, {256, 256, 384}, {512, 512, 512}};
+  const int row = nq <= 32768 ? 0 : nq <= 131072 ? 1 : nq <= 786432 ? 2 : nq <= 1572864 ? 3 : 4;
+  c.steps = kSteps[row][size];
   ProfRange p1(mixed ? "sdf_eval_fp32_cull" : "sdf_eval_fp64_cull", s);
   // one lane per query, then one wave per long walk; a small batch one wave
   // per query at once
