@@ -2890,11 +2890,19 @@ int sdf_eval_launch(const axsq_sdf* h, const double* x, const double* y, const d
   //   64,000: 302 257 292 336 379, 567 433 391 443 499, 1045 1021 851 744 727
   //   180,000: 466 333 350 384 426, 1143 641 468 514 552, 2419 2251 1601 1164 1028
   // with 256 / 384 / 512 1M on 81,920 1250 / 1280 / 1350, on 327,680 1660 / 1610 /
-  // 1700, on 2.1M 2590 / 2340 / 2350, 4M on 2.1M 8300 / 6800 / 6500.
+  // 1700, on 2.1M 2590 / 2340 / 2350; with 384 / 512 / 640 / 768 / 1024 4M on
+  // 5,120 1786 1846 1921 1998 2105, on 81,920 (with adjoint) 4244 4183 4262 4376
+  // 4543, on 2.1M 6645 6321 6278 6250 6366, 8M on 1.3M (an iteration) 15819 15151
+  // 14944 14885 15000, but 2M on 2.1M 3665 3544 3512 3567 3680.
   const int size = b->n <= (int64_t(1) << 15) ? 0 : b->n <= (int64_t(1) << 18) ? 1 : 2;
-  static constexpr int32_t kSteps[5][3] = {
-      {96, 128, 128}, {128, 192, 256}, {192, 256, 320}, {256, 256, 384}, {512, 512, 512}};
-  const int row = nq <= 32768 ? 0 : nq <= 131072 ? 1 : nq <= 786432 ? 2 : nq <= 1572864 ? 3 : 4;
+  static constexpr int32_t kSteps[6][3] = {{96, 128, 128},  {128, 192, 256}, {192, 256, 320},
+                                           {256, 256, 384}, {512, 512, 512}, {384, 512, 768}};
+  const int row = nq <= 32768     ? 0
+                  : nq <= 131072  ? 1
+                  : nq <= 786432  ? 2
+                  : nq <= 1572864 ? 3
+                  : nq <= 3145728 ? 4
+                                  : 5;
   c.steps = kSteps[row][size];
   ProfRange p1(mixed ? "sdf_eval_fp32_cull" : "sdf_eval_fp64_cull", s);
   // one lane per query, then one wave per long walk; a small batch one wave
