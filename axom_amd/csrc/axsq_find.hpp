@@ -82,9 +82,11 @@ constexpr uint32_t kFindLeaf = 0x80000000u, kFindSureBit = 0x40000000u;
 constexpr uint32_t kFindPos = 0x3fffffffu;
 constexpr uint32_t kFindEnd = kFindLeaf | kFindPos;  // no leaf has that position
 constexpr uint32_t kFindNone = 0xfc007c00u;  // an invalid child's range, from +inf to -inf
-// Inside by this much of the node's scale is inside the FP64 box: the halves
-// are off by 2^-10 at most, everything else by 2^-12.
-constexpr float kFindSure = 0.00195313f;  // 2^-9
+// Inside by this much of the node's scale is inside the FP64 box: extents are
+// below 2, but with their margins may round out past it, so the halves are off
+// by 2^-9 at most; the margins of a node with the bit set (s up to 2^30) and the
+// query's t by less than 2^-13 together.
+constexpr float kFindSure = 0.00219726562f;  // 2^-9 + 2^-12
 constexpr float kFindFar = 3e38f;  // beyond every far end of a ray's interval
 
 // Halves rounded outward (sign and magnitude, so the next one down or up is

@@ -1,0 +1,75 @@
+"""The candidate searches at the edges of the compact nodes' number range:
+results are integers, equal to the oracle's, order included.
+"""
+import numpy as np
+import pytest
+
+torch = pytest.importorskip("torch")
+
+from axom_amd import spin  # noqa: E402
+from oracle import oracle as orc  # noqa: E402
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+
+
+def _t(a):
+    return torch.as_tensor(np.ascontiguousarray(a), device=DEV)
+
+
+def _check(boxes, scale, dtype, queries):
+    """Searches of the tree over `boxes` against the oracle; queries: kind -> prims."""
+    nd = boxes.shape[1] // 2
+    kw = dict(FloatType=torch.float32) if dtype is np.float32 else {}
+    g = spin.BVH(_t(boxes), scaleFactor=scale, NDIMS=nd, **kw)
+    o = orc.OracleBVH(boxes, scale, ndims=nd, dtype=dtype)
+    for kind, q in queries.items():
+        ooff, ocnt, ocand = o.find(kind, q)
+        n = q.shape[0]
+        off = torch.empty(n, dtype=torch.int32, device=DEV)
+        cnt = torch.empty_like(off)
+        f = {"points": g.findPoints, "boxes": g.findBoundingBoxes, "rays": g.findRays}[kind]
+        cand = f(off, cnt, n, _t(q))
+        assert np.array_equal(cnt.cpu().numpy(), ocnt), kind
+        assert np.array_equal(off.cpu().numpy(), ooff), kind
+        assert np.array_equal(cand.cpu().numpy(), ocand), kind
+
+
+def _beyond_faces(lo, hi, nd, dtype, size, rng):
+    """Points and small boxes from one step to 2^-13 of `size` beyond a face of
+    [lo, hi], or as far inside it, the other coordinates well inside."""
+    n = 400
+    p = lo + (hi - lo) * rng.uniform(0.1, 0.9, (n, nd))
+    ax, side = rng.integers(nd, size=n), rng.integers(2, size=n)
+    face = np.where(side == 0, lo, hi).astype(dtype)
+    by = size * 2.0 ** rng.uniform(-30, -13, n) * rng.choice([-1, 1, 1], n)
+    out = np.where(side == 0, face - by, face + by).astype(dtype)
+    step = np.nextafter(face, np.where(side == 0, -np.inf, np.inf).astype(dtype))
+    out = np.where(rng.random(n) < 0.2, step, out)
+    p = p.astype(dtype)
+    p[np.arange(n), ax] = out
+    b = np.concatenate([p, p], 1)
+    far = np.where(side == 0, out - dtype(0.1 * size), out + dtype(0.1 * size)).astype(dtype)
+    b[np.arange(n), ax + nd * (side == 0)] = out
+    b[np.arange(n), ax + nd * (side == 1)] = far
+    b = np.concatenate([np.minimum(b[:, :nd], b[:, nd:]), np.maximum(b[:, :nd], b[:, nd:])], 1)
+    return p, b.astype(dtype)
+
+
+@pytest.mark.parametrize("eps", [2.0**-24, 2.0**-22, 2.0**-21, 2.0**-19, 2.0**-15])
+@pytest.mark.parametrize("nd,dtype,depth", [
+    (3, np.float64, 0), (2, np.float64, 0), (3, np.float32, 0), (2, np.float32, 0),
+    (3, np.float64, 12), (2, np.float64, 12), (3, np.float64, 27), (2, np.float64, 27)])
+def test_extents_just_below_a_power_of_two(eps, nd, dtype, depth):
+    """A node's extents, with their margins, round out past the range they are
+    scaled to; a query just outside such a face is in no box."""
+    rng = np.random.default_rng([depth, nd])
+    w = (1.0 - eps) * 2.0**-depth  # half width of a cluster around the origin
+    lo = np.full(nd, -w)
+    b = [np.concatenate([lo * 0.9, -lo]), np.concatenate([lo, -lo * 0.9])]
+    if depth:  # two far boxes around it, so that the cluster is small in the tree
+        b.append(np.concatenate([np.full(nd, 0.9), np.full(nd, 1.0)]))
+        b.append(np.concatenate([np.full(nd, -1.0), np.full(nd, -0.9)]))
+    boxes = np.array(b).astype(dtype)
+    p, q = _beyond_faces(-w, w, nd, dtype, w, rng)
+    _check(boxes, 1.0, dtype, {"points": p, "boxes": q})
