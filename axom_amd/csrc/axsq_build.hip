@@ -17,7 +17,8 @@
 // Up to kSmallSortMax boxes bounds, codes and the sort's first histogram are one
 // kernel (k_mcodes_small), the sort's last pass writes the leaves in tree order,
 // and the whole is one graph. Trees of kSegMax leaves or more, and those with a
-// signed-zero box, whose unions depend on the grouping, take the climb instead:
+// signed-zero or NaN box, whose unions depend on the grouping, take the climb
+// instead:
 //   k_karras      the hierarchy
 //   k_refit_*     bottom-up boxes; the second thread to reach a node goes on
 //                 (hand-offs kept inside workgroups by tiers of leaf spans)
@@ -444,7 +445,8 @@ __global__ __launch_bounds__(kBlock) void k_karras(const uint32_t* __restrict__ 
 
 // ---- box unions over leaf ranges (trees below kSegMax leaves) ------------------------------
 // BoundingBox::addBox is associative over boxes without a signed-zero pair
-// (box_signed_zero_pair), so the box of a run of leaves can be put together
+// (box_signed_zero_pair) or a NaN ([0, 1] ++ NaN ++ [5, 6] is [5, 6] from the
+// left, [0, 6] from the right), so the box of a run of leaves can be put together
 // from any split of the run into consecutive pieces, combined left to right
 // as the SEQ refit combines a node's children: the right part's box, then
 // addBox(the left part's box) (the second arrival at a node in leaf order
@@ -1400,9 +1402,9 @@ int bvh_build_into(axsq_bvh* b, const double* boxes, int64_t n_in, double scale,
   for (int k = 0; k < 6; ++k) b->bounds[k] = hp.bounds[k];
   FindSpace fs;
   b->find_ok = b->searched && !(hp.quirky & 2) && find_space(b->bounds, fs);
-  if (segs && (hp.quirky & 1)) {
-    // a leaf box with a signed-zero pair: unions may depend on the grouping,
-    // so the boxes come from the climb, in the SEQ order
+  if (segs && hp.quirky) {
+    // a leaf box with a signed-zero pair or a NaN: unions may depend on the
+    // grouping, so the boxes come from the climb, in the SEQ order
     AXSQ_TRY(climb_and_emit());
     AXSQ_CHECK_HIP(hipStreamSynchronize(s));
   }

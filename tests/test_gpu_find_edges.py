@@ -73,3 +73,27 @@ def test_extents_just_below_a_power_of_two(eps, nd, dtype, depth):
     boxes = np.array(b).astype(dtype)
     p, q = _beyond_faces(-w, w, nd, dtype, w, rng)
     _check(boxes, 1.0, dtype, {"points": p, "boxes": q})
+
+
+@pytest.mark.parametrize("nd,dtype", [(3, np.float64), (2, np.float64), (3, np.float32)])
+@pytest.mark.parametrize("n", [4, 64, 600, 4097, 262_145, 300_001])
+def test_boxes_with_nan_coordinates(n, nd, dtype):
+    """A box's NaN bound gives way to any other in a union, so which boxes an inner
+    node holds depends on how its union is put together: as the reference's."""
+    rng = np.random.default_rng([n, nd])
+    h = 0.5 / n ** (1.0 / nd)
+    c = rng.random((n, nd))
+    e = rng.uniform(0.2 * h, h, (n, nd))
+    boxes = np.concatenate([c - e, c + e], 1)
+    k = np.flatnonzero(rng.random(n) < 0.2)
+    k = k if k.size else np.array([n // 2])
+    boxes[k, rng.integers(2 * nd, size=k.size)] = np.nan
+    boxes[k[::3]] = np.nan
+    # the root's bounds, from minima whose order is open, hold whatever it is
+    boxes[[0, -1]] = [-0.2] * nd + [1.2] * nd
+    p = rng.random((2000, nd))
+    q = np.concatenate([p - h, p + h], 1)
+    d = rng.normal(size=(200, nd))
+    r = np.concatenate([p[:200], d / np.linalg.norm(d, axis=1, keepdims=True)], 1)
+    _check(boxes.astype(dtype), 1.000123, dtype,
+           {"points": p.astype(dtype), "boxes": q.astype(dtype), "rays": r.astype(dtype)})
