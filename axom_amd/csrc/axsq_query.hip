@@ -405,10 +405,11 @@ __global__ __launch_bounds__(kWaveLanes) void k_ray_fill(FindArgs a) {
 }
 
 // The fill pass for queries with at most kstash (<= 64) candidates: the ids of
-// the leaf positions the count pass kept, at offsets[i]. The ids of a wave's 64
-// queries are one run of the output, which its lanes take 64 at a time, each
-// finding its query among the 64 offsets; four such steps' loads are in flight
-// at once. Where no query has more than 4 ids a lane copies its own.
+// the leaf positions the count pass kept, at offsets[i]. What a wave's 64
+// queries kept is taken as one run, 64 ids at a time, each lane finding its
+// query among the 64 places in the run; four such steps' loads are in flight at
+// once. Queries with more ids have no place in it, however many those are. Where
+// no query has more than 4 ids a lane copies its own.
 // 1M queries of 12 ids: 84 us with a query at a time over the wave, 48 here.
 template <bool PAIRS>
 __global__ __launch_bounds__(kBlock) void k_stash_copy(const int32_t* __restrict__ stash,
@@ -417,9 +418,10 @@ __global__ __launch_bounds__(kBlock) void k_stash_copy(const int32_t* __restrict
                                                         const int32_t* __restrict__ offsets,
                                                         const int32_t* __restrict__ leaf_ids,
                                                         int64_t nq, int32_t* __restrict__ cands) {
-  __shared__ int32_t s_off[kBlock];
+  __shared__ int32_t s_at[kBlock], s_off[kBlock];
   const int lane = (int)__lane_id();
-  int32_t* off = s_off + (threadIdx.x - lane);
+  int32_t* at = s_at + (threadIdx.x - lane);    // a query's place in the run
+  int32_t* off = s_off + (threadIdx.x - lane);  // and in the output
   const int64_t base = (int64_t)blockIdx.x * blockDim.x + threadIdx.x - lane;  // the wave's first
   if (base >= nq) return;  // the whole wave
   auto put = [&](int32_t k, int64_t i, int32_t id) {
@@ -429,38 +431,42 @@ __global__ __launch_bounds__(kBlock) void k_stash_copy(const int32_t* __restrict
       cands[k] = id;
   };
   const int64_t mine = base + lane;
-  const int32_t c = (mine < nq) ? stash_cnt[mine] : 0;
-  const int32_t o = (mine < nq) ? offsets[mine] : 0x7fffffff;
-  if (__ballot(c > 4 && c <= kstash) == 0) {  // few ids everywhere
-    if (c <= kstash)
-      for (int32_t k = 0; k < c; ++k) put(o + k, mine, leaf_ids[stash[mine * kstash + k]]);
+  int32_t c = (mine < nq) ? stash_cnt[mine] : 0;
+  const int32_t o = (mine < nq) ? offsets[mine] : 0;
+  if (c > kstash) c = 0;  // listed: searched again
+  if (__ballot(c > 4) == 0) {  // few ids everywhere
+    for (int32_t k = 0; k < c; ++k) put(o + k, mine, leaf_ids[stash[mine * kstash + k]]);
     return;
   }
+  int32_t end = c;  // of this lane's part of the run, at most 64 * 64
+  for (int step = 1; step < kWaveLanes; step <<= 1) {
+    const int32_t v = __shfl_up(end, step);
+    if (lane >= step) end += v;
+  }
+  at[lane] = end - c;
   off[lane] = o;
   wave_sync();
-  const int last = (int)min(nq - base, (int64_t)kWaveLanes) - 1;
-  const int32_t lo = __shfl(o, 0), hi = __shfl(o, last) + __shfl(c, last);
-  const uint64_t listed = __ballot(c > kstash);  // searched again
-  for (int32_t j0 = lo + lane; j0 - lane < hi; j0 += 4 * kWaveLanes) {
-    int32_t id[4];
+  const int32_t run = __shfl(end, kWaveLanes - 1);
+  for (int32_t j0 = lane; j0 - lane < run; j0 += 4 * kWaveLanes) {
+    int32_t id[4], to[4];
     int q[4];
-    bool take[4];
 #pragma unroll
     for (int u = 0; u < 4; ++u) {
       const int32_t j = j0 + u * kWaveLanes;
-      q[u] = 0;  // the last query whose ids start at or before j
+      q[u] = 0;  // the last query whose part starts at or before j
 #pragma unroll
       for (int step = kWaveLanes / 2; step > 0; step >>= 1)
-        if (off[q[u] + step] <= j) q[u] += step;
-      take[u] = j < hi && !((listed >> q[u]) & 1);
-      id[u] = take[u] ? stash[(base + q[u]) * kstash + (j - off[q[u]])] : 0;
+        if (at[q[u] + step] <= j) q[u] += step;
+      const int32_t k = j - at[q[u]];
+      to[u] = j < run ? off[q[u]] + k : 0;
+      id[u] = j < run ? stash[(base + q[u]) * kstash + k] : 0;
     }
 #pragma unroll
     for (int u = 0; u < 4; ++u)
-      if (take[u]) id[u] = leaf_ids[id[u]];
+      if (j0 + u * kWaveLanes < run) id[u] = leaf_ids[id[u]];
 #pragma unroll
     for (int u = 0; u < 4; ++u)
-      if (take[u]) put(j0 + u * kWaveLanes, base + q[u], id[u]);
+      if (j0 + u * kWaveLanes < run) put(to[u], base + q[u], id[u]);
   }
 }
 

@@ -97,3 +97,49 @@ def test_boxes_with_nan_coordinates(n, nd, dtype):
     r = np.concatenate([p[:200], d / np.linalg.norm(d, axis=1, keepdims=True)], 1)
     _check(boxes.astype(dtype), 1.000123, dtype,
            {"points": p.astype(dtype), "boxes": q.astype(dtype), "rays": r.astype(dtype)})
+
+
+def _search(g, p):
+    off = torch.empty(p.shape[0], dtype=torch.int32, device=DEV)
+    cnt = torch.empty_like(off)
+    return off, cnt, g.findPoints(off, cnt, p.shape[0], p)
+
+
+@pytest.mark.parametrize("nq", [1, 63, 64, 65, 1000])
+def test_kept_ids_beside_queries_with_more(nq):
+    """Waves whose queries have none, few, all that are kept and more than are kept."""
+    rng = np.random.default_rng(nq)
+    sizes = [500, 64, 65, 63, 10, 3, 1]
+    boxes = np.concatenate([np.tile([[2.0 * k] * 3 + [2.0 * k + 1] * 3], (m, 1))
+                            for k, m in enumerate(sizes)])
+    rng.shuffle(boxes)
+    p = rng.integers(0, len(sizes) + 2, nq)[:, None] * 2.0 + rng.uniform(0.1, 0.9, (nq, 3))
+    g, o = spin.BVH(_t(boxes)), orc.OracleBVH(boxes, 1.000123)
+    ooff, ocnt, ocand = o.find("points", p)
+    for _ in range(2):  # the first search of a tree fills by a second walk
+        off, cnt, cand = _search(g, _t(p))
+        assert np.array_equal(cnt.cpu().numpy(), ocnt)
+        assert np.array_equal(off.cpu().numpy(), ooff)
+        assert np.array_equal(cand.cpu().numpy(), ocand)
+
+
+def test_candidate_total_next_to_the_int32_limit():
+    """The kept ids of the last queries end 5 below 2^31 - 1."""
+    many, few = 65536, 10
+    boxes = torch.tensor([[0.0] * 3 + [1.0] * 3], dtype=torch.float64, device=DEV)
+    boxes = torch.cat([boxes.repeat(many, 1), boxes.repeat(few, 1) + 2.0])
+    na, nb = 32767, 6553
+    p = torch.full((na + nb, 3), 0.5, dtype=torch.float64, device=DEV)
+    p[na:] = 2.5
+    total = na * many + nb * few
+    assert total == 2**31 - 6
+    g = spin.BVH(boxes)
+    for _ in range(2):
+        off, cnt, cand = _search(g, p)
+        assert cand.numel() == total
+        assert bool((cnt[:na] == many).all()) and bool((cnt[na:] == few).all())
+        ids = torch.arange(many + few, dtype=torch.int32, device=DEV)
+        assert bool((cand[na * many:].view(nb, few) == ids[many:]).all())
+        a = cand[:na * many].view(na, many)
+        assert all(bool((a[r:r + 2048] == ids[:many]).all()) for r in range(0, na, 2048))
+        del cand, a
