@@ -30,7 +30,10 @@
 namespace axsq {
 
 // Coordinates of the searches: (x - o) * scale, the root box's longest side
-// between 1 and 2. ok: finite and in range; else the FP64 nodes are walked.
+// between 1 and 2. ok: finite, in range and not a point, from which no size of
+// the tree could be told (100,000 equal boxes without extent, 10,000 points
+// elsewhere: every node visited, 75 ms; 0.07 with the FP64 nodes); else the FP64
+// nodes are walked.
 struct FindSpace {
   double o[3];
   double scale;
@@ -45,13 +48,10 @@ __host__ __device__ inline bool find_space(const double b[6], FindSpace& fs) {
     if (e > ext) ext = e;
     fs.o[d] = 0.5 * (b[d] + b[3 + d]);
   }
-  fs.scale = 1.0;
-  if (ext > 0.0) {
-    int e2 = 0;
-    (void)frexp(ext, &e2);
-    ok = ok && e2 > -330;
-    fs.scale = ldexp(1.0, 1 - (e2 > -330 ? e2 : -330));
-  }
+  int e2 = 0;
+  (void)frexp(ext, &e2);
+  ok = ok && ext > 0.0 && e2 > -330;
+  fs.scale = ldexp(1.0, 1 - (e2 > -330 ? e2 : -330));
   return ok;
 }
 
@@ -135,10 +135,12 @@ __device__ __forceinline__ FindNode make_find_node(const FindSpace& fs, int dims
     if (dims == 2) c[d] = __uint_as_float(__float_as_uint(c[d]) & ~7u);
     if ((flags & 3) && d < dims) m = fmax(m, fmax(fabs(lo - c[d]), fabs(hi - c[d])));
   }
-  int e2 = -59;
+  // extents below 2; a smaller node, down to a point, spans its margin of at
+  // most 2^15, which a half holds
+  int e2 = -58;
   if (m > 0.0) (void)frexp(m, &e2);
-  e2 = e2 < -59 ? -59 : e2 > 3 ? 3 : e2;
-  const double s = ldexp(1.0, 1 - e2);  // extents below 2
+  e2 = e2 < -58 ? -58 : e2 > 3 ? 3 : e2;
+  const double s = ldexp(1.0, 1 - e2);
   const double margin = 9.5367431640625e-07 + s * 5.684341886080802e-14;  // 2^-20 + s 2^-44
   n.s = (float)s;
   for (int d = 0; d < 3; ++d) {
@@ -169,7 +171,7 @@ __device__ __forceinline__ void store_find_node(FindNode* __restrict__ nodes, in
     nodes[i] = n;
     return;
   }
-  const uint32_t code = (__float_as_uint(n.s) >> 23) - 125u;  // s = 2^-2 .. 2^60: 0 .. 62
+  const uint32_t code = (__float_as_uint(n.s) >> 23) - 125u;  // s = 2^-2 .. 2^59: 0 .. 61
   FindNode2 m;
   m.cs[0] = (__float_as_uint(n.cs[0]) & ~7u) | (code >> 3);
   m.cs[1] = (__float_as_uint(n.cs[1]) & ~7u) | (code & 7u);

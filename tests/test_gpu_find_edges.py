@@ -143,3 +143,52 @@ def test_candidate_total_next_to_the_int32_limit():
         a = cand[:na * many].view(na, many)
         assert all(bool((a[r:r + 2048] == ids[:many]).all()) for r in range(0, na, 2048))
         del cand, a
+
+
+@pytest.mark.parametrize("nd,dtype", [(3, np.float64), (2, np.float64), (3, np.float32),
+                                      (2, np.float32)])
+@pytest.mark.parametrize("n", [1, 2, 3, 65, 4097])
+@pytest.mark.parametrize("others", [False, True])
+def test_equal_boxes_without_extent(n, others, nd, dtype):
+    """Boxes that are all one point, and the same among others: queries at the
+    point, one step from it and elsewhere."""
+    rng = np.random.default_rng([n, nd])
+    at = np.full((1, nd), 0.7)
+    boxes = np.repeat(np.concatenate([at, at], 1), n, 0)
+    if others:
+        c = rng.random((n, nd))
+        boxes = np.concatenate([boxes, np.concatenate([c - 0.01, c + 0.01], 1)])
+        rng.shuffle(boxes)
+    boxes = boxes.astype(dtype)
+    p = np.repeat(at, 60, 0).astype(dtype)
+    p[20:40] = np.nextafter(p[20:40], rng.choice([0.0, 1.0], (20, nd)).astype(dtype))
+    p[40:] = rng.random((20, nd))
+    q = np.concatenate([p, p], 1)
+    q[::3, nd:] += dtype(0.01)
+    d = rng.normal(size=(60, nd)).astype(dtype)
+    r = np.concatenate([p - d * (np.arange(60)[:, None] % 2).astype(dtype), d], 1)
+    _check(boxes, 1.000123, dtype, {"points": p, "boxes": q, "rays": r})
+
+
+def test_equal_boxes_without_extent_are_passed_over():
+    """A search that misses such a tree ends at its root: 20,000 points and 200,000
+    boxes took 149 ms where every node was visited, 0.1 at the root."""
+    rng = np.random.default_rng(3)
+    n = 200_000
+    c = rng.random((n, 3))
+    p = _t(rng.random((20_000, 3)) + 2.0)
+
+    def best(boxes):
+        g, t = spin.BVH(_t(boxes)), []
+        for _ in range(4):
+            a, b = (torch.cuda.Event(enable_timing=True) for _ in range(2))
+            a.record()
+            _, cnt, _ = _search(g, p)
+            b.record()
+            torch.cuda.synchronize()
+            t.append(a.elapsed_time(b))
+        assert int(cnt.sum()) == 0
+        return min(t)
+
+    spread = best(np.concatenate([c, c], 1))
+    assert best(np.full((n, 6), 0.5)) < 10.0 + 20.0 * spread
