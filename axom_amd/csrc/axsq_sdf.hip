@@ -566,9 +566,10 @@ struct CullQuery {
     // 1e-6: ties (checkCandidate); 1.1 2^-21 R: projections; 2^-50 qmax: q - o
     slack = 1.01e-6f * scale + R * 5.25e-7f + qmax * 8.8817842e-16f;
     // a query at most a0 + a1 / |D| from a node's order plane reads the boxes:
-    // FP64 right_first is decided to 2^-49 R^2 / |D| and the plane's float form
-    // to 2^-20 R; the FP32 form's own decision is near_plane's
-    a0 = (MIXED ? R + qmax : R) * 1.9073486e-6f;
+    // FP64 right_first is decided to 2^-49 R^2 / |D|, the plane's float form to
+    // 2^-20 R and its place (m, of the boxes' rounded centroids) to 2^-52 qmax;
+    // the FP32 form's own decision is near_plane's
+    a0 = MIXED ? (R + qmax) * 1.9073486e-6f : fmaf(R, 1.9073486e-6f, qmax * 8.8817842e-16f);
     a1 = MIXED ? 0.0f : R * R * 1.7763568e-15f;
     qm = qmax * 1.001f;  // the boxes are scaled by 1.000123
     thr = 3.402823466e38f;
