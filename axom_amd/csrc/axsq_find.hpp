@@ -222,12 +222,13 @@ __device__ __forceinline__ void load_find_node(const FindNode* __restrict__ node
 
 // A query's two corners in the search's coordinates, as float pairs (a
 // point's are equal). Far coordinates are clamped: outside every box either
-// way.
+// way, and finite times every node's scale (an infinite t less the infinite
+// range of an invalid child would be a NaN, which the maximum drops).
 template <bool BOX>
 struct FindQuery {
   float lh[3], ll[3], hh[BOX ? 3 : 1], hl[BOX ? 3 : 1];
   __device__ __forceinline__ static void split(double x, float& h, float& l) {
-    x = x > 1e30 ? 1e30 : x < -1e30 ? -1e30 : x;  // a NaN stays
+    x = x > 1e18 ? 1e18 : x < -1e18 ? -1e18 : x;  // a NaN stays
     h = (float)x;
     l = (float)(x - (double)h);
   }

@@ -192,3 +192,19 @@ def test_equal_boxes_without_extent_are_passed_over():
 
     spread = best(np.concatenate([c, c], 1))
     assert best(np.full((n, 6), 0.5)) < 10.0 + 20.0 * spread
+
+
+@pytest.mark.parametrize("nd,dtype", [(3, np.float64), (2, np.float64), (3, np.float32)])
+@pytest.mark.parametrize("depth", [5, 28, 29, 30, 31, 50])
+def test_boundless_queries_beside_an_invalid_box(depth, nd, dtype):
+    """A query that holds everything, at a small node one of whose children is
+    invalid."""
+    w = 1.5 * 2.0**-depth
+    far = np.finfo(dtype).max / 8
+    boxes = np.array([[-1.0] * nd + [-0.9] * nd, [-w] * nd + [w] * nd, [far] * nd + [-far] * nd,
+                      [0.9] * nd + [1.0] * nd]).astype(dtype)
+    big = np.array([1.0, 1e15, 1e20, 1e25, 1e30, 1e36, far, np.inf])
+    q = np.repeat(big[:, None], 2 * nd, 1)
+    q[:, :nd] *= -1.0
+    p = np.concatenate([q[:, nd:], q[:, :nd], q[:, :nd] * (-1.0) ** np.arange(nd)])
+    _check(boxes, 1.0, dtype, {"points": p.astype(dtype), "boxes": q.astype(dtype)})
