@@ -38,7 +38,10 @@ __global__ __launch_bounds__(kBlock) void k_pack_verts(const double* __restrict_
 // Triangle corners (A B C, TriRec), the corner box (BoundingBox{A, B, C},
 // compute_bounding_box.hpp:110-114, BoundingBox.hpp:405-422,464-482) and the
 // degenerate flag (Triangle::degenerate, Triangle.hpp:104-109,327-330). verts:
-// k_pack_verts' records, or NULL.
+// k_pack_verts' records, or NULL. A triangle that refers to a vertex outside
+// [0, nverts) sets bit 1 of *status and gets an invalid box: taken at vertex 0,
+// a connectivity of such triangles would be as many boxes on one point, and the
+// walk test all their pairs before the call ends with the error.
 // 2.6M triangles of 1.3M vertices: 247 us from the three arrays, 186 with the
 // records (15 of it making them).
 __global__ __launch_bounds__(kBlock) void k_tri_setup(const double* __restrict__ x,
@@ -56,10 +59,11 @@ __global__ __launch_bounds__(kBlock) void k_tri_setup(const double* __restrict__
   if (c >= n) return;
   TriRec r;
   double* t = r.v;
+  bool bad = false;
   for (int k = 0; k < 3; ++k) {
     int32_t v = conn[3 * c + k];
     if (v < 0 || v >= nverts) {
-      atomicOr(status, 2);
+      bad = true;
       v = 0;
     }
     if (verts) {
@@ -80,6 +84,13 @@ __global__ __launch_bounds__(kBlock) void k_tri_setup(const double* __restrict__
       if (p < b[d]) b[d] = p;
       if (p > b[3 + d]) b[3 + d] = p;
     }
+  if (bad) {
+    atomicOr(status, 2);
+    for (int d = 0; d < 3; ++d) {
+      b[d] = kDblMax;
+      b[3 + d] = -kDblMax;
+    }
+  }
   double nrm[3];
   tri_normal(t, nrm);
   degen[c] = tri_degenerate(nrm) ? 1 : 0;
@@ -345,7 +356,6 @@ __global__ __launch_bounds__(kBlock) void k_tri_tri(const double* __restrict__ t
                : 0;
 }
 
-// Device allocations of one call, freed on every exit path.
 // Bounding box of each cell of `npc` nodes (primal::compute_bounding_box of
 // the cell's points: BoundingBox::addPoint of each, BoundingBox.hpp:466-482,
 // a coordinate replaces the bound it is strictly below / above). A node index
@@ -388,6 +398,7 @@ __global__ __launch_bounds__(kBlock) void k_expand_first(const int32_t* __restri
   for (int32_t j = 0; j < c; ++j) first[o + j] = (int32_t)i;
 }
 
+// Device allocations of one call, freed on every exit path.
 struct Scratch {
   std::vector<void*> ptrs;
   axsq_alloc_fn fn = nullptr;  // the caller's, whose blocks stay its own
@@ -560,7 +571,7 @@ int self_intersections(const double* x, const double* y, const double* z, int64_
     r.status[1] = status;
     ReadValues v;
     AXSQ_TRY(read_back(r, &v, s));
-    if (v.status[1]) {  // such a vertex was taken as vertex 0 up to here
+    if (v.status[1]) {
       set_error("axsq_mesh_self_intersections: connectivity refers to a vertex outside [0, %lld)",
                 (long long)nverts);
       return AXSQ_ERR_INVALID_ARG;

@@ -1,12 +1,15 @@
 """The candidate searches at the edges of the compact nodes' number range:
 results are integers, equal to the oracle's, order included.
 """
+import time
+
 import numpy as np
 import pytest
 
 torch = pytest.importorskip("torch")
 
-from axom_amd import spin  # noqa: E402
+from axom_amd import _lib as L  # noqa: E402
+from axom_amd import quest, spin  # noqa: E402
 from oracle import oracle as orc  # noqa: E402
 
 pytestmark = pytest.mark.gpu
@@ -208,3 +211,20 @@ def test_boundless_queries_beside_an_invalid_box(depth, nd, dtype):
     q[:, :nd] *= -1.0
     p = np.concatenate([q[:, nd:], q[:, :nd], q[:, :nd] * (-1.0) ** np.arange(nd)])
     _check(boxes, 1.0, dtype, {"points": p.astype(dtype), "boxes": q.astype(dtype)})
+
+
+@pytest.mark.parametrize("ntris", [1, 7, 2_000_000])
+@pytest.mark.parametrize("some", [False, True])
+def test_vertex_ids_out_of_range_cost_no_pairs(ntris, some):
+    """Refused as before, in the time of a tree build: no pair is tested for
+    triangles without vertices, however many they are."""
+    rng = np.random.default_rng(ntris)
+    v = rng.random((99, 3))
+    t = np.full((ntris, 3), 99, np.int32)
+    t[ntris // 2:] = -1
+    if some:
+        t[: min(ntris - 1, 33)] = np.arange(99).reshape(33, 3)[: min(ntris - 1, 33)]
+    a = time.perf_counter()
+    with pytest.raises(L.AxsqError, match="outside"):
+        quest.findTriMeshIntersectionsBVH(_t(v), _t(t))
+    assert time.perf_counter() - a < 5.0
