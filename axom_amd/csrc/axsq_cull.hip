@@ -20,6 +20,11 @@ constexpr int kSmallNode = 8;
 constexpr int kLargeNode = 1024;
 constexpr int kMaxLargePath = 256;  // large nodes over one 1,024-leaf chunk
 constexpr int kCullWave = 64;
+constexpr int kClassSamples = 256;
+// ctl: [0] unusable, [1] [2] list lengths; k_cull_class: [3] loose samples, [4 + k]
+// and [8 + k] nodes of size k whose boxes are over 2 and 1.5 times as thick, [12]
+// joined samples
+constexpr int kCullCtl = 16;
 
 __device__ __forceinline__ void mesh_coords(const CullSpace& cs, const double* V, float x[3]) {
   for (int d = 0; d < 3; ++d) x[d] = (float)((V[d] - cs.o[d]) * cs.scale);
@@ -116,8 +121,8 @@ __device__ __forceinline__ float tri_tau(const double T[9], double reach) {
   return (float)(tau * 1.000001);
 }
 
-// Per leaf: tau, its triangles' NormRec, and the running sum of normals within
-// its block of 256.
+// Per leaf: tau, its triangles' NormRec (norms given), and the running sum of
+// normals within its block of 256.
 template <bool CELLS>
 __global__ __launch_bounds__(kBlock) void k_cull_leaf(const TriRec* __restrict__ tris, int64_t n,
                                                        double reach, double tau_max, double scale,
@@ -139,11 +144,13 @@ __global__ __launch_bounds__(kBlock) void k_cull_leaf(const TriRec* __restrict__
       t = (te < 0.0f || t < 0.0f) ? -1.0f : fmaxf(t, te);
       tri_normal(T, m);
       for (int d = 0; d < 3; ++d) nr[d] += m[d];
-      NormRec r;
-      unit3(m, r.un);
-      const bool flat = tri_degenerate(m);
-      for (int k = 0; k < 3; ++k) r.angle[k] = flat ? -1.0 : tri_angle(T, k);
-      norms[CELLS ? 2 * pos + e : pos] = r;
+      if (norms) {
+        NormRec r;
+        unit3(m, r.un);
+        const bool flat = tri_degenerate(m);
+        for (int k = 0; k < 3; ++k) r.angle[k] = flat ? -1.0 : tri_angle(T, k);
+        norms[CELLS ? 2 * pos + e : pos] = r;
+      }
     }
     if (!(t >= 0.0f && t <= tau_max)) {
       atomicOr(&ctl[0], 1);
@@ -194,6 +201,122 @@ __global__ __launch_bounds__(1024) void k_cull_scan(double* __restrict__ totals,
   }
 }
 
+// The unit mean normal of a node's triangles, from the prefix sums (pre within
+// blocks, base over them); x where it vanishes.
+__device__ __forceinline__ void mean_normal(const Node64& nd, const double* __restrict__ pre,
+                                            const double* __restrict__ base, double w[3]) {
+  double len = 0.0;
+  for (int d = 0; d < 3; ++d) {
+    const double hi = pre[3 * (int64_t)nd.hi + d] + base[3 * (int64_t)(nd.hi / kBlock) + d];
+    const double lo = nd.lo > 0 ? pre[3 * (int64_t)(nd.lo - 1) + d] +
+                                      base[3 * (int64_t)((nd.lo - 1) / kBlock) + d]
+                                : 0.0;
+    w[d] = hi - lo;
+    len += w[d] * w[d];
+  }
+  const double il = len > 0.0 ? 1.0 / sqrt(len) : 0.0;
+  if (il > 0.0 && il < 1e300) {
+    for (int d = 0; d < 3; ++d) w[d] *= il;
+  } else {
+    w[0] = 1.0;
+    w[1] = w[2] = 0.0;
+  }
+}
+
+// What oriented boxes gain on this mesh, from the nodes over kClassSamples leaves
+// spread over the tree: four waves each descend to the node of at most 32,768,
+// 4,096, 512 and 64 leaves over such a leaf and compare the extent of the
+// axis-aligned box along the mean normal with that of what the node holds,
+// tolerances included (of larger nodes 1,024 leaves are looked at). A sample is
+// loose where most leaves' tolerances are more than a quarter of their triangles'
+// height, joined where most of its 64 triangles share a corner with another one.
+// Bound by latency: a descent of up to 16 dependent loads, 16 leaf loads a lane.
+template <bool CELLS>
+__global__ __launch_bounds__(4 * kCullWave) void k_cull_class(CullSpace cs,
+                                                               const Node64* __restrict__ nodes,
+                                                               int32_t ninner,
+                                                               const TriRec* __restrict__ tris,
+                                                               const float* __restrict__ tau,
+                                                               const double* __restrict__ pre,
+                                                               const double* __restrict__ base,
+                                                               int32_t* __restrict__ ctl) {
+  const int lane = (int)threadIdx.x % kCullWave, k = (int)threadIdx.x / kCullWave;
+  const int32_t p = (int32_t)((2 * (int64_t)blockIdx.x + 1) * (ninner + 1) / (2 * kClassSamples));
+  const int32_t cap = 32768 >> (3 * k);
+  Node64 nd = nodes[0];
+  while (nd.hi - nd.lo + 1 > cap) {  // a child holds fewer leaves
+    const int32_t next = p <= nd.mid ? nd.lc : nd.rc;
+    if (next < 0 || next >= ninner) break;
+    nd = nodes[next];
+  }
+  double w[3];
+  mean_normal(nd, pre, base, w);
+  const int32_t size = nd.hi - nd.lo + 1, step = (size + 1023) / 1024;
+  double lo = INFINITY, hi = -INFINITY;
+  int32_t loose = 0, seen = 0;
+#pragma unroll 4
+  for (int32_t q = nd.lo + lane * step; q <= nd.hi; q += kCullWave * step) {
+    const double e = tau[q];
+    const int nrec = CELLS ? tris[2 * (int64_t)q].pad : 1;
+    for (int r = 0; r < nrec; ++r) {
+      const double* T = tris[CELLS ? 2 * (int64_t)q + r : (int64_t)q].v;
+      double l2 = 0.0;
+      for (int c = 0; c < 3; ++c) {
+        double t = 0.0, d2 = 0.0;
+        for (int d = 0; d < 3; ++d) {
+          t += (T[3 * c + d] - cs.o[d]) * cs.scale * w[d];
+          const double g = T[(3 * c + 3 + d) % 9] - T[3 * c + d];
+          d2 += g * g;
+        }
+        lo = fmin(lo, t - e);
+        hi = fmax(hi, t + e);
+        l2 = fmax(l2, d2);
+      }
+      double m[3];
+      tri_normal(T, m);
+      const double h = sqrt((m[0] * m[0] + m[1] * m[1] + m[2] * m[2]) / l2) * cs.scale;
+      ++seen;
+      loose += e > 0.25 * h;
+    }
+  }
+  for (int o = kCullWave / 2; o > 0; o >>= 1) {
+    lo = fmin(lo, __shfl_xor(lo, o));
+    hi = fmax(hi, __shfl_xor(hi, o));
+    loose += __shfl_xor(loose, o);
+    seen += __shfl_xor(seen, o);
+  }
+  double box = 0.0;
+  for (int d = 0; d < 3; ++d) {
+    const double l0 = (nd.flags & 1) ? nd.l[d] : nd.r[d], l1 = (nd.flags & 1) ? nd.l[3 + d] : nd.r[3 + d];
+    const double r0 = (nd.flags & 2) ? nd.r[d] : l0, r1 = (nd.flags & 2) ? nd.r[3 + d] : l1;
+    box += fabs(w[d]) * (fmax(l1, r1) - fmin(l0, r0)) * cs.scale;
+  }
+  // the walk's slack on both sides: ties, and projections at a unit's distance
+  const double own = hi - lo + 2e-6 * (cs.scale + 1.0);
+  if (lane == 0 && box > 2.0 * own) atomicAdd(&ctl[4 + k], 1);
+  if (lane == 0 && box > 1.5 * own) atomicAdd(&ctl[8 + k], 1);
+  if (k < 3) return;
+  // at most 64 leaves, one a lane
+  const bool has = lane < size;
+  const int32_t q = nd.lo + (has ? lane : 0);
+  const double* T = tris[CELLS ? 2 * (int64_t)q : (int64_t)q].v;
+  double v[9];
+  for (int c = 0; c < 9; ++c) v[c] = T[c];
+  bool meets = false;
+  const int32_t held = min(size, kCullWave);
+  for (int o = 0; o < held; ++o)
+    for (int c = 0; c < 9; c += 3) {
+      const double x = __shfl(v[c], o), y = __shfl(v[c + 1], o), z = __shfl(v[c + 2], o);
+      const bool eq = (x == v[0] && y == v[1] && z == v[2]) ||
+                      (x == v[3] && y == v[4] && z == v[5]) ||
+                      (x == v[6] && y == v[7] && z == v[8]);
+      meets = meets || (o != lane && eq);
+    }
+  const int32_t shared = __popcll(__ballot(has && meets));
+  if (lane == 0 && 2 * loose > seen) atomicAdd(&ctl[3], 1);
+  if (lane == 0 && 2 * shared > held) atomicAdd(&ctl[12], 1);
+}
+
 __device__ __forceinline__ uint32_t ordered(float f) {
   const uint32_t b = __float_as_uint(f);
   return (b & 0x80000000u) ? ~b : (b | 0x80000000u);
@@ -234,22 +357,8 @@ __global__ __launch_bounds__(kBlock) void k_cull_nodes(CullSpace cs,
     CullNode n;
     n.lc = nd.lc;
     n.rc = nd.rc;
-    double w[3], len = 0.0;
-    for (int d = 0; d < 3; ++d) {
-      const double hi = pre[3 * (int64_t)nd.hi + d] + base[3 * (int64_t)(nd.hi / kBlock) + d];
-      const double lo = nd.lo > 0 ? pre[3 * (int64_t)(nd.lo - 1) + d] +
-                                        base[3 * (int64_t)((nd.lo - 1) / kBlock) + d]
-                                  : 0.0;
-      w[d] = hi - lo;
-      len += w[d] * w[d];
-    }
-    const double il = len > 0.0 ? 1.0 / sqrt(len) : 0.0;
-    if (il > 0.0 && il < 1e300) {
-      for (int d = 0; d < 3; ++d) w[d] *= il;
-    } else {
-      w[0] = 1.0;
-      w[1] = w[2] = 0.0;
-    }
+    double w[3];
+    mean_normal(nd, pre, base, w);
     double cl[3], cr[3], D[3], dl = 0.0, tw = 0.0;
     for (int d = 0; d < 3; ++d) {  // centroids as in BoxTests::right_first
       cl[d] = 0.5 * (nd.l[d] + nd.l[3 + d]);
@@ -476,8 +585,8 @@ __global__ __launch_bounds__(kBlock) void k_cull_large_end(const Node64* __restr
 }
 
 template <bool CELLS>
-int build(const axsq_bvh* b, const TriRec* tris, const CullSpace& cs, double diag, CullNode* out,
-          NormRec* norms, Workspace& ws, int32_t* bad, hipStream_t s) {
+int build(const axsq_bvh* b, const TriRec* tris, const CullSpace& cs, double diag, int parts,
+          CullNode* out, NormRec* norms, CullResult* res, Workspace& ws, hipStream_t s) {
   const int64_t n = b->n;
   const int32_t ninner = (int32_t)(n - 1);
   const int64_t nb = grid_for(n);
@@ -485,55 +594,87 @@ int build(const axsq_bvh* b, const TriRec* tris, const CullSpace& cs, double dia
   AXSQ_TRY(ws.k1.ensure(sizeof(int32_t) * (size_t)ninner));
   AXSQ_TRY(ws.v0.ensure(sizeof(double) * 3 * (size_t)n));
   AXSQ_TRY(ws.v1.ensure(sizeof(double) * 3 * (size_t)nb));
-  AXSQ_TRY(ws.cnt.ensure(sizeof(int32_t) * 4));
+  AXSQ_TRY(ws.cnt.ensure(sizeof(int32_t) * kCullCtl));
   float* tau = ws.k0.as<float>();
   double* pre = ws.v0.as<double>();
   double* totals = ws.v1.as<double>();
   int32_t* ctl = ws.cnt.as<int32_t>();
-  int32_t* mid_list = ws.k1.as<int32_t>();
-  // nodes over 1,024 leaves: few in a balanced tree, up to ninner - 1,023 in a
-  // chain, each with 12 running extents
-  const size_t nlarge = (size_t)std::max<int64_t>((int64_t)ninner - kLargeNode + 1, 1);
-  AXSQ_TRY(ws.redo.ensure(sizeof(int32_t) * nlarge));
-  AXSQ_TRY(ws.misc.ensure(sizeof(uint32_t) * 12 * nlarge));
-  int32_t* large_list = ws.redo.as<int32_t>();
-  uint32_t* acc = ws.misc.as<uint32_t>();
-  AXSQ_TRY(fill_i32(ctl, 0, 4, s));
-  k_cull_leaf<CELLS><<<(unsigned)nb, kBlock, 0, s>>>(tris, n, kCullReach * diag,
-                                                     diag * (1.0 / 1024.0), cs.scale, tau, pre, totals,
-                                                     norms, ctl);
-  AXSQ_CHECK_HIP(hipGetLastError());
-  k_cull_scan<<<1, 1024, 0, s>>>(totals, nb);
-  AXSQ_CHECK_HIP(hipGetLastError());
-  k_cull_nodes<CELLS><<<grid_for(ninner), kBlock, 0, s>>>(cs, b->nodes, ninner, tris, tau, pre,
-                                                          totals, out, mid_list, large_list, acc,
-                                                          ctl);
-  AXSQ_CHECK_HIP(hipGetLastError());
-  if (n > kSmallNode) {
-    const unsigned g = (unsigned)std::min<int64_t>((n / 6 + 3) / 4 + 1, 8192);
-    k_cull_mid<CELLS><<<g, kBlock, 0, s>>>(cs, b->nodes, tris, tau, mid_list, ctl, out);
+  if (parts & kCullLeaves) {
+    AXSQ_TRY(fill_i32(ctl, 0, kCullCtl, s));
+    k_cull_leaf<CELLS><<<(unsigned)nb, kBlock, 0, s>>>(tris, n, kCullReach * diag,
+                                                       diag * (1.0 / 1024.0), cs.scale, tau, pre,
+                                                       totals, norms, ctl);
+    AXSQ_CHECK_HIP(hipGetLastError());
+    k_cull_scan<<<1, 1024, 0, s>>>(totals, nb);
     AXSQ_CHECK_HIP(hipGetLastError());
   }
-  if (n > kLargeNode) {
-    k_cull_large<CELLS><<<(unsigned)((n + kLargeNode - 1) / kLargeNode), kBlock, 0, s>>>(
-        cs, b->nodes, ninner, tris, tau, out, acc, ctl);
-    AXSQ_CHECK_HIP(hipGetLastError());
-    k_cull_large_end<<<(unsigned)std::min<int64_t>(n / kLargeNode / kBlock + 1, 256), kBlock, 0,
-                       s>>>(b->nodes, large_list, ctl, acc, out);
+  if (parts & kCullClass) {
+    k_cull_class<CELLS><<<kClassSamples, 4 * kCullWave, 0, s>>>(cs, b->nodes, ninner, tris, tau, pre,
+                                                            totals, ctl);
     AXSQ_CHECK_HIP(hipGetLastError());
   }
-  AXSQ_CHECK_HIP(hipMemcpyAsync(bad, ctl, sizeof(int32_t), hipMemcpyDeviceToHost, s));
+  if (parts & kCullBoxes) {
+    int32_t* mid_list = ws.k1.as<int32_t>();
+    // nodes over 1,024 leaves: few in a balanced tree, up to ninner - 1,023 in a
+    // chain, each with 12 running extents
+    const size_t nlarge = (size_t)std::max<int64_t>((int64_t)ninner - kLargeNode + 1, 1);
+    AXSQ_TRY(ws.redo.ensure(sizeof(int32_t) * nlarge));
+    AXSQ_TRY(ws.misc.ensure(sizeof(uint32_t) * 12 * nlarge));
+    int32_t* large_list = ws.redo.as<int32_t>();
+    uint32_t* acc = ws.misc.as<uint32_t>();
+    k_cull_nodes<CELLS><<<grid_for(ninner), kBlock, 0, s>>>(cs, b->nodes, ninner, tris, tau, pre,
+                                                            totals, out, mid_list, large_list,
+                                                            acc, ctl);
+    AXSQ_CHECK_HIP(hipGetLastError());
+    if (n > kSmallNode) {
+      const unsigned g = (unsigned)std::min<int64_t>((n / 6 + 3) / 4 + 1, 8192);
+      k_cull_mid<CELLS><<<g, kBlock, 0, s>>>(cs, b->nodes, tris, tau, mid_list, ctl, out);
+      AXSQ_CHECK_HIP(hipGetLastError());
+    }
+    if (n > kLargeNode) {
+      k_cull_large<CELLS><<<(unsigned)((n + kLargeNode - 1) / kLargeNode), kBlock, 0, s>>>(
+          cs, b->nodes, ninner, tris, tau, out, acc, ctl);
+      AXSQ_CHECK_HIP(hipGetLastError());
+      k_cull_large_end<<<(unsigned)std::min<int64_t>(n / kLargeNode / kBlock + 1, 256), kBlock, 0,
+                         s>>>(b->nodes, large_list, ctl, acc, out);
+      AXSQ_CHECK_HIP(hipGetLastError());
+    }
+  }
+  int32_t h[kCullCtl];
+  AXSQ_CHECK_HIP(hipMemcpyAsync(h, ctl, sizeof(h), hipMemcpyDeviceToHost, s));
   AXSQ_CHECK_HIP(hipStreamSynchronize(s));
+  res->bad = h[0] != 0;
+  // Of a curved, tilted or gently uneven surface nearly every node of some size is
+  // less than half as thick as its box. Of a flat one along the axes, or of a
+  // rough one whose parts are as thick as their boxes at any size, none is. In
+  // between lie strong noise on a curved ground, whose larger nodes are thinner by
+  // half, and large flat facets along the axes, where only those over an edge are;
+  // the small nodes tell these apart. Nodes over 2x at 64, 512, 4,096 leaves / over
+  // 1.5x at 4,096, 32,768 / over 1.5x at 64, per cent:
+  //   spheres, tori, hills, tilted planes   100 90-100 57-100
+  //   noise of 1/20 on a sphere              4  0 44 /  88 100 / 30
+  //   noise of 12 cells on hills             0  0  0 /  26  82 / 26
+  //   height fields with noise               0  0  0 /   0 0-6 / 11-20
+  //   cubes, 196,608 and 786,432             0  0  4 / 46-63 100 / 7-12
+  // Triangles at random (0 0 0 / 0 0 / 16) are another matter: they fill space, and
+  // most queries are near one.
+  const int third = kClassSamples / 3;
+  const bool thin = std::max({h[5], h[6], h[7]}) > third;
+  const bool uneven = std::max(h[8], h[9]) > third && 5 * h[11] > kClassSamples;
+  const bool joined = 2 * h[12] > kClassSamples;
+  res->plain = joined && !thin && !uneven;
+  res->crowd = !joined && !thin;
+  res->loose = 2 * h[3] > kClassSamples && h[7] <= third;
   return AXSQ_OK;
 }
 
 }  // namespace
 
 int cull_build(const axsq_bvh* b, const TriRec* tris, bool cells, const CullSpace& cs, double diag,
-               CullNode* out, NormRec* norms, int32_t* bad, hipStream_t s) {
+               int parts, CullNode* out, NormRec* norms, CullResult* res, hipStream_t s) {
   Workspace& ws = workspace();
-  return cells ? build<true>(b, tris, cs, diag, out, norms, ws, bad, s)
-               : build<false>(b, tris, cs, diag, out, norms, ws, bad, s);
+  return cells ? build<true>(b, tris, cs, diag, parts, out, norms, res, ws, s)
+               : build<false>(b, tris, cs, diag, parts, out, norms, res, ws, s);
 }
 
 }  // namespace axsq

@@ -268,6 +268,8 @@ struct axsq_sdf {
   axsq::CullNode* cull = nullptr;
   axsq::NormRec* cull_norms = nullptr;  // with cull: one per triangle record
   int cull_state = 0;
+  // CullResult's, once asked
+  bool cull_classed = false, cull_plain = false, cull_loose = false, cull_crowd = false;
   std::atomic<bool> evaluated{false};  // since the vertices were set
   std::mutex cull_mu;       // held while a call builds them
   bool walk_fixed = false;  // created with a setting of the reference walk: no culled walk
@@ -281,11 +283,21 @@ int bvh_build_into(axsq_bvh* b, const double* boxes, int64_t n, double scale, in
                    hipStream_t s, int dims = 3, bool f32 = false,
                    const float* boxes_f32 = nullptr);
 void bvh_release(axsq_bvh* b);
-// Builds the oriented child boxes of a tree over `tris` (cs: its mesh
-// coordinates, diag: the mesh's diagonal) into out, n - 1 records; *bad is set
-// when they must not be used. Returns after the stream has run them.
+// The oriented child boxes of a tree over `tris` (cs: its mesh coordinates,
+// diag: the mesh's diagonal), in parts that a call may take one after the other
+// on the same workspace: the leaves' tolerances and normals (norms: their table,
+// or NULL), what oriented boxes gain on this mesh, and the boxes (out, n - 1
+// records). Returns after the stream has run them.
+constexpr int kCullLeaves = 1, kCullClass = 2, kCullBoxes = 4;
+struct CullResult {
+  bool bad;    // the boxes must not be used
+  bool plain;  // with kCullClass: on this surface they are hardly thinner than
+               // axis-aligned ones
+  bool crowd;  // and: nor among triangles that do not meet
+  bool loose;  // and: at the leaves they are no thinner, and the tolerances as large
+};
 int cull_build(const axsq_bvh* b, const TriRec* tris, bool cells, const CullSpace& cs, double diag,
-               CullNode* out, NormRec* norms, int32_t* bad, hipStream_t s);
+               int parts, CullNode* out, NormRec* norms, CullResult* res, hipStream_t s);
 // n 2-D boxes (4 doubles) -> 3-D boxes with z range [0, 0] (6 doubles)
 int widen_boxes2d(const double* boxes2d, int64_t n, double* out, hipStream_t s);
 // Candidate search launches (axsq_query.hip). mode 0: count pass (keeping the

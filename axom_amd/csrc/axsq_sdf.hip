@@ -2750,37 +2750,84 @@ static int sdf_eval_reference(const axsq_sdf* h, SdfArgs a, bool list, const uin
 //    beside the first pass and report them (axsq_sdf_last_early), which the
 //    culled walk has no use for. Speed alone would take them too (50,000
 //    queries on 1.3M triangles: 38 ms, culled 2.0 ms with the boxes), and a
-//    second call on the same vertices does.
+//    second call on the same vertices does;
+//  - and the meshes on which they gain too little (cull_pays).
 static bool cull_wanted(const axsq_sdf* h, double diag, int64_t nq, bool first) {
   if (h->walk_fixed || !(diag >= 0.01 && diag <= 1e15)) return false;
   return h->early_walks == 0 || !first || nq <= 32768 || 24 * nq >= h->ntris;
 }
 
+// Batches and trees up to which the culled walk is taken whatever its boxes gain
+// (cull_pays), and trees that are not asked at all.
+constexpr int64_t kPlainQueries = 65536, kPlainLeaves = 131072, kLooseQueries = 524288;
+constexpr int64_t kClassLeaves = 8192, kClassQueries = 32768;
+
+// Whether the oriented boxes gain enough for a call of nq queries.
+//  - plain: hardly a node is thinner than its axis-aligned box. A visit here
+//    costs as much as the reference walk's, and float extents and margins
+//    separate less. Milliseconds a call, reference / culled, on flat and noisy
+//    height fields of 1.28M triangles: 64,000 queries 0.2 to 0.9 / 0.3 to 1.0, 1M
+//    0.58 / 1.00 and 2.4 / 8.3, 4M 1.6 / 3.0 and 8.1 / 19; a cube of 786,432
+//    1M 1.0 / 1.4. On smaller trees (80,000) the culled walk is the faster one
+//    with a higher hand-on limit (c.steps).
+//  - loose: slender triangles along an axis whose closest points are known to no
+//    better than their height. A cylinder of 100,000: 300,000 queries 12.5 / 8.6,
+//    1M 18 / 25, 4M 41 / 104 (tilted 192 / 11, 627 / 32, 2500 / 133).
+static bool cull_pays(const axsq_sdf* h, int64_t nq) {
+  if (h->cull_plain && h->bvh->n > kPlainLeaves && nq > kPlainQueries) return false;
+  return !(h->cull_loose && nq > kLooseQueries);
+}
+
 // The tree's oriented boxes, built by the first call that wants them after
 // the mesh was set or moved; *out stays NULL where they do not hold (a
-// triangle without a useful tolerance, no memory).
-static int sdf_cull_nodes(axsq_sdf* h, const CullSpace& cs, double diag, hipStream_t s,
+// triangle without a useful tolerance, no memory) or gain too little.
+static int sdf_cull_nodes(axsq_sdf* h, const CullSpace& cs, double diag, int64_t nq, hipStream_t s,
                           const CullNode** out) {
   std::lock_guard<std::mutex> lock(h->cull_mu);
-  if (h->cull_state == 0) {
-    const size_t n = (size_t)(h->bvh->n - 1);
-    const size_t nrec = (n + 1) * (h->cells ? 2 : 1);
-    if (!h->cull && (hipMalloc((void**)&h->cull, sizeof(CullNode) * n) != hipSuccess ||
-                     hipMalloc((void**)&h->cull_norms, sizeof(NormRec) * nrec) != hipSuccess)) {
-      (void)hipGetLastError();
-      (void)hipFree(h->cull);
-      h->cull = nullptr;
-      h->cull_norms = nullptr;
-      h->cull_state = -1;
-    } else {
-      int32_t bad = 0;
-      ProfRange pr("sdf_cull_build", s);
-      AXSQ_TRY(cull_build(h->bvh, h->tris, h->cells, cs, diag, h->cull, h->cull_norms, &bad,
-                          s));
-      h->cull_state = bad ? -1 : 1;
+  const size_t n = (size_t)(h->bvh->n - 1);
+  const size_t nrec = (n + 1) * (h->cells ? 2 : 1);
+  if (h->cull_state == 0 && !h->cull &&
+      (hipMalloc((void**)&h->cull, sizeof(CullNode) * n) != hipSuccess ||
+       hipMalloc((void**)&h->cull_norms, sizeof(NormRec) * nrec) != hipSuccess)) {
+    (void)hipGetLastError();
+    (void)hipFree(h->cull);
+    h->cull = nullptr;
+    h->cull_norms = nullptr;
+    h->cull_state = -1;
+  }
+  if (h->cull_state < 0) return AXSQ_OK;
+  const bool ask = !h->cull_classed && (int64_t)n + 1 > kClassLeaves && nq > kClassQueries;
+  int parts = h->cull_state == 0 ? kCullLeaves | kCullBoxes : 0;
+  if (ask || parts) {
+    ProfRange pr("sdf_cull_build", s);
+    NormRec* const norms = parts ? h->cull_norms : nullptr;
+    CullResult res{};
+    auto build = [&](int p) -> int {
+      AXSQ_TRY(cull_build(h->bvh, h->tris, h->cells, cs, diag, p, h->cull, norms, &res, s));
+      if (res.bad) h->cull_state = -1;
+      if (p & kCullClass) {
+        h->cull_classed = true;
+        h->cull_plain = res.plain;
+        h->cull_loose = res.loose;
+        h->cull_crowd = res.crowd;
+      }
+      return AXSQ_OK;
+    };
+    // first what they gain, where that may make them unnecessary
+    const bool may_not = nq > kLooseQueries ||
+                         ((int64_t)n + 1 > kPlainLeaves && nq > kPlainQueries);
+    if (ask && (may_not || !parts)) {
+      AXSQ_TRY(build(kCullLeaves | kCullClass));
+      parts &= ~kCullLeaves;
+    } else if (ask) {
+      parts |= kCullClass;
+    }
+    if (h->cull_state == 0 && cull_pays(h, nq)) {
+      AXSQ_TRY(build(parts));
+      if (h->cull_state == 0) h->cull_state = 1;
     }
   }
-  if (h->cull_state == 1) *out = h->cull;
+  if (h->cull_state == 1 && cull_pays(h, nq)) *out = h->cull;
   return AXSQ_OK;
 }
 
@@ -2828,7 +2875,7 @@ int sdf_eval_launch(const axsq_sdf* h, const double* x, const double* y, const d
     int e2 = 0;
     (void)std::frexp(diag, &e2);  // diag in [2^(e2 - 1), 2^e2)
     cs.scale = std::ldexp(1.0, 1 - e2);
-    AXSQ_TRY(sdf_cull_nodes(hm, cs, diag, s, &cull));
+    AXSQ_TRY(sdf_cull_nodes(hm, cs, diag, nq, s, &cull));
   }
   // a wave per query (below) needs no order: 5,000 queries 103 us sorted, 75 not
   if (h->sort_queries && nq > (cull ? kCoopQueries : 4096)) {
@@ -2846,7 +2893,10 @@ int sdf_eval_launch(const axsq_sdf* h, const double* x, const double* y, const d
     // axis, and no more: each 8 are a pass. 16 bits for up to 262,144 queries (50
     // a cell), 21 above (80 for 4M). The whole call with 16 / 21 / 30 bits: 60,000
     // near a surface 270 / 280 / 301 us, 1M 820 / 825 / 854, 4M 5885 / 5670 / 5688.
-    const int bits = nq <= 262144 ? 16 : 21;
+    // The reference walk alone, whose waves are as fast as their lanes are close,
+    // takes all 30 (4M over a flat surface of 1.28M triangles: 21 / 30 bits 1650 /
+    // 1560).
+    const int bits = !cull ? 30 : nq <= 262144 ? 16 : 21;
     ProfRange pq("sdf_query_order", s);
     k_query_codes<<<grid_for(nq), kBlock, 0, s>>>(x, y, z, stride, nq, h->domain[0],
                                                   h->domain[1], h->domain[2], inv[0], inv[1],
@@ -2905,6 +2955,15 @@ int sdf_eval_launch(const axsq_sdf* h, const double* x, const double* y, const d
                   : nq <= 3145728 ? 4
                                   : 5;
   c.steps = kSteps[row][size];
+  // Where boxes gain little, lanes stay together longer and few walks are worth a
+  // wave. Noisy height fields of 20,000 and 80,000: 130,000 queries with 128 / 256 /
+  // 384 616 / 369 / 478 us (the reference walk 546), 100,000 192 / 256 / 384 582 /
+  // 466 / 478 (554), 300,000 192 / 512 860 / 657 (742), 1M 256 / 512 2027 / 1279
+  // (1483). 20,000 large triangles at random, 1M 256 / 1024 8.6 / 6.0 ms (9.2), 4M
+  // 512 / without limit 28.8 / 12.6 (27.1).
+  if (nq > kClassQueries && h->cull_plain && b->n <= kPlainLeaves)
+    c.steps = std::max<int32_t>(c.steps, nq <= 131072 ? 256 : 512);
+  if (nq > 786432 && h->cull_crowd) c.steps = 4096;
   ProfRange p1(mixed ? "sdf_eval_fp32_cull" : "sdf_eval_fp64_cull", s);
   // one lane per query, then one wave per long walk; a small batch one wave
   // per query at once
