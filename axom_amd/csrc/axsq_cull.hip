@@ -656,6 +656,7 @@ int build(const axsq_bvh* b, const TriRec* tris, const CullSpace& cs, double dia
   //   noise of 12 cells on hills             0  0  0 /  26  82 / 26
   //   height fields with noise               0  0  0 /   0 0-6 / 11-20
   //   cubes, 196,608 and 786,432             0  0  4 / 46-63 100 / 7-12
+  //   flat along the axes                    0  0  0 /   0   0 / 0
   // Triangles at random (0 0 0 / 0 0 / 16) are another matter: they fill space, and
   // most queries are near one.
   const int third = kClassSamples / 3;
@@ -663,6 +664,7 @@ int build(const axsq_bvh* b, const TriRec* tris, const CullSpace& cs, double dia
   const bool uneven = std::max(h[8], h[9]) > third && 5 * h[11] > kClassSamples;
   const bool joined = 2 * h[12] > kClassSamples;
   res->plain = joined && !thin && !uneven;
+  res->flat = res->plain && 50 * h[11] < kClassSamples;
   res->crowd = !joined && !thin;
   res->loose = 2 * h[3] > kClassSamples && h[7] <= third;
   return AXSQ_OK;

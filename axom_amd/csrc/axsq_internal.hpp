@@ -269,7 +269,8 @@ struct axsq_sdf {
   axsq::NormRec* cull_norms = nullptr;  // with cull: one per triangle record
   int cull_state = 0;
   // CullResult's, once asked
-  bool cull_classed = false, cull_plain = false, cull_loose = false, cull_crowd = false;
+  bool cull_classed = false, cull_plain = false, cull_flat = false, cull_loose = false,
+       cull_crowd = false;
   std::atomic<bool> evaluated{false};  // since the vertices were set
   std::mutex cull_mu;       // held while a call builds them
   bool walk_fixed = false;  // created with a setting of the reference walk: no culled walk
@@ -293,8 +294,9 @@ struct CullResult {
   bool bad;    // the boxes must not be used
   bool plain;  // with kCullClass: on this surface they are hardly thinner than
                // axis-aligned ones
-  bool crowd;  // and: nor among triangles that do not meet
-  bool loose;  // and: at the leaves they are no thinner, and the tolerances as large
+  bool flat;   // and not at all
+  bool crowd;  // hardly thinner, and the triangles do not meet
+  bool loose;  // at the leaves no thinner, and the tolerances as large
 };
 int cull_build(const axsq_bvh* b, const TriRec* tris, bool cells, const CullSpace& cs, double diag,
                int parts, CullNode* out, NormRec* norms, CullResult* res, hipStream_t s);

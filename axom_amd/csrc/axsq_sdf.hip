@@ -2759,22 +2759,28 @@ static bool cull_wanted(const axsq_sdf* h, double diag, int64_t nq, bool first) 
 
 // Batches and trees up to which the culled walk is taken whatever its boxes gain
 // (cull_pays), and trees that are not asked at all.
-constexpr int64_t kPlainQueries = 65536, kPlainLeaves = 131072, kLooseQueries = 524288;
-constexpr int64_t kClassLeaves = 8192, kClassQueries = 32768;
+constexpr int64_t kFlatQueries = kCoopQueries, kPlainQueries = 65536, kLooseQueries = 131072;
+constexpr int64_t kPlainLeaves = 131072, kClassLeaves = 8192, kClassQueries = 32768;
 
 // Whether the oriented boxes gain enough for a call of nq queries.
 //  - plain: hardly a node is thinner than its axis-aligned box. A visit here
 //    costs as much as the reference walk's, and float extents and margins
-//    separate less. Milliseconds a call, reference / culled, on flat and noisy
-//    height fields of 1.28M triangles: 64,000 queries 0.2 to 0.9 / 0.3 to 1.0, 1M
-//    0.58 / 1.00 and 2.4 / 8.3, 4M 1.6 / 3.0 and 8.1 / 19; a cube of 786,432
-//    1M 1.0 / 1.4. On smaller trees (80,000) the culled walk is the faster one
-//    with a higher hand-on limit (c.steps).
+//    separate less, the more so the farther the queries. Milliseconds a call,
+//    reference / culled, queries all around height fields of 1.28M triangles: flat
+//    100,000 0.22 / 0.31, 1M 0.58 / 1.00; noisy 64,000 0.79 to 0.93 / 0.58 to
+//    1.00, 100,000 0.72 to 0.92 / 0.65 to 1.33, 1M 1.8 to 2.4 / 2.5 to 8.3. Near
+//    the surface (1 part in 200 of the mesh) 1M about 320,000 2.4 / 1.6, but on the
+//    tallest noise 2.4 / 2.6; 2.5 diagonals away 1.7 to 2.0 / 2.3 to 3.1, flat 30,000
+//    0.20 / 0.41. On smaller trees (80,000) the culled walk is the faster one with
+//    a higher hand-on limit (c.steps).
 //  - loose: slender triangles along an axis whose closest points are known to no
-//    better than their height. A cylinder of 100,000: 300,000 queries 12.5 / 8.6,
-//    1M 18 / 25, 4M 41 / 104 (tilted 192 / 11, 627 / 32, 2500 / 133).
+//    better than their height. A cylinder of 100,000: 100,000 queries 8 to 12 / 4,
+//    300,000 all around 10 to 13 / 9, near 1.1 / 2.6, far 9.6 / 13.6; 1M 18 / 25,
+//    4M 41 / 104 (tilted 192 / 11, 627 / 32, 2500 / 133).
 static bool cull_pays(const axsq_sdf* h, int64_t nq) {
-  if (h->cull_plain && h->bvh->n > kPlainLeaves && nq > kPlainQueries) return false;
+  if (h->cull_plain && h->bvh->n > kPlainLeaves &&
+      nq > (h->cull_flat ? kFlatQueries : kPlainQueries))
+    return false;
   return !(h->cull_loose && nq > kLooseQueries);
 }
 
@@ -2796,7 +2802,9 @@ static int sdf_cull_nodes(axsq_sdf* h, const CullSpace& cs, double diag, int64_t
     h->cull_state = -1;
   }
   if (h->cull_state < 0) return AXSQ_OK;
-  const bool ask = !h->cull_classed && (int64_t)n + 1 > kClassLeaves && nq > kClassQueries;
+  const int64_t leaves = (int64_t)n + 1;
+  const bool ask = !h->cull_classed && leaves > kClassLeaves &&
+                   nq > (leaves > kPlainLeaves ? kFlatQueries : kClassQueries);
   int parts = h->cull_state == 0 ? kCullLeaves | kCullBoxes : 0;
   if (ask || parts) {
     ProfRange pr("sdf_cull_build", s);
@@ -2808,14 +2816,14 @@ static int sdf_cull_nodes(axsq_sdf* h, const CullSpace& cs, double diag, int64_t
       if (p & kCullClass) {
         h->cull_classed = true;
         h->cull_plain = res.plain;
+        h->cull_flat = res.flat;
         h->cull_loose = res.loose;
         h->cull_crowd = res.crowd;
       }
       return AXSQ_OK;
     };
     // first what they gain, where that may make them unnecessary
-    const bool may_not = nq > kLooseQueries ||
-                         ((int64_t)n + 1 > kPlainLeaves && nq > kPlainQueries);
+    const bool may_not = nq > kLooseQueries || (leaves > kPlainLeaves && nq > kFlatQueries);
     if (ask && (may_not || !parts)) {
       AXSQ_TRY(build(kCullLeaves | kCullClass));
       parts &= ~kCullLeaves;
