@@ -192,7 +192,7 @@ struct axsq_bvh {
                                     // the FP64 node's 128-B line
   axsq::FindNode* fnodes = nullptr; // n-1 compact nodes of the point and box searches
   bool searched = true;             // built with them (not the tree inside an axsq_sdf)
-  bool find_ok = false;             // and they hold: finite boxes within find_space's range
+  bool find_ok = false;             // and they hold: finite boxes in find_space's range, large enough in it
   double* leaf_boxes = nullptr;     // n scaled leaf boxes in leaf order (AoS)
   int32_t* leaf_ids = nullptr;      // n: leaf position -> original id
   uint32_t* mcodes = nullptr;       // n sorted Morton codes

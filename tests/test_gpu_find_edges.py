@@ -228,3 +228,45 @@ def test_vertex_ids_out_of_range_cost_no_pairs(ntris, some):
     with pytest.raises(L.AxsqError, match="outside"):
         quest.findTriMeshIntersectionsBVH(_t(v), _t(t))
     assert time.perf_counter() - a < 5.0
+
+
+def _cells(n, nd):
+    """n^nd cells of the unit cube in order, a little apart."""
+    c = np.stack(np.meshgrid(*[np.arange(n)] * nd, indexing="ij"), -1).reshape(-1, nd)
+    return np.concatenate([c + 0.1, c + 0.9], 1) / n
+
+
+@pytest.mark.parametrize("nd,dtype", [(3, np.float64), (2, np.float64), (3, np.float32)])
+@pytest.mark.parametrize("far", [1e4, 1e9, 1e11, 1e12, 1e15, 1e30])
+def test_small_boxes_in_large_bounds(far, nd, dtype):
+    """A box of 10^4 to 10^30 times the others' extent among them."""
+    rng = np.random.default_rng(nd)
+    boxes = np.concatenate([_cells(11, nd), [[-far] * nd + [far] * nd]]).astype(dtype)
+    p = rng.uniform(-0.1, 1.1, (500, nd))
+    p[::50] *= far
+    h = rng.uniform(0.0, 0.1, (500, 1))
+    d = rng.normal(size=(100, nd))
+    _check(boxes, 1.000123, dtype,
+           {"points": p.astype(dtype), "boxes": np.concatenate([p - h, p + h], 1).astype(dtype),
+            "rays": np.concatenate([p[:100], d], 1).astype(dtype)})
+
+
+def test_small_boxes_in_large_bounds_are_told_apart():
+    """100,000 points among 64,000 cells and a box for everything: 52 ms where each
+    point visited every node, 0.2 with the nodes that tell the cells apart."""
+    cells = _cells(40, 3)
+    p = _t(np.random.default_rng(1).random((100_000, 3)))
+
+    def best(boxes):
+        g, t = spin.BVH(_t(boxes)), []
+        for _ in range(4):
+            a, b = (torch.cuda.Event(enable_timing=True) for _ in range(2))
+            a.record()
+            _search(g, p)
+            b.record()
+            torch.cuda.synchronize()
+            t.append(a.elapsed_time(b))
+        return min(t)
+
+    alone = best(cells)
+    assert best(np.concatenate([cells, [[-1e15] * 3 + [1e15] * 3]])) < 2.0 + 20.0 * alone
