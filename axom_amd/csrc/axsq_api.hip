@@ -1155,7 +1155,7 @@ int axsq_sdf_update_vertices(axsq_sdf* h, const double* x, const double* y, cons
   hipStream_t s = (hipStream_t)stream;
   const size_t nb = sizeof(double) * h->nverts;
   h->cull_state = 0;
-  h->cull_classed = h->cull_plain = h->cull_flat = h->cull_loose = h->cull_crowd = false;
+  h->cull_classed = false;
   h->evaluated = false;
   AXSQ_CHECK_HIP(hipMemcpyAsync(h->vx, x, nb, hipMemcpyDefault, s));
   AXSQ_CHECK_HIP(hipMemcpyAsync(h->vy, y, nb, hipMemcpyDefault, s));

@@ -268,9 +268,9 @@ struct axsq_sdf {
   axsq::CullNode* cull = nullptr;
   axsq::NormRec* cull_norms = nullptr;  // with cull: one per triangle record
   int cull_state = 0;
-  // CullResult's, once asked
-  bool cull_classed = false, cull_plain = false, cull_flat = false, cull_loose = false,
-       cull_crowd = false;
+  // CullResult's, asked for the current vertices (classed) or earlier ones (known)
+  bool cull_classed = false, cull_known = false;
+  bool cull_plain = false, cull_flat = false, cull_loose = false, cull_crowd = false;
   std::atomic<bool> evaluated{false};  // since the vertices were set
   std::mutex cull_mu;       // held while a call builds them
   bool walk_fixed = false;  // created with a setting of the reference walk: no culled walk

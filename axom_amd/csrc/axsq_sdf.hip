@@ -2814,7 +2814,7 @@ static int sdf_cull_nodes(axsq_sdf* h, const CullSpace& cs, double diag, int64_t
       AXSQ_TRY(cull_build(h->bvh, h->tris, h->cells, cs, diag, p, h->cull, norms, &res, s));
       if (res.bad) h->cull_state = -1;
       if (p & kCullClass) {
-        h->cull_classed = true;
+        h->cull_classed = h->cull_known = true;
         h->cull_plain = res.plain;
         h->cull_flat = res.flat;
         h->cull_loose = res.loose;
@@ -2822,8 +2822,10 @@ static int sdf_cull_nodes(axsq_sdf* h, const CullSpace& cs, double diag, int64_t
       }
       return AXSQ_OK;
     };
-    // first what they gain, where that may make them unnecessary
-    const bool may_not = nq > kLooseQueries || (leaves > kPlainLeaves && nq > kFlatQueries);
+    // first what they gain, where that may make them unnecessary and did not fail
+    // to before the vertices moved
+    const bool may_not = (nq > kLooseQueries || (leaves > kPlainLeaves && nq > kFlatQueries)) &&
+                         !(h->cull_known && cull_pays(h, nq));
     if (ask && (may_not || !parts)) {
       AXSQ_TRY(build(kCullLeaves | kCullClass));
       parts &= ~kCullLeaves;

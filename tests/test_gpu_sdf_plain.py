@@ -97,6 +97,21 @@ def test_flat_quad_cells(monkeypatch, size):
         assert np.array_equal(g[k], r[k]), k
 
 
+def test_a_curved_surface_that_becomes_flat(monkeypatch):
+    """What the boxes gained before the vertices moved does not decide afterwards."""
+    flat, t = _mesh("flat")
+    hill = flat + np.array([0.0, 0.0, 0.3]) * np.sin(3.0 * flat[:, [0]]) * np.cos(2.0 * flat[:, [1]])
+    q = np.random.default_rng(4).uniform(-1.5, 1.5, (70_000, 3))
+    a, b = _handles(monkeypatch, hill, t)
+    for v in (hill, flat, flat, hill):
+        a.updateVertices(_t(v))
+        b.updateVertices(_t(v))
+        for n in (70_000, 17_000):
+            g, r = _eval(a, q[:n]), _eval(b, q[:n])
+            for k in ("dist", "cp", "elem", "normal"):
+                assert np.array_equal(g[k], r[k]), (n, k)
+
+
 def _best(sdf, q):
     t = []
     for _ in range(6):
