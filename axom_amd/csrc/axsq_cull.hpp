@@ -9,10 +9,12 @@
 // normal, split direction, their cross product). A subtree whose oriented
 // box is farther than the running minimum holds no triangle the walk could
 // use, and leaving it out leaves 13 triangles and 75 nodes, and 18 and 118.
-// Forward and adjoint of 4M queries on the 81,920-triangle sphere: 33.2 ms
-// with the reference walk alone, 4.7 ms; a shape-fit iteration on 1.3M
-// triangles, 8M queries: 227 and 17.7 ms; 1,000 queries on 5,120 triangles:
-// 1.6 and 0.07 ms.
+// Forward and adjoint of 4M queries on the 81,920-triangle sphere: 33.0 ms
+// with the reference walk alone, 4.2 ms; a shape-fit iteration on 1.3M
+// triangles, 8M queries: 226 and 15.0 ms; 1,000 queries on 5,120 triangles:
+// 1.28 and 0.046 ms. Surfaces whose patches are as thick as their boxes gain
+// nothing: the build tells them (k_cull_class), and large batches on them take
+// the reference walk.
 //
 // Why the result is the reference walk's, bit for bit. Let s be the running
 // minimum (squared) and p the closest point when the reference checks leaf Y.

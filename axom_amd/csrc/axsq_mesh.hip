@@ -5,11 +5,12 @@
 // boxes and degenerate flags, a BVH over the boxes, runs findBoundingBoxes
 // for every box (count, scan, fill of all candidates), keeps the pairs i < j
 // and tests them. Here the triangle test is the traversal's leaf action
-// (the custom leaf action of quest/examples/quest_bvh_two_pass.cpp:144-232):
-// triangle i's box walks the tree and each reached triangle j > i is tested on
-// the spot, keeping kPairSlots hits of i. A scan of the hit counts places every
-// triangle's pairs; triangles with more hits walk again to write them all. The
-// candidate lists are never stored. The output
+// (the custom leaf action of quest/examples/quest_bvh_two_pass.cpp:144-232): a wave
+// walks for the triangles at neighbouring leaves, meets each pair once, from its
+// lower leaf, and tests it on the spot, keeping kPairSlots hits of the smaller
+// index. A scan of the hit counts places every triangle's pairs; triangles with
+// more hits walk again to write them all. The candidate lists are never stored
+// (the walk's own list, of leaves and triangles, is in LDS). The output
 // order is the sequential path's: pairs grouped by the first triangle, the
 // second in the first's BVH traversal order; degenerate indices ascending.
 #include <hip/hip_runtime.h>
@@ -494,8 +495,10 @@ int self_intersections(const double* x, const double* y, const double* z, int64_
   } else {
     const int64_t n = ntris;
     Workspace& ws = workspace();
-    // records of the vertices where the three arrays outgrow an XCD's L2 (4 MB)
-    const bool pack = nverts >= 131072;
+    // records of the vertices where the three arrays outgrow the L2s: crossing noisy
+    // spheres of 163,842 / 327,684 / 655,362 / 1,310,724 vertices, a call with them 517 /
+    // 728 / 1130 / 2016 us, without 508 / 717 / 1158 / 2076
+    const bool pack = nverts >= 524288;
     AXSQ_TRY(ws.mesh_tri.ensure(sizeof(TriRec) * n + (pack ? 32 * (size_t)nverts : 0)));
     AXSQ_TRY(ws.mesh_box.ensure(sizeof(double) * 6 * n));
     AXSQ_TRY(ws.mesh_int.ensure(sizeof(int32_t) * (5 * n + 2) + 2 * sizeof(int64_t) + 64));

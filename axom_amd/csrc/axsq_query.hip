@@ -8,15 +8,14 @@
 // the count gets an error and no write past its buffer). In the one-call
 // search the count pass also keeps each query's first kstash candidate ids and
 // lists the queries that have more, so the fill copies the kept ids and
-// searches again only for the listed queries. The walk runs on the vote
-// schedule (a lane's order of node visits and leaf actions is the one-lane
-// walk's, so the candidate order is too): 11% faster for boxes and 34% for
-// rays than the loop-by-loop schedule on 100,000 boxes, the same for points.
+// searches again only for the listed queries.
 //
 // Points and boxes walk the compact nodes of axsq_find.hpp in either traversal
-// form (k_find_compact), unless the tree's coordinates are out of their range or
-// visits are counted (k_find, on the FP64 nodes); rays do too, a wave for several
-// rays (k_ray_count) or for one (k_ray_fill). Lists and order are the same in all.
+// form (k_find_compact), rays too, a wave for several rays (k_ray_count) or for
+// one (k_ray_fill). Trees whose coordinates are out of those nodes' range or below
+// their resolution, and searches whose visits are counted, walk the FP64 nodes, a
+// lane per query on the vote schedule (k_find). A query's nodes are met left
+// before right in all of them, so lists and order are the same.
 #include "axsq_internal.hpp"
 #include "axsq_traverse.hpp"
 

@@ -490,9 +490,9 @@ __global__ __launch_bounds__(kSdfBlock) AXSQ_SDF_WAVES_ATTR void k_sdf_eval(SdfA
 // list or stack is full. A walk still going when its wave has taken
 // CullArgs::steps node steps (queries with much of the surface at nearly one
 // distance) is handed to k_sdf_coop.
-// 4M queries on 81,920 triangles: 3.7 ms, 75 visits and 13 checks a query in
-// 175 and 33 steps a wave. The vector L1's return path is busy 90% of that
-// time and the VALUs 80%. Before: 7.4 ms with 128-byte records, a stack whose
+// 4M queries on 81,920 triangles: 3.65 ms, 75 visits and 13 checks a query in
+// 175 and 33 steps a wave. The vector L1's return path is busy 84% of that
+// time and the VALUs 73%, with 32% of their lanes. Before: 7.4 ms with 128-byte records, a stack whose
 // entries past the 24th were private (so was its address) and the state
 // copied at each step.
 #ifndef AXSQ_CULL_LDS
@@ -2288,8 +2288,10 @@ __global__ __launch_bounds__(kBlock) void k_bwd_query(
 // a few gathers, one reached by few shares one with its neighbours.
 // 4M queries on 81,920, 8M on 1.3M and 1M on 327,680 triangles (49, 6 and 3 a
 // triangle): 112 / 417 / 74 us with one triangle a wave, 180 / 222 / 32 with
-// seven, 150 / 461 / 53 with 16 lanes a triangle that load for themselves. So
-// seven below 16 queries a triangle, one above.
+// seven, 150 / 461 / 53 with 16 lanes a triangle that load for themselves. The
+// whole adjoint with seven / one, at 8, 12, 16, 24 queries a triangle: 20,480
+// triangles 94/93 100/99 123/119 138/132 us, 81,920 162/168 187/190 211/220
+// 273/261, 327,680 349/397 457/501 596/629. So seven below 16, one from there.
 constexpr int kBwdWave = 64;
 template <int TRIS>
 __global__ __launch_bounds__(kBwdWave) void k_bwd_tri(int64_t nt,

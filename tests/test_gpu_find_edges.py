@@ -270,3 +270,21 @@ def test_small_boxes_in_large_bounds_are_told_apart():
 
     alone = best(cells)
     assert best(np.concatenate([cells, [[-1e15] * 3 + [1e15] * 3]])) < 2.0 + 20.0 * alone
+
+
+@pytest.mark.parametrize("nverts", [524_287, 524_288, 524_289])
+def test_self_intersections_either_side_of_the_vertex_records(nverts):
+    """From 524,288 vertices on the triangles are read through packed records."""
+    rng = np.random.default_rng(nverts)
+    n = 3000
+    v = rng.random((nverts, 3))
+    ids = rng.choice(nverts - 1, size=3 * n, replace=False).astype(np.int32)
+    ids[-1] = nverts - 1
+    t = ids.reshape(n, 3)
+    v[t[:, 1:]] = v[t[:, :1]] + rng.normal(0.0, 0.03, (n, 2, 3))
+    t[7, 1] = t[7, 0]  # no area
+    pairs, degen = quest.findTriMeshIntersectionsBVH(_t(v), _t(t))
+    opairs, odegen = orc.mesh_self_intersections(v, t, nthreads=8)
+    assert opairs.shape[0] > 50 and odegen.tolist() == [7]
+    assert np.array_equal(pairs.cpu().numpy(), opairs)
+    assert np.array_equal(degen.cpu().numpy(), odegen)
