@@ -1669,8 +1669,8 @@ __global__ __launch_bounds__(kWaveLanes) AXSQ_RESUME_WAVES_ATTR void k_sdf_resum
         after_visit();
         if (err) break;
       } else if (phase == kLeaf) {
-        const int32_t k = -found - 1 - clo;
-        if ((uint32_t)k > (uint32_t)(chi - clo) || ((m_eff >> k) & 1u)) break;
+        const int32_t k = -found - 1 - clo;  // (before the first fill the memo is empty)
+        if ((uint32_t)k >= (uint32_t)(chi - clo + 1) || ((m_eff >> k) & 1u)) break;
         ++leaves;  // a leaf that changes nothing
         after_leaf();
         if (err) break;
