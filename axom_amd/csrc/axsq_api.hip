@@ -1156,6 +1156,7 @@ int axsq_sdf_update_vertices(axsq_sdf* h, const double* x, const double* y, cons
   const size_t nb = sizeof(double) * h->nverts;
   h->cull_state = 0;
   h->cull_classed = false;
+  ++h->cull_moves;
   h->evaluated = false;
   AXSQ_CHECK_HIP(hipMemcpyAsync(h->vx, x, nb, hipMemcpyDefault, s));
   AXSQ_CHECK_HIP(hipMemcpyAsync(h->vy, y, nb, hipMemcpyDefault, s));

@@ -270,6 +270,7 @@ struct axsq_sdf {
   int cull_state = 0;
   // CullResult's, asked for the current vertices (classed) or earlier ones (known)
   bool cull_classed = false, cull_known = false;
+  int cull_moves = 0;  // of the vertices since
   bool cull_plain = false, cull_flat = false, cull_loose = false, cull_crowd = false;
   std::atomic<bool> evaluated{false};  // since the vertices were set
   std::mutex cull_mu;       // held while a call builds them
